@@ -38,10 +38,21 @@ thread_local int t_last_path = 0;
 thread_local char t_last_kernel[96] = "";
 thread_local std::string t_hip_error;
 
-// Batches narrower than this go to the generic kernel: the tiled SpMM puts
-// one batch column on each of 64 lanes.
+// Batches narrower than this are not the tile-by-tile kernel's: it puts one batch column on each of 64 lanes.
 constexpr int SPMM_TILED_MIN_BATCH = 24;
-// The rows-along-lanes kernel is the automatic choice from this many of its tiles (workgroups) and this batch.
+
+// Which kernel serves a product, for both entry points that launch one.
+enum class SpFamily { generic, thin, tiled, unsupported };
+SpFamily spmm_family(const DiaView &A, long long ldb, long long ldd, int batch, bool trans, int forced)
+{
+    if (forced == CUVDIA_PATH_GENERIC) return SpFamily::generic;
+    const bool tiled_possible = spmm_tiled_ok(A, ldb, ldd, trans);
+    if (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_WINDOW)
+        return tiled_possible ? SpFamily::tiled : SpFamily::unsupported;
+    if (forced == CUVDIA_PATH_TILED && !tiled_possible) return SpFamily::unsupported;
+    if (spmm_thin_ok(A, trans) && (batch < SPMM_TILED_MIN_BATCH || !tiled_possible)) return SpFamily::thin;
+    return tiled_possible && (batch >= SPMM_TILED_MIN_BATCH || forced == CUVDIA_PATH_TILED) ? SpFamily::tiled : SpFamily::generic;
+}
 // Largest h, w and |offset| the kernels' 32-bit row arithmetic allows.
 constexpr long long DIM_LIMIT = 1LL << 30;
 
@@ -426,28 +437,22 @@ int cuvdia_spmm_layer_f32(const cuvdia_desc *desc, const float *A_vals, const fl
 
     const int forced = g_path.load();
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool tiled_possible = spmm_tiled_ok(desc->view, ldb, ldd, trans);
-    bool tiled;
-    if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK ||
-        forced == CUVDIA_PATH_WINDOW) {
-        if (!tiled_possible) return CUVDIA_EUNSUPPORTED;
-        tiled = true;
-    } else if (forced == CUVDIA_PATH_GENERIC) {
-        tiled = false;
-    } else {
-        tiled = tiled_possible && batch >= SPMM_TILED_MIN_BATCH;
-    }
+    const SpFamily family = spmm_family(desc->view, ldb, ldd, batch, trans, forced);
+    if (family == SpFamily::unsupported) return CUVDIA_EUNSUPPORTED;
+    const bool tiled = family == SpFamily::tiled;
     bool walked = false;
     const int walk = forced == CUVDIA_PATH_WALK ? 1
                      : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WINDOW) ? -1 : 0;
     const hipError_t e = tiled
         ? launch_spmm_tiled(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s, walk, &walked)
+        : family == SpFamily::thin
+        ? launch_spmm_thin(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
         : launch_spmm_generic(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s);
     if (tiled && walk > 0 && e == hipErrorNotSupported) {
         (void)hipGetLastError();
         return CUVDIA_EUNSUPPORTED;
     }
-    t_last_path = !tiled ? CUVDIA_PATH_GENERIC : walked ? CUVDIA_PATH_WALK : CUVDIA_PATH_TILED;
+    t_last_path = family == SpFamily::generic ? CUVDIA_PATH_GENERIC : walked ? CUVDIA_PATH_WALK : CUVDIA_PATH_TILED;
     return e == hipSuccess ? CUVDIA_OK : hip_fail(e, "spmm kernel launch");
 }
 
@@ -699,25 +704,19 @@ int cuvdia_spmm_offsets_noalloc_f32(const float *A_vals, const int *offsets_host
     // the kernel family is chosen by the rule of cuvdia_spmm_layer_f32
     const int forced = g_path.load();
     if (forced == CUVDIA_PATH_WALK) return CUVDIA_EUNSUPPORTED;
-    const bool tiled_possible = spmm_tiled_ok(view, ldb, ldd, trans);
-    bool tiled;
-    if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WINDOW) {
-        if (!tiled_possible) return CUVDIA_EUNSUPPORTED;
-        tiled = true;
-    } else if (forced == CUVDIA_PATH_GENERIC) {
-        tiled = false;
-    } else {
-        tiled = tiled_possible && batch >= SPMM_TILED_MIN_BATCH;
-    }
+    const SpFamily family = spmm_family(view, ldb, ldd, batch, trans, forced);
+    if (family == SpFamily::unsupported) return CUVDIA_EUNSUPPORTED;
+    const bool tiled = family == SpFamily::tiled, thin = family == SpFamily::thin;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // the tiled kernels read the chunk table only, the generic kernel the offset table only
-    if (tiled) e = noalloc_upload(tables + NOALLOC_CHUNKS_AT, chunks.data(), chunks.size() * sizeof(Chunk), s);
+    // the tiled and thin kernels read the chunk table only, the generic kernel the offset table only
+    if (tiled || thin) e = noalloc_upload(tables + NOALLOC_CHUNKS_AT, chunks.data(), chunks.size() * sizeof(Chunk), s);
     else e = noalloc_upload(tables, offsets_host, (size_t)nd * sizeof(int), s);
     if (e != hipSuccess) return hip_fail(e, "table fill kernel launch");
     const SpEpilogue ep{nullptr, CUVDIA_ACT_NONE, 0u, 0u};
     e = tiled ? launch_spmm_tiled(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
+        : thin ? launch_spmm_thin(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
               : launch_spmm_generic(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s);
-    t_last_path = tiled ? CUVDIA_PATH_TILED : CUVDIA_PATH_GENERIC;
+    t_last_path = tiled || thin ? CUVDIA_PATH_TILED : CUVDIA_PATH_GENERIC;
     return e == hipSuccess ? CUVDIA_OK : hip_fail(e, "spmm kernel launch");
 }
 

@@ -1,0 +1,108 @@
+// Device helpers shared by the translation units that hold kernels.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "kernels.hpp"
+
+namespace cuvdia {
+namespace {
+
+// Results leave through non-temporal stores: they are streamed past the
+// caches instead of waiting there, dirty, for the write-back at the kernel's
+// end, which every store of a one-round kernel would otherwise meet at once.
+template <class V>
+__device__ __forceinline__ void stream_store(V *p, V v)
+{
+    __builtin_nontemporal_store(v, p);
+}
+// Four consecutive floats as one 16-byte store; 4-byte alignment is all a 16-byte global store needs.
+__device__ __forceinline__ void stream_store4(float *p, float a, float b, float c, float d)
+{
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    __builtin_nontemporal_store(f4u{a, b, c, d}, reinterpret_cast<f4u *>(p));
+}
+
+// Hardware hands consecutive workgroup ids to the 8 XCDs round-robin, and each
+// XCD has its own L2.  Remap so that every XCD works on contiguous spans of
+// tiles: neighbouring row tiles share dense-operand rows (the halo and the
+// bands +-px apart), which then hit in that XCD's L2.  The tiles are dealt out
+// in groups of 8 spans of XCD_SPAN, one span per XCD and group, so that work
+// which varies along the rows (chunks falling outside the operand) still
+// spreads evenly; the last, partial group is split into 8 near-equal spans.
+// The very last span is dealt backwards: the tiles at the high end of the
+// rows take the slower body for tiles at the operand's ends, exactly like the
+// first tiles of the first span, and dealt in order they would be the last to
+// start as well -- a launch of one or two rounds then ends when they do.
+constexpr int XCD_SPAN = 64;
+__device__ __forceinline__ int xcd_tile(int bid, int nblk)
+{
+    constexpr int XCDS = 8, GROUP = XCDS * XCD_SPAN;
+    const int full = nblk / GROUP * GROUP;           // tiles in whole groups
+    if (bid < full) {
+        const int g = bid / GROUP, in = bid - g * GROUP;
+        const int xcd = in % XCDS;
+        int slot = in / XCDS;
+        if (xcd == XCDS - 1 && (g + 1) * GROUP == nblk) slot = XCD_SPAN - 1 - slot;
+        return g * GROUP + xcd * XCD_SPAN + slot;
+    }
+    const int rest = nblk - full, b = bid - full;
+    const int q = rest / XCDS, r = rest % XCDS;
+    const int xcd = b % XCDS;
+    int slot = b / XCDS;
+    if (xcd == XCDS - 1) slot = q - 1 - slot;        // the last span has q tiles (r < XCDS)
+    return full + xcd * q + (xcd < r ? xcd : r) + slot;
+}
+
+// Orders this wave's LDS writes before its later LDS reads (and the reverse)
+// for data exchanged between lanes of ONE wave.  The LDS unit executes a
+// wave's instructions in order, so only the compiler needs restraining.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Philox4x32-10 (Salmon, Moraes, Dror, Shaw: "Parallel random numbers: as easy
+// as 1, 2, 3", SC'11): a counter-based generator, 4 x 32 random bits per
+// 128-bit counter and 64-bit key, no state.  The result element (row, col)
+// draws word col & 3 of the block with counter (row, col >> 2, 0, 0) and key
+// (seed_lo, seed_hi), so a sample depends on the seed and the element's
+// position only -- not on which kernel, tile or lane produced it.
+struct SpRand4 { unsigned w[4]; };
+__device__ __forceinline__ SpRand4 sp_philox(unsigned row, unsigned colblock, unsigned k0, unsigned k1)
+{
+    unsigned c0 = row, c1 = colblock, c2 = 0u, c3 = 0u;
+#pragma unroll
+    for (int r = 0; r < 10; ++r) {
+        const unsigned hi0 = __umulhi(0xD2511F53u, c0), lo0 = 0xD2511F53u * c0;
+        const unsigned hi1 = __umulhi(0xCD9E8D57u, c2), lo1 = 0xCD9E8D57u * c2;
+        c0 = hi1 ^ c1 ^ k0;
+        c1 = lo1;
+        c2 = hi0 ^ c3 ^ k1;
+        c3 = lo0;
+        k0 += 0x9E3779B9u;
+        k1 += 0xBB67AE85u;
+    }
+    return SpRand4{{c0, c1, c2, c3}};
+}
+// 24 random bits -> a uniform variate in [0, 1), exactly representable
+__device__ __forceinline__ float sp_uniform(unsigned word) { return (float)(word >> 8) * 0x1p-24f; }
+
+// Last step of an SpMM result element: optional per-row bias, optional
+// logistic sigmoid 1/(1+exp(-v)) (src/cuv/tensor_ops/functors.hpp:122),
+// optional Bernoulli sample of that probability, v > u
+// (src/cuv/random/random.cu:86-91).
+__device__ __forceinline__ float sp_finish(float v, float bias, int act, unsigned word = 0u)
+{
+    v += bias;
+    if (act == 0) return v;
+    // v_exp_f32 and v_rcp_f32 (1 ulp each) instead of the library's exp and an
+    // IEEE division: p is off by < 1e-7 absolute, inside what the sum's own
+    // rounding allows, and the store costs a dozen instructions less per element
+    const float p = __builtin_amdgcn_rcpf(1.f + __expf(-v));
+    return act == 2 ? (p > sp_uniform(word) ? 1.f : 0.f) : p;
+}
+
+}  // namespace
+}  // namespace cuvdia

@@ -80,6 +80,13 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
                              float alpha, float beta, SpEpilogue ep, hipStream_t stream,
                              int walk = 0, bool *walked = nullptr);
 
+// Same contract, row_fact == 1 only: rows along the lanes, chunks dealt to the waves (spmm_thin.hip).  For few batch
+// columns and for few output rows; no limit on the operands' sizes.
+bool spmm_thin_ok(const DiaView &A, bool trans);
+hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B, long long ldb,
+                            float *dst, long long ldd, int batch, bool trans,
+                            float alpha, float beta, SpEpilogue ep, hipStream_t stream);
+
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.
 hipError_t launch_momentum(float *W, float *M, const float *dW, long long n, float lr, float mw, float l2,
                            hipStream_t stream);

@@ -1,0 +1,79 @@
+"""The product kernel for few batch columns (rows along the lanes), against the oracle where it can go wrong: row counts
+around its blocks of 64 and 256 rows, every chunk length, column counts that its column blocks do not divide, tables
+that reach past both ends of the dense operand, and each of its launch shapes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _dia(oracle, rng, h, w, offsets):
+    A = oracle.Dia(h, w, offsets, max(h, w), 1)
+    A.vals[:] = np.nan                                   # padding must never be read
+    valid = oracle.valid_mask(A)
+    A.vals[valid] = rng.uniform(-1, 1, int(valid.sum())).astype(np.float32)
+    return A
+
+
+def _check(oracle, seed, h, w, offsets, batch, alpha, beta, kernel):
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    rng = np.random.default_rng(seed)
+    A = _dia(oracle, rng, h, w, offsets)
+    for trans in ("n", "t"):
+        n_in, n_out = (h, w) if trans == "t" else (w, h)
+        B = np.asfortranarray(rng.uniform(-1, 1, (n_in, batch)).astype(np.float32))
+        dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32)) if beta else None
+        gu.check_prod(oracle, A, B, dst, trans, alpha, beta, _lib.PATH_AUTO, "%dx%d %s batch %d" % (h, w, trans, batch))
+        assert _lib.lib().cuvdia_last_kernel().decode().startswith(kernel)
+
+
+@pytest.mark.parametrize("run", range(1, 14))
+@pytest.mark.parametrize("rows", [3, 63, 64, 257, 1021])
+def test_rows_runs_and_columns(oracle, run, rows):
+    # a band of `run` diagonals, one of run - 1 (mixed lengths), and two that leave the matrix early at either end
+    offsets = [d - run // 2 for d in range(run)] + [40 + d for d in range(max(run - 1, 1))] + [-rows + 2, rows - 2]
+    offsets = sorted(set(offsets))
+    for batch in (1, 2, 3, 7, 23):
+        _check(oracle, 100 * run + rows + batch, rows, rows + 5, offsets, batch, 0.75, -1.5 if batch % 2 else 0.0, "spmm_thin_kernel")
+
+
+@pytest.mark.parametrize("h,w,runs,batch,shape", [
+    (300, 290, 20, 9, "2, 4>"),              # few rows, many chunks: 64 rows per workgroup
+    (300, 290, 20, 1, "1, 4>"),
+    (98307, 98301, 17, 5, "8, 1>"),          # eight columns per lane, four waves
+    (33029, 33030, 65, 4, "4, 1>"),          # four columns per lane, sixteen waves
+    (5000, 5003, 3, 14, "2, 1>"),
+])
+def test_launch_shapes(oracle, h, w, runs, batch, shape):
+    offsets = [37 * (r - runs // 2) + d for r in range(runs) for d in range(3)]
+    from cuv_amd import _lib
+    _check(oracle, h + batch, h, w, offsets, batch, 1.0, 0.5, "spmm_thin_kernel<3, ")
+    assert _lib.lib().cuvdia_last_kernel().decode().endswith(shape)
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+def test_non_finite_values_and_sampling(oracle, trans):
+    """An Inf or NaN of the dense operand reaches the rows that reference it and no other, chunks of mixed length
+    included; the fused sample draws what the oracle draws."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng = np.random.default_rng(3)
+    n, batch = 700, 13
+    A = _dia(oracle, rng, n, n, list(range(-3, 4)) + [100, 101])
+    B = np.asfortranarray(rng.uniform(-1, 1, (n, batch)).astype(np.float32))
+    B[2, 5], B[300, 3], B[697, 12] = -np.inf, np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        ref = oracle.prod(A, B, None, trans)
+    got, _ = gu.gpu_prod(A, B, None, trans)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    B = np.asfortranarray(rng.uniform(-1, 1, (n, batch)).astype(np.float32))
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    p = oracle.prod_bias_act(A, B, None, trans, 1.0, 0.0, bias, True)
+    u = oracle.sample_uniform(n, batch, 77)
+    out = torch.empty(batch, n, device="cuda:0")
+    D.prod_bias_act(out, gu.make_dev_dia(A), D.to_device_colmajor(B), trans, bias=torch.from_numpy(bias).cuda(),
+                    act=_lib.ACT_SIGMOID_SAMPLE, seed=77)
+    decided = np.abs(p.astype(np.float64) - u) > 1e-5
+    assert np.array_equal(D.to_host_colmajor(out)[decided], oracle.rnd_binarize(p, u)[decided])
