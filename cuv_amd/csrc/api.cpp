@@ -35,7 +35,6 @@ namespace {
 
 std::atomic_int g_path{CUVDIA_PATH_AUTO};
 thread_local int t_last_path = 0;
-thread_local char t_last_kernel[96] = "";
 thread_local std::string t_hip_error;
 
 // Batches narrower than this are not the tile-by-tile kernel's: it puts one batch column on each of 64 lanes.
@@ -111,12 +110,35 @@ int validate_shape(const int *offsets, int nd, int h, int w, int stride, int rf)
 }  // namespace
 
 namespace cuvdia {
-void note_kernel(const char *fmt, ...)
+KernelNote &kernel_note()
 {
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(t_last_kernel, sizeof t_last_kernel, fmt, ap);
-    va_end(ap);
+    thread_local KernelNote note;
+    return note;
+}
+
+namespace {
+// What a thread waits on: one event per device it has waited on, given back when the thread ends.
+struct Waiter {
+    bool armed = false;
+    int device = -1;
+    hipEvent_t current = nullptr;
+    bool launched = false;
+    unsigned waits = 0;
+    std::vector<std::pair<int, hipEvent_t>> events;
+    ~Waiter()
+    {
+        for (auto &e : events) (void)hipEventDestroy(e.second);
+    }
+};
+thread_local Waiter t_wait;
+constexpr unsigned WAIT_ON_STREAM_EVERY = 64;
+}  // namespace
+
+hipEvent_t launch_event()
+{
+    if (!t_wait.armed) return nullptr;
+    t_wait.launched = true;
+    return t_wait.current;
 }
 }  // namespace cuvdia
 
@@ -151,7 +173,54 @@ int cuvdia_set_path(int path)
 }
 
 int cuvdia_last_path(void) { return t_last_path; }
-const char *cuvdia_last_kernel(void) { return t_last_kernel; }
+const char *cuvdia_last_kernel(void)
+{
+    thread_local char text[96] = "";
+    const KernelNote &n = kernel_note();
+    if (n.text) n.text(n, text, sizeof text);
+    return text;
+}
+
+int cuvdia_wait_begin(void)
+{
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return CUVDIA_ENODEVICE;
+    }
+    Waiter &w = t_wait;
+    if (device != w.device) {
+        w.current = nullptr;
+        for (auto &e : w.events)
+            if (e.first == device) w.current = e.second;
+        if (!w.current) {
+            hipEvent_t event = nullptr;
+            const hipError_t e = hipEventCreateWithFlags(&event, hipEventDisableTiming);
+            if (e != hipSuccess) return hip_fail(e, "hipEventCreateWithFlags");
+            try {
+                w.events.emplace_back(device, event);
+            } catch (const std::bad_alloc &) {
+                (void)hipEventDestroy(event);
+                return CUVDIA_ENOMEM;
+            }
+            w.current = event;
+        }
+        w.device = device;
+    }
+    // The runtime keeps a record of every launch until something waits for the stream as a whole; now and then we do.
+    w.armed = ++w.waits % WAIT_ON_STREAM_EVERY != 0;
+    w.launched = false;
+    return CUVDIA_OK;
+}
+
+int cuvdia_wait_end(void *stream)
+{
+    Waiter &w = t_wait;
+    const bool launched = w.armed && w.launched;
+    w.armed = false;
+    const hipError_t e = launched ? hipEventSynchronize(w.current) : hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? CUVDIA_OK : hip_fail(e, "waiting for the stream");
+}
 
 int cuvdia_plan_chunks_max(const int *offsets_host, int nd, int transposed, int max_len,
                            int *s0, int *len, int *slot, int cap)

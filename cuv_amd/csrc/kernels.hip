@@ -2845,7 +2845,7 @@ hipError_t launch_spmm_generic(const DiaView &A, const float *vals, const float 
         const int slab = batch - done < 65535 * CB ? batch - done : 65535 * CB;
         const dim3 grid(gx, (unsigned)((slab + CB - 1) / CB));
         note_kernel("spmm_generic_kernel<%d>", CB);
-        hipLaunchKernelGGL(spmm_generic_kernel<CB>, grid, dim3(256), 0, stream,
+        launch_kernel(spmm_generic_kernel<CB>, grid, dim3(256), 0, stream,
                            A.offsets_dev, A.nd, vals, A.stride, A.h, A.w, A.rf,
                            B + (long long)done * ldb, ldb, dst + (long long)done * ldd, ldd,
                            n_out, slab, trans ? 1 : 0, alpha, beta, ep);
@@ -2936,7 +2936,7 @@ hipError_t spmm_tiled_launch_10_13(const SpLaunch &L);
 #define CUVDIA_SPMM_ARGS L.chunks, L.nchunks, L.vals, L.stride, L.ashift, L.B, L.ldb, L.dst, L.ldd, L.n_out, L.n_in, \
                          L.batch, L.alpha, L.beta, L.col_tiles, L.col_group, L.a_bytes, L.s_min, L.s_max, L.period_tiles, L.slot_step, L.ep
 #define CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, EP, MIXED)                                                                    \
-    hipLaunchKernelGGL((spmm_tiled_kernel<K, 8, NTAB, EP, MIXED>), L.grid, dim3(512), 0, L.stream, CUVDIA_SPMM_ARGS)
+    launch_kernel((spmm_tiled_kernel<K, 8, NTAB, EP, MIXED>), L.grid, dim3(512), 0, L.stream, CUVDIA_SPMM_ARGS)
 #define CUVDIA_SPMM_LAUNCH_TAB(K, NTAB)                                                                               \
     do {                                                                                                              \
         if (K > 1 && L.mixed) {                                                                                       \
@@ -3003,8 +3003,8 @@ hipError_t spmm_walk_launch(const WalkLaunch &L)
     note_kernel("spmm_walk_kernel<%d, %d, 8, %d, %s>", L.lck, L.lck, L.lck == 7 ? 1 : L.lck == 5 ? 2 : 3, fused ? "true" : "false");
 #define CUVDIA_WALK_LAUNCH(LCK, SH)                                                                                    \
     do {                                                                                                               \
-        if (fused) hipLaunchKernelGGL((spmm_walk_kernel<LCK, LCK, 8, SH, true>), grid, dim3(512), 0, L.stream, CUVDIA_WALK_ARGS); \
-        else hipLaunchKernelGGL((spmm_walk_kernel<LCK, LCK, 8, SH, false>), grid, dim3(512), 0, L.stream, CUVDIA_WALK_ARGS); \
+        if (fused) launch_kernel((spmm_walk_kernel<LCK, LCK, 8, SH, true>), grid, dim3(512), 0, L.stream, CUVDIA_WALK_ARGS); \
+        else launch_kernel((spmm_walk_kernel<LCK, LCK, 8, SH, false>), grid, dim3(512), 0, L.stream, CUVDIA_WALK_ARGS); \
     } while (0)
     if (L.lck == 7) CUVDIA_WALK_LAUNCH(7, 1);
     else if (L.lck == 5) CUVDIA_WALK_LAUNCH(5, 2);
@@ -3025,10 +3025,10 @@ hipError_t dd2dia_window_launch(const DwLaunch &L)
                        L.alpha, L.beta, L.a_bytes, L.b_bytes, L.c_bytes, L.txn, L.tyn, L.ndb
 #define CUVDIA_DW_LAUNCH_SUBS(LC, SUBS)                                                                               \
     do {                                                                                                              \
-        if (sh == 0) hipLaunchKernelGGL((dd2dia_window_kernel<LC, 0, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
-        else if (sh == 1) hipLaunchKernelGGL((dd2dia_window_kernel<LC, 1, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
-        else if (sh == 2) hipLaunchKernelGGL((dd2dia_window_kernel<LC, 2, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
-        else hipLaunchKernelGGL((dd2dia_window_kernel<LC, 3, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
+        if (sh == 0) launch_kernel((dd2dia_window_kernel<LC, 0, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
+        else if (sh == 1) launch_kernel((dd2dia_window_kernel<LC, 1, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
+        else if (sh == 2) launch_kernel((dd2dia_window_kernel<LC, 2, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
+        else launch_kernel((dd2dia_window_kernel<LC, 3, SUBS>), grid, dim3(256 * SUBS), 0, L.stream, CUVDIA_DW_ARGS); \
     } while (0)
 #define CUVDIA_DW_LAUNCH(LC)                                                                                          \
     case LC:                                                                                                          \
@@ -3061,8 +3061,8 @@ hipError_t dd2dia_window_long_launch(const DwLaunch &L)
                         L.alpha, L.beta, L.a_bytes, L.b_bytes, L.c_bytes, L.txn, L.tyn, L.ndb
 #define CUVDIA_DWL_LAUNCH_NW(LC, SH)                                                                                   \
     do {                                                                                                               \
-        if (nw == 5) hipLaunchKernelGGL((dd2dia_window_long_kernel<LC, SH, 5>), grid, dim3(320), 0, L.stream, CUVDIA_DWL_ARGS); \
-        else hipLaunchKernelGGL((dd2dia_window_long_kernel<LC, SH, 7>), grid, dim3(448), 0, L.stream, CUVDIA_DWL_ARGS); \
+        if (nw == 5) launch_kernel((dd2dia_window_long_kernel<LC, SH, 5>), grid, dim3(320), 0, L.stream, CUVDIA_DWL_ARGS); \
+        else launch_kernel((dd2dia_window_long_kernel<LC, SH, 7>), grid, dim3(448), 0, L.stream, CUVDIA_DWL_ARGS); \
     } while (0)
 #define CUVDIA_DWL_LAUNCH(LC)                                                                                          \
     case LC:                                                                                                           \
@@ -3175,7 +3175,7 @@ hipError_t launch_dd2dia_generic(const DiaView &C, float *vals, const float *A, 
     while (done < C.nd) {
         const int slab = C.nd - done < 65535 ? C.nd - done : 65535;
         note_kernel("dd2dia_generic_kernel");
-        hipLaunchKernelGGL(dd2dia_generic_kernel, dim3(gx, (unsigned)slab), dim3(256), 0, stream,
+        launch_kernel(dd2dia_generic_kernel, dim3(gx, (unsigned)slab), dim3(256), 0, stream,
                            C.offsets_dev + done, vals + (long long)done * C.stride, C.stride,
                            C.h, C.w, C.rf, A, lda, B, ldb, batch, alpha, beta);
         done += slab;
@@ -3188,7 +3188,7 @@ hipError_t launch_avg_diagonals(const DiaView &A, const float *vals, float *dst,
     int done = 0;
     while (done < A.nd) {
         const int slab = A.nd - done < 65535 ? A.nd - done : 65535;
-        hipLaunchKernelGGL(avg_diagonals_kernel, dim3((unsigned)slab), dim3(AVG_THREADS), 0, stream,
+        launch_kernel(avg_diagonals_kernel, dim3((unsigned)slab), dim3(AVG_THREADS), 0, stream,
                            A.offsets_dev + done, vals + (long long)done * A.stride, A.stride, A.h, A.w, dst + done);
         done += slab;
     }
@@ -3205,7 +3205,7 @@ hipError_t launch_axpby(float *W, const float *dW, long long n, float alpha, flo
     long long blocks = (items + AXPBY_THREADS - 1) / AXPBY_THREADS;
     if (blocks > 256 * 16) blocks = 256 * 16;         // 16 workgroups per CU, grid-stride beyond that
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(axpby_kernel, dim3((unsigned)blocks), dim3(AXPBY_THREADS), 0, stream, W, dW, n, alpha, beta,
+    launch_kernel(axpby_kernel, dim3((unsigned)blocks), dim3(AXPBY_THREADS), 0, stream, W, dW, n, alpha, beta,
                        (int)head, (int)vec);
     return hipGetLastError();
 }
@@ -3222,7 +3222,7 @@ hipError_t launch_momentum(float *W, float *M, const float *dW, long long n, flo
     long long blocks = (items + AXPBY_THREADS - 1) / AXPBY_THREADS;
     if (blocks > 256 * 16) blocks = 256 * 16;
     if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(momentum_kernel, dim3((unsigned)blocks), dim3(AXPBY_THREADS), 0, stream, W, M, dW, n, lr, mw, l2,
+    launch_kernel(momentum_kernel, dim3((unsigned)blocks), dim3(AXPBY_THREADS), 0, stream, W, M, dW, n, lr, mw, l2,
                        (int)head, (int)vec);
     return hipGetLastError();
 }
@@ -3376,19 +3376,19 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
 #define CUVDIA_DD_LAUNCH(L)                                                                              \
     case L:                                                                                              \
         if (shifted) {                                                                                   \
-            hipLaunchKernelGGL((dd2dia_tiled_kernel<L, true, true, DD_SHIFTED>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
+            launch_kernel((dd2dia_tiled_kernel<L, true, true, DD_SHIFTED>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
         } else if (wide) {                                                                               \
-            hipLaunchKernelGGL((dd2dia_tiled_kernel<L, true, true, DD_WIDE>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
+            launch_kernel((dd2dia_tiled_kernel<L, true, true, DD_WIDE>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
         } else if (pairs) {                                                                              \
-            hipLaunchKernelGGL((dd2dia_tiled_kernel<L, true, true>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
+            launch_kernel((dd2dia_tiled_kernel<L, true, true>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
         } else {                                                                                         \
-            if (a_vec) hipLaunchKernelGGL((dd2dia_tiled_kernel<L, true, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
-            else hipLaunchKernelGGL((dd2dia_tiled_kernel<L, false, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);       \
+            if (a_vec) launch_kernel((dd2dia_tiled_kernel<L, true, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
+            else launch_kernel((dd2dia_tiled_kernel<L, false, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);       \
         }                                                                                                \
         break;
 #define CUVDIA_DD_LAUNCH_LONG(L)                                                                         \
     case L:                                                                                              \
-        hipLaunchKernelGGL((dd2dia_tiled_kernel<L, true, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);      \
+        launch_kernel((dd2dia_tiled_kernel<L, true, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);      \
         break;
     if (lc > CHUNK_MAX) note_kernel("dd2dia_tiled_kernel<%d, true, false, 0>", lc);
     else note_kernel("dd2dia_tiled_kernel<%d, %s, %s, %d>", lc, (shifted || wide || pairs || a_vec) ? "true" : "false",
@@ -3456,7 +3456,7 @@ hipError_t noalloc_upload(unsigned char *dst_dev, const void *src_host, size_t b
         const size_t n = bytes - at < NOALLOC_PIECE_BYTES ? bytes - at : NOALLOC_PIECE_BYTES;
         NoallocPiece piece{};
         std::memcpy(piece.w, src + at, n);
-        hipLaunchKernelGGL(noalloc_fill_kernel, dim3(1), dim3(256), 0, stream, piece,
+        launch_kernel(noalloc_fill_kernel, dim3(1), dim3(256), 0, stream, piece,
                            reinterpret_cast<unsigned *>(dst_dev + at), (int)((n + 3) / 4));
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;

@@ -5,10 +5,39 @@
 #include <hip/hip_runtime_api.h>
 
 #include <cstddef>
+#include <cstdio>
+#include <new>
+#include <tuple>
+#include <type_traits>
 
 #include "plan.hpp"
 
 namespace cuvdia {
+
+// The name of the kernel this host thread launched last, for cuvdia_last_kernel(), written the way a profiler prints
+// it ("spmm_tiled_kernel<7, 8, 1, false>").  A launcher only leaves the format and its arguments here (a few stores);
+// the text is made when somebody asks for it.
+struct KernelNote {
+    void (*text)(const KernelNote &, char *, size_t) = nullptr;
+    const char *fmt = "";
+    alignas(8) unsigned char args[64];
+};
+KernelNote &kernel_note();
+template <class... A>
+void note_kernel(const char *fmt, A... a)
+{
+    using Args = std::tuple<A...>;
+    static_assert(sizeof(Args) <= sizeof(KernelNote::args) && std::is_trivially_destructible<Args>::value, "room for the arguments");
+    KernelNote &n = kernel_note();
+    n.fmt = fmt;
+    new (n.args) Args(a...);
+    n.text = [](const KernelNote &k, char *out, size_t cap) {
+        std::apply([&](auto... x) { std::snprintf(out, cap, k.fmt, x...); }, *reinterpret_cast<const Args *>(k.args));
+    };
+}
+
+// The event that this host thread's launches carry between cuvdia_wait_begin() and cuvdia_wait_end(), or nullptr.
+hipEvent_t launch_event();
 
 // Device form of a window table (plan_walk) for one traversal; tab_dev == nullptr: not a window table.
 struct WalkView {
@@ -66,9 +95,6 @@ hipError_t launch_spmm_generic(const DiaView &A, const float *vals, const float 
 // -1 -- never the walking kernel.  *walked (if not null) tells which ran.
 // Output rows per tile of the walking kernel's instantiation for a window of k rows of lck diagonals whose first
 // shift is s0; 0 when there is none.
-// Records the name of the kernel a launcher is about to launch, written the way a profiler prints it
-// ("spmm_tiled_kernel<7, 8, 1, false>"), for cuvdia_last_kernel(); per host thread.
-void note_kernel(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 int spmm_walk_tile_rows(int lck, int k, int s0);
 // Tiles per segment of the walking launch for such a window on n_out x n_in rows and col_tiles tiles of 64 batch
 // columns, and the launch's workgroups; 0 when the walking kernel does not run there (no instantiation, row

@@ -199,7 +199,7 @@ hipError_t launch_one(const ThinLaunch &L, int waves)
     if (row_blocks * col_groups > 0x7fffffffLL) return hipErrorInvalidValue;
     const size_t lds = (size_t)waves * G * CB * (ROWS + (thin_staged(LC, CB, G) ? 4 * ((LC + 2) / 4) : 0)) * sizeof(float);
     note_kernel("spmm_thin_kernel<%d, %d, %d>", LC, CB, G);
-    hipLaunchKernelGGL((spmm_thin_kernel<LC, CB, G>), dim3((unsigned)(row_blocks * col_groups)), dim3(64 * waves), lds, L.stream,
+    launch_kernel((spmm_thin_kernel<LC, CB, G>), dim3((unsigned)(row_blocks * col_groups)), dim3(64 * waves), lds, L.stream,
                        L.chunks, L.nchunks, L.vals, L.stride, L.ashift, L.X, L.ldx, L.Y, L.ldy, L.n_out, L.n_in, L.batch,
                        (int)row_blocks, (int)col_groups, L.s_min, L.s_max, L.alpha, L.beta, L.ep);
     return hipGetLastError();

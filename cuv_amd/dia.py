@@ -14,6 +14,12 @@ import torch
 
 from . import _lib
 
+try:
+    from . import _native
+except ImportError as e:
+    raise ImportError("cuv_amd/_native.so is not built or does not fit this torch (%s); run `make -j8 -C cuv_amd/csrc` "
+                      "or __graft_entry__.build()" % e) from e
+
 
 def _stream_ptr():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -172,6 +178,7 @@ class dev_dia_matrix_f(_dia_matrix_f):
 
     def __init__(self, h, w, num_dia, stride, row_fact=1, device="cuda:0"):
         self._desc = None
+        self._desc_ptr = 0                       # the same as a plain number, for _native; 0: none yet
         self._init_shape(h, w, num_dia, stride, row_fact)
         self._device = device
         self.vec = None
@@ -196,7 +203,7 @@ class dev_dia_matrix_f(_dia_matrix_f):
         if getattr(self, "_desc", None):
             torch.cuda.synchronize()
             _lib.lib().cuvdia_desc_destroy(self._desc)
-            self._desc = None
+            self._desc, self._desc_ptr = None, 0
 
     def _init_shape(self, h, w, num_dia, stride, row_fact):
         self._drop_desc()
@@ -213,7 +220,7 @@ class dev_dia_matrix_f(_dia_matrix_f):
                 _lib.check(_lib.lib().cuvdia_desc_create(
                     ctypes.byref(d), self._offsets.ctypes.data_as(ctypes.POINTER(ctypes.c_int)),
                     self.num_dia, self.h, self.w, self.stride, self.row_fact), "cuvdia_desc_create")
-            self._desc = d
+            self._desc, self._desc_ptr = d, d.value
         return self._desc
 
     def info(self):
@@ -378,6 +385,8 @@ class dev_block_descriptor_f:
 
 def prod(dst, A, B, transA="n", transB="n", factAB=1.0, factC=0.0, sync=True):
     """dst = factC*dst + factAB*op(A)*B (src/cuv/matrix_ops/spmv.cu:221-247)."""
+    if transB == "n" and _native.product(dst, A, B, transA, factAB, factC, None, 0, 0, sync):
+        return dst
     if transB != "n":
         raise RuntimeError("transB == 'n'")
     if transA not in ("n", "t"):
@@ -401,6 +410,8 @@ def prod_bias_act(dst, A, B, transA="n", factAB=1.0, factC=0.0, bias=None, act=_
     RBM/MLP layer update in one launch (examples/rbm/base.py:48-54,127-136).  act = ACT_SIGMOID_SAMPLE also
     replaces each probability by a Bernoulli sample of it (rnd_binarize, src/cuv/random/random.cu:139-142),
     drawn from Philox4x32-10 keyed by `seed` and the element's (row, column)."""
+    if _native.product(dst, A, B, transA, factAB, factC, bias, act, seed, sync):
+        return dst
     if transA not in ("n", "t"):
         raise RuntimeError("transA must be 'n' or 't'")
     n_out, n_in = (A.w, A.h) if transA == "t" else (A.h, A.w)
@@ -424,6 +435,8 @@ def prod_bias_act(dst, A, B, transA="n", factAB=1.0, factC=0.0, bias=None, act=_
 def densedense_to_dia(C, bd, A, B, factAB=1.0, factC=0.0, sync=True):
     """C = factC*C + factAB*proj(A*B') on C's stored diagonals
     (src/cuv/matrix_ops/densedense_to_sparse.hpp:107-129)."""
+    if _native.projection(C, A, B, factAB, factC, sync):
+        return C
     ba, lda = _check_dense(A, C.h, "A")
     bb, ldb = _check_dense(B, C.w, "B")
     if ba != bb:
@@ -458,6 +471,8 @@ def learn_step_weight_decay(W, dW, learnrate, decay=0.0, sync=True):
     (the whole value vector is updated, as the reference's call on dia.vec() does) or float32 CUDA tensors."""
     w = W.vec if isinstance(W, dev_dia_matrix_f) else W
     d = dW.vec if isinstance(dW, dev_dia_matrix_f) else dW
+    if _native.weight_step(w, None, d, learnrate, 0.0, decay, sync):
+        return W
     for t in (w, d):
         if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
             raise RuntimeError("W.ptr() / dW.ptr(): contiguous float32 CUDA tensors")
@@ -476,6 +491,8 @@ def learn_step_weight_decay_momentum(W, momentum, dW, learnrate, momentum_weight
     """m = momentum_weight*momentum - learnrate*(dW + decay*W); W += m; momentum = m
     (src/cuv/tensor_ops/rprop.cu:158-170,369-376).  Operands as in learn_step_weight_decay."""
     w, m, d = (t.vec if isinstance(t, dev_dia_matrix_f) else t for t in (W, momentum, dW))
+    if _native.weight_step(w, m, d, learnrate, momentum_weight, decay, sync):
+        return W
     for t in (w, m, d):
         if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
             raise RuntimeError("W.ptr() / dW.ptr(): contiguous float32 CUDA tensors")

@@ -368,6 +368,18 @@ int cuvdia_last_path(void);
  * No counterpart in the reference. */
 const char *cuvdia_last_kernel(void);
 
+/* Compute calls that wait.  Every call above only enqueues; a caller that
+ * wants the results at once brackets the call: cuvdia_wait_begin() makes the
+ * kernels that this host thread launches carry a completion event, and
+ * cuvdia_wait_end() returns when the last of them -- and with it everything
+ * enqueued on its stream before it -- is done.  Cheaper than
+ * hipStreamSynchronize(stream), which is what cuvdia_wait_end() does when
+ * nothing was launched in between.  All the calls in between go to `stream`,
+ * on the current device, which is not capturing.  cuvdia_wait_end() always
+ * ends the bracket.  No counterpart in the reference. */
+int cuvdia_wait_begin(void);
+int cuvdia_wait_end(void *stream);
+
 /* Static string for an error code. */
 const char *cuvdia_strerror(int code);
 
