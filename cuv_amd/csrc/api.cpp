@@ -593,7 +593,17 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
         }
     }
     bool tiled;
-    if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK ||
+    bool rows = false;               // of the tiled family: the kernel with rows along the lanes
+    if (batch > 0 && dd2dia_rows_ok(desc->view) && (forced == CUVDIA_PATH_AUTO || forced == CUVDIA_PATH_TILED)) {
+        // (16-byte pieces of A, as the kernels that share staged operands load them)
+        const bool aligned = reinterpret_cast<std::uintptr_t>(A) % 16 == 0 && lda % 4 == 0 && desc->h % 4 == 0;
+        const long long wgs = dd2dia_window_workgroups(desc->view, slab);
+        const bool by_window = wgs > 0 && dd2dia_window_by_size(desc->view, slab, wgs);
+        rows = !tiled_possible || dd2dia_rows_by_size(desc->view, batch, aligned, by_window);
+    }
+    if (rows) {
+        tiled = true;
+    } else if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK ||
         forced == CUVDIA_PATH_WINDOW) {
         if (!tiled_possible) return CUVDIA_EUNSUPPORTED;
         tiled = true;
@@ -605,7 +615,9 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
     bool windowed = false;
-    if (!tiled) {
+    if (rows) {
+        e = launch_dd2dia_rows(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
+    } else if (!tiled) {
         e = launch_dd2dia_generic(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
     } else {
         const int window = forced == CUVDIA_PATH_WINDOW ? 1

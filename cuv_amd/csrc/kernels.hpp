@@ -130,6 +130,15 @@ hipError_t launch_dd2dia_generic(const DiaView &C, float *vals, const float *A, 
                                  const float *B, long long ldb, int batch,
                                  float alpha, float beta, hipStream_t stream);
 
+// Same contract, row_fact == 1 only: rows along the lanes, each wave on its own (dd2dia_rows.hip).  Any alignment, no
+// limit on the operands' sizes.
+bool dd2dia_rows_ok(const DiaView &C);
+// Whether the automatic choice takes that kernel; `aligned`: both operands' bases, leading dimensions and row counts
+// are multiples of 16 bytes; `windowed`: the window-table projection would run otherwise.
+bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowed);
+hipError_t launch_dd2dia_rows(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
+                              int batch, float alpha, float beta, hipStream_t stream);
+
 // Whether the tiled dd2dia can serve these operands (row_fact 1, operand
 // extents within its 32-bit buffer addressing).
 bool dd2dia_tiled_ok(const DiaView &C, long long lda, long long ldb, int batch);
