@@ -27,6 +27,7 @@ struct cuvdia_desc {
     std::vector<int> offsets;        // host copy, table order
     long long nnz;
     int n_chunks_n, n_chunks_t;
+    std::vector<int> walk_n, walk_t; // group rows of the window-table forms
     void *dev_block;                 // one allocation: offsets | chunks_n | chunks_t
     DiaView view;
 };
@@ -46,9 +47,11 @@ SpFamily spmm_family(const DiaView &A, long long ldb, long long ldd, int batch, 
 {
     if (forced == CUVDIA_PATH_GENERIC) return SpFamily::generic;
     const bool tiled_possible = spmm_tiled_ok(A, ldb, ldd, trans);
-    if (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_WINDOW)
+    if (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_WINDOW ||
+        forced == CUVDIA_PATH_PLANE)
         return tiled_possible ? SpFamily::tiled : SpFamily::unsupported;
     if (forced == CUVDIA_PATH_TILED && !tiled_possible) return SpFamily::unsupported;
+    if (forced == CUVDIA_PATH_THIN) return spmm_thin_ok(A, trans) ? SpFamily::thin : SpFamily::unsupported;
     if (spmm_thin_ok(A, trans) && (batch < SPMM_TILED_MIN_BATCH || !tiled_possible)) return SpFamily::thin;
     return tiled_possible && (batch >= SPMM_TILED_MIN_BATCH || forced == CUVDIA_PATH_TILED) ? SpFamily::tiled : SpFamily::generic;
 }
@@ -166,7 +169,8 @@ const char *cuvdia_last_hip_error(void) { return t_hip_error.c_str(); }
 int cuvdia_set_path(int path)
 {
     if (path != CUVDIA_PATH_AUTO && path != CUVDIA_PATH_GENERIC && path != CUVDIA_PATH_TILED &&
-        path != CUVDIA_PATH_TILED_NOWALK && path != CUVDIA_PATH_WALK && path != CUVDIA_PATH_WINDOW)
+        path != CUVDIA_PATH_TILED_NOWALK && path != CUVDIA_PATH_WALK && path != CUVDIA_PATH_WINDOW &&
+        path != CUVDIA_PATH_PLANE && path != CUVDIA_PATH_THIN)
         return CUVDIA_EINVAL;
     g_path.store(path);
     return CUVDIA_OK;
@@ -314,7 +318,7 @@ long long cuvdia_plan_window_launch(const int *offsets_host, int nd, int stride,
     bool rows4 = true;
     for (int r : wp.group_rows) rows4 = rows4 && r % 4 == 0;
     view.h = h; view.w = w; view.nd = nd; view.stride = stride; view.rf = 1;
-    view.walk_n = WalkView{&not_null, wp.ngroups, wp.period, wp.s0, wp.k, wp.lck, wp.astep4, rows4};
+    view.walk_n = WalkView{&not_null, wp.ngroups, wp.period, wp.s0, wp.k, wp.lck, wp.astep4, rows4, wp.group_rows.data()};
     if (!dd2dia_tiled_ok(view, h, w, batch)) return 0;
     const long long workgroups = dd2dia_window_workgroups(view, batch);
     return workgroups > 0 && dd2dia_window_by_size(view, batch, workgroups) ? workgroups : 0;
@@ -436,11 +440,15 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     auto walk_view = [&](const WalkPlan &p, size_t at) {
         bool rows4 = true;
         for (int r : p.group_rows) rows4 = rows4 && r % 4 == 0;
-        return p.ok ? WalkView{reinterpret_cast<const int *>(base + at), p.ngroups, p.period, p.s0, p.k, p.lck, p.astep4, rows4}
-                    : WalkView{nullptr, 0, 0, 0, 0, 0, 0, false};
+        return p.ok ? WalkView{reinterpret_cast<const int *>(base + at), p.ngroups, p.period, p.s0, p.k, p.lck, p.astep4, rows4, p.group_rows.data()}
+                    : WalkView{};
     };
     d->view.walk_n = walk_view(wn, wn_at);
     d->view.walk_t = walk_view(wt, wt_at);
+    d->walk_n.swap(wn.group_rows);                   // (the views point at them)
+    d->walk_t.swap(wt.group_rows);
+    d->view.walk_n.rows_host = d->walk_n.data();
+    d->view.walk_t.rows_host = d->walk_t.data();
     auto span = [](const std::vector<Chunk> &t, int &max_len, int &s_min, int &s_max, int *min_len = nullptr) {
         max_len = 0;
         if (min_len) {
@@ -509,19 +517,17 @@ int cuvdia_spmm_layer_f32(const cuvdia_desc *desc, const float *A_vals, const fl
     const SpFamily family = spmm_family(desc->view, ldb, ldd, batch, trans, forced);
     if (family == SpFamily::unsupported) return CUVDIA_EUNSUPPORTED;
     const bool tiled = family == SpFamily::tiled;
-    bool walked = false;
-    const int walk = forced == CUVDIA_PATH_WALK ? 1
-                     : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WINDOW) ? -1 : 0;
+    int ran = CUVDIA_PATH_TILED;
     const hipError_t e = tiled
-        ? launch_spmm_tiled(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s, walk, &walked)
+        ? launch_spmm_tiled(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s, forced, &ran)
         : family == SpFamily::thin
         ? launch_spmm_thin(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
         : launch_spmm_generic(desc->view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s);
-    if (tiled && walk > 0 && e == hipErrorNotSupported) {
+    if (tiled && e == hipErrorNotSupported) {
         (void)hipGetLastError();
         return CUVDIA_EUNSUPPORTED;
     }
-    t_last_path = family == SpFamily::generic ? CUVDIA_PATH_GENERIC : walked ? CUVDIA_PATH_WALK : CUVDIA_PATH_TILED;
+    t_last_path = family == SpFamily::generic ? CUVDIA_PATH_GENERIC : ran;
     return e == hipSuccess ? CUVDIA_OK : hip_fail(e, "spmm kernel launch");
 }
 
@@ -604,7 +610,7 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     if (rows) {
         tiled = true;
     } else if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK ||
-        forced == CUVDIA_PATH_WINDOW) {
+        forced == CUVDIA_PATH_WINDOW || forced == CUVDIA_PATH_PLANE) {
         if (!tiled_possible) return CUVDIA_EUNSUPPORTED;
         tiled = true;
     } else if (forced == CUVDIA_PATH_GENERIC) {
@@ -621,7 +627,7 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
         e = launch_dd2dia_generic(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
     } else {
         const int window = forced == CUVDIA_PATH_WINDOW ? 1
-                           : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK) ? -1 : 0;
+                           : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_PLANE) ? -1 : 0;
         for (int c0 = 0; c0 < batch && e == hipSuccess; c0 += slab) {
             bool this_one = false;
             e = launch_dd2dia_tiled(desc->view, C_vals, A + (long long)c0 * lda, lda, B + (long long)c0 * ldb, ldb,
@@ -784,7 +790,7 @@ int cuvdia_spmm_offsets_noalloc_f32(const float *A_vals, const int *offsets_host
 
     // the kernel family is chosen by the rule of cuvdia_spmm_layer_f32
     const int forced = g_path.load();
-    if (forced == CUVDIA_PATH_WALK) return CUVDIA_EUNSUPPORTED;
+    if (forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_PLANE) return CUVDIA_EUNSUPPORTED;
     const SpFamily family = spmm_family(view, ldb, ldd, batch, trans, forced);
     if (family == SpFamily::unsupported) return CUVDIA_EUNSUPPORTED;
     const bool tiled = family == SpFamily::tiled, thin = family == SpFamily::thin;

@@ -115,5 +115,36 @@ __device__ __forceinline__ float sp_finish(float v, float bias, int act, unsigne
     return act == 2 ? (p > sp_uniform(word) ? 1.f : 0.f) : p;
 }
 
+// Loads that deliver straight into LDS (no vector register in between): lane i
+// of the wave writes its 16 bytes at lds_byte_addr + 16*i; an
+// out-of-range lane writes zeros, an inactive lane writes nothing.  They are
+// vector-memory operations and complete in order with the wave's other loads
+// (s_waitcnt vmcnt).  Written in assembly so that the waits can be
+// placed by hand: the loops keep them in flight across
+// barriers, which no automatic placement allows.  M0 is written inside the
+// statement without appearing among its clobbers: the compiler treats M0 as a
+// reserved register (it never keeps a value there across other code, and sets
+// it immediately before each instruction of its own that reads it), and it
+// rejects reserved registers in a clobber list with a warning.
+typedef int sp_int4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ sp_int4 raw_rsrc(const void *base, unsigned bytes)
+{
+    const unsigned long long b = reinterpret_cast<unsigned long long>(base);
+    return sp_int4{(int)(unsigned)b, (int)((unsigned)(b >> 32) & 0xffffu), (int)bytes, 0x00020000};
+}
+__device__ __forceinline__ void lds_load_b128(sp_int4 rsrc, unsigned lds_byte_addr, unsigned voff, unsigned soff)
+{
+    // all three are wave-uniform by construction; this keeps them in scalar registers whatever the compiler infers
+    lds_byte_addr = __builtin_amdgcn_readfirstlane(lds_byte_addr);
+    soff = __builtin_amdgcn_readfirstlane(soff);
+    rsrc = sp_int4{__builtin_amdgcn_readfirstlane(rsrc.x), __builtin_amdgcn_readfirstlane(rsrc.y),
+                   __builtin_amdgcn_readfirstlane(rsrc.z), __builtin_amdgcn_readfirstlane(rsrc.w)};
+    asm volatile("s_mov_b32 m0, %0\n\t"
+                 "s_nop 0\n\t"
+                 "buffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds_byte_addr), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+constexpr unsigned OOB_OFFSET = 0x80000000u;     // >= every resource size used here
+
 }  // namespace
 }  // namespace cuvdia

@@ -31,6 +31,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "cuvdia.h"
 #include "device.hpp"
 #include "kernels.hpp"
 
@@ -550,7 +551,6 @@ __device__ __forceinline__ float4 buffer_load_f32x4(__amdgpu_buffer_rsrc_t r, un
 {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
-constexpr unsigned OOB_OFFSET = 0x80000000u;     // >= every resource size used here
 
 // The body for tiles at the operand's ends.  The dense rows [a0, a0 + 80) of
 // the 64 columns are fetched with 16-byte buffer loads into registers (20
@@ -795,35 +795,6 @@ __device__ __forceinline__ void spmm_tile_edge(
     }
 }
 
-// Loads that deliver straight into LDS (no vector register in between): lane i
-// of the wave writes its 16 bytes at lds_byte_addr + 16*i; an
-// out-of-range lane writes zeros, an inactive lane writes nothing.  They are
-// vector-memory operations and complete in order with the wave's other loads
-// (s_waitcnt vmcnt).  Written in assembly so that the waits below can be
-// placed by hand: the loop keeps two chunks of them in flight across
-// barriers, which no automatic placement allows.  M0 is written inside the
-// statement without appearing among its clobbers: the compiler treats M0 as a
-// reserved register (it never keeps a value there across other code, and sets
-// it immediately before each instruction of its own that reads it), and it
-// rejects reserved registers in a clobber list with a warning.
-typedef int sp_int4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ sp_int4 raw_rsrc(const void *base, unsigned bytes)
-{
-    const unsigned long long b = reinterpret_cast<unsigned long long>(base);
-    return sp_int4{(int)(unsigned)b, (int)((unsigned)(b >> 32) & 0xffffu), (int)bytes, 0x00020000};
-}
-__device__ __forceinline__ void lds_load_b128(sp_int4 rsrc, unsigned lds_byte_addr, unsigned voff, unsigned soff)
-{
-    // all three are wave-uniform by construction; this keeps them in scalar registers whatever the compiler infers
-    lds_byte_addr = __builtin_amdgcn_readfirstlane(lds_byte_addr);
-    soff = __builtin_amdgcn_readfirstlane(soff);
-    rsrc = sp_int4{__builtin_amdgcn_readfirstlane(rsrc.x), __builtin_amdgcn_readfirstlane(rsrc.y),
-                   __builtin_amdgcn_readfirstlane(rsrc.z), __builtin_amdgcn_readfirstlane(rsrc.w)};
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(lds_byte_addr), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
 // the same with 4 bytes per lane: lane i writes at lds_byte_addr + 4*i
 __device__ __forceinline__ void lds_load_b32(sp_int4 rsrc, unsigned lds_byte_addr, unsigned voff)
 {
@@ -3124,9 +3095,9 @@ hipError_t spmm_tiled_launch_10_13(const SpLaunch &L)
 #if CUVDIA_IN_PART(4)
 hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B, long long ldb,
                              float *dst, long long ldd, int batch, bool trans,
-                             float alpha, float beta, SpEpilogue ep, hipStream_t stream, int walk, bool *walked)
+                             float alpha, float beta, SpEpilogue ep, hipStream_t stream, int path, int *ran)
 {
-    if (walked) *walked = false;
+    if (ran) *ran = CUVDIA_PATH_TILED;
     const int n_out = trans ? A.w : A.h;
     const int n_in = trans ? A.h : A.w;
     const long long row_tiles = (n_out + SP_ROWS - 1) / SP_ROWS;
@@ -3140,17 +3111,29 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
     // A window table on a product of many tiles: the walking kernel (with the bias, the sigmoid and the sample at
     // its tiles' exit, if asked for).
     const WalkView &wk = trans ? A.walk_t : A.walk_n;
-    if (walk >= 0 && wk.tab_dev != nullptr) {
+    if ((path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_TILED || path == CUVDIA_PATH_WALK) && wk.tab_dev != nullptr) {
         WalkLaunch W{wk.tab_dev, wk.ngroups, wk.period, wk.s0, wk.astep4, wk.lck, wk.k, 0, vals, B, ldb, dst, ldd,
                      n_out, n_in, batch, alpha, beta, (int)col_tiles, (unsigned)((long long)A.nd * A.stride * 4), stream, ep};
-        const int seg_tiles = spmm_walk_plan(wk.lck, wk.k, wk.s0, wk.period, n_out, n_in, col_tiles, walk > 0, nullptr);
+        const int seg_tiles = spmm_walk_plan(wk.lck, wk.k, wk.s0, wk.period, n_out, n_in, col_tiles, path == CUVDIA_PATH_WALK, nullptr);
         if (seg_tiles > 0) {
             W.seg_tiles = seg_tiles;
-            if (walked) *walked = true;
+            if (ran) *ran = CUVDIA_PATH_WALK;
             return spmm_walk_launch(W);
         }
     }
-    if (walk > 0) return hipErrorNotSupported;
+    if (path == CUVDIA_PATH_WALK) return hipErrorNotSupported;
+    // One of another width, or with a larger window: the plane's walk on the matrix cores.
+    if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_PLANE) {
+        PlaneLaunch P{};
+        if (spmm_plane_plan(wk, n_out, n_in, batch, ep.bias != nullptr || ep.act != 0, path == CUVDIA_PATH_PLANE, P)) {
+            if (ran) *ran = CUVDIA_PATH_PLANE;
+            P.tab = wk.tab_dev; P.ngroups = wk.ngroups; P.period = wk.period; P.s0 = wk.s0; P.astep4 = wk.astep4; P.k = wk.k;
+            P.vals = vals; P.B = B; P.ldb = ldb; P.dst = dst; P.ldd = ldd; P.n_out = n_out; P.n_in = n_in; P.batch = batch;
+            P.alpha = alpha; P.beta = beta; P.a_bytes = (unsigned)((long long)A.nd * A.stride * 4); P.ep = ep; P.stream = stream;
+            return spmm_plane_launch(P);
+        }
+        if (path == CUVDIA_PATH_PLANE) return hipErrorNotSupported;
+    }
     const SpLaunch L{trans ? A.chunks_t_dev : A.chunks_n_dev,
                      trans ? A.n_chunks_t : A.n_chunks_n,
                      vals, A.stride, trans ? 1 : 0, B, ldb, dst, ldd, n_out, n_in, batch, alpha, beta,

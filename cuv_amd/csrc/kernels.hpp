@@ -44,6 +44,7 @@ struct WalkView {
     const int *tab_dev;          // group_rows[ngroups], then aoff4[ngroups * k]
     int ngroups, period, s0, k, lck, astep4;
     bool rows4;                  // every group_rows[g] is a multiple of 4
+    const int *rows_host;        // group_rows[ngroups] in host memory
 };
 
 struct DiaView {
@@ -101,10 +102,11 @@ int spmm_walk_tile_rows(int lck, int k, int s0);
 // counts its tiles do not divide, or -- unless forced -- too few workgroups to fill the chip).
 int spmm_walk_plan(int lck, int k, int s0, int period, long long n_out, long long n_in, long long col_tiles,
                    bool forced, long long *workgroups);
+// path: CUVDIA_PATH_*, as forced; *ran: the one that served the call.
 hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B, long long ldb,
                              float *dst, long long ldd, int batch, bool trans,
                              float alpha, float beta, SpEpilogue ep, hipStream_t stream,
-                             int walk = 0, bool *walked = nullptr);
+                             int path = 0, int *ran = nullptr);
 
 // Same contract, row_fact == 1 only: rows along the lanes, chunks dealt to the waves (spmm_thin.hip).  For few batch
 // columns and for few output rows; no limit on the operands' sizes.
@@ -112,6 +114,32 @@ bool spmm_thin_ok(const DiaView &A, bool trans);
 hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B, long long ldb,
                             float *dst, long long ldd, int batch, bool trans,
                             float alpha, float beta, SpEpilogue ep, hipStream_t stream);
+
+// Same contract, window tables on row_fact == 1: the window's plane walked on the matrix cores (spmm_plane.hip).
+constexpr int PLANE_MAX_SEGMENTS = 96;
+struct PlaneCuts {
+    int at[PLANE_MAX_SEGMENTS + 1];      // first map row of every segment, and the end
+};
+struct PlaneLaunch {
+    const int *tab;
+    int ngroups, period, s0, astep4, k;
+    int tp, nseg;
+    PlaneCuts cuts;
+    const float *vals, *B;
+    long long ldb;
+    float *dst;
+    long long ldd;
+    int n_out, n_in, batch;
+    float alpha, beta;
+    int col_tiles;
+    unsigned a_bytes;
+    SpEpilogue ep;
+    hipStream_t stream;
+};
+// Fills in the launch's shape; false: the kernel does not serve this table and these sizes, or (not force) would not be ahead.
+bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int batch, bool fused, bool force,
+                     PlaneLaunch &L);
+hipError_t spmm_plane_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.
 hipError_t launch_momentum(float *W, float *M, const float *dW, long long n, float lr, float mw, float l2,

@@ -1,0 +1,481 @@
+// The product with a window table on the matrix cores: the window's plane, walked down column by column.
+//
+// A window table pairs output row i = (y, x) = (i / period, i mod period) with dense rows (y + dy, x + dx) for K window
+// rows dy of LC diagonals dx.  A workgroup owns 32 output positions x of 64 batch columns and walks down the map rows of
+// a segment.  At step u it has dense row block u in LDS -- the 32 + LC - 1 rows of map row y0 + u + (first dy) -- which all
+// of the K tiles u - K + 1 .. u use, tile m with its window row u - m.  Those tiles are what the matrix instruction's four
+// rows are: v_mfma_f32_4x4x1 multiplies four values (of four tiles, for one x and dx, from 4 lanes that its ABID field
+// names) with 64 values (dense row x + dx, a batch column per lane) and adds to 4 x 64 sums.  Every product that it makes
+// is one that the table has -- a band tiled along x instead would multiply zeros, and a zero times an infinity of the
+// dense operand is a NaN --; a slot whose tile has not started or has left only collects values nobody reads.  Of K = 5,
+// 9 and 13 tiles one is left over by groups of four: its FMAs go to the vector unit, the value broadcast by DPP.
+//
+// Per step and wave (8 rows): LC * 8 * ceil(K / 4) matrix instructions of 8 clocks for LC * K * 8 * 64 multiplications,
+// 22 - 26 per clock and SIMD where the DPP form of the tile-by-tile kernel does 15, and one staging of the dense rows for
+// K window rows.  The walk costs K - 1 steps in which not all tiles are alive (groups of four without any are skipped).
+//
+// Bound: on large windows the matrix cores (13 x 13: two thirds of a launch's time), on small ones the dense rows' way
+// from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
+// 13 x 13 on 256 x 256, batch 256 1131 -> 825 us (50 -> 69 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
+// 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
+// 229 -> 181; level or behind where the rule below says no.
+//
+// Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
+// ascending, acc = fma(a, x, acc).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
+#include "device.hpp"
+#include "kernels.hpp"
+
+namespace cuvdia {
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned plane_u4 __attribute__((ext_vector_type(4)));
+
+// A workgroup's tile: 32 rows x 64 columns, 8 rows per wave.  Up to four workgroups share a CU, each with barriers of its
+// own: while one waits for its block the others multiply.
+constexpr int PLANE_XT = 4;
+constexpr int PLANE_WAVES = 4, PLANE_ROWS = 8 * PLANE_WAVES;
+
+template <int LC, int K>
+struct PlaneShape {
+    static constexpr int TAIL = K % 4 == 1 ? 1 : 0;  // a tile on its own: its FMAs go to the vector unit
+    static constexpr int NG = (K - TAIL + 3) / 4;    // groups of 4 tiles
+    static constexpr int NQX = (PLANE_ROWS + LC - 1 + 3) / 4;       // 16-byte pieces of a column
+    static constexpr int XQ = NQX | 1;                              // ... and from column to column (odd: no bank conflicts)
+    static constexpr int XW = (8 + LC - 1 + 3) / 4;                 // pieces of a lane's window
+    static constexpr int AROW = PLANE_ROWS + 8, AQ = AROW / 4;      // floats from diagonal to diagonal: 40 banks on ...
+    static constexpr int ASLOT = LC * AROW + (16 + 64 - LC * AROW % 32) % 32;   // ... and from tile to tile 16 or 48 banks on
+    static constexpr int AIT = (AQ * LC + 63) / 64;                 // load instructions per tile
+    static constexpr int X_FLOATS = 64 * XQ * 4, STAGE = X_FLOATS + K * ASLOT;
+    static constexpr int XIT = (XQ + PLANE_WAVES - 1) / PLANE_WAVES;    // load instructions per wave
+    static constexpr int FIT = 160 * 1024 / (2 * 4 * STAGE), MOST = K <= 5 ? 4 : 3;     // (in LDS; in registers)
+    static constexpr int PER_CU = FIT < MOST ? FIT : MOST;          // workgroups per CU, a wave per SIMD each
+};
+
+template <int I, int N, class F>
+__device__ __forceinline__ void plane_for(F &&f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        plane_for<I + 1, N>(f);
+    }
+}
+
+// acc[r] += a(lane 16 n + LANE0 + r) * x[r]: the value broadcast inside each row of 16 lanes
+template <int LANE0>
+__device__ __forceinline__ void plane_fma8(float (&acc)[8], float a, const float *x)
+{
+#define PLANE_FMA(r)                                                                                        \
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc[r]) : "v"(a), "v"(x[r]), "n"(LANE0 + r));
+    PLANE_FMA(0) PLANE_FMA(1) PLANE_FMA(2) PLANE_FMA(3) PLANE_FMA(4) PLANE_FMA(5) PLANE_FMA(6) PLANE_FMA(7)
+#undef PLANE_FMA
+}
+
+template <int LC, int K, bool EP>
+__global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC, K>::PER_CU)) void spmm_plane_kernel(
+    const int *__restrict__ tab, int ngroups, int period, int s0, int astep4, int tp, int nseg, PlaneCuts cuts,
+    const float *__restrict__ vals, const float *__restrict__ X, long long ldx, float *__restrict__ Y, long long ldy,
+    int n_out, int n_in, int batch, float alpha, float beta, int col_tiles, unsigned a_bytes, SpEpilogue ep)
+{
+    using S = PlaneShape<LC, K>;
+    __shared__ __attribute__((aligned(16))) float lds[2 * S::STAGE];
+
+    // A unit -- a segment of PLANE_XT neighbouring walks -- stays on one XCD with all its column tiles: they share the
+    // diagonals' values, and the cache lines that tiles side by side have in common.
+    const int xcd = blockIdx.x % 8, k8 = blockIdx.x / 8, xgroups = (tp + PLANE_XT - 1) / PLANE_XT;
+    const int unit = (k8 / (PLANE_XT * col_tiles)) * 8 + xcd, within = k8 % (PLANE_XT * col_tiles);
+    const int xg = unit / nseg, seg = unit - xg * nseg, xt = xg * PLANE_XT + within / col_tiles, coltile = within % col_tiles;
+    if (xg >= xgroups || xt >= tp) return;
+    constexpr int waves = PLANE_WAVES, rows = PLANE_ROWS, nqx = S::NQX;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int xs = min(xt * rows, period - rows), skip = xt * rows - xs;       // (the last tile of a row is moved up)
+    const int seg0 = cuts.at[seg], tiles = cuts.at[seg + 1] - seg0;
+    if (tiles <= 0) return;
+    const int row_first = xs + seg0 * period;
+    const int col0 = coltile * 64, cols = min(64, batch - col0);
+    const float *const xbase = X + (long long)col0 * ldx;
+    const sp_int4 xrsrc = raw_rsrc(xbase, (unsigned)(((long long)(cols - 1) * ldx + n_in) * 4));
+    const sp_int4 arsrc = raw_rsrc(vals, a_bytes);
+    const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(Y + (long long)col0 * ldy, 0, (unsigned)(((long long)(cols - 1) * ldy + n_out) * 4), 0x00020000);
+    const int amin = min(0, astep4 * (LC - 1));
+    const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)&lds[0];
+
+    // this lane's share of a block's requests: byte offsets that stay the same for the whole walk
+    unsigned x_off[S::XIT], a_off[S::AIT];
+#pragma unroll
+    for (int it = 0; it < S::XIT; ++it) {
+        const int p = 64 * (wave + waves * it) + lane, col = p / S::XQ, q = p - col * S::XQ;
+        x_off[it] = q < nqx ? (unsigned)min(col, cols - 1) * ((unsigned)ldx * 4u) + 16u * q : OOB_OFFSET;
+    }
+#pragma unroll
+    for (int it = 0; it < S::AIT; ++it) {
+        const int p = 64 * it + lane, dx = p / S::AQ, q = p - dx * S::AQ;
+        a_off[it] = dx < LC && q < 2 * waves ? (unsigned)(astep4 * dx - amin) + 16u * q : OOB_OFFSET;
+    }
+    auto block_row = [&](int u, int g) { return row_first + s0 + tab[g] + u * period; };
+    auto outside = [&](int u, int g) { const int x0 = block_row(u, g); return x0 + rows + LC - 1 <= 0 || x0 >= n_in; };
+
+    // requests block (u, g): its dense rows, and the values of the tiles that use them
+    auto issue = [&](int u, int g, int buf) {
+        const int x0 = block_row(u, g);
+        const unsigned base = lds0 + (unsigned)(buf * S::STAGE * 4);
+        const bool inside = x0 >= 0 && x0 + 4 * nqx <= n_in;
+        if (inside) {
+#pragma unroll
+            for (int it = 0; it < S::XIT; ++it) {
+                const int i = wave + waves * it;
+                if (i < S::XQ) lds_load_b128(xrsrc, base + 1024u * i, x_off[it], (unsigned)x0 * 4u);
+            }
+        } else {
+            // the block crosses an end of the operand: element by element, what does not exist is 0
+            for (int i = wave; i < S::XQ; i += waves) {
+                const int p = 64 * i + lane, col = p / S::XQ, q = p - col * S::XQ;
+                const float *c = xbase + (long long)min(col, cols - 1) * ldx;
+                f4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = x0 + 4 * q + e;
+                    v[e] = q < nqx && r >= 0 && r < n_in ? c[r] : 0.f;
+                }
+                *reinterpret_cast<f4 *>(lds + buf * S::STAGE + 4 * p) = v;
+            }
+        }
+        for (int s = wave; s < K; s += waves) {
+            const int d = (u - s + K * 64) % K, m = u - d;           // the tile in slot s, and its window row
+            if (m < 0 || m >= tiles) continue;
+            const int at = tab[ngroups + g * K + d] + 4 * (row_first + m * period);
+            const unsigned to = base + (unsigned)((S::X_FLOATS + s * S::ASLOT) * 4);
+            if (inside) {
+#pragma unroll
+                for (int it = 0; it < S::AIT; ++it)
+                    if (256 * (it + 1) <= S::ASLOT || 256 * it + 4 * lane < S::ASLOT)
+                        lds_load_b128(arsrc, to + 1024u * it, a_off[it], (unsigned)(at + amin));
+            } else {
+                for (int it = 0; it < S::AIT; ++it) {
+                    const int p = 64 * it + lane, dx = p / S::AQ, q = p - dx * S::AQ;
+                    if (dx >= LC) continue;
+                    f4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int r = 4 * q + e, xr = x0 + r + dx;
+                        v[e] = r < rows && xr >= 0 && xr < n_in ? vals[(long long)(at / 4) + (long long)(astep4 / 4) * dx + r] : 0.f;
+                    }
+                    *reinterpret_cast<f4 *>(lds + buf * S::STAGE + S::X_FLOATS + s * S::ASLOT + 4 * p) = v;
+                }
+            }
+        }
+    };
+
+    f4 acc[S::NG][8];                                // tiles 4 g + i of rows r in acc[g][r][i]; a lane is a column
+    float tail[8];                                   // the tile that no group has
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+#pragma unroll
+        for (int g = 0; g < S::NG; ++g) acc[g][r] = f4{0.f, 0.f, 0.f, 0.f};
+        tail[r] = 0.f;
+    }
+    // where this lane reads values: lane 4 b + i of a group's register: row b % 8, diagonal 2 q + b / 8, tile i
+    const int lane_a = (lane % 4) * S::ASLOT + (lane / 32) * S::AROW + (lane / 4) % 8 + 8 * wave;
+    const int lane_t = (S::NG * 4) * S::ASLOT + (lane % 16 / 8) * S::AROW + lane % 8 + 8 * wave;
+
+    auto multiply = [&](int u, int buf) {
+        const float *const st = lds + buf * S::STAGE;
+        float x[4 * S::XW];
+#pragma unroll
+        for (int q = 0; q < S::XW; ++q) {
+            const f4 v = *reinterpret_cast<const f4 *>(st + lane * (4 * S::XQ) + 8 * wave + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[4 * q + e] = v[e];
+        }
+        // tiles alive at this step: max(0, u - K + 1) .. min(u, tiles - 1)
+        const int lo = max(0, u - K + 1), n = min(u, tiles - 1) - lo + 1, s_lo = lo % K;
+        const unsigned ones = (1u << n) - 1u, alive = (ones << s_lo) | (ones >> (K - s_lo));
+        plane_for<0, S::NG>([&](auto g_) {
+            constexpr int g = decltype(g_)::value;
+            if (!((alive >> (4 * g)) & 15u)) return;
+            plane_for<0, (LC + 1) / 2>([&](auto q_) {
+                constexpr int q = decltype(q_)::value;
+                // (slots past the last tile, diagonals past the last one: any value, never used)
+                const int at = S::X_FLOATS + lane_a + 4 * g * S::ASLOT + 2 * q * S::AROW;
+                const float a = st[4 * g + 3 < K ? at : min(at, S::STAGE - 1)];
+                plane_for<0, 16>([&](auto b_) {
+                    constexpr int b = decltype(b_)::value, r = b % 8, dx = 2 * q + b / 8;
+                    if constexpr (dx < LC) acc[g][r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, x[r + dx], acc[g][r], 4, b, 0);
+                });
+            });
+        });
+        if constexpr (S::TAIL) {
+            if ((alive >> (4 * S::NG)) & 1u) {
+                plane_for<0, (LC + 1) / 2>([&](auto q_) {
+                    constexpr int q = decltype(q_)::value;
+                    const float a = st[min(S::X_FLOATS + lane_t + 2 * q * S::AROW, S::STAGE - 1)];
+                    plane_fma8<0>(tail, a, x + 2 * q);
+                    if constexpr (2 * q + 1 < LC) plane_fma8<8>(tail, a, x + 2 * q + 1);
+                });
+            }
+        }
+    };
+
+    // A finished tile leaves through LDS, in the place of a block that is done with, so that a column's 32 rows are
+    // written together: lane (c, q) holds rows 4 q .. 4 q + 3 of columns 16 wave + c and 16 wave + 8 + c.
+    constexpr int OPITCH = PLANE_ROWS + 4;
+    static_assert(64 * OPITCH <= S::STAGE, "a tile fits a block's place");
+    const int my_row = 4 * (lane % 8), my_col = 16 * wave + lane / 8;
+    auto place = [&](int m, int c, int r) { return Y + (long long)(col0 + c) * ldy + row_first + (long long)m * period + r; };
+    f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto read_old = [&](int m) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (my_col + 8 * k >= cols) continue;
+            const float *p = place(m, my_col + 8 * k, my_row);
+            if (my_row >= skip) {
+                old[k] = *reinterpret_cast<const f4u *>(p);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (my_row + i >= skip) old[k][i] = p[i];
+            }
+        }
+    };
+    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
+        __builtin_amdgcn_s_barrier();                // nobody reads the block any more
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int r = 0; r < 8; r += 4) *reinterpret_cast<f4 *>(out + lane * OPITCH + 8 * wave + r) = f4{v[r], v[r + 1], v[r + 2], v[r + 3]};
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (EP && ep.act == 2) {
+            // sampled: a lane takes a row and 8 columns, two blocks of the generator
+            const int r = lane % 32, c0 = 16 * wave + 8 * (lane / 32), row = row_first + m * period + r;
+            const float bias = ep.bias ? ep.bias[row] : 0.f;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const SpRand4 w = sp_philox((unsigned)row, (unsigned)(col0 + c0) / 4u + h, ep.seed_lo, ep.seed_hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = c0 + 4 * h + i;
+                    if (c >= cols || r < skip) continue;
+                    float *p = place(m, c, r);
+                    const float s = out[c * OPITCH + r];
+                    *p = sp_finish(beta == 0.f ? alpha * s : beta * (*p) + alpha * s, bias, 2, w.w[i]);
+                }
+            }
+            return false;
+        }
+        float bias[4] = {0.f, 0.f, 0.f, 0.f};
+        if (EP && ep.bias) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bias[i] = ep.bias[row_first + m * period + my_row + i];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            f4 s = *reinterpret_cast<const f4 *>(out + (my_col + 8 * k) * OPITCH + my_row);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[i] = beta == 0.f ? alpha * s[i] : beta * old[k][i] + alpha * s[i];
+                if (EP) s[i] = sp_finish(s[i], bias[i], ep.act);
+            }
+            if (skip == 0) {
+                // (every lane's store is issued, those past the batch out of the resource's range: the count is certain)
+                const unsigned at = my_col + 8 * k < cols ? (unsigned)(my_col + 8 * k) * ((unsigned)ldy * 4u) + 4u * my_row : OOB_OFFSET;
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(plane_u4, s), yrsrc, at, (unsigned)(row_first + m * period) * 4u, 0);
+            } else if (my_col + 8 * k < cols) {
+                float *p = place(m, my_col + 8 * k, my_row);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (my_row + i >= skip) p[i] = s[i];
+            }
+        }
+        return skip == 0;
+    };
+
+    // the blocks (u, g) in order, one requested ahead
+    const int steps = tiles + K - 1;
+    int nu = 0, ng = -1;                             // the block requested last
+    auto advance = [&]() {
+        do {
+            if (++ng == ngroups) {
+                ng = 0;
+                ++nu;
+            }
+        } while (nu < steps && outside(nu, ng));
+    };
+    advance();
+    int buf = 0;
+    bool stores = false;                             // two stores of a finished tile are behind the block's requests
+    if (nu < steps) issue(nu, ng, 0);
+    int slot = 0;                                    // u % K
+    for (int u = 0; u < steps; ++u) {
+        plane_for<0, K>([&](auto s_) {
+            constexpr int s = decltype(s_)::value;
+            if (slot == s && u < tiles) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    if constexpr (s < 4 * S::NG) acc[s / 4][r][s % 4] = 0.f;
+                    else tail[r] = 0.f;
+                }
+            }
+        });
+        const int done = u - (K - 1);                // the tile that ends with this step
+        bool old_read = done < 0 || beta == 0.f || (EP && ep.act == 2);
+        while (nu == u) {
+            // (loads and stores complete in order)
+            if (stores) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            stores = false;
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            advance();
+            if (nu < steps) issue(nu, ng, buf ^ 1);
+            if (!old_read) {
+                read_old(done);
+                old_read = true;
+            }
+            multiply(u, buf);
+            buf ^= 1;
+        }
+        if (done >= 0) {
+            if (!old_read) read_old(done);
+            const int leaving = slot + 1 == K ? 0 : slot + 1;
+            float v[8];
+            plane_for<0, K>([&](auto s_) {
+                constexpr int s = decltype(s_)::value;
+                if (leaving == s) {
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) {
+                        if constexpr (s < 4 * S::NG) v[r] = acc[s / 4][r][s % 4];
+                        else v[r] = tail[r];
+                        asm volatile("" : "+v"(v[r]));       // (keeps the compiler from indexing the sums in memory)
+                    }
+                }
+            });
+            stores = finish(done, v, lds + (buf ^ 1) * S::STAGE);
+        }
+        slot = slot + 1 == K ? 0 : slot + 1;
+    }
+}
+
+template <int LC, int K>
+hipError_t plane_launch_one(const PlaneLaunch &L)
+{
+    const bool fused = L.ep.bias != nullptr || L.ep.act != 0;
+    const long long units = (long long)L.nseg * ((L.tp + PLANE_XT - 1) / PLANE_XT);
+    const unsigned grid = (unsigned)((units + 7) / 8 * 8 * PLANE_XT * L.col_tiles);
+    note_kernel("spmm_plane_kernel<%d, %d, %s>", LC, K, fused ? "true" : "false");
+    auto go = [&](auto kernel) {
+        launch_kernel(kernel, dim3(grid), dim3(64 * PLANE_WAVES), 0, L.stream, L.tab, L.ngroups, L.period, L.s0, L.astep4, L.tp,
+                      L.nseg, L.cuts, L.vals, L.B, L.ldb, L.dst, L.ldd, L.n_out, L.n_in, L.batch, L.alpha, L.beta,
+                      L.col_tiles, L.a_bytes, L.ep);
+    };
+    if (fused) go(spmm_plane_kernel<LC, K, true>);
+    else go(spmm_plane_kernel<LC, K, false>);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t spmm_plane_launch(const PlaneLaunch &L)
+{
+    switch (L.k) {
+        case 5: return plane_launch_one<5, 5>(L);
+        case 7: return plane_launch_one<7, 7>(L);
+        case 8: return plane_launch_one<8, 8>(L);
+        case 9: return plane_launch_one<9, 9>(L);
+        case 11: return plane_launch_one<11, 11>(L);
+        case 13: return plane_launch_one<13, 13>(L);
+        default: return hipErrorNotSupported;
+    }
+}
+
+bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int batch, bool fused, bool force, PlaneLaunch &L)
+{
+    if (wk.tab_dev == nullptr || wk.lck != wk.k) return false;
+    int per_cu = 1;
+    switch (wk.k) {
+        case 5: per_cu = PlaneShape<5, 5>::PER_CU; break;
+        case 7: per_cu = PlaneShape<7, 7>::PER_CU; break;
+        case 8: per_cu = PlaneShape<8, 8>::PER_CU; break;
+        case 9: per_cu = PlaneShape<9, 9>::PER_CU; break;
+        case 11: per_cu = PlaneShape<11, 11>::PER_CU; break;
+        case 13: per_cu = PlaneShape<13, 13>::PER_CU; break;
+        default: return false;
+    }
+    if (wk.period < PLANE_ROWS || n_out % wk.period != 0) return false;
+    L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
+    L.col_tiles = (batch + 63) / 64;
+    const int walk_len = (int)(n_out / wk.period);
+
+    // Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut
+    // where that work divides evenly.  Between two ends of groups' ranges the groups are the same.
+    std::vector<int> ends{0, walk_len};
+    auto range = [&](int g, long long &lo, long long &hi) {      // map rows whose middle window row lies in the operand
+        const long long at = (long long)wk.s0 + wk.rows_host[g] + (long long)(wk.k / 2) * wk.period;
+        lo = (std::max(0LL, -at) + wk.period - 1) / wk.period;
+        hi = std::min<long long>(walk_len, (n_in - at + wk.period - 1) / wk.period);
+    };
+    for (int g = 0; g < wk.ngroups; ++g) {
+        long long lo, hi;
+        range(g, lo, hi);
+        if (lo > 0 && lo < walk_len) ends.push_back((int)lo);
+        if (hi > 0 && hi < walk_len) ends.push_back((int)hi);
+    }
+    std::sort(ends.begin(), ends.end());
+    std::vector<int> groups(ends.size(), 0);
+    long long work = 0;
+    int most = 1;
+    for (size_t i = 0; i + 1 < ends.size(); ++i) {
+        for (int g = 0; g < wk.ngroups; ++g) {
+            long long lo, hi;
+            range(g, lo, hi);
+            groups[i] += lo <= ends[i] && ends[i + 1] <= hi;
+        }
+        work += (long long)groups[i] * (ends[i + 1] - ends[i]);
+        most = std::max(most, groups[i]);
+    }
+    // How many: workgroups run in rounds of 32 CUs per XCD, a unit of PLANE_XT walks with its column tiles on one XCD.
+    const int full = L.tp / PLANE_XT, part = L.tp % PLANE_XT, cap = 32 * per_cu;
+    auto rounds = [&](int segs) {
+        const int wgs = ((segs * full + 7) / 8 * PLANE_XT + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles;
+        return (wgs + cap - 1) / cap;
+    };
+    double best = -1;
+    int n = 1;
+    for (int i = 1; i <= PLANE_MAX_SEGMENTS && i <= walk_len; ++i) {
+        const double cost = rounds(i) * ((double)work / i + 0.9 * (wk.k - 1) * most);
+        if (best < 0 || cost < best) {
+            best = cost;
+            n = i;
+        }
+    }
+    // Taken where the steps come to at most 1.65 times the segments' work (5 x 5 and 7 x 7 windows: 1.4 times), with two column
+    // tiles at least -- with one, the values are most of the traffic, and the tile-by-tile kernel fetches them in pieces twice
+    // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
+    // Measured on 90 layers: 1.0 - 1.6 times the tile-by-tile kernel's rate where taken (one of 30: 0.88), 0.44 - 1.1 elsewhere.
+    const double over = best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
+    if (work == 0) return false;
+    if (!force && (L.col_tiles < 2 || over > (wk.k >= 8 ? 1.65 : 1.4) || (wk.k >= 9 && fused))) return false;
+    L.nseg = n;
+    long long done = 0;
+    size_t i = 0;
+    L.cuts.at[0] = 0;
+    for (int s = 1; s < n; ++s) {
+        const long long want = work * s / n;
+        while (i + 2 < ends.size() && done + (long long)groups[i] * (ends[i + 1] - ends[i]) <= want) {
+            done += (long long)groups[i] * (ends[i + 1] - ends[i]);
+            ++i;
+        }
+        L.cuts.at[s] = groups[i] ? ends[i] + (int)((want - done) / groups[i]) : ends[i];
+    }
+    L.cuts.at[n] = walk_len;
+    return true;
+}
+
+}  // namespace cuvdia

@@ -49,10 +49,12 @@ extern "C" {
 /* Kernel families, for cuvdia_set_path / cuvdia_last_path. */
 #define CUVDIA_PATH_AUTO     0  /* pick by shape (default)                        */
 #define CUVDIA_PATH_GENERIC  1  /* one-thread-per-output kernels, any row_fact    */
-#define CUVDIA_PATH_TILED    2  /* LDS-staged, register-blocked kernels (rf == 1) */
+#define CUVDIA_PATH_TILED    2  /* LDS-staged, register-blocked kernels on the vector unit (rf == 1) */
 #define CUVDIA_PATH_WALK     3  /* of the tiled family: the walking kernel for window tables (products only) */
 #define CUVDIA_PATH_TILED_NOWALK 4  /* the tiled family without its kernels for window tables                  */
 #define CUVDIA_PATH_WINDOW   5  /* of the tiled family: the projection tiled in the window's plane (window tables) */
+#define CUVDIA_PATH_PLANE    6  /* of the tiled family: the product walked on the matrix cores (window tables)     */
+#define CUVDIA_PATH_THIN     8  /* of the tiled family: the product with rows along the lanes                      */
 
 /* Activation applied by cuvdia_spmm_bias_act_f32. */
 #define CUVDIA_ACT_NONE      0
@@ -343,12 +345,14 @@ int cuvdia_cache_clear(void);
 /* Forces a kernel family for subsequent calls (process-wide; tests use it to
  * run both families on the same inputs).  CUVDIA_PATH_TILED on a request the
  * tiled kernels cannot serve (row_fact > 1) returns CUVDIA_EUNSUPPORTED from
- * the compute call.  CUVDIA_PATH_WALK, CUVDIA_PATH_WINDOW and
- * CUVDIA_PATH_TILED_NOWALK choose inside the tiled family: a kernel for
+ * the compute call.  CUVDIA_PATH_WALK, CUVDIA_PATH_PLANE, CUVDIA_PATH_WINDOW
+ * and CUVDIA_PATH_TILED_NOWALK choose inside the tiled family: a kernel for
  * window tables whatever the size of the operands, or none of them.
  * CUVDIA_PATH_WALK: the walking product (CUVDIA_EUNSUPPORTED for a table
  * that is no window table with a walking kernel; densedense_to_dia treats it
- * as CUVDIA_PATH_TILED_NOWALK).  CUVDIA_PATH_WINDOW: the kernels tiled in the
+ * as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_PLANE likewise, for the product
+ * walked on the matrix cores; CUVDIA_PATH_THIN: the product with rows along
+ * the lanes at any batch (densedense_to_dia: as CUVDIA_PATH_AUTO).  CUVDIA_PATH_WINDOW: the kernels tiled in the
  * window's plane, which serve densedense_to_dia (CUVDIA_EUNSUPPORTED when
  * they do not serve the request: no window table of chunks of 2 to 13
  * diagonals, a period, channel distances or row counts that are no multiples
@@ -357,7 +361,8 @@ int cuvdia_set_path(int path);
 
 /* Which family the most recent compute call on this thread launched
  * (CUVDIA_PATH_GENERIC, CUVDIA_PATH_TILED, CUVDIA_PATH_WALK for a product
- * served by the walking kernel, CUVDIA_PATH_WINDOW for a projection served
+ * served by the walking kernel, CUVDIA_PATH_PLANE by the one on the matrix
+ * cores, CUVDIA_PATH_WINDOW for a projection served
  * by the kernel tiled in the window's plane; 0 before any call). */
 int cuvdia_last_path(void);
 

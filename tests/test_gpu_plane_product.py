@@ -1,0 +1,130 @@
+"""The product that walks the window's plane on the matrix cores, against the oracle: every window it is built for, both
+transposes, maps whose width its tiles of 32 positions do not divide, several groups, ragged batches, a destination that is
+read, bias / sigmoid / sample at the tiles' exit, non-finite operands, padded leading dimensions, graph replay."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [                    # (px, py, window, maps in, maps out, batch)
+    (37, 40, 5, 1, 1, 70),
+    (75, 23, 5, 3, 4, 33),    # several groups; 3 tiles of 32 positions, the last moved up
+    (32, 50, 7, 1, 1, 64),
+    (150, 20, 8, 2, 1, 40),
+    (41, 33, 9, 2, 2, 129),
+    (100, 37, 11, 1, 2, 30),
+    (33, 60, 13, 1, 1, 24),
+    (64, 31, 13, 2, 1, 64),
+]
+
+
+def _case(oracle, seed, px, py, fs, maps_in, maps_out, batch, trans):
+    from cuv_amd import dia as D
+    rng = np.random.default_rng(seed)
+    h, w = px * py * maps_in, px * py * maps_out
+    A = oracle.Dia(h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets(), max(h, w), 1)
+    A.vals[:] = np.nan                                   # padding must never be read
+    valid = oracle.valid_mask(A)
+    A.vals[valid] = rng.uniform(-1, 1, int(valid.sum())).astype(np.float32)
+    n_in, n_out = (h, w) if trans == "t" else (w, h)
+    B = np.asfortranarray(rng.uniform(-1, 1, (n_in, batch)).astype(np.float32))
+    dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
+    return rng, A, B, dst
+
+
+@pytest.fixture
+def plane():
+    from cuv_amd import _lib
+    L = _lib.lib()
+    _lib.check(L.cuvdia_set_path(_lib.PATH_PLANE), "set_path")
+    yield L
+    L.cuvdia_set_path(_lib.PATH_AUTO)
+
+
+def _ran():
+    from cuv_amd import _lib
+    return _lib.lib().cuvdia_last_path() == _lib.PATH_PLANE
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_windows_maps_and_batches(oracle, shape, trans):
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    _, A, B, dst = _case(oracle, sum(shape), *shape, trans)
+    for beta in (0.0, -1.5):
+        _, ran = gu.check_prod(oracle, A, B, dst if beta else None, trans, 0.75, beta, _lib.PATH_PLANE, str(shape))
+        assert ran == _lib.PATH_PLANE
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+def test_bias_sigmoid_sample_and_non_finite_values(oracle, plane, trans):
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng, A, B, dst = _case(oracle, 5, 35, 40, 9, 1, 1, 70, trans)
+    n, batch = dst.shape
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    dev, Bd, bd = gu.make_dev_dia(A), D.to_device_colmajor(B), torch.from_numpy(bias).cuda()
+    for beta in (0.0, 0.5):
+        p = oracle.prod_bias_act(A, B, dst if beta else None, trans, 1.0, beta, bias, True)
+        out = D.to_device_colmajor(dst)
+        D.prod_bias_act(out, dev, Bd, trans, 1.0, beta, bias=bd, act=_lib.ACT_SIGMOID)
+        assert _ran()
+        np.testing.assert_allclose(D.to_host_colmajor(out), p, rtol=0, atol=2e-5)
+        out = D.to_device_colmajor(dst)
+        D.prod_bias_act(out, dev, Bd, trans, 1.0, beta, bias=bd, act=_lib.ACT_SIGMOID_SAMPLE, seed=99)
+        u = oracle.sample_uniform(n, batch, 99)
+        decided = np.abs(p.astype(np.float64) - u) > 5e-5
+        assert _ran() and np.array_equal(D.to_host_colmajor(out)[decided], oracle.rnd_binarize(p, u)[decided])
+    for r, c, v in ((3, 5, -np.inf), (n // 2, 0, np.inf), (n - 2, 69, np.nan), (777, 33, np.nan)):
+        B[r, c] = v
+    with np.errstate(invalid="ignore"):
+        ref = oracle.prod(A, B, None, trans)
+    got, ran = gu.gpu_prod(A, B, None, trans, path=_lib.PATH_PLANE)
+    assert ran == _lib.PATH_PLANE and np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+
+
+def test_padded_operands_and_graph_replay(oracle, plane):
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import dia as D
+    _, A, B, _ = _case(oracle, 6, 45, 40, 8, 1, 1, 66, "n")
+    n, batch = B.shape
+    dev = gu.make_dev_dia(A)
+    X = torch.full((batch + 1, n + 7), float("nan"), device="cuda:0")
+    X[:batch, :n] = D.to_device_colmajor(B)
+    out = torch.full((batch + 2, n + 3), -7.0, device="cuda:0")
+    view = out[1:batch + 1, :n]
+    D.prod(view, dev, X[:batch, :n], "n")
+    assert _ran()
+    gu.assert_close_mag(D.to_host_colmajor(view), oracle.prod(A, B), oracle.prod_mag(A, B), "padded")
+    assert torch.all(out[:, n:] == -7.0) and torch.all(out[0] == -7.0) and torch.all(out[batch + 1] == -7.0)
+    eager = view.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        D.prod(view, dev, X[:batch, :n], "n", sync=False)
+    for _ in range(3):
+        view.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(view, eager)
+
+
+def test_the_automatic_choice_takes_it_for_large_products(oracle):
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    A = oracle.Dia(75 * 1500, 75 * 1500, D.filter_factory_float(75, 1500, 8, 1, 1).offsets(), 75 * 1500, 1)
+    A.vals[:] = np.random.default_rng(7).uniform(-1, 1, A.vals.shape)
+    dev, B = gu.make_dev_dia(A), torch.rand((130, A.w), device="cuda:0")
+    out, ref = torch.empty_like(B), torch.empty_like(B)
+    L = _lib.lib()
+    D.prod(out, dev, B, "n")
+    assert L.cuvdia_last_path() == _lib.PATH_PLANE
+    _lib.check(L.cuvdia_set_path(_lib.PATH_TILED_NOWALK), "set_path")
+    try:
+        D.prod(ref, dev, B, "n")
+    finally:
+        L.cuvdia_set_path(_lib.PATH_AUTO)
+    torch.testing.assert_close(out, ref, rtol=1e-5, atol=2e-5)
