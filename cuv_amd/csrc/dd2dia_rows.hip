@@ -17,7 +17,8 @@
 // 6.5 GB: one thread per slot before) 4470 -> 377; 96 x 96, 5 x 5, 3 maps to 4, batch 14 33 -> 11.
 //
 // Accumulation order: range r of S sums its steps r, r + S, ... of DR_COLS columns in ascending order,
-// acc = fma(a, b, acc); total = ((p0 + p1) + p2) + ...
+// acc = fma(a, b, acc), in blocks of DR_BLOCK columns (one running sum over a batch of a thousand loses a digit where two
+// such gradients are subtracted; the blocks' sums wait in LDS); total = ((p0 + p1) + p2) + ... of blocks and ranges.
 #include <hip/hip_runtime.h>
 
 #include "device.hpp"
@@ -31,6 +32,7 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int DR_MAX_WAVES = 8, DR_ROWS = 256;
 constexpr int DR_COLS = 2;                           // batch columns in flight per wave (4 take registers two waves need)
+constexpr int DR_BLOCK = 128;                        // batch columns per running sum
 constexpr int dr_halo(int lc) { return lc > 1 ? (lc + 2) / 4 : 1; }
 
 // 4 consecutive rows from `row` of a column of n rows.  `plain`: the 16 bytes lie inside the allocation (rows outside
@@ -50,7 +52,7 @@ template <int LC>
 __global__ __launch_bounds__(64 * DR_MAX_WAVES) void dd2dia_rows_kernel(
     const Chunk *__restrict__ chunks, int nchunks, float *__restrict__ C, int stride, const float *__restrict__ A,
     long long lda, const float *__restrict__ B, long long ldb, int h, int w, int batch, float alpha, float beta,
-    int row_blocks, int unit_groups, int splits)
+    int row_blocks, int unit_groups, int splits, int blocks_at)
 {
     constexpr int NQ = (LC + 6) / 4, HQ = dr_halo(LC), PITCH = DR_ROWS + 4 * HQ, CU = DR_COLS;
     static_assert(CU * HQ <= 64, "the halo is one piece per lane");
@@ -95,6 +97,9 @@ __global__ __launch_bounds__(64 * DR_MAX_WAVES) void dd2dia_rows_kernel(
                 hv = dr_rows(B + (long long)c * ldb, plain ? hrow : x0 + hk, w, plain);
             }
         };
+        // blocks_at: where in LDS the blocks' sums are (0: a range is one block)
+        f4 *const total = reinterpret_cast<f4 *>(lds + blocks_at) + wave * LC * 64 + lane;
+        int steps = 0, blocks = 0;
         int c0 = split * CU;
         if (c0 < batch) request(c0);
         for (; c0 < batch; c0 += splits * CU) {
@@ -120,6 +125,19 @@ __global__ __launch_bounds__(64 * DR_MAX_WAVES) void dd2dia_rows_kernel(
                         for (int i = 0; i < 4; ++i) acc[j][i] = __builtin_fmaf(now[u][i], x[(i + j) / 4][(i + j) % 4], acc[j][i]);
                 }
             }
+            if (blocks_at != 0 && ++steps == DR_BLOCK / CU) {
+#pragma unroll
+                for (int j = 0; j < LC; ++j) {
+                    total[j * 64] = blocks == 0 ? acc[j] : total[j * 64] + acc[j];
+                    acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+                }
+                steps = 0;
+                ++blocks;
+            }
+        }
+        if (blocks > 0) {
+#pragma unroll
+            for (int j = 0; j < LC; ++j) acc[j] = total[j * 64] + acc[j];
         }
     }
 
@@ -212,11 +230,13 @@ hipError_t dr_launch(const DrLaunch &L)
     const int waves = splits > 4 ? splits : 4, per = waves / splits;
     const long long groups = (L.nchunks + per - 1) / per;
     if (row_blocks * groups > 0x7fffffffLL) return hipErrorInvalidValue;
-    const size_t stage = (size_t)waves * DR_COLS * PITCH * sizeof(float), meet = splits > 1 ? (size_t)waves * LC * 1024 : 0;
+    const bool blocks = L.batch > splits * DR_BLOCK;
+    const size_t staged = (size_t)waves * DR_COLS * PITCH * sizeof(float), sums = (size_t)waves * LC * 1024;
+    const size_t stage = blocks ? staged + sums : staged, meet = splits > 1 ? sums : 0;
     note_kernel("dd2dia_rows_kernel<%d>", LC);
     launch_kernel(dd2dia_rows_kernel<LC>, dim3((unsigned)(row_blocks * groups)), dim3(64 * waves), stage > meet ? stage : meet,
                   L.stream, L.chunks, L.nchunks, L.C, L.stride, L.A, L.lda, L.B, L.ldb, L.h, L.w, L.batch, L.alpha, L.beta,
-                  (int)row_blocks, (int)groups, splits);
+                  (int)row_blocks, (int)groups, splits, blocks ? (int)(staged / sizeof(float)) : 0);
     return hipGetLastError();
 }
 

@@ -32,6 +32,7 @@ def test_rows_runs_and_batches(oracle, run, rows):
 
 @pytest.mark.parametrize("h,w,runs,batch", [
     (301, 2000, 5, 300),                     # eight ranges of the batch
+    (303, 2000, 5, 1100),                    # ... each summed in blocks of columns
     (30001, 30003, 20, 70),                  # several rounds of waves, four ranges
     (70001, 69999, 60, 9),                   # one range
 ])
