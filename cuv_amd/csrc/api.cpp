@@ -620,26 +620,26 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
-    bool windowed = false;
+    int ran = CUVDIA_PATH_TILED;
     if (rows) {
         e = launch_dd2dia_rows(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
     } else if (!tiled) {
         e = launch_dd2dia_generic(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
     } else {
-        const int window = forced == CUVDIA_PATH_WINDOW ? 1
-                           : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_PLANE) ? -1 : 0;
+        const int window = forced == CUVDIA_PATH_WINDOW ? 1 : forced == CUVDIA_PATH_PLANE ? -2
+                           : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK) ? -1 : 0;
         for (int c0 = 0; c0 < batch && e == hipSuccess; c0 += slab) {
-            bool this_one = false;
+            int this_one = CUVDIA_PATH_TILED;
             e = launch_dd2dia_tiled(desc->view, C_vals, A + (long long)c0 * lda, lda, B + (long long)c0 * ldb, ldb,
                                     std::min(slab, batch - c0), alpha, c0 == 0 ? beta : 1.f, s, window, &this_one);
-            windowed = windowed || this_one;
+            if (this_one != CUVDIA_PATH_TILED) ran = this_one;
         }
         if (window > 0 && e == hipErrorNotSupported) {
             (void)hipGetLastError();
             return CUVDIA_EUNSUPPORTED;
         }
     }
-    t_last_path = !tiled ? CUVDIA_PATH_GENERIC : windowed ? CUVDIA_PATH_WINDOW : CUVDIA_PATH_TILED;
+    t_last_path = !tiled ? CUVDIA_PATH_GENERIC : ran;
     return e == hipSuccess ? CUVDIA_OK : hip_fail(e, "dd2dia kernel launch");
 }
 

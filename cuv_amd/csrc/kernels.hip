@@ -3296,15 +3296,24 @@ bool dd2dia_window_by_size(const DiaView &C, int batch, long long workgroups)
 
 hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, long long lda,
                                const float *B, long long ldb, int batch,
-                               float alpha, float beta, hipStream_t stream, int window, bool *windowed)
+                               float alpha, float beta, hipStream_t stream, int window, int *ran)
 {
-    if (windowed) *windowed = false;
+    if (ran) *ran = CUVDIA_PATH_TILED;
+    auto plane = [&](bool force) {
+        const hipError_t e = launch_dd2dia_plane(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
+        if (e != hipErrorNotSupported && ran) *ran = CUVDIA_PATH_PLANE;
+        return e;
+    };
+    if (window == -2)
+        if (const hipError_t e = plane(true); e != hipErrorNotSupported) return e;
     if (window >= 0) {
         int txn = 0, tyn = 0, ndb = 0;
         long long wgs = dd2dia_window_workgroups(C, batch, &txn, &tyn, &ndb);
         // (a lane's byte offsets run up to 16 columns past the batch and must stay below 2^32)
         if (((long long)batch + 16) * std::max(lda, ldb) * 4 >= (1LL << 32)) wgs = 0;
         if (wgs > 0 && (window > 0 || dd2dia_window_by_size(C, batch, wgs))) {
+            if (window == 0)
+                if (const hipError_t e = plane(false); e != hipErrorNotSupported) return e;
             const WalkView &wk = C.walk_n;
             const DwLaunch L{wk.tab_dev, wk.ngroups, wk.k, wk.period, wk.s0, wk.astep4 / 4, wk.lck, vals, A, lda, B, ldb,
                              C.h, C.w, batch, alpha, beta,
@@ -3312,7 +3321,7 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
                              (unsigned)((((long long)batch - 1) * ldb + C.w) * 4),
                              (unsigned)((long long)C.nd * C.stride * 4), txn, tyn, ndb,
                              dd2dia_window_subs(C, wgs), stream};
-            if (windowed) *windowed = true;
+            if (ran) *ran = CUVDIA_PATH_WINDOW;
             return dd2dia_window_launch(L);
         }
     }

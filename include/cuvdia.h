@@ -53,7 +53,7 @@ extern "C" {
 #define CUVDIA_PATH_WALK     3  /* of the tiled family: the walking kernel for window tables (products only) */
 #define CUVDIA_PATH_TILED_NOWALK 4  /* the tiled family without its kernels for window tables                  */
 #define CUVDIA_PATH_WINDOW   5  /* of the tiled family: the projection tiled in the window's plane (window tables) */
-#define CUVDIA_PATH_PLANE    6  /* of the tiled family: the product walked on the matrix cores (window tables)     */
+#define CUVDIA_PATH_PLANE    6  /* of the tiled family: the kernels on the matrix cores (window tables)            */
 #define CUVDIA_PATH_THIN     8  /* of the tiled family: the product with rows along the lanes                      */
 
 /* Activation applied by cuvdia_spmm_bias_act_f32. */
@@ -351,7 +351,8 @@ int cuvdia_cache_clear(void);
  * CUVDIA_PATH_WALK: the walking product (CUVDIA_EUNSUPPORTED for a table
  * that is no window table with a walking kernel; densedense_to_dia treats it
  * as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_PLANE likewise, for the product
- * walked on the matrix cores; CUVDIA_PATH_THIN: the product with rows along
+ * walked on the matrix cores (densedense_to_dia: the projection on the matrix
+ * cores for windows of 9 x 9 and 11 x 11, else as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_THIN: the product with rows along
  * the lanes at any batch (densedense_to_dia: as CUVDIA_PATH_AUTO).  CUVDIA_PATH_WINDOW: the kernels tiled in the
  * window's plane, which serve densedense_to_dia (CUVDIA_EUNSUPPORTED when
  * they do not serve the request: no window table of chunks of 2 to 13
@@ -361,7 +362,7 @@ int cuvdia_set_path(int path);
 
 /* Which family the most recent compute call on this thread launched
  * (CUVDIA_PATH_GENERIC, CUVDIA_PATH_TILED, CUVDIA_PATH_WALK for a product
- * served by the walking kernel, CUVDIA_PATH_PLANE by the one on the matrix
+ * served by the walking kernel, CUVDIA_PATH_PLANE by the ones on the matrix
  * cores, CUVDIA_PATH_WINDOW for a projection served
  * by the kernel tiled in the window's plane; 0 before any call). */
 int cuvdia_last_path(void);
