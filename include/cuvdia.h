@@ -134,7 +134,9 @@ int cuvdia_plan_units(const int *offsets_host, int nd, int *c1, int *c2, int cap
  * periods of at least 192: 4096; or 1024 (512 on periods of at least 256)
  * when the blocks of window rows are at least nine tenths full (13 and 14
  * rows; 9, 10 and 15 in blocks of 5); or 1024 when window rows x channel
- * groups are at least 22.
+ * groups are at least 22.  Of these launches, windows of 9 x 9 and 11 x 11 at
+ * a batch of at least 24 run on the matrix cores instead where their tiles of
+ * 8 x 64 positions fill rounds of one per CU to three quarters.
  * Negative: an error.
  * cuvdia_set_path(CUVDIA_PATH_WINDOW) waives the conditions on the period's
  * size, the workgroups and the batch.  No counterpart in the reference. */
