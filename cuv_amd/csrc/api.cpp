@@ -425,7 +425,7 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     }
     unsigned char *base = static_cast<unsigned char *>(d->dev_block);
     d->view = DiaView{};
-    d->view.h = h; d->view.w = w; d->view.nd = nd; d->view.stride = stride; d->view.rf = row_fact;
+    d->view.h = h; d->view.w = w; d->view.nd = nd; d->view.stride = stride; d->view.rf = row_fact; d->view.nnz = d->nnz;
     d->view.offsets_dev = reinterpret_cast<const int *>(base);
     d->view.chunks_n_dev = reinterpret_cast<const Chunk *>(base + off_bytes);
     d->view.n_chunks_n = d->n_chunks_n;
@@ -769,6 +769,7 @@ int cuvdia_spmm_offsets_noalloc_f32(const float *A_vals, const int *offsets_host
     // requested traversal is described (and uploaded); the other one is left empty.
     DiaView view{};
     view.h = h; view.w = w; view.nd = nd; view.stride = stride; view.rf = row_fact;
+    view.nnz = count_valid(offsets_host, nd, h, w, row_fact);
     view.offsets_dev = reinterpret_cast<const int *>(tables);
     const Chunk *chunks_dev = reinterpret_cast<const Chunk *>(tables + NOALLOC_CHUNKS_AT);
     int max_len = 0, min_len = chunks.front().len, s_min = chunks.front().s0, s_max = s_min;
@@ -800,7 +801,7 @@ int cuvdia_spmm_offsets_noalloc_f32(const float *A_vals, const int *offsets_host
     else e = noalloc_upload(tables, offsets_host, (size_t)nd * sizeof(int), s);
     if (e != hipSuccess) return hip_fail(e, "table fill kernel launch");
     const SpEpilogue ep{nullptr, CUVDIA_ACT_NONE, 0u, 0u};
-    e = tiled ? launch_spmm_tiled(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
+    e = tiled ? launch_spmm_tiled(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s, forced)
         : thin ? launch_spmm_thin(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s)
               : launch_spmm_generic(view, A_vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, s);
     t_last_path = tiled || thin ? CUVDIA_PATH_TILED : CUVDIA_PATH_GENERIC;

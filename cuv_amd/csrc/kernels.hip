@@ -3134,6 +3134,8 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
         }
         if (path == CUVDIA_PATH_PLANE) return hipErrorNotSupported;
     }
+    if (path == CUVDIA_PATH_AUTO && spmm_thin_by_size(A, trans, batch))
+        return launch_spmm_thin(A, vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, stream);
     const SpLaunch L{trans ? A.chunks_t_dev : A.chunks_n_dev,
                      trans ? A.n_chunks_t : A.n_chunks_n,
                      vals, A.stride, trans ? 1 : 0, B, ldb, dst, ldd, n_out, n_in, batch, alpha, beta,

@@ -49,6 +49,7 @@ struct WalkView {
 
 struct DiaView {
     int h, w, nd, stride, rf;
+    long long nnz;               // stored elements
     const int *offsets_dev;      // nd ints, table order
     const Chunk *chunks_n_dev;   // the products' tables (chunks of up to SP_CHUNK_MAX): shifts = offsets
     int n_chunks_n;
@@ -111,6 +112,8 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
 // Same contract, row_fact == 1 only: rows along the lanes, chunks dealt to the waves (spmm_thin.hip).  For few batch
 // columns and for few output rows; no limit on the operands' sizes.
 bool spmm_thin_ok(const DiaView &A, bool trans);
+// Whether the automatic choice takes it for a product that would otherwise run tile by tile.
+bool spmm_thin_by_size(const DiaView &A, bool trans, int batch);
 hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B, long long ldb,
                             float *dst, long long ldd, int batch, bool trans,
                             float alpha, float beta, SpEpilogue ep, hipStream_t stream);

@@ -1,4 +1,4 @@
-// The product for few batch columns: rows along the lanes, chunks dealt to the waves.
+// The product for few batch columns, and for few tiles of many chunks: rows along the lanes, chunks dealt to the waves.
 //
 //   dst[r, c] = sum over chunks, over their diagonals j:  A(slot_j)[r] * X[r + s0 + j, c]
 //
@@ -218,6 +218,23 @@ hipError_t launch_lc(const ThinLaunch &L, int cb, int g, int waves)
 bool spmm_thin_ok(const DiaView &A, bool trans)
 {
     return A.rf == 1 && (trans ? A.n_chunks_t : A.n_chunks_n) <= NOALLOC_MAX_CHUNKS;
+}
+
+bool spmm_thin_by_size(const DiaView &A, bool trans, int batch)
+{
+    const int n_out = trans ? A.w : A.h, lc = trans ? A.max_len_t : A.max_len_n;
+    if (!spmm_thin_ok(A, trans) || lc < 3) return false;
+    // The tile-by-tile kernel works through a tile's chunks one after another, 1 - 2 us apart, and always for 64 columns;
+    // here eight waves share the chunks and the columns are the ones that exist.  So few tiles of many chunks belong here,
+    // and many where a good part of their columns is not there.  Measured on 33500 products of windows of 3 x 3 to 13 x 13,
+    // batch 24 to 300, with and without the fused layer update: 1.1 - 4 times the tile-by-tile kernel's rate where the
+    // tiles' number decides (median 1.8; 0.1 % below 0.97), 0.9 - 1.7 where the columns do (median 1.3, a tenth below 1.0);
+    // one step beyond these lines a tenth of the products falls below 0.9.
+    const double tiles = (n_out + 63) / 64 * (batch / 64.0);     // of the columns that exist
+    const double chunks = (double)A.nnz / n_out / lc;            // per tile, those outside the operand left out
+    const double there = batch / 64.0 / ((batch + 63) / 64);
+    const double most = chunks < 6 ? 40 : chunks < 9.5 ? 56 : chunks < 14 ? 90 : chunks < 24 ? 110 : chunks < 40 ? 120 : 190;
+    return tiles < most || (chunks >= 14 && there <= (lc <= 5 ? 0.8 : 0.7));
 }
 
 hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B, long long ldb,

@@ -77,3 +77,19 @@ def test_non_finite_values_and_sampling(oracle, trans):
                     act=_lib.ACT_SIGMOID_SAMPLE, seed=77)
     decided = np.abs(p.astype(np.float64) - u) > 1e-5
     assert np.array_equal(D.to_host_colmajor(out)[decided], oracle.rnd_binarize(p, u)[decided])
+
+
+@pytest.mark.parametrize("px,k,maps_in,maps_out,batch,kernel", [
+    (40, 7, 1, 1, 24, "spmm_thin_kernel<7"),             # 25 row tiles: few of them, whatever the batch up to ...
+    (40, 7, 1, 1, 140, "spmm_thin_kernel<7"),            # 55 tiles' worth of columns
+    (40, 7, 1, 1, 150, "spmm_tiled_kernel<7"),           # 59
+    (64, 5, 3, 4, 70, "spmm_thin_kernel<5"),             # many tiles, 58 of 128 columns not there
+    (64, 5, 3, 4, 128, "spmm_tiled_kernel<5"),           # all there
+    (64, 13, 2, 2, 88, "spmm_thin_kernel<13"),           # runs longer than 5: up to 70 % there
+    (64, 13, 2, 2, 92, "spmm_tiled_kernel<13"),
+])
+def test_automatic_choice_by_tiles_and_columns(oracle, px, k, maps_in, maps_out, batch, kernel):
+    n = px * px
+    offsets = sorted(m * n + dy * px + dx for m in range(1 - maps_in, maps_out)
+                     for dy in range(-(k // 2), k - k // 2) for dx in range(-(k // 2), k - k // 2))
+    _check(oracle, px + batch, n * maps_in, n * maps_out, offsets, batch, 0.75, 0.5 if batch % 4 else 0.0, kernel)
