@@ -58,8 +58,10 @@ SpFamily spmm_family(const DiaView &A, long long ldb, long long ldd, int batch, 
 // Largest h, w and |offset| the kernels' 32-bit row arithmetic allows.
 constexpr long long DIM_LIMIT = 1LL << 30;
 
+// (The runtime keeps the error for the next hipGetLastError(), which every launch ends with: it is reported here.)
 int hip_fail(hipError_t e, const char *what)
 {
+    (void)hipGetLastError();
     t_hip_error = std::string(what) + ": " + hipGetErrorString(e);
     return CUVDIA_EHIP;
 }
