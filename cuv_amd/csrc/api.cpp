@@ -196,11 +196,10 @@ int cuvdia_wait_begin(void)
     }
     Waiter &w = t_wait;
     if (device != w.device) {
-        w.current = nullptr;
+        hipEvent_t event = nullptr;
         for (auto &e : w.events)
-            if (e.first == device) w.current = e.second;
-        if (!w.current) {
-            hipEvent_t event = nullptr;
+            if (e.first == device) event = e.second;
+        if (!event) {
             const hipError_t e = hipEventCreateWithFlags(&event, hipEventDisableTiming);
             if (e != hipSuccess) return hip_fail(e, "hipEventCreateWithFlags");
             try {
@@ -209,8 +208,8 @@ int cuvdia_wait_begin(void)
                 (void)hipEventDestroy(event);
                 return CUVDIA_ENOMEM;
             }
-            w.current = event;
         }
+        w.current = event;                           // (both or neither: the next call may be on the former device)
         w.device = device;
     }
     // The runtime keeps a record of every launch until something waits for the stream as a whole; now and then we do.
