@@ -4,7 +4,9 @@
 // the stream, argument conversion --, more than the kernels of a small layer take.  Here the same steps read the
 // tensors' fields directly (under 1 us).  Every function returns True when it has done the call, and False -- having
 // done nothing -- for operands that are not the usual ones (wrong shapes or types, another device, a matrix without
-// a descriptor yet, a capturing stream): dia.py then takes its general way, which also words the errors.
+// a descriptor yet, a capturing stream): dia.py then takes its general way, which also words the errors.  Once the
+// library has been called a failure is raised, as _lib.CuvDiaError: kernels may be queued, and the general way would
+// do the call a second time.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -94,17 +96,36 @@ bool stream_of(int device, bool sync, hipStream_t &s)
     return true;
 }
 
-// Runs call() and, if asked to, waits for it without holding the interpreter.
-template <class Call>
-bool run(bool sync, hipStream_t s, Call &&call)
+PyObject *no() { Py_RETURN_FALSE; }
+
+// Raises _lib.CuvDiaError(code, what); returns nullptr.
+PyObject *raise(int code, const char *what)
 {
-    if (!sync) return call() == CUVDIA_OK;
-    if (cuvdia_wait_begin() != CUVDIA_OK) return false;
-    int rc = call(), waited = CUVDIA_OK;
-    Py_BEGIN_ALLOW_THREADS
-    waited = cuvdia_wait_end(s);
-    Py_END_ALLOW_THREADS
-    return rc == CUVDIA_OK && waited == CUVDIA_OK;
+    PyObject *lib = PyImport_ImportModule("cuv_amd._lib");
+    PyObject *type = lib ? PyObject_GetAttrString(lib, "CuvDiaError") : nullptr;
+    PyObject *error = type ? PyObject_CallFunction(type, "is", code, what) : nullptr;
+    if (error) PyErr_SetObject(type, error);
+    Py_XDECREF(error);
+    Py_XDECREF(type);
+    Py_XDECREF(lib);
+    return nullptr;
+}
+
+// Runs call(), named `what`, and, if asked to, waits for it without holding the interpreter.
+template <class Call>
+PyObject *run(bool sync, hipStream_t s, const char *what, Call &&call)
+{
+    if (sync && cuvdia_wait_begin() != CUVDIA_OK) return no();
+    const int rc = call();
+    int waited = CUVDIA_OK;
+    if (sync) {
+        Py_BEGIN_ALLOW_THREADS
+        waited = cuvdia_wait_end(s);
+        Py_END_ALLOW_THREADS
+    }
+    if (rc != CUVDIA_OK) return raise(rc, what);
+    if (waited != CUVDIA_OK) return raise(waited, "cuvdia_wait_end");
+    Py_RETURN_TRUE;
 }
 
 // 'n' or 't' from a one-character string, 0 otherwise
@@ -122,8 +143,6 @@ bool number(PyObject *o, float &v)
     if (PyErr_Occurred()) { PyErr_Clear(); return false; }
     return true;
 }
-
-PyObject *no() { Py_RETURN_FALSE; }
 
 // product(dst, A, B, transA, factAB, factC, bias, act, seed, sync)
 PyObject *product(PyObject *, PyObject *const *a, Py_ssize_t n)
@@ -148,9 +167,9 @@ PyObject *product(PyObject *, PyObject *const *a, Py_ssize_t n)
     const bool sync = PyObject_IsTrue(a[9]) == 1;
     hipStream_t s;
     if (!stream_of(dst.device, sync, s)) return no();
-    return PyBool_FromLong(run(sync, s, [&] {
+    return run(sync, s, "cuvdia_spmm_layer_f32", [&] {
         return cuvdia_spmm_layer_f32(A.desc, A.vals, B.p, B.ld, dst.p, dst.ld, (int)B.batch, trans, alpha, beta, bias, act, seed, s);
-    }));
+    });
 }
 
 // projection(C, A, B, factAB, factC, sync)
@@ -164,9 +183,9 @@ PyObject *projection(PyObject *, PyObject *const *a, Py_ssize_t n)
     const bool sync = PyObject_IsTrue(a[5]) == 1;
     hipStream_t s;
     if (!stream_of(C.device, sync, s)) return no();
-    return PyBool_FromLong(run(sync, s, [&] {
+    return run(sync, s, "cuvdia_dd2dia_f32", [&] {
         return cuvdia_dd2dia_f32(C.desc, C.vals, A.p, A.ld, B.p, B.ld, (int)A.batch, alpha, beta, s);
-    }));
+    });
 }
 
 // weight_step(w, m or None, dw, learnrate, momentum_weight, decay, sync): the value vectors themselves
@@ -186,10 +205,10 @@ PyObject *weight_step(PyObject *, PyObject *const *a, Py_ssize_t n)
     if (!stream_of(device, sync, s)) return no();
     float *wp = static_cast<float *>(w->data_ptr());
     const float *dp = static_cast<const float *>(d->data_ptr());
-    return PyBool_FromLong(run(sync, s, [&] {
+    return run(sync, s, m ? "cuvdia_learn_step_weight_decay_momentum_f32" : "cuvdia_learn_step_weight_decay_f32", [&] {
         return m ? cuvdia_learn_step_weight_decay_momentum_f32(wp, static_cast<float *>(m->data_ptr()), dp, count, lr, mw, decay, s)
                  : cuvdia_learn_step_weight_decay_f32(wp, dp, count, lr, decay, s);
-    }));
+    });
 }
 
 PyMethodDef g_methods[] = {

@@ -3,6 +3,44 @@
 import _fake_hip
 
 
+CALLS = """
+A, G = matrix(64, 64, [-1, 0, 1]), matrix(64, 64, [-1, 0, 1])
+x, y, w, m, d = tensor(4, 64), tensor(4, 64), tensor(100), tensor(100), tensor(100)
+CALLS = [lambda sync: D.prod(y, A, x, "n", "n", 1.0, 0.5, sync=sync),
+         lambda sync: D.prod_bias_act(y, A, x, "n", 1.0, 0.5, act=1, sync=sync),
+         lambda sync: D.densedense_to_dia(G, None, x, y, 1.0, 1.0, sync=sync),
+         lambda sync: D.learn_step_weight_decay(w, d, 0.1, sync=sync),
+         lambda sync: D.learn_step_weight_decay_momentum(w, m, d, 0.1, sync=sync)]
+for call in CALLS:
+    call(True)
+    call(False)
+assert flag("fake_launches") == 10
+"""
+
+
+def test_a_call_that_fails_after_its_launch_is_raised_and_not_done_again(tmp_path):
+    _fake_hip.run(tmp_path, CALLS + """
+general = []
+real, _lib.lib = _lib.lib, lambda: general.append(1) or real()
+for fail in ("fake_fail_wait", "fake_fail_launch"):
+    for k, call in enumerate(CALLS):
+        for sync in (True, False):
+            if fail == "fake_fail_wait" and not sync: continue
+            before = flag("fake_launches")
+            flag(fail, 1)
+            try:
+                call(sync)
+                raise SystemExit("no error: %s of call %d" % (fail, k))
+            except _lib.CuvDiaError as e:
+                assert e.code == _lib.EHIP and "a failure asked for" in str(e), e
+            finally:
+                flag(fail, 0)
+            assert flag("fake_launches") == before + 1, (fail, k, sync)
+            call(sync)                                   # and the next call is an ordinary one
+            assert flag("fake_launches") == before + 2
+""")
+
+
 def test_a_wait_that_cannot_begin_leaves_the_call_undone(tmp_path):
     _fake_hip.run(tmp_path, """
 A, x, y = matrix(64, 64, [-1, 0, 1]), tensor(4, 64), tensor(4, 64)
