@@ -4,7 +4,7 @@
 // the stream, argument conversion --, more than the kernels of a small layer take.  Here the same steps read the
 // tensors' fields directly (under 1 us).  Every function returns True when it has done the call, and False -- having
 // done nothing -- for operands that are not the usual ones (wrong shapes or types, another device, a matrix without
-// a descriptor yet, a capturing stream): dia.py then takes its general way, which also words the errors.  Once the
+// a descriptor yet, a capturing stream, a tensor without memory of its own): dia.py then takes its general way, which also words the errors.  Once the
 // library has been called a failure is raised, as _lib.CuvDiaError: kernels may be queued, and the general way would
 // do the call a second time.
 #define PY_SSIZE_T_CLEAN
@@ -13,6 +13,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include "cuvdia.h"
 
@@ -33,7 +34,7 @@ bool float_tensor(PyObject *o, const at::Tensor *&t)
 {
     if (!THPVariable_Check(o)) return false;
     t = &THPVariable_Unpack(o);
-    return t->is_cuda() && t->scalar_type() == at::kFloat && t->layout() == at::kStrided;
+    return t->has_storage() && t->is_cuda() && t->scalar_type() == at::kFloat && t->layout() == at::kStrided;
 }
 
 bool dense(PyObject *o, Dense &d)
@@ -45,7 +46,7 @@ bool dense(PyObject *o, Dense &d)
     d.ld = d.batch > 1 ? t->stride(0) : d.rows;
     d.device = t->get_device();
     d.p = static_cast<float *>(t->data_ptr());
-    return d.batch > 0 && d.batch <= 0x7fffffff && d.rows > 0 && d.ld >= d.rows;
+    return d.p && d.batch > 0 && d.batch <= 0x7fffffff && d.rows > 0 && d.ld >= d.rows;
 }
 
 struct Matrix {
@@ -71,16 +72,13 @@ bool matrix(PyObject *o, Matrix &m)
     long long desc = 0;
     if (!read_int(o, g_names.desc, desc) || desc == 0 || !read_int(o, g_names.h, m.h) || !read_int(o, g_names.w, m.w)) return false;
     m.desc = reinterpret_cast<const cuvdia_desc *>(desc);
-    PyObject *vec = PyObject_GetAttr(o, g_names.vec);
+    THPObjectPtr vec(PyObject_GetAttr(o, g_names.vec));      // (the matrix holds it)
     if (!vec) { PyErr_Clear(); return false; }
     const at::Tensor *t;
-    const bool ok = float_tensor(vec, t);
-    if (ok) {
-        m.vals = static_cast<float *>(t->data_ptr());
-        m.device = t->get_device();
-    }
-    Py_DECREF(vec);                                  // (the matrix holds it)
-    return ok;
+    if (!float_tensor(vec.get(), t)) return false;
+    m.vals = static_cast<float *>(t->data_ptr());
+    m.device = t->get_device();
+    return m.vals != nullptr;
 }
 
 // The stream to launch on; false when `device` is not the current one or -- for a call that waits -- is being captured.
@@ -159,6 +157,7 @@ PyObject *product(PyObject *, PyObject *const *a, Py_ssize_t n)
         const at::Tensor *t;
         if (!float_tensor(a[6], t) || !t->is_contiguous() || t->numel() != n_out || t->get_device() != dst.device) return no();
         bias = static_cast<const float *>(t->data_ptr());
+        if (!bias) return no();
     }
     if (!PyLong_CheckExact(a[7]) || !PyLong_CheckExact(a[8])) return no();
     const int act = (int)PyLong_AsLong(a[7]);
@@ -205,17 +204,34 @@ PyObject *weight_step(PyObject *, PyObject *const *a, Py_ssize_t n)
     if (!stream_of(device, sync, s)) return no();
     float *wp = static_cast<float *>(w->data_ptr());
     const float *dp = static_cast<const float *>(d->data_ptr());
-    return run(sync, s, m ? "cuvdia_learn_step_weight_decay_momentum_f32" : "cuvdia_learn_step_weight_decay_f32", [&] {
-        return m ? cuvdia_learn_step_weight_decay_momentum_f32(wp, static_cast<float *>(m->data_ptr()), dp, count, lr, mw, decay, s)
+    float *mp = m ? static_cast<float *>(m->data_ptr()) : nullptr;
+    if (!wp || !dp || (m && !mp)) return no();
+    return run(sync, s, mp ? "cuvdia_learn_step_weight_decay_momentum_f32" : "cuvdia_learn_step_weight_decay_f32", [&] {
+        return mp ? cuvdia_learn_step_weight_decay_momentum_f32(wp, mp, dp, count, lr, mw, decay, s)
                  : cuvdia_learn_step_weight_decay_f32(wp, dp, count, lr, decay, s);
     });
 }
 
-PyMethodDef g_methods[] = {
-    {"product", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(product)), METH_FASTCALL, nullptr},
-    {"projection", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(projection)), METH_FASTCALL, nullptr},
-    {"weight_step", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(weight_step)), METH_FASTCALL, nullptr},
-    {nullptr, nullptr, 0, nullptr}};
+// The functions as Python calls them.  Reading a tensor's fields throws where there are none to read (a wrapper seen
+// inside a transform, a fake tensor); the library's own calls, which come last, do not throw.
+template <PyObject *(*Function)(PyObject *, PyObject *const *, Py_ssize_t)>
+PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t n)
+{
+    try {
+        return Function(self, a, n);
+    } catch (const std::exception &) {
+        PyErr_Clear();
+        return no();
+    }
+}
+
+template <PyObject *(*Function)(PyObject *, PyObject *const *, Py_ssize_t)>
+PyMethodDef method(const char *name)
+{
+    return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<Function>)), METH_FASTCALL, nullptr};
+}
+PyMethodDef g_methods[] = {method<product>("product"), method<projection>("projection"), method<weight_step>("weight_step"),
+                           {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", "Direct calls into libcuvdia.so.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -72,3 +72,42 @@ assert wait_begin() == 0
 second = event()
 assert second and second != first and wait_end(None) == 0 and flag("fake_waited_event", kind=ctypes.c_void_p) == second
 """)
+
+
+def test_tensors_without_memory_are_left_to_the_general_way(tmp_path):
+    """Wrappers that torch hands out inside a transform, and fake tensors: a Python exception, as the general way words it."""
+    _fake_hip.run(tmp_path, """
+import torch._subclasses.fake_tensor as ft
+ft.init_gpu_context = lambda *a: None
+A, x, v = matrix(64, 64, [-1, 0, 1]), tensor(4, 64), tensor(100)
+with ft.FakeTensorMode():
+    fake, fake_v = torch.empty(4, 64, device="cuda:0"), torch.empty(100, device="cuda:0")
+assert fake.is_cuda
+N = D._native
+def calls(t, u):
+    return [(lambda: N.product(t, A, x, "n", 1.0, 0.0, None, 0, 0, True), lambda: D.prod(t, A, x)),
+            (lambda: N.product(x, A, t, "n", 1.0, 0.0, None, 0, 0, True), lambda: D.prod(x, A, t)),
+            (lambda: N.product(x, A, x, "n", 1.0, 0.0, u[:64], 0, 0, True), lambda: D.prod_bias_act(x, A, x, bias=u[:64])),
+            (lambda: N.projection(A, t, x, 1.0, 0.0, True), lambda: D.densedense_to_dia(A, None, t, x)),
+            (lambda: N.projection(A, x, t, 1.0, 0.0, True), lambda: D.densedense_to_dia(A, None, x, t)),
+            (lambda: N.weight_step(u, None, v, 0.1, 0.0, 0.0, True), lambda: D.learn_step_weight_decay(u, v, 0.1)),
+            (lambda: N.weight_step(v, u, v, 0.1, 0.9, 0.0, True), lambda: D.learn_step_weight_decay_momentum(v, u, v, 0.1)),
+            (lambda: N.weight_step(v, None, u, 0.1, 0.0, 0.0, True), lambda: D.learn_step_weight_decay(v, u, 0.1))]
+assert not any(direct() for direct, _ in calls(fake, fake_v))
+def check(t, u):
+    for k, (direct, whole) in enumerate(calls(t, u)):
+        assert direct() is False
+        try:
+            whole()
+            raise SystemExit("no error: call %d" % k)
+        except (RuntimeError, TypeError):
+            pass
+    return torch.zeros(1)
+torch.func.vmap(check)(tensor(3, 4, 64), tensor(3, 100))
+torch.func.functionalize(lambda t, u: any(direct() for direct, _ in calls(t, u)) and 1 / 0)(x, v)
+class Holder: pass
+h = Holder()                                             # a matrix whose values are such a tensor
+h.h, h.w, h._desc_ptr, h.vec = 64, 64, A._desc_ptr, fake_v
+assert N.product(x, h, x, "n", 1.0, 0.0, None, 0, 0, True) is False and N.projection(h, x, x, 1.0, 0.0, True) is False
+assert flag("fake_launches") == 0
+""")
