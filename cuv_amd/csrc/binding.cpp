@@ -109,18 +109,17 @@ PyObject *raise(int code, const char *what)
     return nullptr;
 }
 
-// Runs call(), named `what`, and, if asked to, waits for it without holding the interpreter.
+// Runs call(), named `what`, and, if asked to, waits for it, both without holding the interpreter: a launch, too, blocks
+// where the stream's queue is full.
 template <class Call>
 PyObject *run(bool sync, hipStream_t s, const char *what, Call &&call)
 {
     if (sync && cuvdia_wait_begin() != CUVDIA_OK) return no();
-    const int rc = call();
-    int waited = CUVDIA_OK;
-    if (sync) {
-        Py_BEGIN_ALLOW_THREADS
-        waited = cuvdia_wait_end(s);
-        Py_END_ALLOW_THREADS
-    }
+    int rc = CUVDIA_OK, waited = CUVDIA_OK;
+    Py_BEGIN_ALLOW_THREADS
+    rc = call();
+    if (sync) waited = cuvdia_wait_end(s);
+    Py_END_ALLOW_THREADS
     if (rc != CUVDIA_OK) return raise(rc, what);
     if (waited != CUVDIA_OK) return raise(waited, "cuvdia_wait_end");
     Py_RETURN_TRUE;

@@ -111,3 +111,17 @@ h.h, h.w, h._desc_ptr, h.vec = 64, 64, A._desc_ptr, fake_v
 assert N.product(x, h, x, "n", 1.0, 0.0, None, 0, 0, True) is False and N.projection(h, x, x, 1.0, 0.0, True) is False
 assert flag("fake_launches") == 0
 """)
+
+
+def test_other_threads_run_during_launches_and_waits(tmp_path):
+    _fake_hip.run(tmp_path, CALLS + """
+import threading, time
+for call in CALLS:
+    for sync in (True, False):
+        flag("fake_hold_launch", 1)                      # the call stays in its launch until the other thread lets it go on
+        other = threading.Thread(target=lambda: (time.sleep(0.02), flag("fake_hold_launch", 0)))
+        other.start()
+        call(sync)
+        other.join()
+assert flag("fake_held") == 0
+""")
