@@ -81,15 +81,23 @@ bool matrix(PyObject *o, Matrix &m)
     return m.vals != nullptr;
 }
 
-// The stream to launch on; false when `device` is not the current one or -- for a call that waits -- is being captured.
+// Whether a runtime call succeeded; takes its error from the runtime, where the general way's launch would find it.
+bool ok(hipError_t e)
+{
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
+// The stream to launch on; false when `device` is not the current one or -- for a call that waits -- is being captured
+// (or cannot be asked: the default stream while another thread captures).
 bool stream_of(int device, bool sync, hipStream_t &s)
 {
     int current = -1;
-    if (hipGetDevice(&current) != hipSuccess || current != device) return false;
+    if (!ok(hipGetDevice(&current)) || current != device) return false;
     s = c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream();
     if (sync) {
         hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return false;
+        if (!ok(hipStreamIsCapturing(s, &status)) || status != hipStreamCaptureStatusNone) return false;
     }
     return true;
 }

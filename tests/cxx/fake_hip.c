@@ -11,7 +11,7 @@ typedef struct { uint32_t x, y, z; } dim3_;
 
 int fake_device = 0, fake_devices = 2;
 int fake_launches = 0;                   /* kernels launched so far */
-int fake_fail_launch = 0, fake_fail_event_create = 0, fake_fail_wait = 0;
+int fake_fail_launch = 0, fake_fail_event_create = 0, fake_fail_wait = 0, fake_fail_capturing = 0;
 void *fake_last_event = NULL;            /* the event of the last launch, and ... */
 void *fake_waited_event = NULL;          /* ... the one waited for last */
 volatile int fake_hold_launch = 0;       /* launches and waits stay in their call until it is 0, at most 10 s */
@@ -43,7 +43,7 @@ int hipEventCreateWithFlags(void **e, unsigned flags)
 int hipEventDestroy(void *e) { free(e); return SUCCESS; }
 int hipEventSynchronize(void *e) { hold(); fake_waited_event = e; return result(fake_fail_wait || !e); }
 int hipStreamSynchronize(void *s) { hold(); return result(fake_fail_wait); }
-int hipStreamIsCapturing(void *s, int *status) { *status = 0; return SUCCESS; }
+int hipStreamIsCapturing(void *s, int *status) { *status = 0; return result(fake_fail_capturing); }
 int hipExtLaunchKernel(const void *f, dim3_ grid, dim3_ block, void **args, size_t lds, void *stream, void *start, void *stop, int flags)
 {
     hold();

@@ -48,6 +48,10 @@ flag("fake_fail_event_create", 1)
 assert D._native.product(y, A, x, "n", 1.0, 0.0, None, 0, 0, True) is False and flag("fake_launches") == 0
 flag("fake_fail_event_create", 0)
 assert D._native.product(y, A, x, "n", 1.0, 0.0, None, 0, 0, True) is True and flag("fake_launches") == 1
+flag("fake_fail_capturing", 1)                           # the stream cannot be asked whether it is being captured
+assert D._native.product(y, A, x, "n", 1.0, 0.0, None, 0, 0, True) is False and flag("fake_launches") == 1
+flag("fake_fail_capturing", 0)
+assert D._native.product(y, A, x, "n", 1.0, 0.0, None, 0, 0, True) is True and flag("fake_launches") == 2
 """)
 
 
