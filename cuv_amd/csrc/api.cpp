@@ -55,6 +55,37 @@ SpFamily spmm_family(const DiaView &A, long long ldb, long long ldd, int batch, 
     if (spmm_thin_ok(A, trans) && (batch < SPMM_TILED_MIN_BATCH || !tiled_possible)) return SpFamily::thin;
     return tiled_possible && (batch >= SPMM_TILED_MIN_BATCH || forced == CUVDIA_PATH_TILED) ? SpFamily::tiled : SpFamily::generic;
 }
+
+// How a projection is served: what cuvdia_dd2dia_f32 runs and cuvdia_plan_window_launch tells.
+struct DdChoice {
+    bool tiled;          // the kernels that stage operands can address them, `slab` columns at a time
+    int slab;
+    bool rows;           // the automatic choice: the kernel with rows along the lanes; ...
+    long long window;    // ... if not, workgroups of a slab's window-table projection, 0: another kernel
+};
+// `aligned`: A fits 16-byte pieces, as the kernels that share staged operands load it.
+DdChoice dd2dia_choose(const DiaView &C, long long lda, long long ldb, int batch, bool aligned)
+{
+    DdChoice d{dd2dia_tiled_ok(C, lda, ldb, batch), batch, false, 0};
+    if (batch < 1) return d;
+    // The staging kernels address their operands with 32-bit byte offsets.  A batch whose operands are larger is
+    // walked in slabs of columns that fit.
+    if (!d.tiled && batch > DD2DIA_SLAB_MIN) {
+        const int fit = dd2dia_slab_columns(C, lda, ldb);
+        if (fit >= DD2DIA_SLAB_MIN && dd2dia_tiled_ok(C, lda, ldb, fit)) {
+            // slabs of about equal width rather than full ones and a sliver
+            const int count = (batch + fit - 1) / fit;
+            const int even = ((batch + count - 1) / count + DD2DIA_SLAB_MIN - 1) / DD2DIA_SLAB_MIN * DD2DIA_SLAB_MIN;
+            d.slab = std::min(fit, even);
+            d.tiled = true;
+        }
+    }
+    if (d.tiled) d.window = dd2dia_window_grid(C, lda, ldb, d.slab, false);
+    d.rows = dd2dia_rows_ok(C) && (!d.tiled || dd2dia_rows_by_size(C, batch, aligned, d.window > 0));
+    if (d.rows) d.window = 0;
+    return d;
+}
+
 // Largest h, w and |offset| the kernels' 32-bit row arithmetic allows.
 constexpr long long DIM_LIMIT = 1LL << 30;
 
@@ -320,9 +351,7 @@ long long cuvdia_plan_window_launch(const int *offsets_host, int nd, int stride,
     for (int r : wp.group_rows) rows4 = rows4 && r % 4 == 0;
     view.h = h; view.w = w; view.nd = nd; view.stride = stride; view.rf = 1;
     view.walk_n = WalkView{&not_null, wp.ngroups, wp.period, wp.s0, wp.k, wp.lck, wp.astep4, rows4, wp.group_rows.data()};
-    if (!dd2dia_tiled_ok(view, h, w, batch)) return 0;
-    const long long workgroups = dd2dia_window_workgroups(view, batch);
-    return workgroups > 0 && dd2dia_window_by_size(view, batch, workgroups) ? workgroups : 0;
+    return dd2dia_choose(view, h, w, batch, h % 4 == 0).window;
 }
 
 int cuvdia_plan_units(const int *offsets_host, int nd, int *c1, int *c2, int cap)
@@ -583,31 +612,11 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     if (const int rc = check_device(desc)) return rc;
 
     const int forced = g_path.load();
-    // The tiled kernel addresses its operands with 32-bit byte offsets.  A batch whose operands are larger is
-    // walked in slabs of columns that fit: the sum over the batch is the sum of the slabs' sums, so the first slab
-    // runs with the caller's beta and every later one adds to what is there (beta = 1), one launch after the other
-    // on the caller's stream.
-    int slab = batch;
-    bool tiled_possible = dd2dia_tiled_ok(desc->view, lda, ldb, batch);
-    if (!tiled_possible && batch > DD2DIA_SLAB_MIN) {
-        const int fit = dd2dia_slab_columns(desc->view, lda, ldb);
-        if (fit >= DD2DIA_SLAB_MIN && dd2dia_tiled_ok(desc->view, lda, ldb, fit)) {
-            // slabs of about equal width rather than full ones and a sliver
-            const int count = (batch + fit - 1) / fit;
-            const int even = ((batch + count - 1) / count + DD2DIA_SLAB_MIN - 1) / DD2DIA_SLAB_MIN * DD2DIA_SLAB_MIN;
-            slab = std::min(fit, even);
-            tiled_possible = true;
-        }
-    }
+    const bool aligned = reinterpret_cast<std::uintptr_t>(A) % 16 == 0 && lda % 4 == 0 && desc->h % 4 == 0;
+    const DdChoice choice = dd2dia_choose(desc->view, lda, ldb, batch, aligned);
+    const bool tiled_possible = choice.tiled;
+    const bool rows = choice.rows && (forced == CUVDIA_PATH_AUTO || forced == CUVDIA_PATH_TILED);
     bool tiled;
-    bool rows = false;               // of the tiled family: the kernel with rows along the lanes
-    if (batch > 0 && dd2dia_rows_ok(desc->view) && (forced == CUVDIA_PATH_AUTO || forced == CUVDIA_PATH_TILED)) {
-        // (16-byte pieces of A, as the kernels that share staged operands load them)
-        const bool aligned = reinterpret_cast<std::uintptr_t>(A) % 16 == 0 && lda % 4 == 0 && desc->h % 4 == 0;
-        const long long wgs = dd2dia_window_workgroups(desc->view, slab);
-        const bool by_window = wgs > 0 && dd2dia_window_by_size(desc->view, slab, wgs);
-        rows = !tiled_possible || dd2dia_rows_by_size(desc->view, batch, aligned, by_window);
-    }
     if (rows) {
         tiled = true;
     } else if (forced == CUVDIA_PATH_TILED || forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK ||
@@ -629,10 +638,12 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     } else {
         const int window = forced == CUVDIA_PATH_WINDOW ? 1 : forced == CUVDIA_PATH_PLANE ? -2
                            : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK) ? -1 : 0;
-        for (int c0 = 0; c0 < batch && e == hipSuccess; c0 += slab) {
+        // The sum over the batch is the sum of the slabs' sums: the first slab runs with the caller's beta and every
+        // later one adds to what is there (beta = 1), one launch after the other on the caller's stream.
+        for (int c0 = 0; c0 < batch && e == hipSuccess; c0 += choice.slab) {
             int this_one = CUVDIA_PATH_TILED;
             e = launch_dd2dia_tiled(desc->view, C_vals, A + (long long)c0 * lda, lda, B + (long long)c0 * ldb, ldb,
-                                    std::min(slab, batch - c0), alpha, c0 == 0 ? beta : 1.f, s, window, &this_one);
+                                    std::min(choice.slab, batch - c0), alpha, c0 == 0 ? beta : 1.f, s, window, &this_one);
             if (this_one != CUVDIA_PATH_TILED) ran = this_one;
         }
         if (window > 0 && e == hipErrorNotSupported) {

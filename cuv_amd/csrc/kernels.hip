@@ -3237,9 +3237,9 @@ int dd2dia_slab_columns(const DiaView &C, long long lda, long long ldb)
 }
 
 // Workgroups of the window-table projection on these operands, 0 where it does not apply: no window table,
-// chunks longer than CHUNK_MAX or shorter than 2, a period, group rows or row counts that are no multiples of 4
+// chunks longer than SP_CHUNK_MAX or shorter than 2, a period, group rows or row counts that are no multiples of 4
 // (its 16-byte pieces then straddle the operands' ends).
-long long dd2dia_window_workgroups(const DiaView &C, int batch, int *txn, int *tyn, int *ndb)
+static long long dd2dia_window_workgroups(const DiaView &C, int batch, int *txn, int *tyn, int *ndb)
 {
     const WalkView &wk = C.walk_n;
     if (wk.tab_dev == nullptr || wk.lck < 2 || wk.lck > SP_CHUNK_MAX || !wk.rows4 || wk.period % 4 != 0 ||
@@ -3261,7 +3261,7 @@ long long dd2dia_window_workgroups(const DiaView &C, int batch, int *txn, int *t
 // of the batch per tile to get there.  The smaller the window, the less a tile saves over the chunk-by-chunk
 // kernel and the more tiles it takes (measured on 7 x 7, 5 x 5 and 3 x 3 windows of maps 256 to 1024 wide at
 // batch 32 to 512: ahead from 768, 1024 and 1536 tiles on, the 3 x 3 only from batch 128).
-int dd2dia_window_subs(const DiaView &C, long long workgroups)
+static int dd2dia_window_subs(const DiaView &C, long long workgroups)
 {
     const int slots = C.walk_n.k * C.walk_n.lck;
     const long long min_wgs = slots >= 49 ? DW_MIN_WGS : slots >= 25 ? DW_MIN_WGS * 4 / 3 : DW_MIN_WGS * 2;
@@ -3273,7 +3273,7 @@ int dd2dia_window_subs(const DiaView &C, long long workgroups)
 // slots or more, and two ranges only from batch 512 on: a 7 x 7 window on a 256-wide map (256 tiles, 4 ranges)
 // measured 1.2 - 1.5 times the chunk-by-chunk kernel's rate at batch 32 to 2048, on 320- and 384-wide maps (400 and
 // 576 tiles, 2 ranges) 1.1 - 1.6 times from batch 512 and 0.86 - 0.98 below; 5 x 5 windows on those maps 0.6 - 1.0.
-bool dd2dia_window_by_size(const DiaView &C, int batch, long long workgroups)
+static bool dd2dia_window_by_size(const DiaView &C, int batch, long long workgroups)
 {
     const int slots = C.walk_n.k * C.walk_n.lck;
     const long long min_wgs = slots >= 49 ? DW_MIN_WGS : slots >= 25 ? DW_MIN_WGS * 4 / 3 : DW_MIN_WGS * 2;
@@ -3296,6 +3296,14 @@ bool dd2dia_window_by_size(const DiaView &C, int batch, long long workgroups)
     return slots >= 49 && batch >= (subs == 2 ? 512 : 32);
 }
 
+long long dd2dia_window_grid(const DiaView &C, long long lda, long long ldb, int batch, bool forced, int *txn, int *tyn, int *ndb)
+{
+    // (a lane's byte offsets run up to 16 columns past the batch and must stay below 2^32)
+    if (((long long)batch + 16) * std::max(lda, ldb) * 4 >= (1LL << 32)) return 0;
+    const long long wgs = dd2dia_window_workgroups(C, batch, txn, tyn, ndb);
+    return wgs > 0 && (forced || dd2dia_window_by_size(C, batch, wgs)) ? wgs : 0;
+}
+
 hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, long long lda,
                                const float *B, long long ldb, int batch,
                                float alpha, float beta, hipStream_t stream, int window, int *ran)
@@ -3310,10 +3318,8 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
         if (const hipError_t e = plane(true); e != hipErrorNotSupported) return e;
     if (window >= 0) {
         int txn = 0, tyn = 0, ndb = 0;
-        long long wgs = dd2dia_window_workgroups(C, batch, &txn, &tyn, &ndb);
-        // (a lane's byte offsets run up to 16 columns past the batch and must stay below 2^32)
-        if (((long long)batch + 16) * std::max(lda, ldb) * 4 >= (1LL << 32)) wgs = 0;
-        if (wgs > 0 && (window > 0 || dd2dia_window_by_size(C, batch, wgs))) {
+        const long long wgs = dd2dia_window_grid(C, lda, ldb, batch, window > 0, &txn, &tyn, &ndb);
+        if (wgs > 0) {
             if (window == 0)
                 if (const hipError_t e = plane(false); e != hipErrorNotSupported) return e;
             const WalkView &wk = C.walk_n;

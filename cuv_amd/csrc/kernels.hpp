@@ -193,12 +193,10 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
 // 16-byte pieces do not fit, or (not force) a launch on which it would not be ahead of the window-table projection.
 hipError_t launch_dd2dia_plane(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
                                int batch, float alpha, float beta, hipStream_t stream, bool force);
-// Workgroups of the window-table projection for these operands (0: it does not apply).
-long long dd2dia_window_workgroups(const DiaView &C, int batch, int *txn = nullptr, int *tyn = nullptr, int *ndb = nullptr);
-// Whether the automatic choice takes that kernel for a launch of so many workgroups.
-bool dd2dia_window_by_size(const DiaView &C, int batch, long long workgroups);
-// Batch ranges per workgroup (1, 2 or 4) of such a launch.
-int dd2dia_window_subs(const DiaView &C, long long workgroups);
+// Workgroups of the window-table projection on these operands, 0 where it does not serve them or -- unless forced --
+// the automatic choice among the kernels that stage operands does not take it.
+long long dd2dia_window_grid(const DiaView &C, long long lda, long long ldb, int batch, bool forced,
+                             int *txn = nullptr, int *tyn = nullptr, int *ndb = nullptr);
 
 // The allocation-free entry point keeps its device tables in a static device
 // array instead of a descriptor's allocation: the offset table at byte 0 (up

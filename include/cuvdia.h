@@ -119,14 +119,17 @@ int cuvdia_plan_units(const int *offsets_host, int nd, int *c1, int *c2, int cap
 
 /* Pure host function: does the automatic choice of cuvdia_dd2dia_f32 run the
  * kernel tiled in the window's plane for an h x w matrix with this table
- * (row_fact 1) and `batch` packed dense columns?  Returns the number of
- * workgroups of that launch (tiles of 4 x 64 positions x blocks of 8 window
+ * (row_fact 1) and `batch` packed dense columns on 16-byte boundaries?
+ * Returns the number of workgroups of that launch -- of each launch, where
+ * operands above 2 GiB take several -- (tiles of 4 x 64 positions x blocks of 8 window
  * rows -- of 7 where a window row has 9 to 13 diagonals, or of 5 where that
  * leaves fewer rows of the last block empty and the staging buffers of three
- * workgroups fit a CU's LDS -- x channel groups), or 0 when the chunk-by-chunk kernel serves: the table is no
+ * workgroups fit a CU's LDS -- x channel groups), or 0 when another kernel serves: the table is no
  * window table (see cuvdia_plan_walk) of chunks of 2 to 13 diagonals, the
  * period, a channel distance or a row count is no multiple of 4, the period
- * is below 64, or the launch has too few workgroups to fill the chip.  For
+ * is below 64, the batch at most 8 on a period that is no multiple of 64 (the
+ * kernel with rows along the lanes), or the launch has too few workgroups to
+ * fill the chip.  For
  * chunks of up to 8 diagonals: 768 for windows of 49 slots or more -- or 384
  * at a batch of at least 512, or 192 at a batch of at least 32: a workgroup
  * then works two or four ranges of the batch side by side --, 1024 from 25

@@ -12,6 +12,7 @@ typedef struct { uint32_t x, y, z; } dim3_;
 int fake_device = 0, fake_devices = 2;
 int fake_launches = 0;                   /* kernels launched so far */
 int fake_fail_launch = 0, fake_fail_event_create = 0, fake_fail_wait = 0, fake_fail_capturing = 0;
+int fake_grid = 0;                       /* workgroups of the last launch */
 void *fake_last_event = NULL;            /* the event of the last launch, and ... */
 void *fake_waited_event = NULL;          /* ... the one waited for last */
 volatile int fake_hold_launch = 0;       /* launches and waits stay in their call until it is 0, at most 10 s */
@@ -48,6 +49,7 @@ int hipExtLaunchKernel(const void *f, dim3_ grid, dim3_ block, void **args, size
 {
     hold();
     ++fake_launches;
+    fake_grid = grid.x;
     fake_last_event = stop;
     return result(fake_fail_launch);
 }
@@ -55,13 +57,15 @@ int hipLaunchKernel(const void *f, dim3_ grid, dim3_ block, void **args, size_t 
 {
     return hipExtLaunchKernel(f, grid, block, args, lds, stream, NULL, NULL, 0);
 }
-int __hipPushCallConfiguration(dim3_ grid, dim3_ block, size_t lds, void *stream) { return SUCCESS; }
+static __thread struct { dim3_ grid, block; size_t lds; void *stream; } s_config;
+int __hipPushCallConfiguration(dim3_ grid, dim3_ block, size_t lds, void *stream)
+{
+    s_config.grid = grid, s_config.block = block, s_config.lds = lds, s_config.stream = stream;
+    return SUCCESS;
+}
 int __hipPopCallConfiguration(dim3_ *grid, dim3_ *block, size_t *lds, void **stream)
 {
-    memset(grid, 0, sizeof *grid);
-    memset(block, 0, sizeof *block);
-    *lds = 0;
-    *stream = NULL;
+    *grid = s_config.grid, *block = s_config.block, *lds = s_config.lds, *stream = s_config.stream;
     return SUCCESS;
 }
 

@@ -129,3 +129,28 @@ for call in CALLS:
         other.join()
 assert flag("fake_held") == 0
 """)
+
+
+def test_the_planned_window_projection_is_the_one_that_runs(tmp_path):
+    """cuvdia_plan_window_launch against what a call on packed operands takes, over maps, windows and batches on both sides
+    of its rules, operands above 2 GiB among them."""
+    _fake_hip.run(tmp_path, """
+import random
+rng, seen = random.Random(2), set()
+cases = [(500, 500, 7, 1, 1, b) for b in (4, 8, 9)] + [(512, 512, 7, 1, 1, 4), (1024, 1024, 5, 1, 1, 700), (1000, 1000, 5, 1, 1, 700)]
+for _ in range(400):
+    px = rng.choice([rng.randint(15, 160) * 4, rng.randint(1, 10) * 64, rng.randint(60, 640)])
+    maps = rng.choice([(1, 1), (1, 1), (2, 2), (1, 4)])
+    cases.append((px, rng.randint(16, 600), rng.choice([3, 5, 7, 8, 9, 10, 11, 13]), *maps, rng.choice([rng.randint(1, 12), rng.randint(13, 700)])))
+for px, py, fs, maps_in, maps_out, batch in cases:
+    h, w = px * py * maps_in, px * py * maps_out
+    C = matrix(h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+    plan = L.cuvdia_plan_window_launch(C._offsets.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), C.num_dia, C.stride, h, w, batch)
+    D.densedense_to_dia(C, None, tensor(batch, h, bytes_at=1 << 41), tensor(batch, w, bytes_at=1 << 42), 1.0, 0.0)
+    ran = L.cuvdia_last_path()
+    what = (px, py, fs, maps_in, maps_out, batch, plan, L.cuvdia_last_kernel())
+    assert (plan > 0) == (ran in (_lib.PATH_WINDOW, _lib.PATH_PLANE)), what
+    assert ran != _lib.PATH_WINDOW or plan == flag("fake_grid"), what
+    seen.add(L.cuvdia_last_kernel().split(b"<")[0])
+assert seen >= {b"dd2dia_window_kernel", b"dd2dia_window_long_kernel", b"dd2dia_rows_kernel", b"dd2dia_tiled_kernel"}, seen
+""")
