@@ -628,6 +628,10 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     } else {
         tiled = tiled_possible;
     }
+    if (batch == 0) {                // only beta is left of the update, and no operand to look at
+        tiled = false;
+        alpha = 0.f;
+    }
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
     int ran = CUVDIA_PATH_TILED;

@@ -154,3 +154,15 @@ for px, py, fs, maps_in, maps_out, batch in cases:
     seen.add(L.cuvdia_last_kernel().split(b"<")[0])
 assert seen >= {b"dd2dia_window_kernel", b"dd2dia_window_long_kernel", b"dd2dia_rows_kernel", b"dd2dia_tiled_kernel"}, seen
 """)
+
+
+def test_an_empty_batch_is_launched_for_the_projection_alone(tmp_path):
+    _fake_hip.run(tmp_path, """
+A = matrix(4096, 4096, [64 * dy + dx for dy in range(-2, 3) for dx in range(-2, 3)])
+D.prod(tensor(0, 4096, bytes_at=1 << 41), A, tensor(0, 4096, bytes_at=1 << 42))
+assert flag("fake_launches") == 0                        # a product of no columns has no result
+for path in (_lib.PATH_AUTO, _lib.PATH_TILED):
+    L.cuvdia_set_path(path)
+    D.densedense_to_dia(A, None, tensor(0, 4096, bytes_at=1 << 41), tensor(0, 4096, bytes_at=1 << 42), 1.0, 0.5)
+assert flag("fake_launches") == 2 and L.cuvdia_last_kernel() == b"dd2dia_generic_kernel"
+""")
