@@ -47,13 +47,10 @@ SpFamily spmm_family(const DiaView &A, long long ldb, long long ldd, int batch, 
 {
     if (forced == CUVDIA_PATH_GENERIC) return SpFamily::generic;
     const bool tiled_possible = spmm_tiled_ok(A, ldb, ldd, trans);
-    if (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK || forced == CUVDIA_PATH_WINDOW ||
-        forced == CUVDIA_PATH_PLANE)
-        return tiled_possible ? SpFamily::tiled : SpFamily::unsupported;
-    if (forced == CUVDIA_PATH_TILED && !tiled_possible) return SpFamily::unsupported;
     if (forced == CUVDIA_PATH_THIN) return spmm_thin_ok(A, trans) ? SpFamily::thin : SpFamily::unsupported;
-    if (spmm_thin_ok(A, trans) && (batch < SPMM_TILED_MIN_BATCH || !tiled_possible)) return SpFamily::thin;
-    return tiled_possible && (batch >= SPMM_TILED_MIN_BATCH || forced == CUVDIA_PATH_TILED) ? SpFamily::tiled : SpFamily::generic;
+    if (forced != CUVDIA_PATH_AUTO) return tiled_possible ? SpFamily::tiled : SpFamily::unsupported;
+    if (tiled_possible && batch >= SPMM_TILED_MIN_BATCH) return SpFamily::tiled;
+    return spmm_thin_ok(A, trans) ? SpFamily::thin : SpFamily::generic;
 }
 
 // How a projection is served: what cuvdia_dd2dia_f32 runs and cuvdia_plan_window_launch tells.
@@ -615,7 +612,7 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     const bool aligned = reinterpret_cast<std::uintptr_t>(A) % 16 == 0 && lda % 4 == 0 && desc->h % 4 == 0;
     const DdChoice choice = dd2dia_choose(desc->view, lda, ldb, batch, aligned);
     const bool tiled_possible = choice.tiled;
-    const bool rows = choice.rows && (forced == CUVDIA_PATH_AUTO || forced == CUVDIA_PATH_TILED);
+    const bool rows = choice.rows && (forced == CUVDIA_PATH_AUTO || forced == CUVDIA_PATH_THIN);
     bool tiled;
     if (rows) {
         tiled = true;
@@ -640,17 +637,16 @@ int cuvdia_dd2dia_f32(const cuvdia_desc *desc, float *C_vals, const float *A, lo
     } else if (!tiled) {
         e = launch_dd2dia_generic(desc->view, C_vals, A, lda, B, ldb, batch, alpha, beta, s);
     } else {
-        const int window = forced == CUVDIA_PATH_WINDOW ? 1 : forced == CUVDIA_PATH_PLANE ? -2
-                           : (forced == CUVDIA_PATH_TILED_NOWALK || forced == CUVDIA_PATH_WALK) ? -1 : 0;
+        const int path = forced == CUVDIA_PATH_THIN ? CUVDIA_PATH_AUTO : forced;
         // The sum over the batch is the sum of the slabs' sums: the first slab runs with the caller's beta and every
         // later one adds to what is there (beta = 1), one launch after the other on the caller's stream.
         for (int c0 = 0; c0 < batch && e == hipSuccess; c0 += choice.slab) {
             int this_one = CUVDIA_PATH_TILED;
             e = launch_dd2dia_tiled(desc->view, C_vals, A + (long long)c0 * lda, lda, B + (long long)c0 * ldb, ldb,
-                                    std::min(choice.slab, batch - c0), alpha, c0 == 0 ? beta : 1.f, s, window, &this_one);
+                                    std::min(choice.slab, batch - c0), alpha, c0 == 0 ? beta : 1.f, s, path, &this_one);
             if (this_one != CUVDIA_PATH_TILED) ran = this_one;
         }
-        if (window > 0 && e == hipErrorNotSupported) {
+        if (forced == CUVDIA_PATH_WINDOW && e == hipErrorNotSupported) {
             (void)hipGetLastError();
             return CUVDIA_EUNSUPPORTED;
         }

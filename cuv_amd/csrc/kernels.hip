@@ -3306,7 +3306,7 @@ long long dd2dia_window_grid(const DiaView &C, long long lda, long long ldb, int
 
 hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, long long lda,
                                const float *B, long long ldb, int batch,
-                               float alpha, float beta, hipStream_t stream, int window, int *ran)
+                               float alpha, float beta, hipStream_t stream, int path, int *ran)
 {
     if (ran) *ran = CUVDIA_PATH_TILED;
     auto plane = [&](bool force) {
@@ -3314,13 +3314,13 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
         if (e != hipErrorNotSupported && ran) *ran = CUVDIA_PATH_PLANE;
         return e;
     };
-    if (window == -2)
+    if (path == CUVDIA_PATH_PLANE)
         if (const hipError_t e = plane(true); e != hipErrorNotSupported) return e;
-    if (window >= 0) {
+    if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_TILED || path == CUVDIA_PATH_WINDOW) {
         int txn = 0, tyn = 0, ndb = 0;
-        const long long wgs = dd2dia_window_grid(C, lda, ldb, batch, window > 0, &txn, &tyn, &ndb);
+        const long long wgs = dd2dia_window_grid(C, lda, ldb, batch, path == CUVDIA_PATH_WINDOW, &txn, &tyn, &ndb);
         if (wgs > 0) {
-            if (window == 0)
+            if (path == CUVDIA_PATH_AUTO)
                 if (const hipError_t e = plane(false); e != hipErrorNotSupported) return e;
             const WalkView &wk = C.walk_n;
             const DwLaunch L{wk.tab_dev, wk.ngroups, wk.k, wk.period, wk.s0, wk.astep4 / 4, wk.lck, vals, A, lda, B, ldb,
@@ -3333,7 +3333,7 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
             return dd2dia_window_launch(L);
         }
     }
-    if (window > 0) return hipErrorNotSupported;
+    if (path == CUVDIA_PATH_WINDOW) return hipErrorNotSupported;
     // 16-byte loads of A need an aligned base and leading dimension and whole
     // groups of 4 rows; row tiles start at multiples of 256 and lanes at
     // multiples of 4 rows.

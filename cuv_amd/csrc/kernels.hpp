@@ -184,11 +184,12 @@ int dd2dia_slab_columns(const DiaView &C, long long lda, long long ldb);
 // Window tables whose tiles fill the chip go to the window-table projection (a tile of 4 x 64 positions of the
 // window's plane per workgroup, both operands staged once for all the slots of up to 8 window rows).
 // Of those, square windows of 9 and 11 rows go to the kernel on the matrix cores (below), by size.
-// `window`: 0 -- that choice is made by size; 1 -- that kernel or hipErrorNotSupported; -1 -- never; -2 -- the matrix
-// cores if they serve the table.  *ran (if not null): the path that did, CUVDIA_PATH_*.
+// path: CUVDIA_PATH_AUTO -- those choices are made by size; _TILED -- likewise, but never the matrix cores; _WINDOW --
+// the window-table projection or hipErrorNotSupported; _PLANE -- the matrix cores if they serve the table; anything
+// else: none of them.  *ran (if not null): the path that did.
 hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, long long lda,
                                const float *B, long long ldb, int batch,
-                               float alpha, float beta, hipStream_t stream, int window = 0, int *ran = nullptr);
+                               float alpha, float beta, hipStream_t stream, int path = 0, int *ran = nullptr);
 // Same contract, square windows of 9 and 11 rows (dd2dia_plane.hip); hipErrorNotSupported: another table, operands that
 // 16-byte pieces do not fit, or (not force) a launch on which it would not be ahead of the window-table projection.
 hipError_t launch_dd2dia_plane(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,

@@ -54,7 +54,7 @@ extern "C" {
 #define CUVDIA_PATH_TILED_NOWALK 4  /* the tiled family without its kernels for window tables                  */
 #define CUVDIA_PATH_WINDOW   5  /* of the tiled family: the projection tiled in the window's plane (window tables) */
 #define CUVDIA_PATH_PLANE    6  /* of the tiled family: the kernels on the matrix cores (window tables)            */
-#define CUVDIA_PATH_THIN     8  /* of the tiled family: the product with rows along the lanes                      */
+#define CUVDIA_PATH_THIN     8  /* the product with rows along the lanes (rf == 1)                                 */
 
 /* Activation applied by cuvdia_spmm_bias_act_f32. */
 #define CUVDIA_ACT_NONE      0
@@ -348,28 +348,36 @@ int cuvdia_spmm_offsets_noalloc_f32(const float *A_vals_device, const int *offse
 int cuvdia_cache_clear(void);
 
 /* Forces a kernel family for subsequent calls (process-wide; tests use it to
- * run both families on the same inputs).  CUVDIA_PATH_TILED on a request the
- * tiled kernels cannot serve (row_fact > 1) returns CUVDIA_EUNSUPPORTED from
- * the compute call.  CUVDIA_PATH_WALK, CUVDIA_PATH_PLANE, CUVDIA_PATH_WINDOW
+ * run several families on the same inputs).  CUVDIA_PATH_TILED, at any batch:
+ * the kernels that stage their operands in LDS, on the vector unit -- the
+ * walking product and the projection tiled in the window's plane by size,
+ * never the kernels with rows along the lanes; CUVDIA_EUNSUPPORTED from the
+ * compute call for a request they cannot serve (row_fact > 1, operands above
+ * 2 GiB that slabs do not help).  CUVDIA_PATH_WALK, CUVDIA_PATH_PLANE, CUVDIA_PATH_WINDOW
  * and CUVDIA_PATH_TILED_NOWALK choose inside the tiled family: a kernel for
  * window tables whatever the size of the operands, or none of them.
  * CUVDIA_PATH_WALK: the walking product (CUVDIA_EUNSUPPORTED for a table
  * that is no window table with a walking kernel; densedense_to_dia treats it
  * as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_PLANE likewise, for the product
  * walked on the matrix cores (densedense_to_dia: the projection on the matrix
- * cores for windows of 9 x 9 and 11 x 11, else as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_THIN: the product with rows along
- * the lanes at any batch (densedense_to_dia: as CUVDIA_PATH_AUTO).  CUVDIA_PATH_WINDOW: the kernels tiled in the
+ * cores for windows of 9 x 9 and 11 x 11, else as CUVDIA_PATH_TILED_NOWALK).
+ * CUVDIA_PATH_WINDOW: the kernels tiled in the
  * window's plane, which serve densedense_to_dia (CUVDIA_EUNSUPPORTED when
  * they do not serve the request: no window table of chunks of 2 to 13
  * diagonals, a period, channel distances or row counts that are no multiples
- * of 4); the products treat it as CUVDIA_PATH_TILED_NOWALK. */
+ * of 4); the products treat it as CUVDIA_PATH_TILED_NOWALK.
+ * CUVDIA_PATH_THIN: the product with rows along the lanes at any batch
+ * (CUVDIA_EUNSUPPORTED for row_fact > 1 or a table of more than 256 chunks);
+ * densedense_to_dia treats it as CUVDIA_PATH_AUTO. */
 int cuvdia_set_path(int path);
 
 /* Which family the most recent compute call on this thread launched
  * (CUVDIA_PATH_GENERIC, CUVDIA_PATH_TILED, CUVDIA_PATH_WALK for a product
  * served by the walking kernel, CUVDIA_PATH_PLANE by the ones on the matrix
  * cores, CUVDIA_PATH_WINDOW for a projection served
- * by the kernel tiled in the window's plane; 0 before any call). */
+ * by the kernel tiled in the window's plane; 0 before any call).  The kernels
+ * with rows along the lanes, of which the automatic choice makes use beside
+ * the tiled ones, count as CUVDIA_PATH_TILED; cuvdia_last_kernel names them. */
 int cuvdia_last_path(void);
 
 /* Name of the kernel the most recent compute call on this thread launched

@@ -71,8 +71,8 @@ if os.environ.get("FAKE_HIP"):                           # in the script's proce
                 self._desc, self._desc_ptr = d, d.value
             return self._desc
 
-    def matrix(h, w, offsets):
-        m = _Matrix(h, w, len(offsets), max(h, w))
+    def matrix(h, w, offsets, row_fact=1):
+        m = _Matrix(h, w, len(offsets), max(h, w), row_fact)
         m.set_offsets(offsets)
         m.desc
         return m

@@ -166,3 +166,34 @@ for path in (_lib.PATH_AUTO, _lib.PATH_TILED):
     D.densedense_to_dia(A, None, tensor(0, 4096, bytes_at=1 << 41), tensor(0, 4096, bytes_at=1 << 42), 1.0, 0.5)
 assert flag("fake_launches") == 2 and L.cuvdia_last_kernel() == b"dd2dia_generic_kernel"
 """)
+
+
+def test_forced_families(tmp_path):
+    """CUVDIA_PATH_TILED runs the kernels that stage operands, at every batch, or nothing; CUVDIA_PATH_THIN is a product's
+    choice alone."""
+    _fake_hip.run(tmp_path, """
+A = matrix(4099, 4099, [64 * dy + dx for dy in range(-2, 3) for dx in range(-2, 3)])
+huge = matrix(1 << 24, 1 << 24, list(range(-20, 20)))    # 2.5 GiB of values
+def ran(path, M, batch):
+    x, y = tensor(batch, M.w, bytes_at=1 << 41), tensor(batch, M.h, bytes_at=1 << 42)
+    L.cuvdia_set_path(path)
+    names = []
+    for call in (lambda: D.prod(y, M, x), lambda: D.densedense_to_dia(M, None, y, x)):
+        try:
+            call()
+            names.append(L.cuvdia_last_kernel().decode().split("<")[0])
+        except _lib.CuvDiaError as e:
+            names.append(e.code)
+    return names
+for batch in (1, 4, 23, 24, 100):
+    assert ran(_lib.PATH_TILED, A, batch) == ["spmm_tiled_kernel", "dd2dia_tiled_kernel"], (batch, L.cuvdia_last_kernel())
+    assert ran(_lib.PATH_AUTO, A, batch)[1] == ran(_lib.PATH_THIN, A, batch)[1] == "dd2dia_rows_kernel"
+    assert ran(_lib.PATH_THIN, A, batch)[0] == "spmm_thin_kernel"
+large = matrix(256 * 512, 256 * 512, D.filter_factory_float(256, 512, 9, 1, 1).offsets())      # matrix cores, by size
+assert ran(_lib.PATH_AUTO, large, 256) == ["spmm_plane_kernel", "dd2dia_plane_kernel"]
+assert ran(_lib.PATH_TILED, large, 256) == ["spmm_tiled_kernel", "dd2dia_window_long_kernel"]
+assert ran(_lib.PATH_TILED, huge, 8) == [_lib.EUNSUPPORTED] * 2
+assert ran(_lib.PATH_AUTO, huge, 8) == ["spmm_thin_kernel", "dd2dia_rows_kernel"]
+rf2 = matrix(100, 50, [-1, 0, 1], 2)
+assert ran(_lib.PATH_TILED, rf2, 8) == [_lib.EUNSUPPORTED] * 2 and ran(_lib.PATH_THIN, rf2, 8)[0] == _lib.EUNSUPPORTED
+""")
