@@ -13,7 +13,6 @@
 #include <list>
 #include <mutex>
 #include <new>
-#include <string>
 #include <vector>
 
 #include "kernels.hpp"
@@ -36,7 +35,7 @@ namespace {
 
 std::atomic_int g_path{CUVDIA_PATH_AUTO};
 thread_local int t_last_path = 0;
-thread_local std::string t_hip_error;
+thread_local char t_hip_error[256] = "";          // (no std::string: a failure to allocate is reported here as well)
 
 // Batches narrower than this are not the tile-by-tile kernel's: it puts one batch column on each of 64 lanes.
 constexpr int SPMM_TILED_MIN_BATCH = 24;
@@ -90,7 +89,7 @@ constexpr long long DIM_LIMIT = 1LL << 30;
 int hip_fail(hipError_t e, const char *what)
 {
     (void)hipGetLastError();
-    t_hip_error = std::string(what) + ": " + hipGetErrorString(e);
+    std::snprintf(t_hip_error, sizeof t_hip_error, "%s: %s", what, hipGetErrorString(e));
     return CUVDIA_EHIP;
 }
 
@@ -114,8 +113,7 @@ int require_device()
     int ndev = 0;
     const hipError_t e = hipGetDeviceCount(&ndev);
     if (e != hipSuccess || ndev < 1) {
-        t_hip_error = std::string("hipGetDeviceCount: ") + hipGetErrorString(e);
-        (void)hipGetLastError();
+        (void)hip_fail(e, "hipGetDeviceCount");
         return CUVDIA_ENODEVICE;
     }
     return CUVDIA_OK;
@@ -194,7 +192,7 @@ const char *cuvdia_strerror(int code)
     }
 }
 
-const char *cuvdia_last_hip_error(void) { return t_hip_error.c_str(); }
+const char *cuvdia_last_hip_error(void) { return t_hip_error; }
 
 int cuvdia_set_path(int path)
 {
@@ -378,14 +376,9 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     const int rc = validate_shape(offsets_host, nd, h, w, stride, row_fact);
     if (rc) return rc;
 
-    int ndev = 0;
-    hipError_t e = hipGetDeviceCount(&ndev);
-    if (e != hipSuccess || ndev < 1) {
-        t_hip_error = std::string("hipGetDeviceCount: ") + hipGetErrorString(e);
-        (void)hipGetLastError();
-        return CUVDIA_ENODEVICE;
-    }
+    if (const int no_device = require_device()) return no_device;
 
+    hipError_t e = hipSuccess;
     cuvdia_desc *d = nullptr;
     std::vector<Chunk> cn, ct, cp;
     std::vector<Unit> un, us;
@@ -427,7 +420,13 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     const size_t cp_at = off_bytes + cn_bytes + ct_bytes, un_at = cp_at + cp_bytes, us_at = un_at + un_bytes;
     const size_t wn_at = (us_at + us_bytes + 63) / 64 * 64, wn_bytes = walk_ints(wn) * sizeof(int);
     const size_t wt_at = (wn_at + wn_bytes + 63) / 64 * 64, wt_bytes = walk_ints(wt) * sizeof(int);
-    std::vector<unsigned char> staging(wt_at + wt_bytes + 64, 0);
+    std::vector<unsigned char> staging;
+    try {
+        staging.resize(wt_at + wt_bytes + 64, 0);
+    } catch (const std::bad_alloc &) {
+        delete d;
+        return CUVDIA_ENOMEM;
+    }
     std::memcpy(staging.data(), offsets_host, (size_t)nd * sizeof(int));
     std::memcpy(staging.data() + off_bytes, cn.data(), cn_bytes);
     std::memcpy(staging.data() + off_bytes + cn_bytes, ct.data(), ct_bytes);

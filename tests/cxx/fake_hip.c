@@ -17,6 +17,8 @@ void *fake_last_event = NULL;            /* the event of the last launch, and ..
 void *fake_waited_event = NULL;          /* ... the one waited for last */
 volatile int fake_hold_launch = 0;       /* launches and waits stay in their call until it is 0, at most 10 s */
 volatile int fake_held = 0;              /* calls that ran into those 10 s */
+int fake_news = 0;                       /* calls of C++'s operator new; ... */
+int fake_fail_new = 0;                   /* ... n > 0: the n-th from now throws std::bad_alloc, and this is 0 */
 
 static int s_error = 0;
 static int result(int fail) { return fail ? (s_error = UNKNOWN) : SUCCESS; }
@@ -24,6 +26,16 @@ static void hold(void)
 {
     for (int i = 0; i < 10000 && fake_hold_launch; ++i) usleep(1000);
     if (fake_hold_launch) ++fake_held;
+}
+
+void _ZSt17__throw_bad_allocv(void);
+void *_Znwm(size_t n)                    /* operator new(size_t) */
+{
+    ++fake_news;
+    if (fake_fail_new > 0 && --fake_fail_new == 0) _ZSt17__throw_bad_allocv();
+    void *p = malloc(n ? n : 1);
+    if (!p) _ZSt17__throw_bad_allocv();
+    return p;
 }
 
 int hipGetDeviceCount(int *n) { *n = fake_devices; return SUCCESS; }

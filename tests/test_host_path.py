@@ -197,3 +197,59 @@ assert ran(_lib.PATH_AUTO, huge, 8) == ["spmm_thin_kernel", "dd2dia_rows_kernel"
 rf2 = matrix(100, 50, [-1, 0, 1], 2)
 assert ran(_lib.PATH_TILED, rf2, 8) == [_lib.EUNSUPPORTED] * 2 and ran(_lib.PATH_THIN, rf2, 8)[0] == _lib.EUNSUPPORTED
 """)
+
+
+MEMORY = """
+ip = ctypes.POINTER(ctypes.c_int)
+def table(offsets): return (ctypes.c_int * len(offsets))(*offsets)
+win = [dy * 40 + dx + 1600 * m for m in range(-1, 2) for dy in range(-2, 3) for dx in range(-2, 3)]
+offs, nd, n = table(win), len(win), 3200
+x, y, v = 1 << 41, 1 << 42, 1 << 43
+A = matrix(n, n, win)
+f = ctypes.c_float
+"""
+
+
+def test_no_memory_is_an_error_code(tmp_path):
+    """Every allocation of every entry point, one after the other, fails: std::bad_alloc must not leave through the C ABI."""
+    _fake_hip.run(tmp_path, MEMORY + """
+def create():
+    d = ctypes.c_void_p()
+    rc = L.cuvdia_desc_create(ctypes.byref(d), offs, nd, n, n, n, 1)
+    return rc if rc else L.cuvdia_desc_destroy(d)
+def offsets_call():
+    rc = L.cuvdia_spmm_offsets_f32(v, offs, nd, n, n, n, 1, x, n, y, n, 30, b"n", 1.0, 0.0, None)
+    return rc if rc else L.cuvdia_cache_clear()
+def waited():
+    rc = L.cuvdia_wait_begin()
+    return rc if rc else L.cuvdia_wait_end(None)
+def failed_launch():
+    flag("fake_fail_launch", 1)
+    rc = L.cuvdia_spmm_f32(A.desc, v, x, n, y, n, 30, b"n", 1.0, 0.0, None)
+    flag("fake_fail_launch", 0)
+    assert rc == _lib.EHIP and b"a failure asked for" in L.cuvdia_last_hip_error()
+    return 0
+L.cuvdia_wait_end.argtypes = [ctypes.c_void_p]
+c1, c2 = table([0] * 100), table([0] * 100)
+calls = dict(create=create, offsets=offsets_call, waited=waited, failed_launch=failed_launch,
+             dd2dia=lambda: L.cuvdia_dd2dia_offsets_f32(v, offs, nd, n, n, n, 1, x, n, y, n, 30, 1.0, 0.0, None) or L.cuvdia_cache_clear(),
+             noalloc=lambda: L.cuvdia_spmm_offsets_noalloc_f32(v, offs, nd, n, n, n, 1, x, n, y, n, 30, b"t", 1.0, 0.0, None),
+             chunks=lambda: min(0, L.cuvdia_plan_chunks(offs, nd, 0, c1, c2, c1, 0)), units=lambda: min(0, L.cuvdia_plan_units(offs, nd, c1, c2, 100)),
+             walk=lambda: min(0, L.cuvdia_plan_walk(offs, nd, n, 0, None, None, None, None)),
+             walk_launch=lambda: min(0, L.cuvdia_plan_walk_launch(offs, nd, n, n, n, 0, 64)),
+             window_launch=lambda: min(0, L.cuvdia_plan_window_launch(offs, nd, n, n, n, 64)))
+for name, call in calls.items():
+    for k in range(1, 400):
+        print(name, k, flush=True)
+        flag("fake_fail_new", k)
+        rc = call()
+        reached = flag("fake_fail_new") == 0
+        flag("fake_fail_new", 0)
+        assert rc in (0, _lib.ENOMEM), (name, k, rc)     # (0: an allocation that there is another way without)
+        if not reached:
+            assert rc == 0
+            break
+    else:
+        raise SystemExit(name)
+    assert call() == 0
+""")
