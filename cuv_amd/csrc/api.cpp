@@ -26,7 +26,8 @@ struct cuvdia_desc {
     std::vector<int> offsets;        // host copy, table order
     long long nnz;
     int n_chunks_n, n_chunks_t;
-    std::vector<int> walk_n, walk_t; // group rows of the window-table forms
+    std::vector<int> walk_n, walk_t; // group rows of the window-table forms, and the map rows of their products
+    PlaneSpans spans_n, spans_t;
     void *dev_block;                 // one allocation: offsets | chunks_n | chunks_t
     DiaView view;
 };
@@ -406,6 +407,8 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     try {
         plan_walk(cn, stride, false, wn);
         plan_walk(ct, stride, true, wt);
+        d->spans_n = plan_plane(wn, h, w);
+        d->spans_t = plan_plane(wt, w, h);
     } catch (const std::bad_alloc &) {
         delete d;
         return CUVDIA_ENOMEM;
@@ -475,6 +478,8 @@ int cuvdia_desc_create(cuvdia_desc **out, const int *offsets_host, int nd,
     d->walk_t.swap(wt.group_rows);
     d->view.walk_n.rows_host = d->walk_n.data();
     d->view.walk_t.rows_host = d->walk_t.data();
+    d->view.walk_n.spans = &d->spans_n;
+    d->view.walk_t.spans = &d->spans_t;
     auto span = [](const std::vector<Chunk> &t, int &max_len, int &s_min, int &s_max, int *min_len = nullptr) {
         max_len = 0;
         if (min_len) {

@@ -3125,7 +3125,7 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
     // One of another width, or with a larger window: the plane's walk on the matrix cores.
     if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_PLANE) {
         PlaneLaunch P{};
-        if (spmm_plane_plan(wk, n_out, n_in, batch, ep.bias != nullptr || ep.act != 0, path == CUVDIA_PATH_PLANE, P)) {
+        if (spmm_plane_plan(wk, n_out, batch, ep.bias != nullptr || ep.act != 0, path == CUVDIA_PATH_PLANE, P)) {
             if (ran) *ran = CUVDIA_PATH_PLANE;
             P.tab = wk.tab_dev; P.ngroups = wk.ngroups; P.period = wk.period; P.s0 = wk.s0; P.astep4 = wk.astep4; P.k = wk.k;
             P.vals = vals; P.B = B; P.ldb = ldb; P.dst = dst; P.ldd = ldd; P.n_out = n_out; P.n_in = n_in; P.batch = batch;

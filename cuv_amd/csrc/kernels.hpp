@@ -45,6 +45,7 @@ struct WalkView {
     int ngroups, period, s0, k, lck, astep4;
     bool rows4;                  // every group_rows[g] is a multiple of 4
     const int *rows_host;        // group_rows[ngroups] in host memory
+    const PlaneSpans *spans = nullptr;   // the map rows of the product, for spmm_plane_plan
 };
 
 struct DiaView {
@@ -140,8 +141,7 @@ struct PlaneLaunch {
     hipStream_t stream;
 };
 // Fills in the launch's shape; false: the kernel does not serve this table and these sizes, or (not force) would not be ahead.
-bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int batch, bool fused, bool force,
-                     PlaneLaunch &L);
+bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L);
 hipError_t spmm_plane_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.

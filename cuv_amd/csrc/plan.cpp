@@ -105,6 +105,37 @@ void plan_walk(const std::vector<Chunk> &chunks, int stride, bool transposed, Wa
     plan.aoff4.swap(aoff4);
 }
 
+PlaneSpans plan_plane(const WalkPlan &walk, long long n_out, long long n_in)
+{
+    PlaneSpans p;
+    if (!walk.ok || n_out % walk.period != 0) return p;
+    const int walk_len = (int)(n_out / walk.period);
+    auto range = [&](int g, long long &lo, long long &hi) {      // map rows whose middle window row lies in the operand
+        const long long at = (long long)walk.s0 + walk.group_rows[g] + (long long)(walk.k / 2) * walk.period;
+        lo = (std::max(0LL, -at) + walk.period - 1) / walk.period;
+        hi = std::min<long long>(walk_len, (n_in - at + walk.period - 1) / walk.period);
+    };
+    p.ends = {0, walk_len};
+    for (int g = 0; g < walk.ngroups; ++g) {
+        long long lo, hi;
+        range(g, lo, hi);
+        if (lo > 0 && lo < walk_len) p.ends.push_back((int)lo);
+        if (hi > 0 && hi < walk_len) p.ends.push_back((int)hi);
+    }
+    std::sort(p.ends.begin(), p.ends.end());
+    p.groups.assign(p.ends.size() - 1, 0);
+    for (size_t i = 0; i < p.groups.size(); ++i) {
+        for (int g = 0; g < walk.ngroups; ++g) {
+            long long lo, hi;
+            range(g, lo, hi);
+            p.groups[i] += lo <= p.ends[i] && p.ends[i + 1] <= hi;
+        }
+        p.work += (long long)p.groups[i] * (p.ends[i + 1] - p.ends[i]);
+        p.most = std::max(p.most, p.groups[i]);
+    }
+    return p;
+}
+
 std::vector<Unit> plan_units(const std::vector<Chunk> &chunks)
 {
     std::vector<Unit> out;

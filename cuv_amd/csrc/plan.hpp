@@ -44,6 +44,15 @@ struct WalkPlan {
 // `chunks`: a table from plan_chunks (shifts ascending).  plan.ok is false when the table is no window table.
 void plan_walk(const std::vector<Chunk> &chunks, int stride, bool transposed, WalkPlan &plan);
 
+// The map rows of a product with a window table, for the kernel that walks them: between ends[i] and ends[i + 1]
+// groups[i] groups have their middle window row in the dense operand.  Empty where n_out is no whole number of map rows.
+struct PlaneSpans {
+    std::vector<int> ends, groups;   // groups: one less
+    long long work = 0;              // sum over the map rows of their groups
+    int most = 1;                    // largest of groups
+};
+PlaneSpans plan_plane(const WalkPlan &walk, long long n_out, long long n_in);
+
 // Sort shifts (stable in table position), cut into maximal runs of
 // consecutive shifts -- a repeated shift starts a new run -- and split each
 // run into near-equal chunks of at most max_len (<= CHUNK_SLOTS).  Positions

@@ -395,9 +395,13 @@ hipError_t spmm_plane_launch(const PlaneLaunch &L)
     }
 }
 
-bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int batch, bool fused, bool force, PlaneLaunch &L)
+bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
 {
-    if (wk.tab_dev == nullptr || wk.lck != wk.k) return false;
+    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.period < PLANE_ROWS) return false;
+    const PlaneSpans &spans = *wk.spans;
+    if (spans.work == 0) return false;
+    L.col_tiles = (batch + 63) / 64;
+    if (!force && (L.col_tiles < 2 || (wk.k >= 9 && fused))) return false;     // (the rule is below)
     int per_cu = 1;
     switch (wk.k) {
         case 5: per_cu = PlaneShape<5, 5>::PER_CU; break;
@@ -408,48 +412,26 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int ba
         case 13: per_cu = PlaneShape<13, 13>::PER_CU; break;
         default: return false;
     }
-    if (wk.period < PLANE_ROWS || n_out % wk.period != 0) return false;
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
-    L.col_tiles = (batch + 63) / 64;
     const int walk_len = (int)(n_out / wk.period);
 
     // Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut
     // where that work divides evenly.  Between two ends of groups' ranges the groups are the same.
-    std::vector<int> ends{0, walk_len};
-    auto range = [&](int g, long long &lo, long long &hi) {      // map rows whose middle window row lies in the operand
-        const long long at = (long long)wk.s0 + wk.rows_host[g] + (long long)(wk.k / 2) * wk.period;
-        lo = (std::max(0LL, -at) + wk.period - 1) / wk.period;
-        hi = std::min<long long>(walk_len, (n_in - at + wk.period - 1) / wk.period);
-    };
-    for (int g = 0; g < wk.ngroups; ++g) {
-        long long lo, hi;
-        range(g, lo, hi);
-        if (lo > 0 && lo < walk_len) ends.push_back((int)lo);
-        if (hi > 0 && hi < walk_len) ends.push_back((int)hi);
-    }
-    std::sort(ends.begin(), ends.end());
-    std::vector<int> groups(ends.size(), 0);
-    long long work = 0;
-    int most = 1;
-    for (size_t i = 0; i + 1 < ends.size(); ++i) {
-        for (int g = 0; g < wk.ngroups; ++g) {
-            long long lo, hi;
-            range(g, lo, hi);
-            groups[i] += lo <= ends[i] && ends[i + 1] <= hi;
-        }
-        work += (long long)groups[i] * (ends[i + 1] - ends[i]);
-        most = std::max(most, groups[i]);
-    }
     // How many: workgroups run in rounds of 32 CUs per XCD, a unit of PLANE_XT walks with its column tiles on one XCD.
+    const std::vector<int> &ends = spans.ends, &groups = spans.groups;
+    const long long work = spans.work;
     const int full = L.tp / PLANE_XT, part = L.tp % PLANE_XT, cap = 32 * per_cu;
     auto rounds = [&](int segs) {
         const int wgs = ((segs * full + 7) / 8 * PLANE_XT + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles;
         return (wgs + cap - 1) / cap;
     };
+    const double walk_ends = 0.9 * (wk.k - 1) * spans.most;
     double best = -1;
     int n = 1;
     for (int i = 1; i <= PLANE_MAX_SEGMENTS && i <= walk_len; ++i) {
-        const double cost = rounds(i) * ((double)work / i + 0.9 * (wk.k - 1) * most);
+        const int r = rounds(i);
+        if (best >= 0 && r * walk_ends >= best) break;       // (more segments never run in fewer rounds)
+        const double cost = r * ((double)work / i + walk_ends);
         if (best < 0 || cost < best) {
             best = cost;
             n = i;
@@ -460,8 +442,7 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, long long n_in, int ba
     // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
     // Measured on 90 layers: 1.0 - 1.6 times the tile-by-tile kernel's rate where taken (one of 30: 0.88), 0.44 - 1.1 elsewhere.
     const double over = best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
-    if (work == 0) return false;
-    if (!force && (L.col_tiles < 2 || over > (wk.k >= 8 ? 1.65 : 1.4) || (wk.k >= 9 && fused))) return false;
+    if (!force && over > (wk.k >= 8 ? 1.65 : 1.4)) return false;
     L.nseg = n;
     long long done = 0;
     size_t i = 0;

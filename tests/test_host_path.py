@@ -210,6 +210,23 @@ f = ctypes.c_float
 """
 
 
+def test_compute_calls_allocate_nothing(tmp_path):
+    _fake_hip.run(tmp_path, MEMORY + """
+calls = [lambda b: L.cuvdia_spmm_f32(A.desc, v, x, n, y, n, b, b"n", 1.0, 0.5, None),
+         lambda b: L.cuvdia_spmm_layer_f32(A.desc, v, x, n, y, n, b, b"t", 1.0, 0.0, v, 2, 7, None),
+         lambda b: L.cuvdia_dd2dia_f32(A.desc, v, x, n, y, n, b, 1.0, 0.0, None),
+         lambda b: L.cuvdia_avg_diagonals_f32(A.desc, v, x, None),
+         lambda b: L.cuvdia_learn_step_weight_decay_momentum_f32(x, y, v, 1000, 0.1, 0.9, 0.0, None)]
+for path in (0, 1, 2, 4, 6, 8):
+    L.cuvdia_set_path(path)
+    for b in (1, 30, 200):
+        before = flag("fake_news")
+        for call in calls:
+            assert call(b) == 0, (path, b)
+            assert flag("fake_news") == before, (path, b, L.cuvdia_last_kernel())
+""")
+
+
 def test_no_memory_is_an_error_code(tmp_path):
     """Every allocation of every entry point, one after the other, fails: std::bad_alloc must not leave through the C ABI."""
     _fake_hip.run(tmp_path, MEMORY + """
