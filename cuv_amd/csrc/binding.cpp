@@ -14,6 +14,11 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
+#include <torch/version.h>
+
+#include <cctype>
+#include <cstring>
+#include <string>
 
 #include "cuvdia.h"
 
@@ -241,10 +246,28 @@ PyMethodDef g_methods[] = {method<product>("product"), method<projection>("proje
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", "Direct calls into libcuvdia.so.", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 
+// Fails to import where torch or Python is not the one this was compiled against: a tensor's fields may lie elsewhere.
+bool fits()
+{
+    PyObject *torch = PyImport_ImportModule("torch");
+    PyObject *version = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+    const char *text = version ? PyUnicode_AsUTF8(version) : nullptr;
+    const size_t n = std::strlen(TORCH_VERSION);                   // (what follows names the build: "+rocm7.0")
+    const bool same_torch = text && std::strncmp(text, TORCH_VERSION, n) == 0 && !std::isdigit((unsigned char)text[n]);
+    const std::string python = std::to_string(PY_MAJOR_VERSION) + "." + std::to_string(PY_MINOR_VERSION) + ".";
+    const bool same_python = std::strncmp(Py_GetVersion(), python.c_str(), python.size()) == 0;
+    if (!PyErr_Occurred() && !(same_torch && same_python))
+        PyErr_Format(PyExc_ImportError, "built for torch %s and Python %sx, this is torch %s and Python %s", TORCH_VERSION, python.c_str(), text ? text : "?", Py_GetVersion());
+    Py_XDECREF(version);
+    Py_XDECREF(torch);
+    return !PyErr_Occurred();
+}
+
 }  // namespace
 
 PyMODINIT_FUNC PyInit__native(void)
 {
+    if (!fits()) return nullptr;
     g_names = {PyUnicode_InternFromString("h"), PyUnicode_InternFromString("w"), PyUnicode_InternFromString("vec"),
                PyUnicode_InternFromString("_desc_ptr")};
     return PyModule_Create(&g_module);

@@ -8,6 +8,7 @@ a tensor of shape (batch, rows) that is contiguous (`t.t()` is the rows x batch
 view).  torch only provides device memory and the stream here.
 """
 import ctypes
+import warnings
 
 import numpy as np
 import torch
@@ -17,8 +18,13 @@ from . import _lib
 try:
     from . import _native
 except ImportError as e:
-    raise ImportError("cuv_amd/_native.so is not built or does not fit this torch (%s); run `make -j8 -C cuv_amd/csrc` "
-                      "or __graft_entry__.build()" % e) from e
+    # Built against another torch or Python, or not at all: the calls go through ctypes, some 8 us later.
+    warnings.warn("cuv_amd/_native.so is not built or does not fit this torch (%s): calls take the slower way through ctypes; "
+                  "run `make -j8 -C cuv_amd/csrc` or __graft_entry__.build()" % e, RuntimeWarning)
+
+    class _native:
+        """Takes no call."""
+        product = projection = weight_step = staticmethod(lambda *args: False)
 
 
 def _stream_ptr():

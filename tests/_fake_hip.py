@@ -8,13 +8,13 @@ import sys
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def run(tmp_path, script):
-    """Runs the script after `from _fake_hip import *` (and _lib); fails with its output if it does not end well."""
+def run(tmp_path, script, first=""):
+    """Runs `first`, then the script after `from _fake_hip import *` (and _lib); fails with its output if it does not end well."""
     lib = os.path.join(str(tmp_path), "libfake_hip.so")
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-w", "-fexceptions", "-o", lib, os.path.join(ROOT, "tests", "cxx", "fake_hip.c"),
                     "-l:libstdc++.so.6"], check=True)
     path = os.pathsep.join([ROOT, os.path.join(ROOT, "tests"), os.environ.get("PYTHONPATH", "")])
-    p = subprocess.run([sys.executable, "-c", "from _fake_hip import *\nfrom _fake_hip import _lib\n" + script], text=True, timeout=300, cwd=str(tmp_path),
+    p = subprocess.run([sys.executable, "-c", first + "\nfrom _fake_hip import *\nfrom _fake_hip import _lib\n" + script], text=True, timeout=300, cwd=str(tmp_path),
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env=dict(os.environ, PYTHONPATH=path, FAKE_HIP=lib))
     assert p.returncode == 0, "exit %d\n%s" % (p.returncode, p.stdout[-6000:])
     return p.stdout

@@ -1,5 +1,7 @@
 """The calls' way through cuv_amd/dia.py, the Python module and the library's dispatch, on a runtime without a GPU
 (tests/cxx/fake_hip.c), so that waits and launches can fail and calls can be held where they are."""
+import pytest
+
 import _fake_hip
 
 
@@ -270,3 +272,14 @@ for name, call in calls.items():
         raise SystemExit(name)
     assert call() == 0
 """)
+
+
+@pytest.mark.parametrize("first", ["sys.modules['cuv_amd._native'] = None", "torch.__version__ = '2.9.1+rocm6.4'",
+                                   "torch.__version__ += '.post1'"])
+def test_without_a_module_that_fits_the_calls_go_through_ctypes(tmp_path, first):
+    fits = "post1" in first
+    out = _fake_hip.run(tmp_path, CALLS + """
+print("module" if D._native.__class__.__name__ == "module" else "ctypes")
+""", "import ctypes, os, sys\nctypes.CDLL(os.environ['FAKE_HIP'], mode=ctypes.RTLD_GLOBAL)\nimport torch\n" + first)
+    assert out.split()[-1] == ("module" if fits else "ctypes")
+    assert ("slower way through ctypes" in out) != fits
