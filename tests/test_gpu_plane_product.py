@@ -128,3 +128,34 @@ def test_the_automatic_choice_takes_it_for_large_products(oracle):
     finally:
         L.cuvdia_set_path(_lib.PATH_AUTO)
     torch.testing.assert_close(out, ref, rtol=1e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_fused_exit_of_every_window(oracle, plane, shape, trans):
+    """Bias, sigmoid and sample of every window the kernel is built for, into a destination that is read or only written."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng, A, B, dst = _case(oracle, 17 + sum(shape), *shape, trans)
+    n, batch = dst.shape
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    dev, Bd, bd = gu.make_dev_dia(A), D.to_device_colmajor(B), torch.from_numpy(bias).cuda()
+    for beta in (0.0, 0.5):
+        old = dst if beta else None
+        p = oracle.prod_bias_act(A, B, old, trans, 0.25, beta, bias, True)
+        # a quarter (the sigmoid's steepest slope) of 1e-5 of the sum's terms, and the sigmoid's own rounding
+        tol = 0.25 * gu.REL_TOL * (oracle.prod_mag(A, B, old, trans, 0.25, beta) + np.abs(bias)[:, None]) + 3e-7
+        out = D.to_device_colmajor(dst if beta else np.full_like(dst, np.nan))
+        D.prod_bias_act(out, dev, Bd, trans, 0.25, beta, bias=bd, act=_lib.ACT_SIGMOID)
+        assert _ran() and _lib.lib().cuvdia_last_kernel().decode().endswith("true>")
+        assert np.all(np.abs(D.to_host_colmajor(out).astype(np.float64) - p) <= tol)
+        out = D.to_device_colmajor(dst if beta else np.full_like(dst, np.nan))
+        D.prod_bias_act(out, dev, Bd, trans, 0.25, beta, bias=bd, act=_lib.ACT_SIGMOID_SAMPLE, seed=5)
+        u = oracle.sample_uniform(n, batch, 5)
+        decided = np.abs(p.astype(np.float64) - u) > tol
+        assert _ran() and np.array_equal(D.to_host_colmajor(out)[decided], oracle.rnd_binarize(p, u)[decided])
+    out = D.to_device_colmajor(dst)
+    D.prod_bias_act(out, dev, Bd, trans, 0.25, 0.5, bias=bd)                   # a bias alone
+    ref = oracle.prod(A, B, dst, trans, 0.25, 0.5) + bias[:, None]
+    gu.assert_close_mag(D.to_host_colmajor(out), ref, oracle.prod_mag(A, B, dst, trans, 0.25, 0.5) + np.abs(bias)[:, None], str(shape))

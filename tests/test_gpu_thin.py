@@ -93,3 +93,59 @@ def test_automatic_choice_by_tiles_and_columns(oracle, px, k, maps_in, maps_out,
     offsets = sorted(m * n + dy * px + dx for m in range(1 - maps_in, maps_out)
                      for dy in range(-(k // 2), k - k // 2) for dx in range(-(k // 2), k - k // 2))
     _check(oracle, px + batch, n * maps_in, n * maps_out, offsets, batch, 0.75, 0.5 if batch % 4 else 0.0, kernel)
+
+
+def _band_reference(vals, offsets, X, trans):
+    """The product of an n x n matrix with few diagonals in float64, a diagonal at a time, and the sums of its |terms|."""
+    import torch
+    n = X.shape[1]
+    out, mag = torch.zeros(X.shape, dtype=torch.float64, device=X.device), torch.zeros(X.shape, dtype=torch.float64, device=X.device)
+    for d, k in enumerate(offsets):
+        lo, hi = max(0, -k), min(n, n - k)               # rows of the matrix
+        src, dst = (slice(lo, hi), slice(lo + k, hi + k)) if trans == "t" else (slice(lo + k, hi + k), slice(lo, hi))
+        term = vals[d, lo:hi].double() * X[:, src].double()
+        out[:, dst] += term
+        mag[:, dst] += term.abs()
+    return out, mag
+
+
+@pytest.mark.parametrize("batch", [5, 40])
+def test_operands_above_2_gib(batch):
+    """Columns 2^26 and more floats apart: byte offsets pass 2^31 and 2^32 inside the batch."""
+    import torch
+    from cuv_amd import _lib, dia as D
+    n, offsets = 4099, [-70, -3, -2, -1, 0, 1, 2, 64, 65]
+    ld = ((1 << 26) + 4) * (8 if batch < 8 else 1)
+    A = D.dev_dia_matrix_f(n, n, len(offsets), n, device="cuda:0")
+    A.set_offsets(offsets)
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(batch)
+    A.vec.uniform_(-1, 1, generator=g)
+    X, Y = (torch.empty(batch, ld, device="cuda:0")[:, :n] for _ in range(2))
+    X.uniform_(-1, 1, generator=g)
+    for trans in ("n", "t"):
+        old = Y.uniform_(-1, 1, generator=g).clone()
+        D.prod(Y, A, X, trans, "n", 1.0, 0.5)
+        assert _lib.lib().cuvdia_last_kernel().decode().startswith("spmm_thin_kernel")
+        ref, mag = _band_reference(A.vec.view(len(offsets), n), offsets, X, trans)
+        assert torch.all((Y.double() - (ref + 0.5 * old)).abs() <= 1e-5 * (mag + 0.5 * old.abs()))
+
+
+def test_values_above_2_gib():
+    """2.2 GiB of values: diagonals 8 MiB apart, the last ones beyond 2^31 bytes."""
+    import torch
+    from cuv_amd import _lib, dia as D
+    n, offsets = (1 << 21) + 3, [300 * r + d for r in range(-22, 22) for d in range(6)]
+    A = D.dev_dia_matrix_f(n, n, len(offsets), n, device="cuda:0")
+    assert A.vec.numel() * 4 > 1 << 31
+    A.set_offsets(offsets)
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(1)
+    A.vec.uniform_(-1, 1, generator=g)
+    X = torch.rand(4, n, generator=g, device="cuda:0")
+    Y = torch.empty_like(X)
+    for trans in ("n", "t"):
+        D.prod(Y, A, X, trans, "n", 1.0, 0.0)
+        assert _lib.lib().cuvdia_last_kernel().decode().startswith("spmm_thin_kernel")
+        ref, mag = _band_reference(A.vec.view(len(offsets), n), offsets, X, trans)
+        assert torch.all((Y.double() - ref).abs() <= 1e-5 * mag)
