@@ -88,11 +88,18 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
     __shared__ __attribute__((aligned(16))) float lds[2 * S::STAGE];
 
     // A unit -- a segment of PLANE_XT neighbouring walks -- stays on one XCD with all its column tiles: they share the
-    // diagonals' values, and the cache lines that tiles side by side have in common.
-    const int xcd = blockIdx.x % 8, k8 = blockIdx.x / 8, xgroups = (tp + PLANE_XT - 1) / PLANE_XT;
-    const int unit = (k8 / (PLANE_XT * col_tiles)) * 8 + xcd, within = k8 % (PLANE_XT * col_tiles);
-    const int xg = unit / nseg, seg = unit - xg * nseg, xt = xg * PLANE_XT + within / col_tiles, coltile = within % col_tiles;
-    if (xg >= xgroups || xt >= tp) return;
+    // diagonals' values, and the cache lines that tiles side by side have in common.  The last walks of a map row, where
+    // there are fewer, are units of their own behind the full ones, without gaps: an XCD deals its workgroups out to its
+    // four shader engines in turn, idle ones among them, and with gaps in step with that two of the engines got more than
+    // fit into one round (13 x 13, 3 maps of 258 x 258 to 4, batch 72, 9 walks: 927 us with gaps, 559 without).
+    const int xcd = blockIdx.x % 8, k8 = blockIdx.x / 8, xgroups = tp / PLANE_XT, full_unit = PLANE_XT * col_tiles;
+    const int full_slots = (nseg * xgroups + 7) / 8 * full_unit;
+    const bool full = k8 < full_slots;
+    const int size = full ? full_unit : tp % PLANE_XT * col_tiles, at = full ? k8 : k8 - full_slots;
+    const int unit = at / size * 8 + xcd, within = at % size;
+    const int xg = full ? unit / nseg : xgroups, seg = full ? unit - xg * nseg : unit;
+    if (full ? xg >= xgroups : seg >= nseg) return;
+    const int xt = xg * PLANE_XT + within / col_tiles, coltile = within % col_tiles;
     constexpr int waves = PLANE_WAVES, rows = PLANE_ROWS, nqx = S::NQX;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
     const int xs = min(xt * rows, period - rows), skip = xt * rows - xs;       // (the last tile of a row is moved up)
@@ -367,8 +374,8 @@ template <int LC, int K>
 hipError_t plane_launch_one(const PlaneLaunch &L)
 {
     const bool fused = L.ep.bias != nullptr || L.ep.act != 0;
-    const long long units = (long long)L.nseg * ((L.tp + PLANE_XT - 1) / PLANE_XT);
-    const unsigned grid = (unsigned)((units + 7) / 8 * 8 * PLANE_XT * L.col_tiles);
+    const long long full = (long long)L.nseg * (L.tp / PLANE_XT), part = L.nseg;       // units (the kernel's head)
+    const unsigned grid = (unsigned)(((full + 7) / 8 * PLANE_XT + (part + 7) / 8 * (L.tp % PLANE_XT)) * 8 * L.col_tiles);
     note_kernel("spmm_plane_kernel<%d, %d, %s>", LC, K, fused ? "true" : "false");
     auto go = [&](auto kernel) {
         launch_kernel(kernel, dim3(grid), dim3(64 * PLANE_WAVES), 0, L.stream, L.tab, L.ngroups, L.period, L.s0, L.astep4, L.tp,

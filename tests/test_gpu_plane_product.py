@@ -159,3 +159,17 @@ def test_fused_exit_of_every_window(oracle, plane, shape, trans):
     D.prod_bias_act(out, dev, Bd, trans, 0.25, 0.5, bias=bd)                   # a bias alone
     ref = oracle.prod(A, B, dst, trans, 0.25, 0.5) + bias[:, None]
     gu.assert_close_mag(D.to_host_colmajor(out), ref, oracle.prod_mag(A, B, dst, trans, 0.25, 0.5) + np.abs(bias)[:, None], str(shape))
+
+
+@pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch", [
+    (150, 61, 7, 1, 2, 70),   # 5 walks of 32 positions: one unit of 4, and 1
+    (262, 40, 7, 2, 1, 76),   # 9 walks: two units of 4, and 1
+    (190, 50, 8, 1, 1, 130),  # 6: 4 and 2, three column tiles
+    (200, 45, 5, 2, 2, 65),   # 7: 4 and 3
+])
+def test_walks_that_units_of_four_do_not_divide(oracle, px, py, fs, maps_in, maps_out, batch):
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    _, A, B, dst = _case(oracle, px + py, px, py, fs, maps_in, maps_out, batch, "t")
+    _, ran = gu.check_prod(oracle, A, B, dst, "t", 1.0, 0.5, _lib.PATH_PLANE, "%d x %d" % (px, py))
+    assert ran == _lib.PATH_PLANE
