@@ -227,9 +227,11 @@ bool spmm_thin_by_size(const DiaView &A, bool trans, int batch)
     // The tile-by-tile kernel works through a tile's chunks one after another, 1 - 2 us apart, and always for 64 columns;
     // here eight waves share the chunks and the columns are the ones that exist.  So few tiles of many chunks belong here,
     // and many where a good part of their columns is not there.  Measured on 33500 products of windows of 3 x 3 to 13 x 13,
-    // batch 24 to 300, with and without the fused layer update: 1.1 - 4 times the tile-by-tile kernel's rate where the
-    // tiles' number decides (median 1.8; 0.1 % below 0.97), 0.9 - 1.7 where the columns do (median 1.3, a tenth below 1.0);
-    // one step beyond these lines a tenth of the products falls below 0.9.
+    // square maps up to 300 wide, batch 24 to 300, with and without the fused layer update: 1.1 - 4 times the tile-by-tile
+    // kernel's rate where the tiles' number decides (median 1.8; 0.1 % below 0.97), 0.93 - 2 where the columns do (1st
+    // percentile; median 1.37, 2.1 % below 0.97, most of them maps whose width is a multiple of 4); one step beyond these
+    // lines a tenth of the products falls below 0.9.  On 2400 products of maps of any shape up to 640 wide, batch up to 640:
+    // none and 1.5 % below 0.97, the least 0.90.
     const double tiles = (n_out + 63) / 64 * (batch / 64.0);     // of the columns that exist
     const double chunks = (double)A.nnz / n_out / lc;            // per tile, those outside the operand left out
     const double there = batch / 64.0 / ((batch + 63) / 64);

@@ -173,3 +173,36 @@ def test_walks_that_units_of_four_do_not_divide(oracle, px, py, fs, maps_in, map
     _, A, B, dst = _case(oracle, px + py, px, py, fs, maps_in, maps_out, batch, "t")
     _, ran = gu.check_prod(oracle, A, B, dst, "t", 1.0, 0.5, _lib.PATH_PLANE, "%d x %d" % (px, py))
     assert ran == _lib.PATH_PLANE
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+@pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch", [
+    (40, 33, 7, 1, 9, 66),    # a map row of 9 groups' tables meets one or two of them
+    (64, 20, 5, 9, 1, 40),
+    (36, 10, 9, 5, 4, 33),    # maps hardly taller than the window
+    (34, 8, 7, 3, 3, 65),
+])
+def test_groups_that_a_segment_does_not_meet(oracle, px, py, fs, maps_in, maps_out, batch, trans):
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    _, A, B, dst = _case(oracle, px + py, px, py, fs, maps_in, maps_out, batch, trans)
+    _, ran = gu.check_prod(oracle, A, B, dst, trans, 1.0, 0.5, _lib.PATH_PLANE, "%d x %d" % (px, py))
+    assert ran == _lib.PATH_PLANE
+
+
+@pytest.mark.parametrize("h,w,offsets", [
+    (40 * 200, 40 * 20, [0]),                  # a map that ends long before the rows do
+    (40 * 150, 40 * 150, [-40 * 90, 40 * 90]), # two maps with nothing between them
+])
+def test_rows_that_no_group_reaches(oracle, h, w, offsets):
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    rng = np.random.default_rng(h + w)
+    window = [o + 40 * dy + dx for o in offsets for dy in range(-3, 4) for dx in range(-3, 4)]
+    A = oracle.Dia(h, w, window, h, 1)
+    A.vals[:] = rng.uniform(-1, 1, A.vals.shape).astype(np.float32)
+    for trans in ("n", "t"):
+        n_in, n_out = (h, w) if trans == "t" else (w, h)
+        B = np.asfortranarray(rng.uniform(-1, 1, (n_in, 66)).astype(np.float32))
+        dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, 66)).astype(np.float32))
+        gu.check_prod(oracle, A, B, dst, trans, 1.0, 0.5, _lib.PATH_PLANE, str((h, w, trans)))
