@@ -88,14 +88,6 @@ hipError_t launch_spmm_generic(const DiaView &A, const float *vals, const float 
                                float *dst, long long ldd, int batch, bool trans,
                                float alpha, float beta, SpEpilogue ep, hipStream_t stream);
 
-// Same contract, row_fact == 1 only: 64 output rows x 64 batch columns per
-// workgroup, dense tile staged through LDS once per run chunk, lanes own
-// batch columns and keep a sliding register window along the rows, diagonal
-// values are broadcast across each 16-lane row by DPP.  Window tables on
-// products of many tiles go to the walking kernel, which stages a block of
-// dense rows once for all the window rows that read it.  `walk`: 0 -- that
-// choice is made by size; 1 -- the walking kernel or hipErrorNotSupported;
-// -1 -- never the walking kernel.  *walked (if not null) tells which ran.
 // Output rows per tile of the walking kernel's instantiation for a window of k rows of lck diagonals whose first
 // shift is s0; 0 when there is none.
 int spmm_walk_tile_rows(int lck, int k, int s0);
@@ -104,7 +96,18 @@ int spmm_walk_tile_rows(int lck, int k, int s0);
 // counts its tiles do not divide, or -- unless forced -- too few workgroups to fill the chip).
 int spmm_walk_plan(int lck, int k, int s0, int period, long long n_out, long long n_in, long long col_tiles,
                    bool forced, long long *workgroups);
-// path: CUVDIA_PATH_*, as forced; *ran: the one that served the call.
+// Same contract, row_fact == 1 only: 64 output rows x 64 batch columns per
+// workgroup, dense tile staged through LDS once per run chunk, lanes own
+// batch columns and keep a sliding register window along the rows, diagonal
+// values are broadcast across each 16-lane row by DPP.  Window tables on
+// products of many tiles go to the walking kernel, which stages a block of
+// dense rows once for all the window rows that read it, or to the plane's walk
+// on the matrix cores (below); products of few tiles and ragged batches to the
+// kernel with rows along the lanes.
+// path: CUVDIA_PATH_AUTO -- those choices are made by size; _TILED -- the
+// walking kernel by size, else tile by tile; _WALK, _PLANE -- that kernel or
+// hipErrorNotSupported; anything else: tile by tile.  *ran (if not null): the
+// path that served the call, CUVDIA_PATH_TILED for rows along the lanes.
 hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B, long long ldb,
                              float *dst, long long ldd, int batch, bool trans,
                              float alpha, float beta, SpEpilogue ep, hipStream_t stream,
@@ -164,8 +167,8 @@ hipError_t launch_dd2dia_generic(const DiaView &C, float *vals, const float *A, 
 // Same contract, row_fact == 1 only: rows along the lanes, each wave on its own (dd2dia_rows.hip).  Any alignment, no
 // limit on the operands' sizes.
 bool dd2dia_rows_ok(const DiaView &C);
-// Whether the automatic choice takes that kernel; `aligned`: both operands' bases, leading dimensions and row counts
-// are multiples of 16 bytes; `windowed`: the window-table projection would run otherwise.
+// Whether the automatic choice takes that kernel; `aligned`: A's base, leading dimension and row count are multiples of
+// 16 bytes, as the kernels that share staged operands load it in pieces; `windowed`: the window-table projection would run otherwise.
 bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowed);
 hipError_t launch_dd2dia_rows(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
                               int batch, float alpha, float beta, hipStream_t stream);

@@ -16,7 +16,7 @@
 //
 // Bound: on large windows the matrix cores (13 x 13: two thirds of a launch's time), on small ones the dense rows' way
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
-// 13 x 13 on 256 x 256, batch 256 1131 -> 825 us (50 -> 69 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
+// 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
 // 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
 // 229 -> 181; level or behind where the rule below says no.
 //

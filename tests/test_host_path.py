@@ -158,6 +158,29 @@ assert seen >= {b"dd2dia_window_kernel", b"dd2dia_window_long_kernel", b"dd2dia_
 """)
 
 
+def test_the_planned_walk_is_the_one_that_runs(tmp_path):
+    """cuvdia_plan_walk_launch against the kernel and the grid of the product, over maps, windows and batches on both sides of
+    its rules."""
+    _fake_hip.run(tmp_path, """
+import random
+rng, seen = random.Random(3), set()
+for _ in range(400):
+    px, py = rng.choice([rng.randint(1, 10) * 64, rng.randint(40, 640)]), rng.randint(16, 700)
+    fs, maps = rng.choice([3, 5, 7, 7, 9]), rng.choice([(1, 1), (1, 1), (2, 2), (1, 4)])
+    batch, trans = rng.choice([rng.randint(1, 40), rng.randint(41, 700)]), rng.choice("nt")
+    h, w = px * py * maps[0], px * py * maps[1]
+    A = matrix(h, w, D.filter_factory_float(px, py, fs, *maps).offsets())
+    plan = L.cuvdia_plan_walk_launch(A._offsets.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), A.num_dia, A.stride, h, w, trans == "t", batch)
+    n_in, n_out = (h, w) if trans == "t" else (w, h)
+    D.prod_bias_act(tensor(batch, n_out, bytes_at=1 << 41), A, tensor(batch, n_in, bytes_at=1 << 42), trans, act=rng.choice([0, 1, 2]))
+    ran = L.cuvdia_last_path()
+    assert (plan > 0) == (ran == _lib.PATH_WALK), (px, py, fs, maps, batch, trans, plan, L.cuvdia_last_kernel())
+    assert ran != _lib.PATH_WALK or plan == flag("fake_grid")
+    seen.add(L.cuvdia_last_kernel().split(b"<")[0])
+assert seen >= {b"spmm_walk_kernel", b"spmm_plane_kernel", b"spmm_thin_kernel", b"spmm_tiled_kernel"}, seen
+""")
+
+
 def test_an_empty_batch_is_launched_for_the_projection_alone(tmp_path):
     _fake_hip.run(tmp_path, """
 A = matrix(4096, 4096, [64 * dy + dx for dy in range(-2, 3) for dx in range(-2, 3)])
