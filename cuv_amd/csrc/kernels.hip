@@ -3310,7 +3310,8 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
 {
     if (ran) *ran = CUVDIA_PATH_TILED;
     auto plane = [&](bool force) {
-        const hipError_t e = launch_dd2dia_plane(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
+        hipError_t e = launch_dd2dia_split(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
+        if (e == hipErrorNotSupported) e = launch_dd2dia_plane(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
         if (e != hipErrorNotSupported && ran) *ran = CUVDIA_PATH_PLANE;
         return e;
     };

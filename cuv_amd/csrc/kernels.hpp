@@ -186,7 +186,7 @@ int dd2dia_slab_columns(const DiaView &C, long long lda, long long ldb);
 // the four waves split the batch and are summed through LDS in wave order.
 // Window tables whose tiles fill the chip go to the window-table projection (a tile of 4 x 64 positions of the
 // window's plane per workgroup, both operands staged once for all the slots of up to 8 window rows).
-// Of those, square windows of 9 and 11 rows go to the kernel on the matrix cores (below), by size.
+// Of those, square windows of 9, 11 and 13 rows go to the kernels on the matrix cores (below), by size.
 // path: CUVDIA_PATH_AUTO -- those choices are made by size; _TILED -- likewise, but never the matrix cores; _WINDOW --
 // the window-table projection or hipErrorNotSupported; _PLANE -- the matrix cores if they serve the table; anything
 // else: none of them.  *ran (if not null): the path that did.
@@ -196,6 +196,9 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
 // Same contract, square windows of 9 and 11 rows (dd2dia_plane.hip); hipErrorNotSupported: another table, operands that
 // 16-byte pieces do not fit, or (not force) a launch on which it would not be ahead of the window-table projection.
 hipError_t launch_dd2dia_plane(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
+                               int batch, float alpha, float beta, hipStream_t stream, bool force);
+// Same contract, square windows of 13 rows (dd2dia_split.hip): fp32 products as bfloat16 ones on the matrix cores; hipErrorNotSupported as above.
+hipError_t launch_dd2dia_split(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
                                int batch, float alpha, float beta, hipStream_t stream, bool force);
 // Workgroups of the window-table projection on these operands, 0 where it does not serve them or -- unless forced --
 // the automatic choice among the kernels that stage operands does not take it.
