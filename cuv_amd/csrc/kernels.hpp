@@ -146,6 +146,11 @@ struct PlaneLaunch {
 // Fills in the launch's shape; false: the kernel does not serve this table and these sizes, or (not force) would not be ahead.
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L);
 hipError_t spmm_plane_launch(const PlaneLaunch &L);
+// Cuts the map rows into segments (L.nseg, L.cuts); tp and col_tiles are set.
+double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, int every, double walk_ends, PlaneLaunch &L);
+// The same, windows of 13 rows, fp32 products as bfloat16 ones (spmm_split.hip); no samples.
+bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, PlaneLaunch &L);
+hipError_t spmm_split_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.
 hipError_t launch_momentum(float *W, float *M, const float *dW, long long n, float lr, float mw, float l2,

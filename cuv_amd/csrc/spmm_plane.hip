@@ -18,7 +18,8 @@
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
 // 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
 // 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
-// 229 -> 181; level or behind where the rule below says no.
+// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has what spmm_split.hip leaves: samples, tables
+// of more than 19 groups, and what the rule there refuses.
 //
 // Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
 // ascending, acc = fma(a, x, acc).
@@ -407,6 +408,48 @@ hipError_t spmm_plane_launch(const PlaneLaunch &L)
     }
 }
 
+// Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut where that
+// work divides evenly, at multiples of `every` from the segment's first.  Between two ends of groups' ranges the groups are the
+// same.  How many: workgroups run in rounds of 32 CUs per XCD, a unit of `unit` walks with its column tiles on one XCD.
+// Returns the rounds' steps, of all places there are, over the segments' own.
+double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, int every, double walk_ends, PlaneLaunch &L)
+{
+    const std::vector<int> &ends = spans.ends, &groups = spans.groups;
+    const long long work = spans.work;
+    const int full = L.tp / unit, part = L.tp % unit, cap = 32 * per_cu;
+    auto rounds = [&](int segs) {
+        const int wgs = ((segs * full + 7) / 8 * unit + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles;
+        return (wgs + cap - 1) / cap;
+    };
+    double best = -1;
+    int n = 1;
+    for (int i = 1; i <= PLANE_MAX_SEGMENTS && i <= walk_len; ++i) {
+        const int r = rounds(i);
+        if (best >= 0 && r * walk_ends >= best) break;       // (more segments never run in fewer rounds)
+        const double cost = r * ((double)work / i + walk_ends);
+        if (best < 0 || cost < best) {
+            best = cost;
+            n = i;
+        }
+    }
+    L.nseg = 0;
+    long long done = 0;
+    size_t i = 0;
+    L.cuts.at[0] = 0;
+    for (int s = 1; s < n; ++s) {
+        const long long want = work * s / n;
+        while (i + 2 < ends.size() && done + (long long)groups[i] * (ends[i + 1] - ends[i]) <= want) {
+            done += (long long)groups[i] * (ends[i + 1] - ends[i]);
+            ++i;
+        }
+        const int at = groups[i] ? ends[i] + (int)((want - done) / groups[i]) : ends[i], last = L.cuts.at[L.nseg];
+        const int cut = last + (at - last + every / 2) / every * every;
+        if (cut > last && cut < walk_len) L.cuts.at[++L.nseg] = cut;
+    }
+    L.cuts.at[++L.nseg] = walk_len;
+    return best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
+}
+
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
 {
     if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.period < PLANE_ROWS) return false;
@@ -427,50 +470,14 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
     const int walk_len = (int)(n_out / wk.period);
 
-    // Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut
-    // where that work divides evenly.  Between two ends of groups' ranges the groups are the same.
-    // How many: workgroups run in rounds of 32 CUs per XCD, a unit of PLANE_XT walks with its column tiles on one XCD.
-    const std::vector<int> &ends = spans.ends, &groups = spans.groups;
-    const long long work = spans.work;
-    const int full = L.tp / PLANE_XT, part = L.tp % PLANE_XT, cap = 32 * per_cu;
-    auto rounds = [&](int segs) {
-        const int wgs = ((segs * full + 7) / 8 * PLANE_XT + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles;
-        return (wgs + cap - 1) / cap;
-    };
-    const double walk_ends = 0.9 * (wk.k - 1) * spans.most;
-    double best = -1;
-    int n = 1;
-    for (int i = 1; i <= PLANE_MAX_SEGMENTS && i <= walk_len; ++i) {
-        const int r = rounds(i);
-        if (best >= 0 && r * walk_ends >= best) break;       // (more segments never run in fewer rounds)
-        const double cost = r * ((double)work / i + walk_ends);
-        if (best < 0 || cost < best) {
-            best = cost;
-            n = i;
-        }
-    }
+    const double over = plane_cut(spans, walk_len, PLANE_XT, per_cu, 1, 0.9 * (wk.k - 1) * spans.most, L);
     // Taken where the steps come to at most 1.65 times the segments' work (5 x 5 and 7 x 7 windows: 1.4 times), with two column
     // tiles at least -- with one, the values are most of the traffic, and the tile-by-tile kernel fetches them in pieces twice
     // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
     // Measured on 12500 random products of 1 to 17 maps, 40 to 640 wide and 16 to 1400 tall, batch 24 to 640: 1543 are taken,
     // at 0.96 - 3.2 times the tile-by-tile kernel's rate (1st and 99th percentile; median 1.29, 1.4 % below 0.97, the least
     // 0.89), 0.44 - 4.2 elsewhere (median 0.91).
-    const double over = best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
-    if (!force && over > (wk.k >= 8 ? 1.65 : 1.4)) return false;
-    L.nseg = n;
-    long long done = 0;
-    size_t i = 0;
-    L.cuts.at[0] = 0;
-    for (int s = 1; s < n; ++s) {
-        const long long want = work * s / n;
-        while (i + 2 < ends.size() && done + (long long)groups[i] * (ends[i + 1] - ends[i]) <= want) {
-            done += (long long)groups[i] * (ends[i + 1] - ends[i]);
-            ++i;
-        }
-        L.cuts.at[s] = groups[i] ? ends[i] + (int)((want - done) / groups[i]) : ends[i];
-    }
-    L.cuts.at[n] = walk_len;
-    return true;
+    return force || over <= (wk.k >= 8 ? 1.65 : 1.4);
 }
 
 }  // namespace cuvdia
