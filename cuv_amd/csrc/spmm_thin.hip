@@ -252,12 +252,23 @@ hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B,
     // values once more --, and where even 2 columns do not, 64 rows per workgroup.  Tables of a chunk per wave are
     // one round of loads whatever the shape: fewer of them per wave end sooner.
     auto wgs = [&](int rows, int cb) { return (((long long)L.n_out + rows - 1) / rows) * ((batch + cb - 1) / cb); };
+    const double chunks = (double)A.nnz / L.n_out / lc;         // per row block, those outside the operand left out
     int cb = batch <= 2 ? batch : (batch > 4 && wgs(256, 8) >= 384) ? 8 : wgs(256, 4) >= 128 ? 4 : 2;
     if (L.nchunks <= 8 && cb > 2 && wgs(256, 2) <= 2048) cb = 2;
     int g = 1, waves = L.nchunks < 8 ? L.nchunks : 8;
     if (L.nchunks >= 16 && wgs(256, 2) <= 160) {
         g = 4;
         if (cb > 2) cb = 2;
+    } else if (cb == 8 && chunks <= (L.nchunks < 16 ? 18 : 9)) {
+        // Few chunks per row block, however many the table has: 8 waves have nothing to share, and their sums' place in LDS
+        // lets two workgroups into a CU.  Measured on 170 random products, up to 16 maps, batch 1 to 140, every shape: of those
+        // that come here the choice below is at 1.00 - 2.4 times the rate of 8 columns by 4 or 8 waves (mean 1.35), within 1.2 of
+        // the best; on 149 others none is below 0.98.  448 x 448, 3 x 3, 1 map to 4, batch 23, transposed 94 -> 45 us; 388 x 388,
+        // 7 x 7, batch 12, transposed 33 -> 17.  Tables of 16 chunks and more had 4 waves before: beyond 9 chunks a row block
+        // 0.89 - 1.1.
+        if (wgs(256, 8) < 4000) cb = 4;
+        const long long n = wgs(256, cb);
+        waves = n >= 16000 ? 1 : n >= 3000 || chunks <= 3 ? 2 : 4;
     } else if (cb == 8 && L.nchunks >= 16) {
         waves = 4;
     } else if (cb == 4 && L.nchunks >= 64 && wgs(256, 4) <= 256) {
