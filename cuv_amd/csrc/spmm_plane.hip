@@ -456,7 +456,6 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
-    if (!force && (L.col_tiles < 2 || (wk.k >= 9 && fused))) return false;     // (the rule is below)
     int per_cu = 1;
     switch (wk.k) {
         case 5: per_cu = PlaneShape<5, 5>::PER_CU; break;
@@ -476,8 +475,16 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
     // Measured on 12500 random products of 1 to 17 maps, 40 to 640 wide and 16 to 1400 tall, batch 24 to 640: 1543 are taken,
     // at 0.96 - 3.2 times the tile-by-tile kernel's rate (1st and 99th percentile; median 1.29, 1.4 % below 0.97, the least
-    // 0.89), 0.44 - 4.2 elsewhere (median 0.91).
-    return force || over <= (wk.k >= 8 ? 1.65 : 1.4);
+    // 0.89).
+    const bool many = L.col_tiles >= 2 && !(wk.k >= 9 && fused) && over <= (wk.k >= 8 ? 1.65 : 1.4);
+    // ... and, up to 11 x 11, where the steps with the columns and positions that only fill tiles up come to at most 1.8 times
+    // the work: of 330 random products of the same ranges that takes 23 more, at 0.98 - 1.9 times the tile-by-tile kernel's rate
+    // (median 1.21; 282 x 282, 7 x 7, 2 maps to 5, batch 128 295 -> 243 us; 517 x 517, 5 x 5, batch 64 629 -> 355; 512 x 555,
+    // 11 x 11 with bias and sigmoid, batch 128 1247 -> 881).  Beyond 1.8 a fifth falls below 0.97, and so do half of the 7 x 7
+    // and 9 x 9 layers with a bias or an activation.
+    const double padded = over * L.col_tiles * 64 / batch * L.tp * PLANE_ROWS / wk.period;
+    const bool full = wk.k <= 11 && (!fused || wk.k == 5 || wk.k == 11) && padded <= 1.8;
+    return force || many || full;
 }
 
 }  // namespace cuvdia

@@ -1,0 +1,40 @@
+"""The automatic choice of the plane's walk on either side of its rule for well-filled tiles, its result against the
+tile-by-tile kernel's."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch,trans,fused,taken", [
+    (282, 282, 7, 2, 5, 128, "n", False, True),
+    (282, 282, 7, 2, 5, 128, "n", True, False),       # with a bias: 5 x 5 and 11 x 11 only
+    (282, 282, 7, 2, 5, 70, "n", False, False),       # most of the second column tile is empty
+    (517, 517, 5, 3, 5, 64, "n", False, True),        # one column tile
+    (300, 620, 11, 2, 1, 192, "t", True, True),
+])
+def test_well_filled_tiles(px, py, fs, maps_in, maps_out, batch, trans, fused, taken):
+    import torch
+    from cuv_amd import _lib, dia as D
+    m = D.filter_factory_float(px, py, fs, maps_in, maps_out).get_dia("cuda:0")
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(1)
+    m.vec.normal_(0.0, 0.1, generator=g)
+    n_in, n_out = (m.h, m.w) if trans == "t" else (m.w, m.h)
+    X = torch.rand((batch, n_in), device="cuda:0", generator=g)
+    bias = torch.rand(n_out, device="cuda:0", generator=g)
+    L, out = _lib.lib(), []
+    for path in (_lib.PATH_AUTO, _lib.PATH_TILED_NOWALK):
+        _lib.check(L.cuvdia_set_path(path), "set_path")
+        try:
+            y = torch.full((batch, n_out), float("nan"), device="cuda:0")
+            if fused:
+                D.prod_bias_act(y, m, X, trans, 1.0, 0.0, bias=bias, act=_lib.ACT_SIGMOID)
+            else:
+                D.prod(y, m, X, trans)
+        finally:
+            L.cuvdia_set_path(_lib.PATH_AUTO)
+        if path == _lib.PATH_AUTO:
+            assert (L.cuvdia_last_path() == _lib.PATH_PLANE) == taken
+        out.append(y)
+    # two fp32 sums of the same terms, at most 1225 of them below 0.6 in magnitude and 0.05 in the mean
+    torch.testing.assert_close(out[0], out[1], rtol=0, atol=1e-5 * 1225 * 0.05)
