@@ -89,7 +89,8 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
 
     // each XCD takes a contiguous stretch of the tiles: neighbours share rows of A and B
-    const int each = gridDim.x / 8, more = gridDim.x % 8, xcd = blockIdx.x % 8;
+    const int ntiles = tiles.first_tile[ngroups], each = ntiles / 8, more = ntiles % 8, xcd = blockIdx.x % 8;
+    if ((int)blockIdx.x >= ntiles) return;                       // (5000 of 8192 on the large layer: no difference in time)
     const int tile = xcd * each + min(xcd, more) + blockIdx.x / 8;
     int g = 0;
     while (g + 1 < ngroups && tile >= tiles.first_tile[g + 1]) ++g;
@@ -319,11 +320,11 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
 
 template <int LC, int K>
 hipError_t ds_launch(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb, int batch,
-                     float alpha, float beta, hipStream_t stream, int txn, const DsTiles &tiles)
+                     float alpha, float beta, hipStream_t stream, long long workgroups, int txn, const DsTiles &tiles)
 {
     const WalkView &wk = C.walk_n;
     note_kernel("dd2dia_split_kernel<%d, %d>", LC, K);
-    launch_kernel((dd2dia_split_kernel<LC, K>), dim3((unsigned)tiles.first_tile[wk.ngroups]), dim3(DS_THREADS), 0, stream,
+    launch_kernel((dd2dia_split_kernel<LC, K>), dim3((unsigned)std::max(workgroups, (long long)tiles.first_tile[wk.ngroups])), dim3(DS_THREADS), 0, stream,
                   wk.tab_dev, wk.ngroups, wk.period, wk.s0, wk.astep4 / 4, vals, A, lda, B, ldb, C.h, C.w, batch, alpha, beta,
                   (unsigned)((((long long)batch - 1) * lda + C.h) * 4), (unsigned)((((long long)batch - 1) * ldb + C.w) * 4),
                   (unsigned)((long long)C.nd * C.stride * 4), txn, tiles);
@@ -370,12 +371,12 @@ bool ds_plan(const DiaView &C, const float *B, long long lda, long long ldb, int
 }  // namespace
 
 hipError_t launch_dd2dia_split(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
-                               int batch, float alpha, float beta, hipStream_t stream, bool force)
+                               int batch, float alpha, float beta, hipStream_t stream, long long workgroups)
 {
     DsTiles tiles;
-    if (!ds_plan(C, B, lda, ldb, batch, force, tiles)) return hipErrorNotSupported;
+    if (!ds_plan(C, B, lda, ldb, batch, workgroups == 0, tiles)) return hipErrorNotSupported;
     const int txn = (C.walk_n.period + DS_XT - 1) / DS_XT;
-    return ds_launch<13, 13>(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, txn, tiles);
+    return ds_launch<13, 13>(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, workgroups, txn, tiles);
 }
 
 }  // namespace cuvdia

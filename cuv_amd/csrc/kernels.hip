@@ -3310,20 +3310,21 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
                                float alpha, float beta, hipStream_t stream, int path, int *ran)
 {
     if (ran) *ran = CUVDIA_PATH_TILED;
-    auto plane = [&](bool force) {
-        hipError_t e = launch_dd2dia_split(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
-        if (e == hipErrorNotSupported) e = launch_dd2dia_plane(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, force);
-        if (e != hipErrorNotSupported && ran) *ran = CUVDIA_PATH_PLANE;
+    auto plane = [&](long long in_place_of) {                    // (workgroups of the window-table projection; 0: forced)
+        hipError_t e = launch_dd2dia_split(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, in_place_of);
+        const bool split = e != hipErrorNotSupported;
+        if (!split) e = launch_dd2dia_plane(C, vals, A, lda, B, ldb, batch, alpha, beta, stream, in_place_of == 0);
+        if (e != hipErrorNotSupported && ran) *ran = split && in_place_of ? CUVDIA_PATH_WINDOW : CUVDIA_PATH_PLANE;
         return e;
     };
     if (path == CUVDIA_PATH_PLANE)
-        if (const hipError_t e = plane(true); e != hipErrorNotSupported) return e;
+        if (const hipError_t e = plane(0); e != hipErrorNotSupported) return e;
     if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_TILED || path == CUVDIA_PATH_WINDOW) {
         int txn = 0, tyn = 0, ndb = 0;
         const long long wgs = dd2dia_window_grid(C, lda, ldb, batch, path == CUVDIA_PATH_WINDOW, &txn, &tyn, &ndb);
         if (wgs > 0) {
             if (path == CUVDIA_PATH_AUTO)
-                if (const hipError_t e = plane(false); e != hipErrorNotSupported) return e;
+                if (const hipError_t e = plane(wgs); e != hipErrorNotSupported) return e;
             const WalkView &wk = C.walk_n;
             const DwLaunch L{wk.tab_dev, wk.ngroups, wk.k, wk.period, wk.s0, wk.astep4 / 4, wk.lck, vals, A, lda, B, ldb,
                              C.h, C.w, batch, alpha, beta,

@@ -146,8 +146,9 @@ struct PlaneLaunch {
 // Fills in the launch's shape; false: the kernel does not serve this table and these sizes, or (not force) would not be ahead.
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L);
 hipError_t spmm_plane_launch(const PlaneLaunch &L);
-// Cuts the map rows into segments (L.nseg, L.cuts); tp and col_tiles are set.
-double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, int every, double walk_ends, PlaneLaunch &L);
+// How many segments of the map rows (L.nseg; tp and col_tiles are set), and the segments (L.nseg, L.cuts).
+double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, double walk_ends, PlaneLaunch &L);
+void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L);
 // The same, windows of 13 rows, fp32 products as bfloat16 ones (spmm_split.hip); no samples.
 bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, PlaneLaunch &L);
 hipError_t spmm_split_launch(const PlaneLaunch &L);
@@ -202,9 +203,11 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
 // 16-byte pieces do not fit, or (not force) a launch on which it would not be ahead of the window-table projection.
 hipError_t launch_dd2dia_plane(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
                                int batch, float alpha, float beta, hipStream_t stream, bool force);
-// Same contract, square windows of 13 rows (dd2dia_split.hip): fp32 products as bfloat16 ones on the matrix cores; hipErrorNotSupported as above.
+// Same contract, square windows of 13 rows (dd2dia_split.hip): fp32 products as bfloat16 ones on the matrix cores;
+// hipErrorNotSupported as above.  It counts as the window-table projection in whose place it runs and is launched with that
+// one's workgroups, which cuvdia_plan_window_launch tells (0: by force, with its own): those past its tiles end at once.
 hipError_t launch_dd2dia_split(const DiaView &C, float *vals, const float *A, long long lda, const float *B, long long ldb,
-                               int batch, float alpha, float beta, hipStream_t stream, bool force);
+                               int batch, float alpha, float beta, hipStream_t stream, long long workgroups);
 // Workgroups of the window-table projection on these operands, 0 where it does not serve them or -- unless forced --
 // the automatic choice among the kernels that stage operands does not take it.
 long long dd2dia_window_grid(const DiaView &C, long long lda, long long ldb, int batch, bool forced,

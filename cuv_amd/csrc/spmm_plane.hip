@@ -409,12 +409,11 @@ hipError_t spmm_plane_launch(const PlaneLaunch &L)
 }
 
 // Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut where that
-// work divides evenly, at multiples of `every` from the segment's first.  Between two ends of groups' ranges the groups are the
-// same.  How many: workgroups run in rounds of 32 CUs per XCD, a unit of `unit` walks with its column tiles on one XCD.
-// Returns the rounds' steps, of all places there are, over the segments' own.
-double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, int every, double walk_ends, PlaneLaunch &L)
+// work divides evenly, at multiples of `every` from the segment's first (plane_cut).  Between two ends of groups' ranges the
+// groups are the same.  How many: workgroups run in rounds of 32 CUs per XCD, a unit of `unit` walks with its column tiles on
+// one XCD (plane_over, which returns the rounds' steps, of all places there are, over the segments' own).
+double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, double walk_ends, PlaneLaunch &L)
 {
-    const std::vector<int> &ends = spans.ends, &groups = spans.groups;
     const long long work = spans.work;
     const int full = L.tp / unit, part = L.tp % unit, cap = 32 * per_cu;
     auto rounds = [&](int segs) {
@@ -432,6 +431,15 @@ double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, in
             n = i;
         }
     }
+    L.nseg = n;
+    return best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
+}
+
+void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
+{
+    const std::vector<int> &ends = spans.ends, &groups = spans.groups;
+    const long long work = spans.work;
+    const int n = L.nseg;
     L.nseg = 0;
     long long done = 0;
     size_t i = 0;
@@ -447,7 +455,6 @@ double plane_cut(const PlaneSpans &spans, int walk_len, int unit, int per_cu, in
         if (cut > last && cut < walk_len) L.cuts.at[++L.nseg] = cut;
     }
     L.cuts.at[++L.nseg] = walk_len;
-    return best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
 }
 
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
@@ -469,7 +476,7 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
     const int walk_len = (int)(n_out / wk.period);
 
-    const double over = plane_cut(spans, walk_len, PLANE_XT, per_cu, 1, 0.9 * (wk.k - 1) * spans.most, L);
+    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, 0.9 * (wk.k - 1) * spans.most, L);
     // Taken where the steps come to at most 1.65 times the segments' work (5 x 5 and 7 x 7 windows: 1.4 times), with two column
     // tiles at least -- with one, the values are most of the traffic, and the tile-by-tile kernel fetches them in pieces twice
     // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
@@ -484,7 +491,9 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     // and 9 x 9 layers with a bias or an activation.
     const double padded = over * L.col_tiles * 64 / batch * L.tp * PLANE_ROWS / wk.period;
     const bool full = wk.k <= 11 && (!fused || wk.k == 5 || wk.k == 11) && padded <= 1.8;
-    return force || many || full;
+    if (!force && !many && !full) return false;
+    plane_cut(spans, walk_len, 1, L);
+    return true;
 }
 
 }  // namespace cuvdia

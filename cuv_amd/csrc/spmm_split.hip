@@ -608,14 +608,17 @@ bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force,
     L.tp = (wk.period + S::XS - 1) / S::XS;
     // (a segment that has the end of a map in it walks both maps' ends)
     const double walk_ends = 0.9 * (wk.k - 1) * spans.most * (spans.groups.size() > 1 ? 2 : 1);
-    const double over = plane_cut(spans, (int)(n_out / wk.period), 128 / S::XS, 2, S::PY, walk_ends, L);
+    const int walk_len = (int)(n_out / wk.period);
+    const double over = plane_over(spans, walk_len, 128 / S::XS, 2, walk_ends, L);
     // Taken where the rounds' steps, with the columns and positions that only fill tiles up, come to at most 1.8 times the segments'
     // own.  Measured on 374 random products of 13 x 13 windows, 1 to 5 maps, 40 to 640 wide, batch 24 to 640, a third of them with
     // bias and sigmoid: of the last 260 it takes 56, at 0.94 - 2.4 times the rate of the kernels that served them (one below
     // 0.97; median 1.17, with bias and sigmoid 1.4); forced on the first 114, at most 1.8: median 1.2, above: 0.48 - 2.2, a fifth
     // below 0.9.
     const double padded = over * L.col_tiles * S::COLS / batch * L.tp * S::XS / wk.period;
-    return force || padded <= 1.8;
+    if (!force && padded > 1.8) return false;
+    plane_cut(spans, walk_len, S::PY, L);
+    return true;
 }
 
 }  // namespace cuvdia

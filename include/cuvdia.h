@@ -362,7 +362,7 @@ int cuvdia_cache_clear(void);
  * that is no window table with a walking kernel; densedense_to_dia treats it
  * as CUVDIA_PATH_TILED_NOWALK); CUVDIA_PATH_PLANE likewise, for the product
  * walked on the matrix cores (densedense_to_dia: the projection on the matrix
- * cores for windows of 9 x 9 and 11 x 11, else as CUVDIA_PATH_TILED_NOWALK).
+ * cores for windows of 9 x 9, 11 x 11 and 13 x 13, else as CUVDIA_PATH_TILED_NOWALK).
  * CUVDIA_PATH_WINDOW: the kernels tiled in the
  * window's plane, which serve densedense_to_dia (CUVDIA_EUNSUPPORTED when
  * they do not serve the request: no window table of chunks of 2 to 13
@@ -377,7 +377,8 @@ int cuvdia_set_path(int path);
  * (CUVDIA_PATH_GENERIC, CUVDIA_PATH_TILED, CUVDIA_PATH_WALK for a product
  * served by the walking kernel, CUVDIA_PATH_PLANE by the ones on the matrix
  * cores, CUVDIA_PATH_WINDOW for a projection served
- * by the kernel tiled in the window's plane; 0 before any call).  The kernels
+ * by the kernels tiled in the window's plane, of which the automatic choice
+ * takes one on the matrix cores for 13 x 13 windows; 0 before any call).  The kernels
  * with rows along the lanes, of which the automatic choice makes use beside
  * the tiled ones, count as CUVDIA_PATH_TILED; cuvdia_last_kernel names them. */
 int cuvdia_last_path(void);
