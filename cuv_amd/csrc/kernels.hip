@@ -3124,9 +3124,11 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
     if (path == CUVDIA_PATH_WALK) return hipErrorNotSupported;
     // One of another width, or with a larger window: the plane's walk on the matrix cores, 13 x 13 ones with split operands.
     if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_PLANE) {
-        PlaneLaunch P{};
-        const bool fused = ep.bias != nullptr || ep.act != 0, split = ep.act != 2 && spmm_split_plan(wk, n_out, batch, path == CUVDIA_PATH_PLANE, P);
-        if (split || spmm_plane_plan(wk, n_out, batch, fused, path == CUVDIA_PATH_PLANE, P)) {
+        PlaneLaunch plane{}, other{};
+        const bool force = path == CUVDIA_PATH_PLANE, walks = spmm_plane_plan(wk, n_out, batch, ep.bias != nullptr || ep.act != 0, force, plane);
+        const bool split = spmm_split_plan(wk, n_out, batch, force, walks, other);
+        if (split || walks) {
+            PlaneLaunch &P = split ? other : plane;
             if (ran) *ran = CUVDIA_PATH_PLANE;
             P.tab = wk.tab_dev; P.ngroups = wk.ngroups; P.period = wk.period; P.s0 = wk.s0; P.astep4 = wk.astep4; P.k = wk.k;
             P.vals = vals; P.B = B; P.ldb = ldb; P.dst = dst; P.ldd = ldd; P.n_out = n_out; P.n_in = n_in; P.batch = batch;

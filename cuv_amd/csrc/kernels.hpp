@@ -149,8 +149,9 @@ hipError_t spmm_plane_launch(const PlaneLaunch &L);
 // How many segments of the map rows (L.nseg; tp and col_tiles are set), and the segments (L.nseg, L.cuts).
 double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, double walk_ends, PlaneLaunch &L);
 void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L);
-// The same, windows of 13 rows, fp32 products as bfloat16 ones (spmm_split.hip); no samples.
-bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, PlaneLaunch &L);
+// The same, windows of 13 rows, fp32 products as bfloat16 ones (spmm_split.hip).
+// walks: whether the former would be taken.
+bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, bool walks, PlaneLaunch &L);
 hipError_t spmm_split_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.

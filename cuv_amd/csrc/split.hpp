@@ -61,9 +61,6 @@ __device__ __forceinline__ unsigned split8(const float (&x)[8], unsigned hi_mask
 // ones (also where numbers above 2^17 meet by chance: the caller's exact way is right for any).
 __device__ __forceinline__ bool split_inexact(unsigned low) { return (low & 0xffffu) != 0u || (low & 0x7f800000u) == 0x7f800000u; }
 
-// The six products, smallest first.
-constexpr int SPLIT_A[6] = {2, 0, 1, 1, 0, 0}, SPLIT_B[6] = {0, 2, 1, 0, 1, 0};
-
 __device__ __forceinline__ split_f4 split_mfma(split_u4 a, split_u4 b, split_f4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split_b8, a), __builtin_bit_cast(split_b8, b), c, 0, 0, 0);

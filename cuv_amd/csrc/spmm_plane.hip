@@ -18,8 +18,8 @@
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
 // 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
 // 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
-// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has what spmm_split.hip leaves: samples, tables
-// of more than 19 groups, and what the rule there refuses.
+// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has what spmm_split.hip leaves: tables of more
+// than 19 groups, and what the rule there refuses.
 //
 // Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
 // ascending, acc = fma(a, x, acc).

@@ -300,6 +300,27 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
         barrier();
         const int thread = here(threadIdx.x), q = thread % S::OQ, x = 4 * q, c = thread / S::OQ;
         constexpr int CSTEP = PS_THREADS / S::OQ, PER_ROW = S::COLS / CSTEP;
+        if (EP && ep.act == 2) {
+            // sampled: a lane takes a position and 4 columns, a block of the generator
+            static_assert(S::COLS / 4 * S::XS == PS_THREADS, "a patch row at a time");
+            const int sx = thread % S::XS, c0 = thread / S::XS * 4;
+#pragma nounroll
+            for (int y = 0; y < PY; ++y) {
+                if (sx < skip || y0 + y >= rows || c0 >= cols) continue;
+                const int row = row_first + (y0 + y) * period + sx;
+                const float bias = ep.bias ? ep.bias[row] : 0.f;
+                const SpRand4 w = sp_philox((unsigned)row, (unsigned)(col0 + c0) / 4u, ep.seed_lo, ep.seed_hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (c0 + i >= cols) continue;
+                    float *const p = Y + (long long)(col0 + c0 + i) * ldy + row;
+                    const float sum = out[(y * S::COLS + c0 + i) * S::OPITCH + sx];
+                    *p = sp_finish(beta == 0.f ? alpha * sum : beta * *p + alpha * sum, bias, 2, w.w[i]);
+                }
+            }
+            barrier();
+            return;
+        }
         f4 s[S::OIT];
         unsigned at[S::OIT];
 #pragma unroll
@@ -598,7 +619,7 @@ hipError_t ps_launch_one(const PlaneLaunch &L)
 
 hipError_t spmm_split_launch(const PlaneLaunch &L) { return ps_launch_one<13, 13>(L); }
 
-bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, PlaneLaunch &L)
+bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, bool walks, PlaneLaunch &L)
 {
     using S = PsShape<13, 13>;
     if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.k != 13 || wk.lck != 13 || wk.ngroups * 13 > 256 || wk.period < 32) return false;
@@ -610,13 +631,14 @@ bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force,
     const double walk_ends = 0.9 * (wk.k - 1) * spans.most * (spans.groups.size() > 1 ? 2 : 1);
     const int walk_len = (int)(n_out / wk.period);
     const double over = plane_over(spans, walk_len, 128 / S::XS, 2, walk_ends, L);
-    // Taken where the rounds' steps, with the columns and positions that only fill tiles up, come to at most 1.8 times the segments'
-    // own.  Measured on 374 random products of 13 x 13 windows, 1 to 5 maps, 40 to 640 wide, batch 24 to 640, a third of them with
-    // bias and sigmoid: of the last 260 it takes 56, at 0.94 - 2.4 times the rate of the kernels that served them (one below
-    // 0.97; median 1.17, with bias and sigmoid 1.4); forced on the first 114, at most 1.8: median 1.2, above: 0.48 - 2.2, a fifth
-    // below 0.9.
+    // Taken where the rounds' steps, with the columns and positions that only fill tiles up, come to at most 2.1 times the
+    // segments' own where the tile-by-tile kernel would run, 1.65 times where the plane's walk would.  Measured on 210 random
+    // products of 13 x 13 windows, 1 to 5 maps, 40 to 640 wide, batch 24 to 640, a third of them with bias and sigmoid: 79 are
+    // taken, at 0.91 - 4.8 times the rate of the kernels that served them (one below 0.97; median 1.29, with bias and sigmoid
+    // 1.43; samples 0.98 - 1.28).  Forced on 111 others: up to these lines 4 % below 0.97 in place of the tile-by-tile kernel, beyond
+    // them more than a third.
     const double padded = over * L.col_tiles * S::COLS / batch * L.tp * S::XS / wk.period;
-    if (!force && padded > 1.8) return false;
+    if (!force && padded > (walks ? 1.65 : 2.1)) return false;
     plane_cut(spans, walk_len, S::PY, L);
     return true;
 }

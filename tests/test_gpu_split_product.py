@@ -114,7 +114,7 @@ def test_graph_replay(oracle):
     (512, 512, 1, 64, "", True),          # one column tile
     (96, 96, 1, 64, "", False),           # few workgroups
     (256, 256, 1, 24, "", False),         # most columns of a tile empty
-    (256, 256, 1, 256, "sample", False),
+    (256, 256, 1, 256, "sample", True),
 ])
 def test_the_automatic_choice(px, py, maps_out, batch, act, taken):
     import torch
