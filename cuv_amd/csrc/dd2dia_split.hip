@@ -18,10 +18,12 @@
 // batch 357 421 -> 327; 200 x 200, 2 maps to 2, batch 256 357 -> 214; 272 x 272 to 2, batch 388 413 -> 346.  Windows of 7 to 11
 // rows have fewer products for the same loads and fewer of them are slots: 0.5 - 0.95 times the kernels that serve them.
 //
-// Accumulation order: of every 16 columns the six products of all columns, smallest first, rounded towards zero as the matrix
-// core does; these sums in fp32, columns ascending.  Error against 64 bits
-// (2-norm, relative; uniform operands in -1 .. 1) at batch 37, 256 and 2048: 0.7, 1.0 and 2.2e-7, where a chain of fp32 FMAs has
-// 1.2, 2.9 and 8.1e-7.
+// Accumulation order: of every 16 columns the six products of all columns, smallest first, rounded as the matrix core does
+// (split.hpp); these sums in fp32, columns ascending.  Error against 64 bits (2-norm, relative; uniform operands in -1 .. 1) at
+// batch 37, 128, 256 and 2048: 0.5, 0.7, 0.9 and 2.2e-7, where a chain of fp32 FMAs has 1.1, 2.0, 2.9 and 8.1e-7.  Sums of 1, 2,
+// 4, 8 and 16 products spread over 128 columns: 3.1, 4.1, 5.1, 5.9 and 6.6e-8, the chain 2.5, 3.1, 4.0, 5.4 and 7.4e-8: a sum of
+// few is rounded where the others' meet the first parts' products and again where the blocks of 16 columns meet.  (First parts'
+// products as a fourth instruction, a sum of their own: 2.5, 3.4, 4.4, 5.4 and 6.2e-8, and 838 -> 918 us on the first case above.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -130,13 +132,12 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
     // As the matrix instruction has its operands: lane (m, kg) holds 8 columns of position m of a patch, of one part for kg < 2
     // and of another for the other half.  A wave's two patches of A lie one below the other.
     const int m16 = lane % 16, kg = lane / 16, at = kg % 2 * 256 + m16 * 16;
-    const unsigned char *const b12 = lds + wave * S::PATCH + at + (kg < 2 ? 0 : S::PART), *const b31 = lds + wave * S::PATCH + at + (kg < 2 ? 2 * S::PART : 0);
+    const unsigned char *const b21 = lds + wave * S::PATCH + at + (kg < 2 ? S::PART : 0), *const b31 = lds + wave * S::PATCH + at + (kg < 2 ? 2 * S::PART : 0);
     const unsigned char *const a11 = lds + (S::NBX * S::NBY + wave) * S::PATCH + at, *const a13 = a11 + (kg < 2 ? 0 : 2 * S::PART);
     unsigned *const flags = reinterpret_cast<unsigned *>(lds + S::FLAGS);
     int *const row_tab = reinterpret_cast<int *>(lds + S::TAB);
     if (threadIdx.x < K) row_tab[threadIdx.x] = tab[ngroups + g * K + threadIdx.x] / 4;
-    unsigned hi_mask;
-    asm volatile("v_mov_b32 %0, 0xffff0000" : "=v"(hi_mask));
+    const SplitConst split_const;
 
     f4 st[8];
     auto request = [&](auto first_, auto last_, int c) __attribute__((always_inline)) {
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             for (int e = 0; e < 4; ++e) {
                 const float v[8] = {st[0][e], st[1][e], st[2][e], st[3][e], st[4][e], st[5][e], st[6][e], st[7][e]};
                 u4 p[3];
-                low |= split8(v, hi_mask, p);
+                low |= split8(v, split_const, p);
                 asm volatile("" : "+v"(low));
 #pragma unroll
                 for (int s = 0; s < 3; ++s) *reinterpret_cast<u4 *>(to + s * S::PART + e * 16) = p[s];
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float *>(lds + S::RAW + j * 1024 + t * 4);
             unsigned char *const there = lds + (S::NBX * S::NBY + quad / (DS_XT / 4) / 4 * (DS_XT / 4) + quad % (DS_XT / 4)) * S::PATCH + 256 + quad / (DS_XT / 4) % 4 * 64 + pos * 16;
             u4 p[3];
-            low |= split8(v, hi_mask, p);
+            low |= split8(v, split_const, p);
 #pragma unroll
             for (int s = 0; s < 3; ++s) *reinterpret_cast<u4 *>(there + s * S::PART) = p[s];
         }
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             constexpr int t = decltype(t_)::value, at = (t / S::BX * S::NBX + t % S::BX) * S::PATCH;
             if constexpr (t < TILES) {
                 bf[t % 2][0] = *reinterpret_cast<const u4 *>(b31 + at);
-                bf[t % 2][1] = *reinterpret_cast<const u4 *>(b12 + at);
+                bf[t % 2][1] = *reinterpret_cast<const u4 *>(b21 + at);
             }
         };
         fetch(std::integral_constant<int, 0>{});
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             request(std::integral_constant<int, S::LOADS * t / TILES>{}, std::integral_constant<int, S::LOADS * (t + 1) / TILES>{}, c + DS_COLS);
             f4 sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
             if (__builtin_expect(!exact, 1)) {
-                // the six products: a1 b3 + a3 b1, a2 b1 + a2 b2, a1 b1 + a1 b2
+                // the six products: a1 b3, a3 b1; a2 b2, a2 b1; a1 b2, a1 b1
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
 #pragma unroll

@@ -1,9 +1,16 @@
 // fp32 products on the matrix cores' bfloat16 instructions.
 //
-// A number is held as the sum of three bfloat16 numbers, its top 8 significant bits, the next 8 and the last 8: exactly, unless
-// it is infinite, a NaN or so small (below 2^-110) that the last part is no bfloat16 number.  Of the nine products of two such
-// sums the six largest are made -- each exact, as 8 bits times 8 bits are 16 --; what is left out is below 2^-24 of the product,
-// 2^-25 on average.
+// A number is held as the sum of three bfloat16 numbers (the triple-bfloat16 splitting of Henry, Tang and Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations", 2019): the nearest one, the one nearest to
+// what that leaves, and the rest, which has at most 7 bits: exactly, unless it is infinite, a NaN, within half a unit of
+// bfloat16's largest number or so small (below 2^-110) that the rest is no bfloat16 number.  Of the nine products of two such sums the six
+// largest are made -- each exact, as 8 bits times 8 bits are 16 --; what is left out is at most 2^-24 of the product, 2^-27.5 in
+// the quadratic mean of uniform numbers, of either sign alike (parts cut off instead: up to 2^-21, 2^-24.7 in the mean, and always
+// towards zero).  Products within 2^-7 of the largest number may overflow, as their first parts' do.
+//
+// What the matrix core does with them, measured: 8 products at a time, columns ascending, what lies more than 24 bits below the
+// largest of the 8 cut off, of the sum so far towards minus infinity; the new sum to the nearest fp32 number.  (Numbers below the normal ones
+// are kept, among the parts and in the sums.)  Hence the small products first: only the first parts' sum is rounded at its own size.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -22,36 +29,58 @@ __device__ __forceinline__ int here(int lane)
     return lane;
 }
 
-// Two numbers' parts, a pair of bfloat16 numbers each.  Returns the last parts' bits, for split_inexact().  hi_mask is
-// 0xffff0000 in a vector register: an instruction with a scalar operand takes twice as long.
-__device__ __forceinline__ unsigned split2(float x0, float x1, unsigned hi_mask, unsigned &p0, unsigned &p1, unsigned &p2)
+// Two numbers to two bfloat16 ones, the nearest each.
+__device__ __forceinline__ unsigned split_near(float x0, float x1)
 {
-    const unsigned b0 = __builtin_bit_cast(unsigned, x0), b1 = __builtin_bit_cast(unsigned, x1);
-    const float r0 = x0 - __builtin_bit_cast(float, b0 & hi_mask), r1 = x1 - __builtin_bit_cast(float, b1 & hi_mask);
-    const unsigned c0 = __builtin_bit_cast(unsigned, r0), c1 = __builtin_bit_cast(unsigned, r1);
-    const unsigned d0 = __builtin_bit_cast(unsigned, r0 - __builtin_bit_cast(float, c0 & hi_mask));
-    const unsigned d1 = __builtin_bit_cast(unsigned, r1 - __builtin_bit_cast(float, c1 & hi_mask));
-    p0 = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-    p1 = __builtin_amdgcn_perm(c1, c0, 0x07060302u);
-    p2 = __builtin_amdgcn_perm(d1, d0, 0x07060302u);
-    return d0 | d1;
+    unsigned p;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(p) : "v"(x0), "v"(x1));
+    return p;
 }
-__device__ __forceinline__ unsigned split4(split_f4 x, unsigned hi_mask, split_u2 (&p)[3])
+// What such a pair leaves of its numbers, exactly.  (Constants in vector registers: an instruction with a scalar operand or one
+// of its own takes twice as long.)
+struct SplitConst {
+    unsigned hi_mask, half;
+    __device__ __forceinline__ SplitConst() { asm volatile("v_mov_b32 %0, 0xffff0000\n\tv_mov_b32 %1, 16" : "=&v"(hi_mask), "=v"(half)); }
+};
+__device__ __forceinline__ void split_rest(unsigned p, const SplitConst &k, float &x0, float &x1)
 {
-    unsigned a, b, c, low = split2(x[0], x[1], hi_mask, a, b, c);
-    p[0][0] = a; p[1][0] = b; p[2][0] = c;
-    low |= split2(x[2], x[3], hi_mask, a, b, c);
-    p[0][1] = a; p[1][1] = b; p[2][1] = c;
+    x0 -= __builtin_bit_cast(float, p << k.half);
+    x1 -= __builtin_bit_cast(float, p & k.hi_mask);
+}
+__device__ __forceinline__ unsigned split_last(float x0, float x1, unsigned &low)
+{
+    const unsigned d0 = __builtin_bit_cast(unsigned, x0), d1 = __builtin_bit_cast(unsigned, x1);
+    low |= d0 | d1;
+    return __builtin_amdgcn_perm(d1, d0, 0x07060302u);
+}
+// Two numbers' parts, a pair of bfloat16 numbers each; the last parts' bits are added to low, for split_inexact().
+__device__ __forceinline__ void split2(float x0, float x1, const SplitConst &k, unsigned &p0, unsigned &p1, unsigned &p2, unsigned &low)
+{
+    p0 = split_near(x0, x1);
+    split_rest(p0, k, x0, x1);
+    p1 = split_near(x0, x1);
+    split_rest(p1, k, x0, x1);
+    p2 = split_last(x0, x1, low);
+}
+__device__ __forceinline__ unsigned split4(split_f4 x, const SplitConst &k, split_u2 (&p)[3])
+{
+    unsigned low = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        unsigned a, b, c;
+        split2(x[2 * i], x[2 * i + 1], k, a, b, c, low);
+        p[0][i] = a; p[1][i] = b; p[2][i] = c;
+    }
     asm volatile("" : "+v"(low));                    // (here: the compiler would keep every last part for later)
     return low;
 }
-__device__ __forceinline__ unsigned split8(const float (&x)[8], unsigned hi_mask, split_u4 (&p)[3])
+__device__ __forceinline__ unsigned split8(const float (&x)[8], const SplitConst &k, split_u4 (&p)[3])
 {
     unsigned low = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         unsigned a, b, c;
-        low |= split2(x[2 * i], x[2 * i + 1], hi_mask, a, b, c);
+        split2(x[2 * i], x[2 * i + 1], k, a, b, c, low);
         p[0][i] = a; p[1][i] = b; p[2][i] = c;
     }
     asm volatile("" : "+v"(low));

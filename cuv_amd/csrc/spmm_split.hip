@@ -18,10 +18,11 @@
 // batch 256 556 -> 407; 448 x 448, 2 maps to 3, batch 64 560 -> 361; 416 x 416, transposed, batch 357 444 -> 426.
 // Windows of 11 rows use 47 % of a patch's products: level with the fp32 kernel.
 //
-// Accumulation order: of every 32 dense rows (16 of two map rows) the products of parts, rounded towards zero as the matrix
-// core does; these sums in fp32, map rows ascending.  Error against 64 bits (2-norm,
-// relative) of 1, 2 and 4 maps' sums, values of a normal distribution: 0.8, 1.0 and 1.2e-7 with uniform rows, 0.7, 0.9 and 1.1e-7
-// with binary ones, where a chain of fp32 FMAs has 2.3, 3.3 and 4.6e-7, 1.7, 2.3 and 3.3e-7.
+// Accumulation order: of every 32 dense rows (16 of two map rows) the products of parts, smallest first, rounded as the matrix
+// core does (split.hpp); these sums in fp32, map rows ascending.  Error against 64 bits (2-norm, relative), normal values, one
+// map's sums of 1, 2, 3, 7, 19 and 169 uniform rows that are not 0: 3.3, 4.2, 4.4, 4.8, 5.7 and 6.4e-8, where a chain of fp32 FMAs
+// has 2.6, 3.6, 4.0, 5.0, 8.0 and 22.6e-8; of binary rows 0.5, 3.6, 4.1, 4.7, 5.7 and 6.3e-8, the chain 0.5, 3.6, 4.0, 5.3, 8.0 and
+// 23.5e-8.  (First parts' products as a sum of their own: 2.6, 3.4, 3.6, 4.1, 5.2 and 7.0e-8, and 2 - 5 % more time.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -96,26 +97,24 @@ __device__ __forceinline__ void ps_load(sp_int4 rsrc, unsigned to, unsigned voff
 
 // A pair of numbers on its way into three parts, a step at a time
 struct PsPair {
-    unsigned b0, b1, c0, c1, d0, d1;
-    __device__ __forceinline__ unsigned first(float x0, float x1, unsigned hi_mask)
+    float x0, x1;
+    unsigned p;
+    __device__ __forceinline__ unsigned first(float v0, float v1)
     {
-        b0 = __builtin_bit_cast(unsigned, x0); b1 = __builtin_bit_cast(unsigned, x1);
-        c0 = __builtin_bit_cast(unsigned, x0 - __builtin_bit_cast(float, b0 & hi_mask));
-        c1 = __builtin_bit_cast(unsigned, x1 - __builtin_bit_cast(float, b1 & hi_mask));
-        return __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        x0 = v0; x1 = v1;
+        return p = split_near(x0, x1);
     }
-    __device__ __forceinline__ unsigned second(unsigned hi_mask)
+    __device__ __forceinline__ unsigned second(const SplitConst &k)
     {
-        const float r0 = __builtin_bit_cast(float, c0), r1 = __builtin_bit_cast(float, c1);
-        d0 = __builtin_bit_cast(unsigned, r0 - __builtin_bit_cast(float, c0 & hi_mask));
-        d1 = __builtin_bit_cast(unsigned, r1 - __builtin_bit_cast(float, c1 & hi_mask));
-        return __builtin_amdgcn_perm(c1, c0, 0x07060302u);
+        split_rest(p, k, x0, x1);
+        return p = split_near(x0, x1);
     }
-    __device__ __forceinline__ unsigned third(unsigned &low)
+    __device__ __forceinline__ unsigned third(const SplitConst &k, unsigned &low)
     {
-        low |= d0 | d1;
+        split_rest(p, k, x0, x1);
+        const unsigned last = split_last(x0, x1, low);
         asm volatile("" : "+v"(low));
-        return __builtin_amdgcn_perm(d1, d0, 0x07060302u);
+        return last;
     }
 };
 
@@ -171,8 +170,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
     auto block_row = [&](int u, int g) { return row_first + s0 + __builtin_amdgcn_readlane(group_lane, g) + 2 * u * period; };
     auto outside = [&](int x0) { return x0 + period + S::XS + LC - 1 <= 0 || x0 >= n_in; };
     auto inside = [&](int x0) { return x0 >= 0 && x0 + period + 4 * S::NQ <= n_in; };
-    unsigned hi_mask;
-    asm volatile("v_mov_b32 %0, 0xffff0000" : "=v"(hi_mask));
+    const SplitConst split_const;
     unsigned *const flags = reinterpret_cast<unsigned *>(lds + S::FLAGS);
 
     // The blocks (u, g) in order: one multiplied, the next one split, the one after that requested.  Of the groups only those
@@ -395,7 +393,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrsrc, c < cols && xr >= 0 && xr < n_in ? (unsigned)c * ldx4 + 4u * xr : OOB_OFFSET, 0, 0));
             }
             u2 p[3];
-            low |= split4(x, hi_mask, p);
+            low |= split4(x, split_const, p);
             more |= p[1][0] | p[1][1];
 #pragma unroll
             for (int s = 0; s < 3; ++s) *reinterpret_cast<u2 *>(lds + buf * S::X_BYTES + s * S::XSB + r * S::XRB + q * S::XQB + c * 8) = p[s];
@@ -500,7 +498,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
             ps_for<0, 8>([&](auto j_) __attribute__((always_inline)) {
                 constexpr int j = decltype(j_)::value;
                 unsigned p0, p1, p2;
-                low |= split2(v[j][0], v[j][1], hi_mask, p0, p1, p2);
+                split2(v[j][0], v[j][1], split_const, p0, p1, p2, low);
                 af[0][j / 4][0][j % 4] = p0; af[0][j / 4][1][j % 4] = p1; af[0][j / 4][2][j % 4] = p2;
             });
             if (__any(split_inexact(low))) exact(std::integral_constant<int, 0>{});
@@ -542,12 +540,12 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 if constexpr (pass == 0) {
                     constexpr int j = 2 * (i / 3), ar = j / 4, aj = j % 4;
                     if constexpr (i % 3 == 0) {
-                        af[1][ar][0][aj] = ap.first(v[j][0], v[j][1], hi_mask);
-                        af[1][ar][0][aj + 1] = aq.first(v[j + 1][0], v[j + 1][1], hi_mask);
+                        af[1][ar][0][aj] = ap.first(v[j][0], v[j][1]);
+                        af[1][ar][0][aj + 1] = aq.first(v[j + 1][0], v[j + 1][1]);
                     }
                     if constexpr (i % 3 == 1) {
-                        af[1][ar][1][aj] = ap.second(hi_mask);
-                        af[1][ar][1][aj + 1] = aq.second(hi_mask);
+                        af[1][ar][1][aj] = ap.second(split_const);
+                        af[1][ar][1][aj + 1] = aq.second(split_const);
                         if constexpr (j == 2) values_at(std::integral_constant<int, 1>{}, 1, u);
                         if constexpr (j < 6) {
                             values_of(std::integral_constant<int, (j + 2) % 4>{}, v[j + 2]);
@@ -555,14 +553,14 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                         }
                     }
                     if constexpr (i % 3 == 2) {
-                        af[1][ar][2][aj] = ap.third(low);
-                        af[1][ar][2][aj + 1] = aq.third(low);
+                        af[1][ar][2][aj] = ap.third(split_const, low);
+                        af[1][ar][2][aj + 1] = aq.third(split_const, low);
                     }
                 }
                 constexpr int xj = i / 3, piece = 2 * pass + xj / 2, xh = xj % 2;
-                if constexpr (i % 3 == 0) xq[0][xh] = xp.first(xst[piece][2 * xh], xst[piece][2 * xh + 1], hi_mask);
-                if constexpr (i % 3 == 1) xq[1][xh] = xp.second(hi_mask);
-                if constexpr (i % 3 == 2) xq[2][xh] = xp.third(low_x);
+                if constexpr (i % 3 == 0) xq[0][xh] = xp.first(xst[piece][2 * xh], xst[piece][2 * xh + 1]);
+                if constexpr (i % 3 == 1) xq[1][xh] = xp.second(split_const);
+                if constexpr (i % 3 == 2) xq[2][xh] = xp.third(split_const, low_x);
                 if constexpr (i % 3 == 2 && xh == 1) {
                     more_x |= xq[1][0] | xq[1][1];
 #pragma unroll
