@@ -150,6 +150,11 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             }
         });
     };
+    // (where a thread of the first four waves puts a position's second 8 columns of A)
+    auto second = [&](int t) __attribute__((always_inline)) {
+        const int quad = t / 4;
+        return lds + (S::NBX * S::NBY + quad / (DS_XT / 4) / 4 * (DS_XT / 4) + quad % (DS_XT / 4)) * S::PATCH + 256 + quad / (DS_XT / 4) % 4 * 64 + t % 4 * 16;
+    };
     auto place = [&]() __attribute__((always_inline)) {
         unsigned low = 0;
         if (ends) {
@@ -174,17 +179,20 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
         }
         // (A's second columns: a position's 8 a thread, four waves)
         if (wave < 4) {
-            const int t = here(thread), quad = t / 4, pos = t % 4;
+            const int t = here(thread);
             float v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const float *>(lds + S::RAW + j * 1024 + t * 4);
-            unsigned char *const there = lds + (S::NBX * S::NBY + quad / (DS_XT / 4) / 4 * (DS_XT / 4) + quad % (DS_XT / 4)) * S::PATCH + 256 + quad / (DS_XT / 4) % 4 * 64 + pos * 16;
+            unsigned char *const there = second(t);
             u4 p[3];
             low |= split8(v, split_const, p);
 #pragma unroll
             for (int s = 0; s < 3; ++s) *reinterpret_cast<u4 *>(there + s * S::PART) = p[s];
         }
-        const bool bad = __any(split_inexact(low));
+        const bool bad = split_inexact<5>(low, [&](int i) __attribute__((always_inline)) {
+            if (i < 4 ? !have : wave >= 4) return u4{0u, 0u, 0u, 0u};
+            return *reinterpret_cast<const u4 *>((i < 4 ? to + i * 16 : second(here(thread))) + 2 * S::PART);
+        });
         if (lane == 0) flags[wave] = bad;
     };
     auto barrier = [&]() __attribute__((always_inline)) {

@@ -53,7 +53,7 @@ __device__ __forceinline__ unsigned split_last(float x0, float x1, unsigned &low
     low |= d0 | d1;
     return __builtin_amdgcn_perm(d1, d0, 0x07060302u);
 }
-// Two numbers' parts, a pair of bfloat16 numbers each; the last parts' bits are added to low, for split_inexact().
+// Two numbers' parts, a pair of bfloat16 numbers each; the last parts' bits are added to low, for split_inexact.
 __device__ __forceinline__ void split2(float x0, float x1, const SplitConst &k, unsigned &p0, unsigned &p1, unsigned &p2, unsigned &low)
 {
     p0 = split_near(x0, x1);
@@ -86,9 +86,22 @@ __device__ __forceinline__ unsigned split8(const float (&x)[8], const SplitConst
     asm volatile("" : "+v"(low));
     return low;
 }
-// Whether, by the last parts' bits, some number was not held exactly: bits below a bfloat16 number's, or an exponent of all
-// ones (also where numbers above 2^17 meet by chance: the caller's exact way is right for any).
-__device__ __forceinline__ bool split_inexact(unsigned low) { return (low & 0xffffu) != 0u || (low & 0x7f800000u) == 0x7f800000u; }
+// Whether some number was not held exactly, by its wave's lanes' last parts: bits below a bfloat16 number's, or a NaN.  low: their
+// bits; last(i), i < N: four pairs of them, asked for only where the exponents make up all ones, as those of numbers on both sides of
+// 2^17 do together.
+template <int N, class Last>
+__device__ __forceinline__ bool split_inexact(unsigned low, Last &&last)
+{
+    if (__builtin_expect(!__any((low & 0xffffu) != 0u || (low & 0x7f800000u) == 0x7f800000u), 1)) return false;
+    unsigned bad = low & 0xffffu;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const split_u4 pairs = last(i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bad |= ((pairs[j] & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+    }
+    return __any(bad != 0u);
+}
 
 __device__ __forceinline__ split_f4 split_mfma(split_u4 a, split_u4 b, split_f4 c)
 {

@@ -373,7 +373,12 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
 
     // A block's flags: 1: not all of its dense rows are held exactly; 2: not all are bfloat16 numbers
     auto raise = [&](int buf, unsigned low, unsigned more) __attribute__((always_inline)) {
-        const unsigned f = (__any(split_inexact(low)) ? 1u : 0u) | (__any(more != 0u) ? 2u : 0u);
+        const bool bad = split_inexact<PIECES / 2>(low, [&](int i) __attribute__((always_inline)) {
+            const unsigned char *const at = x_to + buf * S::X_BYTES + 2 * S::XSB + 2 * i * (8 * S::XC * PS_WAVES);
+            const u2 p0 = *reinterpret_cast<const u2 *>(at), p1 = *reinterpret_cast<const u2 *>(at + 8 * S::XC * PS_WAVES);
+            return u4{p0[0], p0[1], p1[0], p1[1]};
+        });
+        const unsigned f = (bad ? 1u : 0u) | (__any(more != 0u) ? 2u : 0u);
         if (lane == 0) flags[4 * buf + wave] = f;
     };
     // The values of a block that crosses an end of the operand, and such a block's or the first one's dense rows: element by
@@ -501,7 +506,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 split2(v[j][0], v[j][1], split_const, p0, p1, p2, low);
                 af[0][j / 4][0][j % 4] = p0; af[0][j / 4][1][j % 4] = p1; af[0][j / 4][2][j % 4] = p2;
             });
-            if (__any(split_inexact(low))) exact(std::integral_constant<int, 0>{});
+            if (split_inexact<2>(low, [&](int i) __attribute__((always_inline)) { return af[0][i][2]; })) exact(std::integral_constant<int, 0>{});
         }
         request(third);
         ps_for<0, 2>([&](auto pass_) __attribute__((always_inline)) {
@@ -570,7 +575,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 __builtin_amdgcn_sched_barrier(0);
             });
             if constexpr (pass == 0) {
-                if (__any(split_inexact(low))) exact(std::integral_constant<int, 1>{});
+                if (split_inexact<2>(low, [&](int i) __attribute__((always_inline)) { return af[1][i][2]; })) exact(std::integral_constant<int, 1>{});
             }
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
