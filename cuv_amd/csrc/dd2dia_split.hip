@@ -104,8 +104,8 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
     const __amdgpu_buffer_rsrc_t cr = __builtin_amdgcn_make_buffer_rsrc(C, 0, c_bytes, 0x00020000);
     const unsigned lda4 = (unsigned)lda * 4u, ldb4 = (unsigned)ldb * 4u;
 
-    // Columns past the batch and rows outside the operands lie out of the resources' range (0) or in a neighbouring
-    // column (slots that are not stored).
+    // Columns past the batch lie out of the resources' range (0).  Rows outside the operands are not asked for, and are 0 as
+    // well: what memory holds there must not decide whether the split holds a stage's numbers.
 
     // This thread's task of a stage: the first of its 4 rows, its 8 columns, the place of the first row's.
     const int thread = threadIdx.x;
@@ -120,11 +120,13 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
     const int row_wanted = (of_a ? i_tile : i_tile + s_g) + quad_y * period + 4 * quad_x;
     const int row = of_a ? row_wanted : row_wanted < 0 && row_wanted > -4 ? 0 : row_wanted > w - 4 && row_wanted < w ? w - 4 : row_wanted;
     const int moved = row_wanted - row;
-    const unsigned off = have ? (unsigned)row * 4u + (unsigned)(8 * kq) * ld4 : OOB_OFFSET;
+    const bool inside = have && row_wanted > -4 && row_wanted < (of_a ? h : w);
+    const unsigned off = (unsigned)row * 4u + (unsigned)(8 * kq) * ld4;
     unsigned char *const to = lds + ((of_a ? S::NBX * S::NBY : 0) + quad_y / 4 * wide + quad_x) * S::PATCH + kq * 256 + quad_y % 4 * 64;
     // ... and of A's second 8 columns: a quad of the wave's column on its way to LDS, half a task from there
     const sp_int4 a_raw = raw_rsrc(A, a_bytes);
-    const unsigned raw_off = (unsigned)(i_tile + lane / (DS_XT / 4) * period + 4 * (lane % (DS_XT / 4))) * 4u + (unsigned)(8 + wave) * lda4;
+    const int raw_row = i_tile + lane / (DS_XT / 4) * period + 4 * (lane % (DS_XT / 4));
+    const unsigned raw_off = (unsigned)raw_row * 4u + (unsigned)(8 + wave) * lda4;
     const unsigned raw_to = (unsigned)(unsigned long long)(__attribute__((address_space(3))) unsigned char *)&lds[S::RAW] + 1024u * wave;
     // (a tile whose rows of B cross an end of the operand)
     const int b_first = i_tile + s_g, b_last = b_first + (4 * S::NBY - 1) * period + 4 * S::NBX - 1;
@@ -144,9 +146,9 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
         ds_for<decltype(first_)::value, decltype(last_)::value>([&](auto j_) {
             constexpr int j = decltype(j_)::value;
             if constexpr (j == 8) {
-                lds_load_b128(a_raw, raw_to, raw_off + (unsigned)c * lda4, 0);
+                lds_load_b128(a_raw, raw_to, raw_row < h ? raw_off + (unsigned)c * lda4 : OOB_OFFSET, 0);
             } else {
-                st[j] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, have ? off + (unsigned)(c + j) * ld4 : OOB_OFFSET, 0, 0));
+                st[j] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, inside ? off + (unsigned)(c + j) * ld4 : OOB_OFFSET, 0, 0));
             }
         });
     };
