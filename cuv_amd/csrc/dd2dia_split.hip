@@ -7,7 +7,8 @@
 // others are sums of their own that nobody reads, so no value of theirs, infinite or not, reaches a slot.  Every number is split
 // into three bfloat16 ones where it is staged (split.hpp), six of their nine products are made: 16 columns of two pairs of parts
 // fill an instruction's 32, three instructions are 16 columns.  What the split does not hold exactly (an infinity, a NaN, a
-// number below 2^-110) is seen there, and the stage that has it is multiplied in fp32 from memory.
+// number below 2^-110) is seen there, and the stage that has it is multiplied in fp32 from memory, 4.7 times as long where
+// every stage has some (4 maps of 256 x 256 to 4, batch 256: 4.0 ms).
 //
 // Per stage of 16 columns the loads of the next one are on their way to registers; the split, transposed, goes to LDS; a wave
 // works two patches of A.  No branch is taken in the products' loop: each taken branch cost about 30 clocks.

@@ -7,7 +7,8 @@
 // split into three bfloat16 numbers (split.hpp), the rows on their way to LDS, the values on their way from it, between the
 // products; six of the nine products of parts are made, and only the three of the rows' first parts where no row of a step
 // has others (a binary layer's units).  What the split does not hold exactly (an infinity, a NaN, a number below 2^-110) is
-// seen there, and the step that has it is multiplied in fp32.
+// seen there, and the step that has it is multiplied in fp32 on the vector unit: 6 times as long where every step has some (4
+// channels of 256 x 256 maps, batch 256, every eighth column around 2^-126: 4.4 ms), 1.06 where one number in 65536 is one.
 //
 // Two workgroups share a CU, so that one multiplies while the other waits: a step is a chain of waits (its values and rows from
 // LDS, the first pair's split, two barriers) of which a wave alone hides nothing.  Tried: one workgroup of 128 columns with 512
@@ -421,31 +422,45 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
     };
     // An operand that the split does not hold exactly -- an infinity, a NaN, a number next to the smallest ones --: the
     // block's products for a pair of patches one by one, those that the table has and no others; then zeros in its place.
+    // A lane takes a column's dense rows 4 at a time, for all the patch rows that use them.
     auto exact = [&](auto p_) __attribute__((always_inline)) {
         constexpr int p = decltype(p_)::value;
         const int l = here(lane), sx = wave * PX;            // this lane's sums: positions sx .. sx + 3 of patch rows l / 32, + 2
-        ps_for<0, 4 * NT>([&](auto n_) __attribute__((always_inline)) {
-            constexpr int n = decltype(n_)::value / 4, i4 = decltype(n_)::value % 4, a = 2 * p + i4 / 2;
-            const int t = step_of(a, cur.u), y0 = 2 * (cur.u - t), sy = 2 * (i4 % 2) + l / 32;
-            if (t >= S::NS || y0 < 0 || y0 >= rows) return;
-            const float *const col = xbase + (long long)min(32 * n + l % 32, cols - 1) * ldx;
-            f4 sum = {0.f, 0.f, 0.f, 0.f};
+        ps_for<0, NT>([&](auto n_) __attribute__((always_inline)) {
+            constexpr int n = decltype(n_)::value;
+            const unsigned col = (unsigned)min(32 * n + l % 32, cols - 1) * ldx4;
+            auto piece = [&](int xr) __attribute__((always_inline)) {
+                if (xr >= 0 && xr + 4 <= n_in) return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(xrsrc, col, 4 * xr, 0));
+                f4 x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    x[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xrsrc, xr + e >= 0 && xr + e < n_in ? col + 4u * (xr + e) : OOB_OFFSET, 0, 0));
+                return x;
+            };
 #pragma nounroll
             for (int r = 0; r < 2; ++r) {
-                const int d = 2 * t + r - sy;
-                if (d < 0 || d >= K || y0 + sy >= rows) continue;
-                const unsigned char *const from = lds + S::A0 + r * S::HALFB + d * S::SLOTB + 4 * sx;
+                const int x0 = cur.x0 + r * period + sx;
+                f4 x = piece(x0);
 #pragma nounroll
-                for (int dx = 0; dx < LC; ++dx) {
-                    const f4 w = *reinterpret_cast<const f4 *>(from + dx * S::ROWB);
-                    const int xr = cur.x0 + r * period + sx + dx;
+                for (int q = 0; q < LC; q += 4) {
+                    const f4 more = piece(x0 + min(q + 4, LC - 1));
+                    const float xs[7] = {x[0], x[1], x[2], x[3], more[0], more[1], more[2]};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (xr + i >= 0 && xr + i < n_in) sum[i] = fmaf(w[i], col[xr + i], sum[i]);
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        const int t = step_of(2 * p + i4 / 2, cur.u), y0 = 2 * (cur.u - t), sy = 2 * (i4 % 2) + l / 32, d = 2 * t + r - sy;
+                        if (t >= S::NS || y0 < 0 || d < 0 || d >= K || y0 + sy >= rows) continue;
+                        const unsigned char *const from = lds + S::A0 + r * S::HALFB + d * S::SLOTB + 4 * sx + q * S::ROWB;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (q + e >= LC) continue;
+                            const f4 w = *reinterpret_cast<const f4 *>(from + e * S::ROWB);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[p][n][4 * i4 + i] = fmaf(w[i], xs[e + i], acc[p][n][4 * i4 + i]);
+                        }
+                    }
+                    x = more;
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[p][n][4 * i4 + i] += sum[i];
         });
 #pragma unroll
         for (int r = 0; r < 2; ++r)

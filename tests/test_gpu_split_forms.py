@@ -61,3 +61,27 @@ def test_gradient_bits_do_not_depend_on_what_lies_between_the_columns(px, rows, 
         _forced(lambda: D.densedense_to_dia(m, bd, a, b, 0.5, 0.0), b"dd2dia_split_kernel")
         out.append(m.vec.clone())
     assert torch.equal(*out)
+
+
+def test_price_of_numbers_that_no_three_parts_hold():
+    """A product whose every step has them: 6 times an ordinary one's time as measured, and 66 times where each dense row of a column was
+    fetched by itself."""
+    import torch
+    from cuv_amd import dia as D
+    n_in, n_out, batch = 40000 * 2, 40000, 128
+    m = _dia(n_out, n_in, _offsets(200, 200, 1, 2))
+    m.vec.normal_()
+    X, out, best = _rand(1, batch, n_in), torch.empty((batch, n_out), device="cuda:0"), []
+    for tiny in (False, True):
+        if tiny:
+            X[::8] *= 2.0 ** -126
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        times = []
+        for _ in range(4):
+            e[0].record()
+            _forced(lambda: D.prod(out, m, X, "n", sync=False), b"spmm_split_kernel")
+            e[1].record()
+            torch.cuda.synchronize()
+            times.append(e[0].elapsed_time(e[1]))
+        best.append(min(times))
+    assert best[1] < 16 * best[0], best
