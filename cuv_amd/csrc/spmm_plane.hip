@@ -18,8 +18,8 @@
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
 // 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
 // 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
-// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has what spmm_split.hip leaves: tables of more
-// than 19 groups, and what the rule there refuses.
+// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has the products without bias and activation
+// that spmm_split.hip's rule leaves (the bound there on filled tiles).
 //
 // Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
 // ascending, acc = fma(a, x, acc).
@@ -388,8 +388,12 @@ hipError_t plane_launch_one(const PlaneLaunch &L)
                       L.nseg, L.cuts, L.vals, L.B, L.ldb, L.dst, L.ldd, L.n_out, L.n_in, L.batch, L.alpha, L.beta,
                       L.col_tiles, L.a_bytes, L.ep);
     };
-    if (fused) go(spmm_plane_kernel<LC, K, true>);
-    else go(spmm_plane_kernel<LC, K, false>);
+    if constexpr (K < 13) {
+        if (fused) go(spmm_plane_kernel<LC, K, true>);
+        else go(spmm_plane_kernel<LC, K, false>);
+    } else {
+        go(spmm_plane_kernel<LC, K, false>);         // (fused: spmm_plane_plan leaves them to spmm_split.hip)
+    }
     return hipGetLastError();
 }
 
@@ -459,7 +463,7 @@ void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
 
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
 {
-    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.period < PLANE_ROWS) return false;
+    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
