@@ -1,5 +1,5 @@
-"""The automatic choice of the plane's walk on either side of its rule for well-filled tiles, its result against the
-tile-by-tile kernel's."""
+"""The automatic choice of the plane's walk on either side of its rule for well-filled tiles, its result and the tile-by-tile
+kernel's against 64 bits."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 ])
 def test_well_filled_tiles(px, py, fs, maps_in, maps_out, batch, trans, fused, taken):
     import torch
+    import _gpu_util as gu
     from cuv_amd import _lib, dia as D
     m = D.filter_factory_float(px, py, fs, maps_in, maps_out).get_dia("cuda:0")
     g = torch.Generator(device="cuda:0")
@@ -36,5 +37,18 @@ def test_well_filled_tiles(px, py, fs, maps_in, maps_out, batch, trans, fused, t
         if path == _lib.PATH_AUTO:
             assert (L.cuvdia_last_path() == _lib.PATH_PLANE) == taken
         out.append(y)
-    # two fp32 sums of the same terms, at most 1225 of them below 0.6 in magnitude and 0.05 in the mean
-    torch.testing.assert_close(out[0], out[1], rtol=0, atol=1e-5 * 1225 * 0.05)
+    ref, mag = (torch.zeros((batch, n_out), dtype=torch.float64, device="cuda:0") for _ in range(2))
+    offsets = D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets().tolist()
+    vals = m.vec.view(len(offsets), -1)
+    for d, k in enumerate(offsets):
+        rows = slice(max(0, -k), min(m.h, m.w - k))
+        cols = slice(rows.start + k, rows.stop + k)
+        to, of = (cols, rows) if trans == "t" else (rows, cols)
+        term = vals[d, rows].double() * X[:, of].double()
+        ref[:, to] += term
+        mag[:, to] += term.abs()
+    tol = gu.REL_TOL * mag
+    if fused:                                            # a sigmoid's slope is 1/4 at most; itself within 8 units of the last place
+        ref, tol = torch.sigmoid(ref + bias.double()), tol / 4 + 2.0 ** -21
+    for y in out:
+        assert ((y.double() - ref).abs() <= tol).all()

@@ -85,3 +85,98 @@ def test_price_of_numbers_that_no_three_parts_hold():
             times.append(e[0].elapsed_time(e[1]))
         best.append(min(times))
     assert best[1] < 16 * best[0], best
+
+
+def _spans(h, w, offsets):
+    for d, k in enumerate(offsets):
+        rows = slice(max(0, -k), min(h, w - k))
+        if rows.stop > rows.start:
+            yield d, rows, slice(rows.start + k, rows.stop + k)
+
+
+def _exact_product(vals, X, h, w, offsets, trans):
+    """(sums, sums of magnitudes) in 64 bits"""
+    import torch
+    out = [torch.zeros((X.shape[0], w if trans == "t" else h), dtype=torch.float64, device="cuda:0") for _ in range(2)]
+    for d, rows, cols in _spans(h, w, offsets):
+        to, of = (cols, rows) if trans == "t" else (rows, cols)
+        term = vals[d, rows].double() * X[:, of].double()
+        out[0][:, to] += term
+        out[1][:, to] += term.abs()
+    return out
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+@pytest.mark.parametrize("more,lead,pad_x,pad_y,descending", [
+    (1, 0, 1, 5, False),         # value rows, columns at every remainder of 4 numbers
+    (2, 1, 2, 0, True),
+    (3, 2, 0, 3, False),
+    (0, 3, 7, 2, True),
+])
+def test_product(more, lead, pad_x, pad_y, descending, trans):
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import dia as D
+    px, rows, batch, beta = 50, 23, 37, -0.5
+    h, w = px * rows, px * rows * 2
+    offsets = _offsets(px, rows, 1, 2)[::-1 if descending else 1]
+    m = _dia(h, w, offsets, max(h, w) + more)
+    vals = m.vec.view(len(offsets), -1)
+    m.vec.fill_(float("nan"))
+    for i, (d, span, _) in enumerate(_spans(h, w, offsets)):
+        vals[d, span] = _rand(100 + i, span.stop - span.start)
+    n_in, n_out = (h, w) if trans == "t" else (w, h)
+    X, Y = _rand(1, batch, n_in), _rand(2, batch, n_out)
+    x, y = _in_columns(X, n_in + pad_x, lead, float("nan")), _in_columns(Y, n_out + pad_y, lead + 1, -7.0)
+    whole = torch.as_strided(y, (batch * (n_out + pad_y) + lead + 9,), (1,), 0)
+    _forced(lambda: D.prod(y, m, x, trans, "n", 0.75, beta), b"spmm_split_kernel")
+    ref, mag = _exact_product(vals, X, h, w, offsets, trans)
+    gu.assert_close_mag(y.cpu(), (0.75 * ref + beta * Y.double()).cpu(), (0.75 * mag + 0.5 * Y.double().abs()).cpu(), "product")
+    y.fill_(-7.0)
+    assert torch.all(whole == -7.0)                      # nothing was written beside the columns
+
+
+@pytest.mark.parametrize("lead,descending", [(1, False), (2, True), (3, False), (0, True)])
+def test_gradient(lead, descending):
+    """A at every remainder of 16 bytes, columns apart, tables in either order; the padding keeps what it held."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import dia as D
+    px, rows, batch = 44, 19, 37
+    h, w = px * rows * 2, px * rows
+    offsets = _offsets(px, rows, 2, 1)[::-1 if descending else 1]
+    m = _dia(h, w, offsets)
+    m.vec.fill_(float("nan"))
+    vals, old = m.vec.view(len(offsets), -1), {}
+    for d, span, _ in _spans(h, w, offsets):
+        vals[d, span] = old[d] = _rand(200 + d, span.stop - span.start)
+    A, B = _rand(3, batch, h), _rand(4, batch, w)
+    a, b = _in_columns(A, h + 4, lead, float("nan")), _in_columns(B, w + 8, 4, float("nan"))
+    _forced(lambda: D.densedense_to_dia(m, D.dev_block_descriptor_f(m), a, b, 0.5, 0.9), b"dd2dia_split_kernel")
+    written = torch.zeros_like(vals, dtype=torch.bool)
+    for d, span, cols in _spans(h, w, offsets):
+        term = A[:, span].double() * B[:, cols].double()
+        ref, mag = 0.5 * term.sum(0) + 0.9 * old[d].double(), 0.5 * term.abs().sum(0) + 0.9 * old[d].double().abs()
+        assert ((vals[d, span].double() - ref).abs() <= gu.REL_TOL * mag).all()
+        written[d, span] = True
+    assert torch.all(vals[~written].isnan())
+
+
+def test_gradient_graph_replay():
+    import torch
+    from cuv_amd import dia as D
+    px, rows, batch = 64, 24, 50
+    m = _dia(px * rows, px * rows, _offsets(px, rows))
+    bd, A, B = D.dev_block_descriptor_f(m), _rand(5, batch, px * rows), _rand(6, batch, px * rows)
+    _forced(lambda: D.densedense_to_dia(m, bd, A, B, 0.5, 0.0), b"dd2dia_split_kernel")
+    eager, g = m.vec.clone(), torch.cuda.CUDAGraph()
+
+    def capture():
+        with torch.cuda.graph(g):
+            D.densedense_to_dia(m, bd, A, B, 0.5, 0.0, sync=False)
+    _forced(capture, b"dd2dia_split_kernel")
+    for _ in range(3):
+        m.vec.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(m.vec, eager)
