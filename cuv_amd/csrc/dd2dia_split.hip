@@ -15,9 +15,10 @@
 //
 // Bound: the loads.  A stage's products take 4500 clocks of a CU, the split and its way to LDS 2300; with all CUs at work a stage
 // comes to 11000, for 80 KB in segments of 176 bytes (tiles 16 positions wide: 112 bytes, and half as long again).  Measured
-// against the kernel with a wave per window row: 4 maps of 256 x 256 to 4, batch 256 1000 -> 807 us (57 -> 70 TFLOP/s); 416 x 416,
-// batch 357 421 -> 327; 200 x 200, 2 maps to 2, batch 256 357 -> 214; 272 x 272 to 2, batch 388 413 -> 346.  Windows of 7 to 11
-// rows have fewer products for the same loads and fewer of them are slots: 0.5 - 0.95 times the kernels that serve them.
+// against the kernel with a wave per window row: 4 channels of 256 x 256 maps, batch 256 981 -> 837 us (58 -> 68 TFLOP/s); 416 x 416,
+// batch 357 421 -> 322; 200 x 200, 2 maps to 2, batch 256 357 -> 228; 272 x 272 to 2, batch 388 413 -> 329.  (Parts cut off instead
+// of rounded: 825, 332, 228 and 331.)  Windows of 7 to 11 rows have fewer products for the same loads and fewer of them are
+// slots: 0.5 - 0.95 times the kernels that serve them.
 //
 // Accumulation order: of every 16 columns the six products of all columns, smallest first, rounded as the matrix core does
 // (split.hpp); these sums in fp32, columns ascending.  Error against 64 bits (2-norm, relative; uniform operands in -1 .. 1) at
@@ -373,9 +374,11 @@ bool ds_plan(const DiaView &C, const float *B, long long lda, long long ldb, int
     if (n == 0) return false;
     // A tile takes a CU to itself for the whole batch, so a launch comes in rounds of 32 tiles per XCD: taken where at least
     // three quarters of the rounds' positions are the map's, and from 128 columns on, below which the results' way out (8000
-    // clocks and more per tile) is too much of a tile.  Measured on 45 layers of maps 190 to 545 wide, batch 26 to 720, that the
-    // kernel with a wave per window row serves otherwise: 1.02 - 1.69 times its rate where taken (median 1.19), 0.82 - 1.06 below
-    // 128 columns, 0.95 - 1.04 where the rounds are emptier.
+    // clocks and more per tile) is too much of a tile.  Measured on 140 random layers of maps 190 to 545 wide, batch 27 to 720,
+    // against the kernel with a wave per window row: 54 are taken, at 0.93 - 1.49 times its rate (median 1.20, two below 1.0);
+    // forced on others, 0.74 - 1.25 below 128 columns (median 0.94) and 0.88 - 1.13 where the rounds are emptier.  Not
+    // asked where the projection runs chunk by chunk (maps below 256 wide, by that kernel's rule): forced there, 0.89 - 1.38 times
+    // the rate from 128 columns on, ahead where the rounds are full.
     const long long rounds = ((n + 7) / 8 + 31) / 32;
     return force || (batch >= 128 && 4 * n * wk.period >= 3 * rounds * 256 * txn * DS_XT);
 }

@@ -15,8 +15,9 @@
 // registers, its work interleaved by hand (720 - 770 us on the first case below), the values and not the rows in two buffers (780).
 //
 // Bound: that chain, 7500 - 8500 clocks a step where the products take 1600 (rows of bfloat16 numbers) or 3200 of a SIMD's.
-// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256 815 -> 700 us; 200 x 200, 2 maps to 4,
-// batch 256 556 -> 407; 448 x 448, 2 maps to 3, batch 64 560 -> 361; 416 x 416, transposed, batch 357 444 -> 426.
+// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256, binary rows 815 -> 692 us, uniform ones
+// 752 (six products of parts instead of three); 200 x 200, 2 maps to 4, batch 256 556 -> 415 and 450; 448 x 448, 2 maps to 3,
+// batch 64 560 -> 370 and 425.  (Parts cut off instead of rounded: 689, 407 and 367 with binary rows.)
 // Windows of 11 rows use 47 % of a patch's products: level with the fp32 kernel.
 //
 // Accumulation order: of every 32 dense rows (16 of two map rows) the products of parts, smallest first, rounded as the matrix
@@ -652,9 +653,10 @@ bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force,
     // Taken where the rounds' steps, with the columns and positions that only fill tiles up, come to at most 2.1 times the
     // segments' own where the tile-by-tile kernel would run, 1.65 times where the plane's walk would.  Measured on 210 random
     // products of 13 x 13 windows, 1 to 5 maps, 40 to 640 wide, batch 24 to 640, a third of them with bias and sigmoid: 79 are
-    // taken, at 0.91 - 4.8 times the rate of the kernels that served them (one below 0.97; median 1.29, with bias and sigmoid
-    // 1.43; samples 0.98 - 1.28).  Forced on 111 others: up to these lines 4 % below 0.97 in place of the tile-by-tile kernel, beyond
-    // them more than a third.
+    // taken, at 0.90 - 4.7 times the rate of the kernels that served them (one below 0.97; median 1.25, with bias and sigmoid
+    // 1.42; samples 0.98 - 1.28).  Forced on 111 others: up to these lines 4 % below 0.97 in place of the tile-by-tile kernel, beyond
+    // them more than a third.  The line of 1.65 is a cautious one: the plane's walk keeps 20 of the 210, of which 13 would be
+    // up to 1.6 times as fast here and 4 at 0.91 - 0.96.
     const double padded = over * L.col_tiles * S::COLS / batch * L.tp * S::XS / wk.period;
     if (!force && padded > (walks ? 1.65 : 2.1)) return false;
     plane_cut(spans, walk_len, S::PY, L);

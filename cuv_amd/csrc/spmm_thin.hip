@@ -263,7 +263,8 @@ hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B,
         // Few chunks per row block, however many the table has: 8 waves have nothing to share, and their sums' place in LDS
         // lets two workgroups into a CU.  Measured on 170 random products, up to 16 maps, batch 1 to 140, every shape: of those
         // that come here the choice below is at 1.00 - 2.4 times the rate of 8 columns by 4 or 8 waves (mean 1.35), within 1.2 of
-        // the best; on 149 others none is below 0.98.  448 x 448, 3 x 3, 1 map to 4, batch 23, transposed 94 -> 45 us; 388 x 388,
+        // the best.  Of 260 others (batch 1 to 139) 33 come here to 4 columns per lane: 0.94 - 2.0 times (median 1.30; the one below
+        // 0.99 is 144 x 144, 5 x 5, 2 maps to 1, batch 17: 8.4 -> 9.0 us).  448 x 448, 3 x 3, 1 map to 4, batch 23, transposed 94 -> 45 us; 388 x 388,
         // 7 x 7, batch 12, transposed 33 -> 17.  Tables of 16 chunks and more had 4 waves before: beyond 9 chunks a row block
         // 0.89 - 1.1.
         if (wgs(256, 8) < 4000) cb = 4;

@@ -378,7 +378,9 @@ int cuvdia_set_path(int path);
  * served by the walking kernel, CUVDIA_PATH_PLANE by the ones on the matrix
  * cores, CUVDIA_PATH_WINDOW for a projection served
  * by the kernels tiled in the window's plane, of which the automatic choice
- * takes one on the matrix cores for 13 x 13 windows; 0 before any call).  The kernels
+ * takes one on the matrix cores for 13 x 13 windows, among the calls that
+ * cuvdia_plan_window_launch names -- forced by CUVDIA_PATH_PLANE, that kernel
+ * is reported as CUVDIA_PATH_PLANE --; 0 before any call).  The kernels
  * with rows along the lanes, of which the automatic choice makes use beside
  * the tiled ones, count as CUVDIA_PATH_TILED; cuvdia_last_kernel names them. */
 int cuvdia_last_path(void);
