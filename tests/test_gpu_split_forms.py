@@ -180,3 +180,33 @@ def test_gradient_graph_replay():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(m.vec, eager)
+
+
+@pytest.mark.parametrize("where", ["first", "second"])
+@pytest.mark.parametrize("op", ["product", "gradient"])
+def test_numbers_whose_nearest_bfloat16_number_is_infinite(op, where):
+    """The largest fp32 numbers and the last one below them that bfloat16 rounds down, against small ones."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import dia as D
+    px, rows, batch = 40, 24, 40
+    n, offsets = px * rows, _offsets(px, rows)
+    m = _dia(n, n, offsets)
+    bd, vals, X, Y = D.dev_block_descriptor_f(m), _rand(7, len(offsets), n), _rand(8, batch, n), _rand(9, batch, n)
+    first, second = (vals, X) if op == "product" else (X, Y)
+    large, small = (first, second) if where == "first" else (second, first)
+    small *= 2.0 ** -20
+    bits = torch.tensor([0x7f7fffff, 0x7f7f8000, 0x7f7f7fff], dtype=torch.int32, device="cuda:0").view(torch.float32)
+    large.view(-1)[::997] = bits[torch.arange(large.view(-1)[::997].numel(), device="cuda:0") % 3]
+    if op == "product":
+        m.vec.copy_(vals.view(-1))
+        got = _forced(lambda: D.prod(torch.empty((batch, n), device="cuda:0"), m, X, "n"), b"spmm_split_kernel").double()
+        ref, mag = _exact_product(vals, X, n, n, offsets, "n")
+    else:
+        _forced(lambda: D.densedense_to_dia(m, bd, X, Y, 1.0, 0.0), b"dd2dia_split_kernel")
+        got = m.vec.view(len(offsets), n).double()
+        ref, mag = torch.zeros_like(got), torch.zeros_like(got)
+        for d, span, cols in _spans(n, n, offsets):
+            term = X[:, span].double() * Y[:, cols].double()
+            ref[d, span], mag[d, span] = term.sum(0), term.abs().sum(0)
+    assert ((got - ref).abs() <= gu.REL_TOL * mag).all()
