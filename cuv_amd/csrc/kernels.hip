@@ -1376,7 +1376,6 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
     const int col0 = coltile * SP_COLS;
     const int cols_here = min(SP_COLS, batch - col0);
     const int nsteps = ntiles + K - 1;
-    const int nblocks = nsteps * ngroups;
 
     // dense rows: instruction i = wave + WAVES it of a block stages pieces 64 i .. 64 i + 63, piece p = XQ * column + quad
     constexpr int XIT = (XQ + WAVES - 1) / WAVES;
@@ -1422,12 +1421,11 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
         const int j = h * S::DPI + lane / (ROWS / 4);
         a_lane[k] = (n < K * S::AI && j < LCK) ? (unsigned)(16 * (lane % (ROWS / 4)) + j * astep4) : OOB_OFFSET;
     }
-    // Requests block number i = u * ngroups + g (step u, group g) into buffer i & 1: its dense
-    // rows and, for every tile m = u - dy that exists, the values of chunk (g, dy) for the tile's rows.
-    auto issue = [&](int i, int u, int g) __attribute__((always_inline)) {
-        const int a0 = row_first + s0 + stab[g] + u * period;        // first dense row the block's chunks read
-        if (a0 + ROWS + LCK - 1 <= 0 || a0 >= n_in) return;          // wholly outside: nothing to stage (see apply)
-        const unsigned buf = lds0 + (unsigned)(i & 1) * BUF_BYTES;
+    auto block_row = [&](int u, int g) __attribute__((always_inline)) { return row_first + s0 + stab[g] + u * period; };
+    // Requests block (step u, group g), whose chunks read the dense rows from a0 on, into buffer `to`: those rows and,
+    // for every tile m = u - dy that exists, the values of chunk (g, dy) for the tile's rows.
+    auto issue = [&](int to, int u, int g, int a0) __attribute__((always_inline)) {
+        const unsigned buf = lds0 + (unsigned)to * BUF_BYTES;
         const int a0p = a0 - SH;                                     // a multiple of 4
         if ((a0p >= 0) & (a0p + 4 * XQ <= n_in)) {
             // every staged piece exists
@@ -1490,13 +1488,11 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
 #pragma unroll
         for (int t = 0; t < T; ++t) acc[k][t] = 0.f;
 
-    // Applies block i = (u, g) to the tiles that use it; UU = u mod K gives the sets their static names:
-    // tile m = u - dy sits in set (UU - dy) mod K.
-    auto apply = [&](int i, int u, int g, auto uu_c) __attribute__((always_inline)) {
+    // Applies the block of step u in buffer `from` to the tiles that use it; UU = u mod K gives the sets their static
+    // names: tile m = u - dy sits in set (UU - dy) mod K.
+    auto apply = [&](int from, int u, auto uu_c) __attribute__((always_inline)) {
         constexpr int UU = decltype(uu_c)::value;
-        const int a0 = row_first + s0 + stab[g] + u * period;
-        if (a0 + ROWS + LCK - 1 <= 0 || a0 >= n_in) return;
-        const float *buf = &lds[i & 1][0];
+        const float *buf = &lds[from][0];
         float win[4 * WQ];
         {
             const float4 *p4 = reinterpret_cast<const float4 *>(buf + lane * XPITCH + wave * T);
@@ -1559,13 +1555,13 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
         Y + (long long)col0 * ldy, (unsigned)(((long long)(cols_here - 1) * ldy + n_out) * 4));
     const bool by_row = EP && ep.act == 2;      // (kernel-uniform) the sampled result leaves row by row
     // Stores the tile that step u completes (m = u - K + 1, set (UU + 1) mod K) and clears its set for the tile
-    // K steps on.  `ilast` is the step's last block: every wave is through with its buffer (the barrier that
-    // ended the block), and the next request into it comes after the second barrier below.
-    auto finish = [&](int u, int ilast, auto uu_c, const f4u (&ypre)[NST]) __attribute__((always_inline)) {
+    // K steps on, through buffer `idle`: every wave is through with what was in it (the barrier that ended the block),
+    // and the next request into it comes after the second barrier below.
+    auto finish = [&](int u, int idle, auto uu_c, const f4u (&ypre)[NST]) __attribute__((always_inline)) {
         constexpr int SET = (decltype(uu_c)::value + 1) % K;
         const int m = u - (K - 1);
         if (m >= 0 && m < ntiles) {
-            float *out = &lds[ilast & 1][0];
+            float *out = &lds[idle][0];
             static_assert(OPITCH % 4 == 0 && T % 4 == 0, "the sums leave as 16-byte LDS writes");
 #pragma unroll
             for (int t = 0; t < T; t += 4)
@@ -1633,7 +1629,28 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
         for (int t = 0; t < T; ++t) acc[SET][t] = 0.f;
     };
 
-    issue(0, 0, 0);
+    // The blocks in order, one requested ahead; those wholly outside the operand are no blocks.  (Where they were, each
+    // cost a barrier, and the block before it was applied with no request under way: of one map's groups to 8 or 16,
+    // transposed, all but one or two.  7 x 7, 192 x 280, 1 map to 8, batch 265, transposed 657 -> 425 us; 5 x 5, 128 x 148,
+    // 1 to 16, batch 32, sampled 115 -> 60; 7 x 7, 192 x 192, 4 to 6, batch 200 654 -> 581.  With one group 512 x 512, 7 x 7,
+    // batch 512 315 -> 309: a block's row is worked out once.)  Group rows ascend, so the groups with rows in the segment's
+    // steps are a range.
+    int g0 = 0, g1 = ngroups;
+    while (g0 < g1 && block_row(nsteps - 1, g0) + ROWS + LCK - 1 <= 0) ++g0;
+    while (g0 < g1 && block_row(0, g1 - 1) >= n_in) --g1;
+    int nu = g0 < g1 ? 0 : nsteps, ng = g0 - 1, na0 = 0;         // the block requested last, and its first dense row
+    auto advance = [&]() __attribute__((always_inline)) {
+        do {
+            if (++ng >= g1) {
+                ng = g0;
+                ++nu;
+            }
+            na0 = block_row(nu, ng);
+        } while (nu < nsteps && (na0 + ROWS + LCK - 1 <= 0 || na0 >= n_in));
+    };
+    if (nu < nsteps) advance();
+    int buf = 0;                                                 // where it is
+    if (nu < nsteps) issue(buf, nu, ng, na0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     auto step = [&](int u, auto uu_c) __attribute__((always_inline)) {
@@ -1662,17 +1679,15 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
                     ypre[q] = __builtin_bit_cast(f4u, __builtin_amdgcn_raw_buffer_load_b128(yr, y_lane[q], tile_off, 0));
             }
         }
-        int i = u * ngroups;
-        for (int g = 0; g < ngroups; ++g, ++i) {
-            if (i + 1 < nblocks) {
-                const bool last = g + 1 == ngroups;
-                issue(i + 1, last ? u + 1 : u, last ? 0 : g + 1);
-            }
-            apply(i, u, g, uu_c);
+        while (nu == u) {
+            advance();
+            if (nu < nsteps) issue(buf ^ 1, nu, ng, na0);
+            apply(buf, u, uu_c);
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __syncthreads();
+            buf ^= 1;
         }
-        finish(u, i - 1, uu_c, ypre);
+        finish(u, buf ^ 1, uu_c, ypre);
     };
     for (int u0 = 0; u0 < nsteps; u0 += K) walk_steps<K, 0>(step, u0, nsteps);
 }
