@@ -795,18 +795,6 @@ __device__ __forceinline__ void spmm_tile_edge(
     }
 }
 
-// the same with 4 bytes per lane: lane i writes at lds_byte_addr + 4*i
-__device__ __forceinline__ void lds_load_b32(sp_int4 rsrc, unsigned lds_byte_addr, unsigned voff)
-{
-    lds_byte_addr = __builtin_amdgcn_readfirstlane(lds_byte_addr);
-    rsrc = sp_int4{__builtin_amdgcn_readfirstlane(rsrc.x), __builtin_amdgcn_readfirstlane(rsrc.y),
-                   __builtin_amdgcn_readfirstlane(rsrc.z), __builtin_amdgcn_readfirstlane(rsrc.w)};
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "buffer_load_dword %1, %2, 0 offen lds"
-                 :: "s"(lds_byte_addr), "v"(voff), "s"(rsrc) : "memory");
-}
-
 // The lean body (see spmm_tile) with the staging done by loads that write LDS
 // directly.  A chunk stages 76 rows (19 16-byte pieces) of each of the 64
 // columns, column after column without gaps: piece p = 19 * column + quad

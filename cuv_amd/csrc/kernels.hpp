@@ -147,7 +147,7 @@ struct PlaneLaunch {
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L);
 hipError_t spmm_plane_launch(const PlaneLaunch &L);
 // How many segments of the map rows (L.nseg; tp and col_tiles are set), and the segments (L.nseg, L.cuts).
-double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, double walk_ends, PlaneLaunch &L);
+double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, const double *shares, double walk_ends, PlaneLaunch &L);
 void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L);
 // The same, windows of 13 rows, fp32 products as bfloat16 ones (spmm_split.hip).
 // walks: whether the former would be taken.

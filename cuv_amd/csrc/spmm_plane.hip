@@ -14,6 +14,16 @@
 // 22 - 26 per clock and SIMD where the DPP form of the tile-by-tile kernel does 15, and one staging of the dense rows for
 // K window rows.  The walk costs K - 1 steps in which not all tiles are alive (groups of four without any are skipped).
 //
+// A block's requests follow each other without waiting for anything: the chunks' starts are in LDS, a tile's place comes from
+// one of them, blocks at the operand's ends are fetched 4 bytes per lane with what does not exist out of the resource's range
+// (element by element, with a wait for each, the few such blocks at a segment's ends held up the launch), and the next block's
+// place is worked out behind the requests.  Old values and results go through buffer accesses, their 32-bit offsets in few
+// registers: a fourth workgroup per CU for 7 and 8 window rows.  Before -> with all of that, the segments cut for it:
+// 7 x 7, 150 x 150, 4 maps to 6, batch 200 346 -> 259 us; 192 x 192 414 -> 370; 96 x 64, batch 512 185 -> 155; 475 x 475, 1 map,
+// batch 213 177 -> 161; 41 x 37, 3 to 4, batch 70 45 -> 32; 8 x 8, 128 x 128, 3 to 4, batch 203 136 -> 116; 9 x 9, 343 x 343,
+// batch 288 154 -> 147; 5 x 5, 152 x 152, 4 to 4, batch 256 134 -> 127.  Three blocks in LDS instead of two: 318 for 302 with
+// three workgroups per CU either way.
+//
 // Bound: on large windows the matrix cores (13 x 13: two thirds of a launch's time), on small ones the dense rows' way
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
 // 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
@@ -43,6 +53,7 @@ typedef unsigned plane_u4 __attribute__((ext_vector_type(4)));
 // own: while one waits for its block the others multiply.
 constexpr int PLANE_XT = 4;
 constexpr int PLANE_WAVES = 4, PLANE_ROWS = 8 * PLANE_WAVES;
+constexpr int PLANE_TAB = 256;                       // chunks of a table, at most
 
 template <int LC, int K>
 struct PlaneShape {
@@ -51,13 +62,20 @@ struct PlaneShape {
     static constexpr int NQX = (PLANE_ROWS + LC - 1 + 3) / 4;       // 16-byte pieces of a column
     static constexpr int XQ = NQX | 1;                              // ... and from column to column (odd: no bank conflicts)
     static constexpr int XW = (8 + LC - 1 + 3) / 4;                 // pieces of a lane's window
-    static constexpr int AROW = PLANE_ROWS + 8, AQ = AROW / 4;      // floats from diagonal to diagonal: 40 banks on ...
-    static constexpr int ASLOT = LC * AROW + (16 + 64 - LC * AROW % 32) % 32;   // ... and from tile to tile 16 or 48 banks on
+    static constexpr int AROW = PLANE_ROWS, AQ = AROW / 4;          // floats from diagonal to diagonal: 32 banks on ...
     static constexpr int AIT = (AQ * LC + 63) / 64;                 // load instructions per tile
+    static constexpr int ASLOT = std::max(LC * AROW, AIT == 1 ? 256 : 0) + 8;   // ... and from tile to tile 8 or 40 (a whole
+                                                                                // instruction fits: no lane sits it out)
+    static constexpr int NQ = (LC + 1) / 2;                         // registers of values per group: 2 diagonals each
     static constexpr int X_FLOATS = 64 * XQ * 4, STAGE = X_FLOATS + K * ASLOT;
     static constexpr int XIT = (XQ + PLANE_WAVES - 1) / PLANE_WAVES;    // load instructions per wave
-    static constexpr int FIT = 160 * 1024 / (2 * 4 * STAGE), MOST = K <= 5 ? 4 : 3;     // (in LDS; in registers)
-    static constexpr int PER_CU = FIT < MOST ? FIT : MOST;          // workgroups per CU, a wave per SIMD each
+    static constexpr int FIT = 160 * 1024 / ((2 * 4 * STAGE + 4 * PLANE_TAB + 1279) / 1280 * 1280);
+    // Workgroups per CU, a wave per SIMD each: as many as fit in LDS and, with the registers that a wave needs, on a SIMD.
+    static constexpr int per_cu(bool fused)
+    {
+        const int most = K <= 5 ? 4 : K <= 8 ? (fused ? 3 : 4) : 3;
+        return FIT < most ? FIT : most;
+    }
 };
 
 template <int I, int N, class F>
@@ -80,13 +98,14 @@ __device__ __forceinline__ void plane_fma8(float (&acc)[8], float a, const float
 }
 
 template <int LC, int K, bool EP>
-__global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC, K>::PER_CU)) void spmm_plane_kernel(
+__global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) void spmm_plane_kernel(
     const int *__restrict__ tab, int ngroups, int period, int s0, int astep4, int tp, int nseg, PlaneCuts cuts,
     const float *__restrict__ vals, const float *__restrict__ X, long long ldx, float *__restrict__ Y, long long ldy,
     int n_out, int n_in, int batch, float alpha, float beta, int col_tiles, unsigned a_bytes, SpEpilogue ep)
 {
     using S = PlaneShape<LC, K>;
     __shared__ __attribute__((aligned(16))) float lds[2 * S::STAGE];
+    __shared__ int starts[PLANE_TAB];                // where the chunks' values start
 
     // A unit -- a segment of PLANE_XT neighbouring walks -- stays on one XCD with all its column tiles: they share the
     // diagonals' values, and the cache lines that tiles side by side have in common.  The last walks of a map row, where
@@ -115,6 +134,9 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
     const int amin = min(0, astep4 * (LC - 1));
     const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)&lds[0];
 
+    for (int i = threadIdx.x; i < ngroups * K; i += 64 * PLANE_WAVES) starts[i] = tab[ngroups + i];
+    const int group_rows = lane < ngroups ? tab[lane] : 0;          // (5 window rows at least: 51 groups at most)
+
     // this lane's share of a block's requests: byte offsets that stay the same for the whole walk
     unsigned x_off[S::XIT], a_off[S::AIT];
 #pragma unroll
@@ -125,14 +147,13 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
 #pragma unroll
     for (int it = 0; it < S::AIT; ++it) {
         const int p = 64 * it + lane, dx = p / S::AQ, q = p - dx * S::AQ;
-        a_off[it] = dx < LC && q < 2 * waves ? (unsigned)(astep4 * dx - amin) + 16u * q : OOB_OFFSET;
+        a_off[it] = dx < LC ? (unsigned)(astep4 * dx - amin) + 16u * q : OOB_OFFSET;
     }
-    auto block_row = [&](int u, int g) { return row_first + s0 + tab[g] + u * period; };
-    auto outside = [&](int u, int g) { const int x0 = block_row(u, g); return x0 + rows + LC - 1 <= 0 || x0 >= n_in; };
+    auto block_row = [&](int u, int g) { return row_first + s0 + __builtin_amdgcn_readlane(group_rows, g) + u * period; };
 
-    // requests block (u, g): its dense rows, and the values of the tiles that use them
-    auto issue = [&](int u, int g, int buf) {
-        const int x0 = block_row(u, g);
+    // requests the block of step u (u % K: `slot`) whose dense rows start at x0: those rows, and the values of the tiles that
+    // use them; lane d of `first` has where the group's chunk of window row d starts
+    auto issue = [&](int u, int slot, int first, int x0, int buf) {
         const unsigned base = lds0 + (unsigned)(buf * S::STAGE * 4);
         const bool inside = x0 >= 0 && x0 + 4 * nqx <= n_in;
         if (inside) {
@@ -143,22 +164,15 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
             }
         } else {
             // the block crosses an end of the operand: element by element, what does not exist is 0
-            for (int i = wave; i < S::XQ; i += waves) {
-                const int p = 64 * i + lane, col = p / S::XQ, q = p - col * S::XQ;
-                const float *c = xbase + (long long)min(col, cols - 1) * ldx;
-                f4 v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = x0 + 4 * q + e;
-                    v[e] = q < nqx && r >= 0 && r < n_in ? c[r] : 0.f;
-                }
-                *reinterpret_cast<f4 *>(lds + buf * S::STAGE + 4 * p) = v;
+            for (int i = wave; i < 4 * S::XQ; i += waves) {
+                const int p = 64 * i + lane, col = p / (4 * S::XQ), r = p - col * (4 * S::XQ), row = x0 + r;
+                lds_load_b32(xrsrc, base + 256u * i, r < 4 * nqx && (unsigned)row < (unsigned)n_in ? (unsigned)min(col, cols - 1) * ((unsigned)ldx * 4u) + 4u * row : OOB_OFFSET);
             }
         }
         for (int s = wave; s < K; s += waves) {
-            const int d = (u - s + K * 64) % K, m = u - d;           // the tile in slot s, and its window row
+            const int d = slot - s + (slot < s ? K : 0), m = u - d;  // the tile in slot s, and its window row
             if (m < 0 || m >= tiles) continue;
-            const int at = tab[ngroups + g * K + d] + 4 * (row_first + m * period);
+            const int at = __builtin_amdgcn_readlane(first, d) + 4 * (row_first + m * period);
             const unsigned to = base + (unsigned)((S::X_FLOATS + s * S::ASLOT) * 4);
             if (inside) {
 #pragma unroll
@@ -166,16 +180,10 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
                     if (256 * (it + 1) <= S::ASLOT || 256 * it + 4 * lane < S::ASLOT)
                         lds_load_b128(arsrc, to + 1024u * it, a_off[it], (unsigned)(at + amin));
             } else {
-                for (int it = 0; it < S::AIT; ++it) {
-                    const int p = 64 * it + lane, dx = p / S::AQ, q = p - dx * S::AQ;
-                    if (dx >= LC) continue;
-                    f4 v;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int r = 4 * q + e, xr = x0 + r + dx;
-                        v[e] = r < rows && xr >= 0 && xr < n_in ? vals[(long long)(at / 4) + (long long)(astep4 / 4) * dx + r] : 0.f;
-                    }
-                    *reinterpret_cast<f4 *>(lds + buf * S::STAGE + S::X_FLOATS + s * S::ASLOT + 4 * p) = v;
+                for (int it = 0; it < (LC * S::AROW + 63) / 64; ++it) {
+                    const int p = 64 * it + lane, dx = p / S::AROW, r = p % S::AROW;
+                    if (dx < LC)
+                        lds_load_b32(arsrc, to + 256u * it, (unsigned)(x0 + r + dx) < (unsigned)n_in ? (unsigned)(at + astep4 * dx + 4 * r) : OOB_OFFSET);
                 }
             }
         }
@@ -191,6 +199,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
     }
     // where this lane reads values: lane 4 b + i of a group's register: row b % 8, diagonal 2 q + b / 8, tile i
     const int lane_a = (lane % 4) * S::ASLOT + (lane / 32) * S::AROW + (lane / 4) % 8 + 8 * wave;
+    const int lane_last = lane_a - std::max(0, 4 * (S::NG - 1) + lane % 4 - (K - 1)) * S::ASLOT;
     const int lane_t = (S::NG * 4) * S::ASLOT + (lane % 16 / 8) * S::AROW + lane % 8 + 8 * wave;
 
     auto multiply = [&](int u, int buf) {
@@ -202,30 +211,32 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[4 * q + e] = v[e];
         }
+        auto value = [&](int g, int q) {
+            // (slots past the last tile, diagonals past the last one: any value, never used)
+            return st[S::X_FLOATS + (4 * g + 3 < K ? lane_a : lane_last) + 4 * g * S::ASLOT + 2 * q * S::AROW];
+        };
         // tiles alive at this step: max(0, u - K + 1) .. min(u, tiles - 1)
         const int lo = max(0, u - K + 1), n = min(u, tiles - 1) - lo + 1, s_lo = lo % K;
         const unsigned ones = (1u << n) - 1u, alive = (ones << s_lo) | (ones >> (K - s_lo));
         plane_for<0, S::NG>([&](auto g_) {
             constexpr int g = decltype(g_)::value;
             if (!((alive >> (4 * g)) & 15u)) return;
-            plane_for<0, (LC + 1) / 2>([&](auto q_) {
+            plane_for<0, S::NQ>([&](auto q_) {
                 constexpr int q = decltype(q_)::value;
-                // (slots past the last tile, diagonals past the last one: any value, never used)
-                const int at = S::X_FLOATS + lane_a + 4 * g * S::ASLOT + 2 * q * S::AROW;
-                const float a = st[4 * g + 3 < K ? at : min(at, S::STAGE - 1)];
+                const float v = value(g, q);
                 plane_for<0, 16>([&](auto b_) {
                     constexpr int b = decltype(b_)::value, r = b % 8, dx = 2 * q + b / 8;
-                    if constexpr (dx < LC) acc[g][r] = __builtin_amdgcn_mfma_f32_4x4x1f32(a, x[r + dx], acc[g][r], 4, b, 0);
+                    if constexpr (dx < LC) acc[g][r] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, x[r + dx], acc[g][r], 4, b, 0);
                 });
             });
         });
         if constexpr (S::TAIL) {
             if ((alive >> (4 * S::NG)) & 1u) {
-                plane_for<0, (LC + 1) / 2>([&](auto q_) {
+                plane_for<0, S::NQ>([&](auto q_) {
                     constexpr int q = decltype(q_)::value;
-                    const float a = st[min(S::X_FLOATS + lane_t + 2 * q * S::AROW, S::STAGE - 1)];
-                    plane_fma8<0>(tail, a, x + 2 * q);
-                    if constexpr (2 * q + 1 < LC) plane_fma8<8>(tail, a, x + 2 * q + 1);
+                    const float v = st[S::X_FLOATS + lane_t + 2 * q * S::AROW];
+                    plane_fma8<0>(tail, v, x + 2 * q);
+                    if constexpr (2 * q + 1 < LC) plane_fma8<8>(tail, v, x + 2 * q + 1);
                 });
             }
         }
@@ -236,23 +247,24 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
     constexpr int OPITCH = PLANE_ROWS + 4;
     static_assert(64 * OPITCH <= S::STAGE, "a tile fits a block's place");
     const int my_row = 4 * (lane % 8), my_col = 16 * wave + lane / 8;
-    auto place = [&](int m, int c, int r) { return Y + (long long)(col0 + c) * ldy + row_first + (long long)m * period + r; };
-    f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    auto read_old = [&](int m) {
+    // (every lane's stores are issued, those past the batch or before the rows of this walk out of the resource's range: the
+    // count is certain)
+    auto place = [&](int c, int r) { return c < cols && r >= skip ? (unsigned)c * ((unsigned)ldy * 4u) + 4u * r : OOB_OFFSET; };
+    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
+        const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
+        f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        if (beta != 0.f && !(EP && ep.act == 2)) {
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (my_col + 8 * k >= cols) continue;
-            const float *p = place(m, my_col + 8 * k, my_row);
-            if (my_row >= skip) {
-                old[k] = *reinterpret_cast<const f4u *>(p);
-            } else {
+            for (int k = 0; k < 2; ++k) {
+                if (skip == 0) {
+                    old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
+                } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (my_row + i >= skip) old[k][i] = p[i];
+                    for (int i = 0; i < 4; ++i)
+                        old[k][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0));
+                }
             }
         }
-    };
-    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
         __builtin_amdgcn_s_barrier();                // nobody reads the block any more
         asm volatile("" ::: "memory");
 #pragma unroll
@@ -270,10 +282,11 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int c = c0 + 4 * h + i;
-                    if (c >= cols || r < skip) continue;
-                    float *p = place(m, c, r);
-                    const float s = out[c * OPITCH + r];
-                    *p = sp_finish(beta == 0.f ? alpha * s : beta * (*p) + alpha * s, bias, 2, w.w[i]);
+                    const unsigned to = place(c, r);
+                    const float t = alpha * out[c * OPITCH + r];
+                    const float was = beta == 0.f ? 0.f : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, to, tile_at, 0));
+                    const float p = sp_finish(beta == 0.f ? t : beta * was + t, bias, 2, w.w[i]);
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(p), yrsrc, to, tile_at, 0);
                 }
             }
             return false;
@@ -292,14 +305,11 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
                 if (EP) s[i] = sp_finish(s[i], bias[i], ep.act);
             }
             if (skip == 0) {
-                // (every lane's store is issued, those past the batch out of the resource's range: the count is certain)
-                const unsigned at = my_col + 8 * k < cols ? (unsigned)(my_col + 8 * k) * ((unsigned)ldy * 4u) + 4u * my_row : OOB_OFFSET;
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(plane_u4, s), yrsrc, at, (unsigned)(row_first + m * period) * 4u, 0);
-            } else if (my_col + 8 * k < cols) {
-                float *p = place(m, my_col + 8 * k, my_row);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(plane_u4, s), yrsrc, place(my_col + 8 * k, my_row), tile_at, 0);
+            } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (my_row + i >= skip) p[i] = s[i];
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[i]), yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0);
             }
         }
         return skip == 0;
@@ -312,19 +322,31 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
     int g0 = 0, g1 = ngroups;
     while (g0 < g1 && block_row(steps - 1, g0) + rows + LC - 1 <= 0) ++g0;
     while (g0 < g1 && block_row(0, g1 - 1) >= n_in) --g1;
-    int nu = g0 < g1 ? 0 : steps, ng = g0 - 1;       // the block requested last
+    // the block to be requested next: its step, step % K, group, first dense row, and where its chunks' values start
+    int nu = g0 < g1 ? 0 : steps, nslot = 0, ng = g0 - 1, nx0 = 0, first = 0;
     auto advance = [&]() {
         do {
             if (++ng >= g1) {
                 ng = g0;
                 ++nu;
+                nslot = nslot + 1 == K ? 0 : nslot + 1;
             }
-        } while (nu < steps && outside(nu, ng));
+            nx0 = block_row(nu, ng);
+        } while (nu < steps && (nx0 + rows + LC - 1 <= 0 || nx0 >= n_in));
+        first = starts[ng * K + (lane < K ? lane : 0)];
     };
-    advance();
-    int buf = 0;
+    __syncthreads();                                 // (the starts are in place)
+    if (nu < steps) advance();
+    int pu = nu;                                     // the step of the block that was requested last
+    int buf = 0;                                     // its place
     bool stores = false;                             // two stores of a finished tile are behind the block's requests
-    if (nu < steps) issue(nu, ng, 0);
+    auto request = [&](int to) {
+        pu = nu;
+        if (nu >= steps) return;
+        issue(nu, nslot, first, nx0, to);
+        advance();
+    };
+    request(0);
     int slot = 0;                                    // u % K
     for (int u = 0; u < steps; ++u) {
         plane_for<0, K>([&](auto s_) {
@@ -338,25 +360,18 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (EP && K == 9 ? 2 : PlaneShape<LC
             }
         });
         const int done = u - (K - 1);                // the tile that ends with this step
-        bool old_read = done < 0 || beta == 0.f || (EP && ep.act == 2);
-        while (nu == u) {
+        while (pu == u) {
             // (loads and stores complete in order)
             if (stores) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             stores = false;
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            advance();
-            if (nu < steps) issue(nu, ng, buf ^ 1);
-            if (!old_read) {
-                read_old(done);
-                old_read = true;
-            }
+            request(buf ^ 1);
             multiply(u, buf);
             buf ^= 1;
         }
         if (done >= 0) {
-            if (!old_read) read_old(done);
             const int leaving = slot + 1 == K ? 0 : slot + 1;
             float v[8];
             plane_for<0, K>([&](auto s_) {
@@ -414,29 +429,30 @@ hipError_t spmm_plane_launch(const PlaneLaunch &L)
 
 // Every segment walks (its map rows + k - 1) steps of as many blocks as groups have rows there: the map rows are cut where that
 // work divides evenly, at multiples of `every` from the segment's first (plane_cut).  Between two ends of groups' ranges the
-// groups are the same.  How many: workgroups run in rounds of 32 CUs per XCD, a unit of `unit` walks with its column tiles on
-// one XCD (plane_over, which returns the rounds' steps, of all places there are, over the segments' own).
-double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, double walk_ends, PlaneLaunch &L)
+// groups are the same.  How many: workgroups run on 32 CUs per XCD, a unit of `unit` walks with its column tiles on one XCD;
+// shares[n] is how long a CU takes for n workgroups at once, in workgroups of a CU that holds as many as it can, the last entry
+// (plane_over, which returns the time, in steps of such workgroups, over the segments' own).
+double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, const double *shares, double walk_ends, PlaneLaunch &L)
 {
     const long long work = spans.work;
-    const int full = L.tp / unit, part = L.tp % unit, cap = 32 * per_cu;
-    auto rounds = [&](int segs) {
-        const int wgs = ((segs * full + 7) / 8 * unit + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles;
-        return (wgs + cap - 1) / cap;
+    const int full = L.tp / unit, part = L.tp % unit;
+    auto time = [&](int segs) {
+        const int wgs = ((segs * full + 7) / 8 * unit + (segs * (part > 0) + 7) / 8 * part) * L.col_tiles, n = (wgs + 31) / 32;
+        return n / per_cu * shares[per_cu] + shares[n % per_cu];
     };
     double best = -1;
     int n = 1;
     for (int i = 1; i <= PLANE_MAX_SEGMENTS && i <= walk_len; ++i) {
-        const int r = rounds(i);
-        if (best >= 0 && r * walk_ends >= best) break;       // (more segments never run in fewer rounds)
-        const double cost = r * ((double)work / i + walk_ends);
+        const double t = time(i);
+        if (best >= 0 && t * walk_ends >= best) break;       // (more segments never run in less)
+        const double cost = t * ((double)work / i + walk_ends);
         if (best < 0 || cost < best) {
             best = cost;
             n = i;
         }
     }
     L.nseg = n;
-    return best * 8 * cap / std::max(1.0, (double)work * L.tp * L.col_tiles);
+    return best * 8 * 32 / std::max(1.0, (double)work * L.tp * L.col_tiles);
 }
 
 void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
@@ -463,24 +479,26 @@ void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
 
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
 {
-    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
+    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.ngroups * wk.k > PLANE_TAB || wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
+    // (a CU with one workgroup less than it holds is hardly slower on them all together; one alone waits for its blocks)
+    static const double SHARES[][5] = {{0, 1}, {0, 1.3, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}};
     int per_cu = 1;
     switch (wk.k) {
-        case 5: per_cu = PlaneShape<5, 5>::PER_CU; break;
-        case 7: per_cu = PlaneShape<7, 7>::PER_CU; break;
-        case 8: per_cu = PlaneShape<8, 8>::PER_CU; break;
-        case 9: per_cu = PlaneShape<9, 9>::PER_CU; break;
-        case 11: per_cu = PlaneShape<11, 11>::PER_CU; break;
-        case 13: per_cu = PlaneShape<13, 13>::PER_CU; break;
+        case 5: per_cu = PlaneShape<5, 5>::per_cu(fused); break;
+        case 7: per_cu = PlaneShape<7, 7>::per_cu(fused); break;
+        case 8: per_cu = PlaneShape<8, 8>::per_cu(fused); break;
+        case 9: per_cu = PlaneShape<9, 9>::per_cu(fused); break;
+        case 11: per_cu = PlaneShape<11, 11>::per_cu(fused); break;
+        case 13: per_cu = PlaneShape<13, 13>::per_cu(fused); break;
         default: return false;
     }
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
     const int walk_len = (int)(n_out / wk.period);
 
-    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, 0.9 * (wk.k - 1) * spans.most, L);
+    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, SHARES[per_cu - 1], 0.9 * (wk.k - 1) * spans.most, L);
     // Taken where the steps come to at most 1.65 times the segments' work (5 x 5 and 7 x 7 windows: 1.4 times), with two column
     // tiles at least -- with one, the values are most of the traffic, and the tile-by-tile kernel fetches them in pieces twice
     // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).

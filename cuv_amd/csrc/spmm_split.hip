@@ -649,7 +649,8 @@ bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force,
     // (a segment that has the end of a map in it walks both maps' ends)
     const double walk_ends = 0.9 * (wk.k - 1) * spans.most * (spans.groups.size() > 1 ? 2 : 1);
     const int walk_len = (int)(n_out / wk.period);
-    const double over = plane_over(spans, walk_len, 128 / S::XS, 2, walk_ends, L);
+    const double shares[] = {0, 2, 2};               // (a workgroup alone on its CU takes as long as two)
+    const double over = plane_over(spans, walk_len, 128 / S::XS, 2, shares, walk_ends, L);
     // Taken where the rounds' steps, with the columns and positions that only fill tiles up, come to at most 2.1 times the
     // segments' own where the tile-by-tile kernel would run, 1.65 times where the plane's walk would.  Measured on 210 random
     // products of 13 x 13 windows, 1 to 5 maps, 40 to 640 wide, batch 24 to 640, a third of them with bias and sigmoid: 79 are

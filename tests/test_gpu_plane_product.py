@@ -206,3 +206,14 @@ def test_rows_that_no_group_reaches(oracle, h, w, offsets):
         B = np.asfortranarray(rng.uniform(-1, 1, (n_in, 66)).astype(np.float32))
         dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, 66)).astype(np.float32))
         gu.check_prod(oracle, A, B, dst, trans, 1.0, 0.5, _lib.PATH_PLANE, str((h, w, trans)))
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+def test_as_many_groups_as_a_table_has(oracle, plane, trans):
+    """51 groups of 5 window rows: the last of the chunks' starts."""
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    _, A, B, dst = _case(oracle, 5, 32, 6, 5, 26, 26, 25, trans)
+    for alpha, beta, old in ((1.0, 0.0, None), (0.75, -0.5, dst)):
+        _, ran = gu.check_prod(oracle, A, B, old, trans, alpha, beta, _lib.PATH_PLANE, "51 groups")
+        assert ran == _lib.PATH_PLANE
