@@ -3131,7 +3131,7 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
     // One of another width, or with a larger window: the plane's walk on the matrix cores, 13 x 13 ones with split operands.
     if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_PLANE) {
         PlaneLaunch plane{}, other{};
-        const bool force = path == CUVDIA_PATH_PLANE, walks = spmm_plane_plan(wk, n_out, batch, ep.bias != nullptr || ep.act != 0, force, plane);
+        const bool force = path == CUVDIA_PATH_PLANE, walks = spmm_plane_plan(wk, n_out, batch, ep, force, plane);
         const bool split = spmm_split_plan(wk, n_out, batch, force, walks, other);
         if (split || walks) {
             PlaneLaunch &P = split ? other : plane;

@@ -144,7 +144,7 @@ struct PlaneLaunch {
     hipStream_t stream;
 };
 // Fills in the launch's shape; false: the kernel does not serve this table and these sizes, or (not force) would not be ahead.
-bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L);
+bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpilogue &ep, bool force, PlaneLaunch &L);
 hipError_t spmm_plane_launch(const PlaneLaunch &L);
 // How many segments of the map rows (L.nseg; tp and col_tiles are set), and the segments (L.nseg, L.cuts).
 double plane_over(const PlaneSpans &spans, int walk_len, int unit, int per_cu, const double *shares, double walk_ends, PlaneLaunch &L);

@@ -477,14 +477,15 @@ void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
     L.cuts.at[++L.nseg] = walk_len;
 }
 
-bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused, bool force, PlaneLaunch &L)
+bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpilogue &ep, bool force, PlaneLaunch &L)
 {
+    const bool fused = ep.bias != nullptr || ep.act != 0;
     if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.ngroups * wk.k > PLANE_TAB || wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
     // (a CU with one workgroup less than it holds is hardly slower on them all together; one alone waits for its blocks)
-    static const double SHARES[][5] = {{0, 1}, {0, 1.3, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}};
+    static const double SHARES[][5] = {{0, 1}, {0, 2, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}};
     int per_cu = 1;
     switch (wk.k) {
         case 5: per_cu = PlaneShape<5, 5>::per_cu(fused); break;
@@ -499,21 +500,24 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, bool fused,
     const int walk_len = (int)(n_out / wk.period);
 
     const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, SHARES[per_cu - 1], 0.9 * (wk.k - 1) * spans.most, L);
-    // Taken where the steps come to at most 1.65 times the segments' work (5 x 5 and 7 x 7 windows: 1.4 times), with two column
-    // tiles at least -- with one, the values are most of the traffic, and the tile-by-tile kernel fetches them in pieces twice
-    // as long -- and, of the layers with a bias or an activation, only up to 8 x 8 (the larger ones keep fewer waves).
-    // Measured on 12500 random products of 1 to 17 maps, 40 to 640 wide and 16 to 1400 tall, batch 24 to 640: 1543 are taken,
-    // at 0.96 - 3.2 times the tile-by-tile kernel's rate (1st and 99th percentile; median 1.29, 1.4 % below 0.97, the least
-    // 0.89).
-    const bool many = L.col_tiles >= 2 && !(wk.k >= 9 && fused) && over <= (wk.k >= 8 ? 1.65 : 1.4);
-    // ... and, up to 11 x 11, where the steps with the columns and positions that only fill tiles up come to at most 1.8 times
-    // the work: of 330 random products of the same ranges that takes 23 more, at 0.98 - 1.9 times the tile-by-tile kernel's rate
-    // (median 1.21; 282 x 282, 7 x 7, 2 maps to 5, batch 128 295 -> 243 us; 517 x 517, 5 x 5, batch 64 629 -> 355; 512 x 555,
-    // 11 x 11 with bias and sigmoid, batch 128 1247 -> 881).  Beyond 1.8 a fifth falls below 0.97, and so do half of the 7 x 7
-    // and 9 x 9 layers with a bias or an activation.
-    const double padded = over * L.col_tiles * 64 / batch * L.tp * PLANE_ROWS / wk.period;
-    const bool full = wk.k <= 11 && (!fused || wk.k == 5 || wk.k == 11) && padded <= 1.8;
-    if (!force && !many && !full) return false;
+    // Taken by the steps, with the positions that only fill tiles up, over the work: up to these lines, for plain products,
+    // with a bias and a sigmoid, and with a sample (on the vector unit, a few workgroups at a time).  Columns that only fill
+    // tiles up are the tile-by-tile kernel's as well; where they are more than half of those that exist the kernel with rows
+    // along the lanes does without them, and is ahead on a single column tile.
+    // Measured on 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, against the better of those
+    // two kernels: 197 were taken, at 0.79 - 1.6 times its rate (1st and 99th percentile; median 1.15, a tenth below 0.96: 5 x 5
+    // on a single large map, where memory is the bound); beyond the lines about as many fall below 1 as above.
+    static const struct { int k; double plain, fused, sample; } LINES[] = {
+        {5, 1.7, 1.75, 1.5}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 2.1}, {9, 2.2, 2.4, 2.2}, {11, 2.0, 1.8, 1.3}};
+    double line = 0;
+    for (const auto &l : LINES)
+        if (l.k == wk.k) line = ep.act == 2 ? l.sample : fused ? l.fused : l.plain;
+    if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, 1.45) : 0;
+    bool ahead = over * L.tp * PLANE_ROWS / wk.period <= line;
+    // (13 x 13: of what spmm_split.hip's rule leaves; with one column tile the values are most of the traffic, and the
+    // tile-by-tile kernel fetches them in pieces twice as long)
+    if (wk.k == 13) ahead = L.col_tiles >= 2 && over <= 1.65;
+    if (!force && !ahead) return false;
     plane_cut(spans, walk_len, 1, L);
     return true;
 }
