@@ -30,8 +30,9 @@ namespace {
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-constexpr int DR_MAX_WAVES = 8, DR_ROWS = 256;
-constexpr int DR_COLS = 2;                           // batch columns in flight per wave (4 take registers two waves need)
+constexpr int DR_ROWS = 256;
+constexpr int dr_max_waves(int lc) { return lc <= 8 ? 16 : 8; }     // (their sums' place in LDS)
+constexpr int DR_COLS = 2, DR_COLS_FEW = 4;          // batch columns in flight per wave; ... of launches of few waves
 constexpr int DR_BLOCK = 128;                        // batch columns per running sum
 constexpr int dr_halo(int lc) { return lc > 1 ? (lc + 2) / 4 : 1; }
 
@@ -48,13 +49,13 @@ __device__ __forceinline__ f4 dr_rows(const float *col, int row, int n, bool pla
 // The first of the 4 rows to load for a lane whose rows start at `row`: itself as long as one of them exists.
 __device__ __forceinline__ int dr_start(int row, int n) { return row <= -4 ? 0 : row >= n ? n - 4 : row; }
 
-template <int LC>
-__global__ __launch_bounds__(64 * DR_MAX_WAVES) void dd2dia_rows_kernel(
+template <int LC, int CU>
+__global__ __launch_bounds__(64 * dr_max_waves(LC)) void dd2dia_rows_kernel(
     const Chunk *__restrict__ chunks, int nchunks, float *__restrict__ C, int stride, const float *__restrict__ A,
     long long lda, const float *__restrict__ B, long long ldb, int h, int w, int batch, float alpha, float beta,
     int row_blocks, int unit_groups, int splits, int blocks_at)
 {
-    constexpr int NQ = (LC + 6) / 4, HQ = dr_halo(LC), PITCH = DR_ROWS + 4 * HQ, CU = DR_COLS;
+    constexpr int NQ = (LC + 6) / 4, HQ = dr_halo(LC), PITCH = DR_ROWS + 4 * HQ;
     static_assert(CU * HQ <= 64, "the halo is one piece per lane");
     extern __shared__ __attribute__((aligned(16))) float lds[];
 
@@ -224,19 +225,28 @@ hipError_t dr_launch(const DrLaunch &L)
     // columns -- a step takes about 1 us whatever the launch's size --, and up to four rounds of waves where each still
     // has 16 columns (one round and a bit takes as long as two: 4851 tiles, batch 544 take 181 us in 4 ranges, 216 in 2).
     int splits = 1;
-    while (splits < DR_MAX_WAVES && ((2 * splits * tiles <= 4096 && 2 * splits * DR_COLS <= L.batch) ||
-                                     (2 * splits * tiles <= 16384 && 32 * splits <= L.batch)))
+    while (splits < 8 && ((2 * splits * tiles <= 4096 && 2 * splits * DR_COLS <= L.batch) ||
+                          (2 * splits * tiles <= 16384 && 32 * splits <= L.batch)))
         splits *= 2;
+    // 16 where each still has 16 columns (and blocks' sums need no place beside the 16 waves' columns).  With few waves a step
+    // is a trip to memory, and 4 columns of one take as long as 2: 28 x 28, 7 x 7, 2 maps to 2, batch 864 43 -> 29 us with both,
+    // 32 x 32, 1 map to 8, batch 931 45 -> 30; a third of the sizes of few waves 1.05 - 1.5, none below 0.9.
+    if (dr_max_waves(LC) == 16 && splits == 8 && 16 * tiles <= 4096 && L.batch >= 256 && L.batch <= 16 * DR_BLOCK) splits = 16;
     const int waves = splits > 4 ? splits : 4, per = waves / splits;
     const long long groups = (L.nchunks + per - 1) / per;
     if (row_blocks * groups > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool blocks = L.batch > splits * DR_BLOCK;
-    const size_t staged = (size_t)waves * DR_COLS * PITCH * sizeof(float), sums = (size_t)waves * LC * 1024;
+    const bool few = splits * tiles <= 2048 && 2 * splits * DR_COLS_FEW <= L.batch;
+    const size_t staged = (size_t)waves * (few ? DR_COLS_FEW : DR_COLS) * PITCH * sizeof(float), sums = (size_t)waves * LC * 1024;
     const size_t stage = blocks ? staged + sums : staged, meet = splits > 1 ? sums : 0;
     note_kernel("dd2dia_rows_kernel<%d>", LC);
-    launch_kernel(dd2dia_rows_kernel<LC>, dim3((unsigned)(row_blocks * groups)), dim3(64 * waves), stage > meet ? stage : meet,
-                  L.stream, L.chunks, L.nchunks, L.C, L.stride, L.A, L.lda, L.B, L.ldb, L.h, L.w, L.batch, L.alpha, L.beta,
-                  (int)row_blocks, (int)groups, splits, blocks ? (int)(staged / sizeof(float)) : 0);
+    auto go = [&](auto kernel) {
+        launch_kernel(kernel, dim3((unsigned)(row_blocks * groups)), dim3(64 * waves), stage > meet ? stage : meet,
+                      L.stream, L.chunks, L.nchunks, L.C, L.stride, L.A, L.lda, L.B, L.ldb, L.h, L.w, L.batch, L.alpha, L.beta,
+                      (int)row_blocks, (int)groups, splits, blocks ? (int)(staged / sizeof(float)) : 0);
+    };
+    if (few) go(dd2dia_rows_kernel<LC, DR_COLS_FEW>);
+    else go(dd2dia_rows_kernel<LC, DR_COLS>);
     return hipGetLastError();
 }
 
@@ -252,7 +262,17 @@ bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowe
     // plane's kernel 1.0 - 1.8 up to batch 8 where its tiles of 64 positions are not full, 0.6 - 1.1 else; tables of 14
     // chunks or more (several maps) 1.1 - 3 up to batch 64, 0.65 - 1.1 above; pairs in a band of more than 128 rows
     // 1.3 - 1.7 up to batch 128; bands and single windows 0.7 - 1.
-    if (windowed) return batch <= 8 && C.walk_n.period % 64 != 0;
+    // Measured again on 1522 layers with 4 columns in flight and up to 16 ranges: pairs of chunks 1.1 - 1.5 on average up to
+    // batch 64 (128 where there are at most 256 tiles of 256 rows and a chunk, of fewer than 14 chunks; 16 beyond 1024), 1.1
+    // above batch 256 on at most 256 tiles, 0.9 - 1 between; single chunks 0.7 - 0.95, but 1.1 - 1.4 up to batch 16 on more than
+    // 1024 tiles; 9 to 12 wide window rows in the plane's kernel 1.1 - 1.2 up to batch 20, 0.6 - 0.85 above 32.  On 2200 others
+    // 205 came here that had not: 0.88 - 3.8 times the rate (mean 1.21, 7 below 0.97; 32 x 32, 7 x 7, 1 map to 8, batch 931 41.4 ->
+    // 30.2 us; 64 x 64, 1 map, batch 32 6.9 -> 6.0; 46 x 46, 1 to 8, batch 896 76 -> 57).
+    const long long tiles = (long long)((C.h + DR_ROWS - 1) / DR_ROWS) * C.n_chunks_n;
+    if (windowed) return C.walk_n.period % 64 != 0 && batch <= (C.max_len_n > CHUNK_MAX && C.max_len_n < 13 ? 20 : 8);
+    if (batch <= 16 && tiles > 1024 && C.max_len_n <= CHUNK_MAX) return true;
+    const bool pairs = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.max_len_n >= 5;
+    if (pairs && (batch <= (tiles <= 256 && C.n_chunks_n < 14 ? 128 : tiles <= 1024 ? 64 : 16) || (batch > 256 && tiles <= 256))) return true;
     if (C.n_chunks_n >= 14) return batch <= 64;
     const bool wide = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.pair_delta_max > PAIR_NARROW_DELTA && C.pair_delta_max <= PAIR_BAND_DELTA;
     return wide && C.max_len_p >= 4 && batch <= 128;

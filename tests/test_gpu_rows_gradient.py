@@ -40,6 +40,13 @@ def test_ranges_of_the_batch(oracle, h, w, runs, batch):
     _check(oracle, h, h, w, [41 * (r - runs // 2) + d for r in range(runs) for d in range(3)], batch, 0.5)
 
 
+@pytest.mark.parametrize("run", [1, 5, 8, 9, 13])
+@pytest.mark.parametrize("batch", [63, 64, 67, 255, 256, 259, 2048, 2049])     # (16 ranges from 256 to 2048, windows up to 8)
+def test_four_columns_in_flight_and_sixteen_ranges(oracle, run, batch):
+    offsets = sorted([d - run // 2 for d in range(run)] + [40 + d for d in range(max(run - 2, 1))])
+    _check(oracle, run + batch, 301, 299, offsets, batch, 0.9 if batch % 2 else 0.0)
+
+
 def test_several_maps_on_aligned_operands_and_short_batches(oracle):
     # 14 chunks or more at a batch up to 64; a band of 160 rows; the plane's tiles of 64 positions not full
     win = [[m * 1024 + dy * 32 + dx for dy in range(-2, 3) for dx in range(-2, 3)] for m in range(3)]
