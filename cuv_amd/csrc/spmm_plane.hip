@@ -250,21 +250,23 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     // (every lane's stores are issued, those past the batch or before the rows of this walk out of the resource's range: the
     // count is certain)
     auto place = [&](int c, int r) { return c < cols && r >= skip ? (unsigned)c * ((unsigned)ldy * 4u) + 4u * r : OOB_OFFSET; };
-    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
+    const bool reads_old = beta != 0.f && !(EP && ep.act == 2);
+    f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto read_old = [&](int m) {
         const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
-        f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        if (beta != 0.f && !(EP && ep.act == 2)) {
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                if (skip == 0) {
-                    old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
-                } else {
+        for (int k = 0; k < 2; ++k) {
+            if (skip == 0) {
+                old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
+            } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        old[k][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0));
-                }
+                for (int i = 0; i < 4; ++i)
+                    old[k][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0));
             }
         }
+    };
+    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
+        const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
         __builtin_amdgcn_s_barrier();                // nobody reads the block any more
         asm volatile("" ::: "memory");
 #pragma unroll
@@ -347,6 +349,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
         advance();
     };
     request(0);
+    constexpr bool AHEAD = S::per_cu(EP) < 4;
     int slot = 0;                                    // u % K
     for (int u = 0; u < steps; ++u) {
         plane_for<0, K>([&](auto s_) {
@@ -360,6 +363,9 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             }
         });
         const int done = u - (K - 1);                // the tile that ends with this step
+        // (with a fourth workgroup on the CU there are no registers to hold old values for the length of a block, nor need to:
+        // with two 11 x 11, 402 x 310, batch 477, transposed, is 382 us like this, 397 with old values read at the exit)
+        bool old_read = !reads_old || done < 0;
         while (pu == u) {
             // (loads and stores complete in order)
             if (stores) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
@@ -368,10 +374,15 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             request(buf ^ 1);
+            if (AHEAD && !old_read) {
+                read_old(done);
+                old_read = true;
+            }
             multiply(u, buf);
             buf ^= 1;
         }
         if (done >= 0) {
+            if (AHEAD && !old_read) read_old(done);
             const int leaving = slot + 1 == K ? 0 : slot + 1;
             float v[8];
             plane_for<0, K>([&](auto s_) {
@@ -385,6 +396,10 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                     }
                 }
             });
+            if (!AHEAD) {
+                old[0] = old[1] = f4{0.f, 0.f, 0.f, 0.f};            // (not held in between)
+                if (!old_read) read_old(done);
+            }
             stores = finish(done, v, lds + (buf ^ 1) * S::STAGE);
         }
         slot = slot + 1 == K ? 0 : slot + 1;
@@ -484,8 +499,10 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
-    // (a CU with one workgroup less than it holds is hardly slower on them all together; one alone waits for its blocks)
-    static const double SHARES[][5] = {{0, 1}, {0, 2, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}};
+    // (A CU with one workgroup less than it holds is hardly slower on them all together; one alone waits for its blocks.  Not so
+    // 5 x 5 windows, bound by memory and by the tiles' exits: 400 x 400, 4 maps to 4, batch 82 451 us with full rounds, 467 with
+    // these shares; 7 x 7, 96 x 64, 4 to 6, batch 512 187 and 157.)
+    static const double SHARES[][5] = {{0, 1}, {0, 2, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}}, FULL[] = {0, 4, 4, 4, 4};
     int per_cu = 1;
     switch (wk.k) {
         case 5: per_cu = PlaneShape<5, 5>::per_cu(fused); break;
@@ -499,7 +516,7 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
     const int walk_len = (int)(n_out / wk.period);
 
-    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, SHARES[per_cu - 1], 0.9 * (wk.k - 1) * spans.most, L);
+    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, wk.k == 5 ? FULL : SHARES[per_cu - 1], 0.9 * (wk.k - 1) * spans.most, L);
     // Taken by the steps, with the positions that only fill tiles up, over the work: up to these lines, for plain products,
     // with a bias and a sigmoid, and with a sample (on the vector unit, a few workgroups at a time).  Columns that only fill
     // tiles up are the tile-by-tile kernel's as well; where they are more than half of those that exist the kernel with rows
@@ -508,7 +525,7 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     // two kernels: 197 were taken, at 0.79 - 1.6 times its rate (1st and 99th percentile; median 1.15, a tenth below 0.96: 5 x 5
     // on a single large map, where memory is the bound); beyond the lines about as many fall below 1 as above.
     static const struct { int k; double plain, fused, sample; } LINES[] = {
-        {5, 1.7, 1.75, 1.5}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 2.1}, {9, 2.2, 2.4, 2.2}, {11, 2.0, 1.8, 1.3}};
+        {5, 1.7, 1.75, 1.5}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 1.8}, {9, 2.2, 2.4, 1.7}, {11, 2.0, 1.8, 1.3}};
     double line = 0;
     for (const auto &l : LINES)
         if (l.k == wk.k) line = ep.act == 2 ? l.sample : fused ? l.fused : l.plain;
