@@ -269,7 +269,7 @@ bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowe
     // 205 came here that had not: 0.88 - 3.8 times the rate (mean 1.21, 7 below 0.97; 32 x 32, 7 x 7, 1 map to 8, batch 931 41.4 ->
     // 30.2 us; 64 x 64, 1 map, batch 32 6.9 -> 6.0; 46 x 46, 1 to 8, batch 896 76 -> 57).
     const long long tiles = (long long)((C.h + DR_ROWS - 1) / DR_ROWS) * C.n_chunks_n;
-    if (windowed) return C.walk_n.period % 64 != 0 && batch <= (C.max_len_n > CHUNK_MAX && C.max_len_n < 13 ? 20 : 8);
+    if (windowed) return C.walk_n.period % 64 != 0 && batch <= (C.walk_n.lck > CHUNK_MAX && C.walk_n.lck < 13 ? 20 : 8);
     if (batch <= 16 && tiles > 1024 && C.max_len_n <= CHUNK_MAX) return true;
     const bool pairs = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.max_len_n >= 5;
     if (pairs && (batch <= (tiles <= 256 && C.n_chunks_n < 14 ? 128 : tiles <= 1024 ? 64 : 16) || (batch > 256 && tiles <= 256))) return true;
