@@ -29,3 +29,22 @@ def test_shapes(oracle, px, py, fs, maps_in, maps_out, batch, trans, columns):
     dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
     gu.check_prod(oracle, A, B, dst, trans, 0.75, -0.5, _lib.PATH_THIN, "%d x %d" % (px, py))
     assert _lib.lib().cuvdia_last_kernel() == b"spmm_thin_kernel<%d, %d, 1>" % (fs, columns)
+
+
+@pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch,trans,thin", [
+    (201, 192, 7, 1, 1, 32, "n", True),       # half of the 64 columns, 302 tiles by those that exist
+    (201, 190, 7, 1, 1, 32, "t", False),      # 299
+    (201, 192, 7, 1, 1, 36, "n", False),      # more than 0.55 of 64
+])
+def test_few_columns_of_many_tiles(oracle, px, py, fs, maps_in, maps_out, batch, trans, thin):
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng = np.random.default_rng(px + py + batch)
+    h, w = px * py * maps_in, px * py * maps_out
+    A = oracle.Dia(h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets(), max(h, w), 1)
+    A.vals[:] = rng.uniform(-1, 1, A.vals.shape).astype(np.float32)
+    n_in, n_out = (h, w) if trans == "t" else (w, h)
+    B = np.asfortranarray(rng.uniform(-1, 1, (n_in, batch)).astype(np.float32))
+    dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
+    gu.check_prod(oracle, A, B, dst, trans, 1.0, 0.5, _lib.PATH_AUTO, "%d x %d" % (px, py))
+    assert _lib.lib().cuvdia_last_kernel().decode().startswith("spmm_thin_kernel") == thin
