@@ -26,9 +26,9 @@
 //
 // Bound: on large windows the matrix cores (13 x 13: two thirds of a launch's time), on small ones the dense rows' way
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
-// 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 290 -> 217; 8 x 8, 1 map of
-// 448 x 448 to 2, batch 372 592 -> 395; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 524 -> 359; 7 x 7 on 475 x 475, batch 213
-// 229 -> 181; level or behind where the rule below says no.  Of 13 x 13 windows it has the products without bias and activation
+// 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 269 -> 215; 8 x 8, 1 map of
+// 448 x 448 to 2, batch 372 582 -> 346; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 495 -> 340; 7 x 7 on 475 x 475, batch 213
+// 201 -> 162; level or behind where the rule below says no.  Of 13 x 13 windows it has the products without bias and activation
 // that spmm_split.hip's rule leaves (the bound there on filled tiles).
 //
 // Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
@@ -499,10 +499,6 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
-    // (A CU with one workgroup less than it holds is hardly slower on them all together; one alone waits for its blocks.  Not so
-    // 5 x 5 windows, bound by memory and by the tiles' exits: 400 x 400, 4 maps to 4, batch 82 451 us with full rounds, 467 with
-    // these shares; 7 x 7, 96 x 64, 4 to 6, batch 512 187 and 157.)
-    static const double SHARES[][5] = {{0, 1}, {0, 2, 2}, {0, 1.6, 2.3, 3}, {0, 1.9, 2.6, 3.1, 4}}, FULL[] = {0, 4, 4, 4, 4};
     int per_cu = 1;
     switch (wk.k) {
         case 5: per_cu = PlaneShape<5, 5>::per_cu(fused); break;
@@ -516,20 +512,27 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     L.tp = (wk.period + PLANE_ROWS - 1) / PLANE_ROWS;
     const int walk_len = (int)(n_out / wk.period);
 
-    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, wk.k == 5 ? FULL : SHARES[per_cu - 1], 0.9 * (wk.k - 1) * spans.most, L);
+    // A CU with fewer workgroups than it holds takes as long as a full one, but for 7 and 8 window rows, four workgroups of which
+    // hold each other up: 7 x 7, 96 x 64, 4 maps to 6, batch 512 157 us with these shares, 187 with full rounds; 8 x 8, 128 x 128,
+    // 3 to 4, batch 203 117 and 124.  Not so 5 x 5 windows, bound by memory and by the tiles' exits -- 400 x 400, 4 to 4, batch 82
+    // 467 and 451 --, nor three 9 x 9 ones: 475 x 475, batch 213 238 and 215, 64 x 64, 1 to 8, batch 864 112 and 100.
+    static const double PART[] = {0, 1.9, 2.6, 3.1, 4};
+    double shares[5];
+    for (int n = 0; n <= per_cu; ++n) shares[n] = n == 0 ? 0 : per_cu == 4 && wk.k != 5 ? PART[n] : per_cu;
+    const double over = plane_over(spans, walk_len, PLANE_XT, per_cu, shares, 0.9 * (wk.k - 1) * spans.most, L);
     // Taken by the steps, with the positions that only fill tiles up, over the work: up to these lines, for plain products,
     // with a bias and a sigmoid, and with a sample (on the vector unit, a few workgroups at a time).  Columns that only fill
     // tiles up are the tile-by-tile kernel's as well; where they are more than half of those that exist the kernel with rows
     // along the lanes does without them, and is ahead on a single column tile.
-    // Measured on 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, against the better of those
-    // two kernels: 197 were taken, at 0.79 - 1.6 times its rate (1st and 99th percentile; median 1.15, a tenth below 0.96: 5 x 5
-    // on a single large map, where memory is the bound); beyond the lines about as many fall below 1 as above.
+    // Fitted to 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, all kernels timed on each (197
+    // taken, 0.79 - 1.6 times the better other kernel's rate, 1st and 99th percentile; median 1.15); on 2600 others, in turn with
+    // the tree that had the former rules, this kernel's products and the ones that it leaves were at 0.92 and more.
     static const struct { int k; double plain, fused, sample; } LINES[] = {
-        {5, 1.7, 1.75, 1.5}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 1.8}, {9, 2.2, 2.4, 1.7}, {11, 2.0, 1.8, 1.3}};
+        {5, 1.8, 1.85, 1.75}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 1.8}, {9, 2.2, 2.4, 1.7}, {11, 2.0, 1.8, 1.3}};
     double line = 0;
     for (const auto &l : LINES)
         if (l.k == wk.k) line = ep.act == 2 ? l.sample : fused ? l.fused : l.plain;
-    if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, 1.45) : 0;
+    if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, wk.k >= 8 ? 1.65 : 1.45) : 0;
     bool ahead = over * L.tp * PLANE_ROWS / wk.period <= line;
     // (13 x 13: of what spmm_split.hip's rule leaves; with one column tile the values are most of the traffic, and the
     // tile-by-tile kernel fetches them in pieces twice as long)
