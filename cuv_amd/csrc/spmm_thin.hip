@@ -233,13 +233,14 @@ bool spmm_thin_by_size(const DiaView &A, bool trans, int batch)
     // lines a tenth of the products falls below 0.9.  On 2400 products of maps of any shape up to 640 wide, batch up to 640:
     // none and 1.5 % below 0.97, the least 0.90.
     // Measured again on 3000 products and layers of the same maps, in turn with the lines below 14, 24 and 40 chunks at 90, 110
-    // and 120 tiles, above 40 at 190, and up to 35 columns of 64 decided by the tiles alone: 114 came here that had not, at 0.82 -
-    // 2.0 times the rate (mean 1.22, 10 below 0.97).
+    // and 120 tiles, above 40 at 190, and up to 35 columns decided by the tiles alone: 114 came here that had not, at 0.82 - 2.0
+    // times the rate (mean 1.22, 10 below 0.97).  (A second column tile that is nearly empty: 448 x 448, a band of 25, batch 67 59 ->
+    // 85 us.)
     const double tiles = (n_out + 63) / 64 * (batch / 64.0);     // of the columns that exist
     const double chunks = (double)A.nnz / n_out / lc;            // per tile, those outside the operand left out
     const double there = batch / 64.0 / ((batch + 63) / 64);
     const double most = chunks < 6 ? 40 : chunks < 9.5 ? 56 : chunks < 14 ? 115 : chunks < 40 ? 130 : 250;
-    if (there <= 0.55 && tiles >= (chunks < 6 ? 1000 : 300)) return true;
+    if (batch <= 35 && chunks >= 4 && tiles >= (chunks < 6 ? 1000 : 300)) return true;
     return tiles < most || (chunks >= 14 && there <= (lc <= 5 ? 0.8 : 0.7));
 }
 

@@ -34,7 +34,8 @@ def test_shapes(oracle, px, py, fs, maps_in, maps_out, batch, trans, columns):
 @pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch,trans,thin", [
     (201, 192, 7, 1, 1, 32, "n", True),       # half of the 64 columns, 302 tiles by those that exist
     (201, 190, 7, 1, 1, 32, "t", False),      # 299
-    (201, 192, 7, 1, 1, 36, "n", False),      # more than 0.55 of 64
+    (201, 192, 7, 1, 1, 36, "n", False),
+    (201, 100, 7, 1, 1, 67, "n", False),      # the second column tile nearly empty
 ])
 def test_few_columns_of_many_tiles(oracle, px, py, fs, maps_in, maps_out, batch, trans, thin):
     import _gpu_util as gu
