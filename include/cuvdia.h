@@ -127,8 +127,9 @@ int cuvdia_plan_units(const int *offsets_host, int nd, int *c1, int *c2, int cap
  * workgroups fit a CU's LDS -- x channel groups), or 0 when another kernel serves: the table is no
  * window table (see cuvdia_plan_walk) of chunks of 2 to 13 diagonals, the
  * period, a channel distance or a row count is no multiple of 4, the period
- * is below 64, the batch at most 8 on a period that is no multiple of 64 (the
- * kernel with rows along the lanes), or the launch has too few workgroups to
+ * is below 64, the batch at most 8 -- 20 with window rows of 9 to 12 diagonals
+ * -- on a period that is no multiple of 64 (the kernel with rows along the
+ * lanes), or the launch has too few workgroups to
  * fill the chip.  For
  * chunks of up to 8 diagonals: 768 for windows of 49 slots or more -- or 384
  * at a batch of at least 512, or 192 at a batch of at least 32: a workgroup
