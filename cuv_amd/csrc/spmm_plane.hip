@@ -68,8 +68,12 @@ struct PlaneShape {
                                                                                 // instruction fits: no lane sits it out)
     static constexpr int NQ = (LC + 1) / 2;                         // registers of values per group: 2 diagonals each
     static constexpr int X_FLOATS = 64 * XQ * 4, STAGE = X_FLOATS + K * ASLOT;
+    // The last slot's last register of an odd window row holds a diagonal that does not exist in its upper half: its lanes read
+    // on behind the slot, 24 floats behind the last block's of 9, 11 and 13 diagonals.
+    static constexpr int LAST_READ = X_FLOATS + (K - 1) * ASLOT + (2 * NQ - 1) * AROW + PLANE_ROWS - 1;
+    static constexpr int LDS_FLOATS = STAGE + std::max(STAGE, LAST_READ + 1);
     static constexpr int XIT = (XQ + PLANE_WAVES - 1) / PLANE_WAVES;    // load instructions per wave
-    static constexpr int FIT = 160 * 1024 / ((2 * 4 * STAGE + 4 * PLANE_TAB + 1279) / 1280 * 1280);
+    static constexpr int FIT = 160 * 1024 / ((4 * LDS_FLOATS + 4 * PLANE_TAB + 1279) / 1280 * 1280);
     // Workgroups per CU, a wave per SIMD each: as many as fit in LDS and, with the registers that a wave needs, on a SIMD.
     static constexpr int per_cu(bool fused)
     {
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     int n_out, int n_in, int batch, float alpha, float beta, int col_tiles, unsigned a_bytes, SpEpilogue ep)
 {
     using S = PlaneShape<LC, K>;
-    __shared__ __attribute__((aligned(16))) float lds[2 * S::STAGE];
+    __shared__ __attribute__((aligned(16))) float lds[S::LDS_FLOATS];
     __shared__ int starts[PLANE_TAB];                // where the chunks' values start
 
     // A unit -- a segment of PLANE_XT neighbouring walks -- stays on one XCD with all its column tiles: they share the
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             for (int e = 0; e < 4; ++e) x[4 * q + e] = v[e];
         }
         auto value = [&](int g, int q) {
-            // (slots past the last tile, diagonals past the last one: any value, never used)
+            // (slots past the last tile, diagonals past the last one: any value of the array, never used)
             return st[S::X_FLOATS + (4 * g + 3 < K ? lane_a : lane_last) + 4 * g * S::ASLOT + 2 * q * S::AROW];
         };
         // tiles alive at this step: max(0, u - K + 1) .. min(u, tiles - 1)

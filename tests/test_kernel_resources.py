@@ -1,0 +1,33 @@
+"""What the built kernels take of the hardware, and that what they address lies inside what they declare: the library's metadata and
+the kernels' arithmetic, without a GPU."""
+import re
+
+import numpy as np
+import pytest
+
+import _kernel_resources
+
+
+@pytest.mark.parametrize("k", [5, 7, 8, 9, 11, 13])
+def test_plane_walk_reads_values_inside_its_lds(k):
+    """Every lane's place of every value register (spmm_plane.hip, `lane_a`, `lane_last`, `lane_t`), in the block that lies last:
+    windows of 9, 11 and 13 rows have a register whose upper half is a diagonal that does not exist."""
+    rows, waves, chunk_starts = 32, 4, 256 * 4
+    tail = int(k % 4 == 1)
+    groups, registers = (k - tail + 3) // 4, (k + 1) // 2
+    pieces = ((rows + k - 1 + 3) // 4) | 1
+    slot = max(k * rows, 256 if rows // 4 * k <= 64 else 0) + 8
+    dense, stage = 64 * pieces * 4, 64 * pieces * 4 + k * slot
+    lane, wave = np.meshgrid(np.arange(64), np.arange(waves))
+    lane_a = (lane % 4) * slot + (lane // 32) * rows + (lane // 4) % 8 + 8 * wave
+    lane_last = lane_a - np.maximum(0, 4 * (groups - 1) + lane % 4 - (k - 1)) * slot
+    lane_t = 4 * groups * slot + (lane % 16 // 8) * rows + lane % 8 + 8 * wave
+    reads = [(lane_a if 4 * g + 3 < k else lane_last) + 4 * g * slot + 2 * q * rows for g in range(groups) for q in range(registers)]
+    if tail:
+        reads += [lane_t + 2 * q * rows for q in range(registers)]
+    last = stage + dense + max(int(r.max()) for r in reads)
+    found = {n: m for n, m in _kernel_resources.kernels().items() if "spmm_plane_kernelILi%dELi%dE" % (k, k) in n}
+    assert len(found) == (1 if k == 13 else 2)
+    for name, meta in found.items():
+        floats = (meta[".group_segment_fixed_size"] - chunk_starts) // 4
+        assert 2 * stage <= floats and last < floats, (name, last, floats)
