@@ -4,8 +4,8 @@
 //
 // A wave owns 256 rows of one chunk: a lane keeps 4 rows x LC diagonals of running sums and, per batch column, loads
 // its 4 values of A and of B (one 16-byte load each) and gets the LC - 1 values of B that follow its own from its
-// neighbours through a piece of LDS that belongs to the wave; the next DR_COLS columns are in flight meanwhile.  No
-// barrier until the end, and 4-byte alignment is all the loads need -- the kernels that share staged operands between
+// neighbours through a piece of LDS that belongs to the wave; the next CU columns (2, or 4 on launches of few waves) are in
+// flight meanwhile.  No barrier until the end, and 4-byte alignment is all the loads need -- the kernels that share staged operands between
 // waves take 16-byte pieces from 16-byte boundaries, and fall to single-element loads where a map's width, the leading
 // dimension or a pointer is no multiple of 4 -- and 64-bit addresses: no limit on the operands' sizes.  The waves of a
 // workgroup take neighbouring chunks of the same rows (A's values come out of the L1) or, on launches of few tiles,
@@ -16,10 +16,12 @@
 // batch 458 500 -> 170 us; 83 x 90, 5 x 5, 3 maps to 4, batch 192 115 -> 47; 382 x 382, 7 x 7, 1 map to 16, batch 32 (values of
 // 6.5 GB: one thread per slot before) 4470 -> 377; 96 x 96, 5 x 5, 3 maps to 4, batch 14 33 -> 11.
 //
-// Accumulation order: range r of S sums its steps r, r + S, ... of DR_COLS columns in ascending order,
+// Accumulation order: range r of S sums its steps r, r + S, ... of CU columns in ascending order,
 // acc = fma(a, b, acc), in blocks of DR_BLOCK columns (one running sum over a batch of a thousand loses a digit where two
 // such gradients are subtracted; the blocks' sums wait in LDS); total = ((p0 + p1) + p2) + ... of blocks and ranges.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -31,8 +33,11 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int DR_ROWS = 256;
-constexpr int dr_max_waves(int lc) { return lc <= 8 ? 16 : 8; }     // (their sums' place in LDS)
+constexpr int DR_WAVES = 8, DR_WAVES_MOST = 16;      // waves of a workgroup, at most; ... with the batch in 16 ranges,
+constexpr int DR_LC_MOST = 8;                        // ... for whose sums LDS has the place up to here
 constexpr int DR_COLS = 2, DR_COLS_FEW = 4;          // batch columns in flight per wave; ... of launches of few waves
+// 16 waves leave 128 registers to each: 4 columns of 7 and 8 diagonals do not fit (8 and 12 registers spilled)
+constexpr int dr_cols_few(int lc, int waves) { return waves == DR_WAVES_MOST && lc > 6 ? DR_COLS : DR_COLS_FEW; }
 constexpr int DR_BLOCK = 128;                        // batch columns per running sum
 constexpr int dr_halo(int lc) { return lc > 1 ? (lc + 2) / 4 : 1; }
 
@@ -49,8 +54,8 @@ __device__ __forceinline__ f4 dr_rows(const float *col, int row, int n, bool pla
 // The first of the 4 rows to load for a lane whose rows start at `row`: itself as long as one of them exists.
 __device__ __forceinline__ int dr_start(int row, int n) { return row <= -4 ? 0 : row >= n ? n - 4 : row; }
 
-template <int LC, int CU>
-__global__ __launch_bounds__(64 * dr_max_waves(LC)) void dd2dia_rows_kernel(
+template <int LC, int CU, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void dd2dia_rows_kernel(
     const Chunk *__restrict__ chunks, int nchunks, float *__restrict__ C, int stride, const float *__restrict__ A,
     long long lda, const float *__restrict__ B, long long ldb, int h, int w, int batch, float alpha, float beta,
     int row_blocks, int unit_groups, int splits, int blocks_at)
@@ -228,25 +233,35 @@ hipError_t dr_launch(const DrLaunch &L)
     while (splits < 8 && ((2 * splits * tiles <= 4096 && 2 * splits * DR_COLS <= L.batch) ||
                           (2 * splits * tiles <= 16384 && 32 * splits <= L.batch)))
         splits *= 2;
-    // 16 where each still has 16 columns (and blocks' sums need no place beside the 16 waves' columns).  With few waves a step
-    // is a trip to memory, and 4 columns of one take as long as 2: 28 x 28, 7 x 7, 2 maps to 2, batch 864 43 -> 29 us with both,
-    // 32 x 32, 1 map to 8, batch 931 45 -> 30; a third of the sizes of few waves 1.05 - 1.5, none below 0.9.
-    if (dr_max_waves(LC) == 16 && splits == 8 && 16 * tiles <= 4096 && L.batch >= 256 && L.batch <= 16 * DR_BLOCK) splits = 16;
+    // 16 where each still has 16 columns (and blocks' sums need no place beside the 16 waves' columns): 28 x 28, 7 x 7, 2 maps to
+    // 2, batch 864 38 -> 28 us, 32 x 32, 1 map to 8, batch 931 41 -> 30; 8 x 8, 48 x 48, batch 1024 38 -> 33.  With few waves a
+    // step is a trip to memory, and 4 columns of one take as long as 2: 8 waves of 7 and 8 diagonals 59 x 59, batch 4096 188 ->
+    // 153 us, 61 x 61, batch 224 12.8 -> 12.4.  (One bound of 16 waves for all launches, 4 columns with spilled registers in
+    // them: 198 and 13.4, and 48 x 48 36.)
+    if (LC <= DR_LC_MOST && splits == 8 && 16 * tiles <= 4096 && L.batch >= 256 && L.batch <= 16 * DR_BLOCK) splits = 16;
     const int waves = splits > 4 ? splits : 4, per = waves / splits;
     const long long groups = (L.nchunks + per - 1) / per;
     if (row_blocks * groups > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool blocks = L.batch > splits * DR_BLOCK;
     const bool few = splits * tiles <= 2048 && 2 * splits * DR_COLS_FEW <= L.batch;
-    const size_t staged = (size_t)waves * (few ? DR_COLS_FEW : DR_COLS) * PITCH * sizeof(float), sums = (size_t)waves * LC * 1024;
-    const size_t stage = blocks ? staged + sums : staged, meet = splits > 1 ? sums : 0;
-    note_kernel("dd2dia_rows_kernel<%d>", LC);
-    auto go = [&](auto kernel) {
-        launch_kernel(kernel, dim3((unsigned)(row_blocks * groups)), dim3(64 * waves), stage > meet ? stage : meet,
-                      L.stream, L.chunks, L.nchunks, L.C, L.stride, L.A, L.lda, L.B, L.ldb, L.h, L.w, L.batch, L.alpha, L.beta,
-                      (int)row_blocks, (int)groups, splits, blocks ? (int)(staged / sizeof(float)) : 0);
+    auto go = [&](auto cu_, auto most_) {
+        constexpr int CU = decltype(cu_)::value, MOST = decltype(most_)::value;
+        const size_t staged = (size_t)waves * CU * PITCH * sizeof(float), sums = (size_t)waves * LC * 1024;
+        const size_t stage = blocks ? staged + sums : staged, meet = splits > 1 ? sums : 0;
+        note_kernel("dd2dia_rows_kernel<%d, %d, %d>", LC, CU, MOST);
+        launch_kernel((dd2dia_rows_kernel<LC, CU, MOST>), dim3((unsigned)(row_blocks * groups)), dim3(64 * waves),
+                      stage > meet ? stage : meet, L.stream, L.chunks, L.nchunks, L.C, L.stride, L.A, L.lda, L.B, L.ldb, L.h, L.w,
+                      L.batch, L.alpha, L.beta, (int)row_blocks, (int)groups, splits, blocks ? (int)(staged / sizeof(float)) : 0);
     };
-    if (few) go(dd2dia_rows_kernel<LC, DR_COLS_FEW>);
-    else go(dd2dia_rows_kernel<LC, DR_COLS>);
+    auto with_waves = [&](auto most) {
+        constexpr int FEW = dr_cols_few(LC, decltype(most)::value);
+        if (few) go(std::integral_constant<int, FEW>{}, most);
+        else go(std::integral_constant<int, DR_COLS>{}, most);
+    };
+    if constexpr (LC <= DR_LC_MOST) {
+        if (waves == DR_WAVES_MOST) with_waves(std::integral_constant<int, DR_WAVES_MOST>{});
+    }
+    if (waves <= DR_WAVES) with_waves(std::integral_constant<int, DR_WAVES>{});
     return hipGetLastError();
 }
 

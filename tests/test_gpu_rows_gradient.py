@@ -40,11 +40,13 @@ def test_ranges_of_the_batch(oracle, h, w, runs, batch):
     _check(oracle, h, h, w, [41 * (r - runs // 2) + d for r in range(runs) for d in range(3)], batch, 0.5)
 
 
-@pytest.mark.parametrize("run", [1, 5, 8, 9, 13])
+@pytest.mark.parametrize("run", [1, 5, 6, 7, 8, 9, 13])
 @pytest.mark.parametrize("batch", [63, 64, 67, 255, 256, 259, 2048, 2049])     # (16 ranges from 256 to 2048, windows up to 8)
 def test_four_columns_in_flight_and_sixteen_ranges(oracle, run, batch):
     offsets = sorted([d - run // 2 for d in range(run)] + [40 + d for d in range(max(run - 2, 1))])
-    _check(oracle, run + batch, 301, 299, offsets, batch, 0.9 if batch % 2 else 0.0)
+    waves = 16 if run <= 8 and 256 <= batch <= 2048 else 8           # (a range each)
+    columns = 2 if batch < 64 or (waves == 16 and run > 6) else 4    # (two steps of 4 in every range)
+    _check(oracle, run + batch, 301, 299, offsets, batch, 0.9 if batch % 2 else 0.0, "dd2dia_rows_kernel<%d, %d, %d>" % (run, columns, waves))
 
 
 def test_several_maps_on_aligned_operands_and_short_batches(oracle):

@@ -1,7 +1,5 @@
 """What the built kernels take of the hardware, and that what they address lies inside what they declare: the library's metadata and
 the kernels' arithmetic, without a GPU."""
-import re
-
 import numpy as np
 import pytest
 
@@ -31,3 +29,11 @@ def test_plane_walk_reads_values_inside_its_lds(k):
     for name, meta in found.items():
         floats = (meta[".group_segment_fixed_size"] - chunk_starts) // 4
         assert 2 * stage <= floats and last < floats, (name, last, floats)
+
+
+def test_rows_gradient_holds_its_registers():
+    """No vector register of the gradient with rows along the lanes waits in memory: a launch of 16 waves per workgroup has 128, and
+    leaves the others theirs."""
+    found = {n: m for n, m in _kernel_resources.kernels().items() if "dd2dia_rows_kernel" in n}
+    assert len(found) >= 26
+    assert {n: m[".vgpr_spill_count"] for n, m in found.items() if m[".vgpr_spill_count"] or m[".private_segment_fixed_size"]} == {}
