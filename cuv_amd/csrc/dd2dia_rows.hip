@@ -277,17 +277,24 @@ bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowe
     // plane's kernel 1.0 - 1.8 up to batch 8 where its tiles of 64 positions are not full, 0.6 - 1.1 else; tables of 14
     // chunks or more (several maps) 1.1 - 3 up to batch 64, 0.65 - 1.1 above; pairs in a band of more than 128 rows
     // 1.3 - 1.7 up to batch 128; bands and single windows 0.7 - 1.
-    // Measured again on 1522 layers with 4 columns in flight and up to 16 ranges: pairs of chunks 1.1 - 1.5 on average up to
-    // batch 64 (128 where there are at most 256 tiles of 256 rows and a chunk, of fewer than 14 chunks; 16 beyond 1024), 1.1
-    // above batch 256 on at most 256 tiles, 0.9 - 1 between; single chunks 0.7 - 0.95, but 1.1 - 1.4 up to batch 16 on more than
-    // 1024 tiles; 9 to 12 wide window rows in the plane's kernel 1.1 - 1.2 up to batch 20, 0.6 - 0.85 above 32.  On 2200 others
-    // 205 came here that had not: 0.88 - 3.8 times the rate (mean 1.21, 7 below 0.97; 32 x 32, 7 x 7, 1 map to 8, batch 931 41.4 ->
-    // 30.2 us; 64 x 64, 1 map, batch 32 6.9 -> 6.0; 46 x 46, 1 to 8, batch 896 76 -> 57).
+    // Measured again with 4 columns in flight and up to 16 ranges, on 1800 gradients of these kinds that had gone elsewhere:
+    // More than 1024 tiles of 256 rows and a chunk, batch up to 16: 1.2 - 4.7; windows of one map, whose few chunks share little
+    // there, 0.85 - 1.1 above 8 columns of rows up to 4 wide and above 12 of 5 and 6 (5 x 5, 396 x 278, batch 15 11.5 and 13.5 us).
+    // Pairs of chunks on up to 256 tiles: 1.1 - 1.5 up to batch 128 (rows 5 wide 0.96 - 1.05 above 96), 0.9 - 1 up to 256, 1.05 -
+    // 1.25 where 16 ranges run, up to batch 2048, 0.79 - 0.95 above (8 x 8, 28 x 28, batch 4096 130 and 153 us), 0.9 - 0.96 for
+    // 3 columns, two steps of one wave; up to 1024 tiles 1.0 - 1.5 up to batch 48, of rows 5 and 6 wide up to 16 (5 x 5,
+    // 128 x 128, batch 64 6.8 and 8.2).
+    // 9 to 12 wide window rows in the plane's kernel: 1.1 - 1.6 up to batch 20, 0.6 - 0.85 above 32.
+    // Of 1583 gradients that the lines without these distinctions had sent here 230 are left out, at 0.79 - 1.5 (mean 0.92); the
+    // others are at a mean of 1.25, 1 % below 1.0, the least 0.94.
     const long long tiles = (long long)((C.h + DR_ROWS - 1) / DR_ROWS) * C.n_chunks_n;
+    const int run = C.max_len_n;
     if (windowed) return C.walk_n.period % 64 != 0 && batch <= (C.walk_n.lck > CHUNK_MAX && C.walk_n.lck < 13 ? 20 : 8);
-    if (batch <= 16 && tiles > 1024 && C.max_len_n <= CHUNK_MAX) return true;
-    const bool pairs = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.max_len_n >= 5;
-    if (pairs && (batch <= (tiles <= 256 && C.n_chunks_n < 14 ? 128 : tiles <= 1024 ? 64 : 16) || (batch > 256 && tiles <= 256))) return true;
+    if (tiles > 1024 && run <= CHUNK_MAX && C.n_chunks_n > 1 && batch <= (run >= 7 || C.n_chunks_n > run ? 16 : run >= 5 ? 12 : 8)) return true;
+    if (C.n_units < C.n_chunks_p && run <= CHUNK_MAX && run >= 5 && tiles <= 1024 && (batch != 3 || tiles > 256)) {
+        const int most = tiles <= 256 && C.n_chunks_n < 14 ? (run == 5 ? 96 : 128) : run >= 7 ? 48 : 16;
+        if (batch <= most || (tiles <= 256 && batch > 256 && batch <= DR_WAVES_MOST * DR_BLOCK)) return true;
+    }
     if (C.n_chunks_n >= 14) return batch <= 64;
     const bool wide = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.pair_delta_max > PAIR_NARROW_DELTA && C.pair_delta_max <= PAIR_BAND_DELTA;
     return wide && C.max_len_p >= 4 && batch <= 128;

@@ -158,6 +158,34 @@ assert seen >= {b"dd2dia_window_kernel", b"dd2dia_window_long_kernel", b"dd2dia_
 """)
 
 
+def test_the_projections_that_run_with_rows_along_the_lanes(tmp_path):
+    """Both sides of every limit of the choice on operands that any kernel could take."""
+    _fake_hip.run(tmp_path, """
+def rows(M, batch):
+    D.densedense_to_dia(M, None, tensor(batch, M.h, bytes_at=1 << 41), tensor(batch, M.w, bytes_at=1 << 42), 1.0, 0.0)
+    return L.cuvdia_last_kernel().startswith(b"dd2dia_rows_kernel")
+def window(px, py, fs, maps_in=1, maps_out=1):
+    return matrix(px * py * maps_in, px * py * maps_out, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+for M, yes, no in [
+    (window(64, 64, 7), [1, 2, 4, 128, 257, 2048], [3, 129, 256, 2049, 8192]),       # 112 tiles of 256 rows and a chunk
+    (window(64, 64, 5), [96, 257], [97]),
+    (window(64, 64, 7, 1, 2), [64, 300], [65]),                                      # 14 chunks
+    (window(120, 120, 7), [3, 48], [49, 300]),                                       # 399 tiles
+    (window(128, 128, 5), [3, 16], [17, 300]),                                       # 320
+    (window(280, 280, 7), [16], [17]),                                               # 2149
+    (window(356, 356, 5), [12], [13]),                                               # 2480
+    (window(416, 217, 5, 1, 2), [16], [17]),                                         # ..., two maps
+    (window(408, 408, 3), [8], [9]),
+    (window(480, 293, 3, 1, 2), [16], [17]),
+    (matrix(504 * 732, 504 * 732, list(range(-3, 4))), [], [1, 8]),                  # one chunk
+    (window(500, 500, 7), [8], [9]),                                                 # window rows staged for the whole window
+    (window(500, 500, 9), [20], [21]),
+]:
+    for batch in yes + no:
+        assert rows(M, batch) == (batch in yes), (M.h, M.w, M.num_dia, batch, L.cuvdia_last_kernel())
+""")
+
+
 def test_the_planned_walk_is_the_one_that_runs(tmp_path):
     """cuvdia_plan_walk_launch against the kernel and the grid of the product, over maps, windows and batches on both sides of
     its rules."""
