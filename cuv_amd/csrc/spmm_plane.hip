@@ -19,16 +19,15 @@
 // (element by element, with a wait for each, the few such blocks at a segment's ends held up the launch), and the next block's
 // place is worked out behind the requests.  Old values and results go through buffer accesses, their 32-bit offsets in few
 // registers: a fourth workgroup per CU for 7 and 8 window rows.  Before -> with all of that, the segments cut for it:
-// 7 x 7, 150 x 150, 4 maps to 6, batch 200 346 -> 259 us; 192 x 192 414 -> 370; 96 x 64, batch 512 185 -> 155; 475 x 475, 1 map,
-// batch 213 177 -> 161; 41 x 37, 3 to 4, batch 70 45 -> 32; 8 x 8, 128 x 128, 3 to 4, batch 203 136 -> 116; 9 x 9, 343 x 343,
-// batch 288 154 -> 147; 5 x 5, 152 x 152, 4 to 4, batch 256 134 -> 127.  Three blocks in LDS instead of two: 318 for 302 with
-// three workgroups per CU either way.
+// 7 x 7, 150 x 150, 4 maps to 6, batch 200 346 -> 257 us; 96 x 64, batch 512 183 -> 154; 475 x 475, 1 map, batch 213 177 -> 156;
+// 9 x 9, 343 x 343, batch 288 154 -> 139; 5 x 5, 152 x 152, 4 to 4, batch 256 131 -> 119, with a sigmoid on 352 x 352, batch 832
+// 283 -> 268.  Three blocks in LDS instead of two: 318 for 302 with three workgroups per CU either way.
 //
 // Bound: on large windows the matrix cores (13 x 13: two thirds of a launch's time), on small ones the dense rows' way
 // from memory; with few steps per segment the walk's ends.  Measured (tile-by-tile kernel -> this one): 4 channels of
-// 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 269 -> 215; 8 x 8, 1 map of
-// 448 x 448 to 2, batch 372 582 -> 346; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 495 -> 340; 7 x 7 on 475 x 475, batch 213
-// 201 -> 162; level or behind where the rule below says no.  Of 13 x 13 windows it has the products without bias and activation
+// 13 x 13 on 256 x 256, batch 256 1131 -> 800 us (50 -> 71 TFLOP/s); 9 x 9 on 475 x 475, batch 213 264 -> 193; 8 x 8, 1 map of
+// 448 x 448 to 2, batch 372 582 -> 354; 9 x 9, 4 maps of 256 x 256 to 4, batch 114 494 -> 300; 7 x 7 on 475 x 475, batch 213
+// 202 -> 156; level or behind where the rule below says no.  Of 13 x 13 windows it has the products without bias and activation
 // that spmm_split.hip's rule leaves (the bound there on filled tiles).
 //
 // Accumulation order per output element: window rows ascending, groups in table order within a window row, diagonals
@@ -251,8 +250,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     constexpr int OPITCH = PLANE_ROWS + 4;
     static_assert(64 * OPITCH <= S::STAGE, "a tile fits a block's place");
     const int my_row = 4 * (lane % 8), my_col = 16 * wave + lane / 8;
-    // (every lane's stores are issued, those past the batch or before the rows of this walk out of the resource's range: the
-    // count is certain)
+    // (what lies past the batch or before the rows of this walk is out of the resource's range)
     auto place = [&](int c, int r) { return c < cols && r >= skip ? (unsigned)c * ((unsigned)ldy * 4u) + 4u * r : OOB_OFFSET; };
     const bool reads_old = beta != 0.f && !(EP && ep.act == 2);
     f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -269,7 +267,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             }
         }
     };
-    auto finish = [&](int m, const float (&v)[8], float *out) -> bool {
+    auto finish = [&](int m, const float (&v)[8], float *out) {
         const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
         __builtin_amdgcn_s_barrier();                // nobody reads the block any more
         asm volatile("" ::: "memory");
@@ -295,7 +293,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(p), yrsrc, to, tile_at, 0);
                 }
             }
-            return false;
+            return;
         }
         float bias[4] = {0.f, 0.f, 0.f, 0.f};
         if (EP && ep.bias) {
@@ -318,7 +316,6 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s[i]), yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0);
             }
         }
-        return skip == 0;
     };
 
     // The blocks (u, g) in order, one requested ahead.  Of the groups only those with rows anywhere in the segment are
@@ -345,7 +342,6 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     if (nu < steps) advance();
     int pu = nu;                                     // the step of the block that was requested last
     int buf = 0;                                     // its place
-    bool stores = false;                             // two stores of a finished tile are behind the block's requests
     auto request = [&](int to) {
         pu = nu;
         if (nu >= steps) return;
@@ -353,7 +349,12 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
         advance();
     };
     request(0);
-    constexpr bool AHEAD = S::per_cu(EP) < 4;
+    // A tile's old values are requested with the last of its blocks and held for its length, or requested at its exit; the code for
+    // the first is the faster one also where none are read.  11 x 11, 402 x 310, batch 477, transposed 348 us held, 395 at the
+    // exit; 9 x 9 with a sigmoid, 512 x 563, batch 86 116 and 132 (held, 4 registers are spilled; with two workgroups per CU none
+    // are, and 132); 5 x 5 with a sigmoid, 352 x 352, batch 832 268 and 293.  Without bias and activation four workgroups of 5, 7
+    // and 8 window rows have no registers to hold them (level).
+    constexpr bool AHEAD = S::per_cu(EP) < 4 || (EP && K == 5);
     int slot = 0;                                    // u % K
     for (int u = 0; u < steps; ++u) {
         plane_for<0, K>([&](auto s_) {
@@ -367,14 +368,12 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             }
         });
         const int done = u - (K - 1);                // the tile that ends with this step
-        // (with a fourth workgroup on the CU there are no registers to hold old values for the length of a block, nor need to:
-        // with two 11 x 11, 402 x 310, batch 477, transposed, is 382 us like this, 397 with old values read at the exit)
         bool old_read = !reads_old || done < 0;
         while (pu == u) {
-            // (loads and stores complete in order)
-            if (stores) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            stores = false;
+            // (for a finished tile's stores as well: to leave them under way took a branch on whether there are any, and cost more
+            // than their wait: 7 x 7, 475 x 475, batch 213, with a sigmoid 188 us with it, 169 without, plain 162 and 156; 9 x 9,
+            // 256 x 256, 4 maps to 4, batch 114 340 and 300)
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             request(buf ^ 1);
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                 old[0] = old[1] = f4{0.f, 0.f, 0.f, 0.f};            // (not held in between)
                 if (!old_read) read_old(done);
             }
-            stores = finish(done, v, lds + (buf ^ 1) * S::STAGE);
+            finish(done, v, lds + (buf ^ 1) * S::STAGE);
         }
         slot = slot + 1 == K ? 0 : slot + 1;
     }
@@ -517,9 +516,9 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     const int walk_len = (int)(n_out / wk.period);
 
     // A CU with fewer workgroups than it holds takes as long as a full one, but for 7 and 8 window rows, four workgroups of which
-    // hold each other up: 7 x 7, 96 x 64, 4 maps to 6, batch 512 157 us with these shares, 187 with full rounds; 8 x 8, 128 x 128,
-    // 3 to 4, batch 203 117 and 124.  Not so 5 x 5 windows, bound by memory and by the tiles' exits -- 400 x 400, 4 to 4, batch 82
-    // 467 and 451 --, nor three 9 x 9 ones: 475 x 475, batch 213 238 and 215, 64 x 64, 1 to 8, batch 864 112 and 100.
+    // hold each other up: 7 x 7, 96 x 64, 4 maps to 6, batch 512 154 us with these shares, 187 with full rounds; 8 x 8, 128 x 128,
+    // 3 to 4, batch 203 115 and 122.  Not so 5 x 5 windows, bound by memory and by the tiles' exits: 400 x 400, 4 to 4, batch 82
+    // 456 and 441.  With three 9 x 9 ones it is level: 475 x 475, batch 213 196 and 194.
     static const double PART[] = {0, 1.9, 2.6, 3.1, 4};
     double shares[5];
     for (int n = 0; n <= per_cu; ++n) shares[n] = n == 0 ? 0 : per_cu == 4 && wk.k != 5 ? PART[n] : per_cu;
