@@ -527,14 +527,17 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     // with a bias and a sigmoid, and with a sample (on the vector unit, a few workgroups at a time).  Columns that only fill
     // tiles up are the tile-by-tile kernel's as well; where they are more than half of those that exist the kernel with rows
     // along the lanes does without them, and is ahead on a single column tile.
-    // Fitted to 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, all kernels timed on each (197
-    // taken, 0.79 - 1.6 times the better other kernel's rate, 1st and 99th percentile; median 1.15); on 2600 others, in turn with
-    // the tree that had the former rules, this kernel's products and the ones that it leaves were at 0.92 and more.
+    // Fitted to 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, all kernels timed on each.  Timed
+    // again against the kernel otherwise taken, on 1100 others: of 505 that come here the mean is 1.21, 1 % are below 0.93 (the
+    // least, 0.87, on 5 x 5 windows whose segments fill a round badly), 5 % below 0.99.  A sample is taken at every exit, and with
+    // one map there is an exit for every block: 9 x 9 1.0 - 1.1 up to 1.4, 0.77 - 1.1 (mean 0.96) from there to the line of several
+    // maps (396 x 396, batch 576 539 us here and 486).
     static const struct { int k; double plain, fused, sample; } LINES[] = {
         {5, 1.8, 1.85, 1.75}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 1.8}, {9, 2.2, 2.4, 1.7}, {11, 2.0, 1.8, 1.3}};
     double line = 0;
     for (const auto &l : LINES)
         if (l.k == wk.k) line = ep.act == 2 ? l.sample : fused ? l.fused : l.plain;
+    if (wk.k == 9 && ep.act == 2 && wk.ngroups == 1) line = 1.4;
     if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, wk.k >= 8 ? 1.65 : 1.45) : 0;
     bool ahead = over * L.tp * PLANE_ROWS / wk.period <= line;
     // (13 x 13: of what spmm_split.hip's rule leaves; with one column tile the values are most of the traffic, and the

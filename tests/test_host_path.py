@@ -209,6 +209,21 @@ assert seen >= {b"spmm_walk_kernel", b"spmm_plane_kernel", b"spmm_thin_kernel", 
 """)
 
 
+def test_sampled_layers_of_one_map_leave_the_plane_earlier(tmp_path):
+    """9 x 9 windows: a sample at every block's exit with one map, at every second or fourth with more."""
+    _fake_hip.run(tmp_path, """
+def ran(px, py, maps, batch, act):
+    n = px * py * maps
+    A = matrix(n, n, D.filter_factory_float(px, py, 9, maps, maps).offsets())
+    D.prod_bias_act(tensor(batch, n, bytes_at=1 << 41), A, tensor(batch, n, bytes_at=1 << 42), "n", act=act)
+    return L.cuvdia_last_path() == _lib.PATH_PLANE
+assert ran(396, 396, 1, 576, _lib.ACT_SIGMOID), L.cuvdia_last_kernel()
+assert not ran(396, 396, 1, 576, _lib.ACT_SIGMOID_SAMPLE)
+assert ran(345, 345, 2, 128, _lib.ACT_SIGMOID_SAMPLE), L.cuvdia_last_kernel()
+assert ran(509, 444, 1, 329, _lib.ACT_SIGMOID_SAMPLE)
+""")
+
+
 def test_an_empty_batch_is_launched_for_the_projection_alone(tmp_path):
     _fake_hip.run(tmp_path, """
 A = matrix(4096, 4096, [64 * dy + dx for dy in range(-2, 3) for dx in range(-2, 3)])
