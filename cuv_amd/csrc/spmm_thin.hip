@@ -25,6 +25,8 @@
 // total = ((p0 + p1) + p2) + ...
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device.hpp"
 #include "kernels.hpp"
 
@@ -164,15 +166,49 @@ __global__ __launch_bounds__(64 * (CB == 4 ? 16 : 8)) void spmm_thin_kernel(
 #pragma unroll
     for (int c = 0; c < CB; ++c) *reinterpret_cast<f4 *>(part + (slice * CB + c) * ROWS + l4) = acc[c];
     __syncthreads();
+    auto total = [&](int e) {
+        float sum = part[e];
+        for (int s = 1; s < slices; ++s) sum += part[s * CB * ROWS + e];
+        return sum;
+    };
+    // Sampled: a thread takes as many neighbouring columns of a row as leave every thread some, up to the four that a block of the
+    // generator serves.  (With a block for every element -- and its word by index, from memory -- samples took longer than all
+    // else: 452 x 452, 3 x 3, 4 maps to 4, batch 28, transposed 194 -> 123 us; 160 x 160, 7 x 7, 1 to 8, batch 33, transposed
+    // 67 -> 43; 64 x 64, a band of 9, batch 16 8.4 -> 5.9.)
+    auto sampled = [&](auto q_) {
+        constexpr int Q = decltype(q_)::value;
+        for (int e = threadIdx.x; e < CB / Q * ROWS; e += blockDim.x) {
+            const int c = e / ROWS * Q, r = e % ROWS, row = row0 + r, col = col0 + c;
+            if (row < first_row || row >= n_out || col >= batch) continue;
+            const SpRand4 w = sp_philox((unsigned)row, (unsigned)col >> 2, ep.seed_lo, ep.seed_hi);
+            const unsigned upper = 0u - (((unsigned)col >> 1) & 1u), odd = 0u - ((unsigned)col & 1u);    // the first column's place
+            const float bias = ep.bias ? ep.bias[row] : 0.f;
+#pragma unroll
+            for (int i = 0; i < Q; ++i) {
+                if (col + i >= batch) break;
+                unsigned word = w.w[i];
+                if (Q == 2) word = (w.w[i] & ~upper) | (w.w[(2 + i) & 3] & upper);
+                if (Q == 1) word = (((w.w[0] & ~upper) | (w.w[2] & upper)) & ~odd) | (((w.w[1] & ~upper) | (w.w[3] & upper)) & odd);
+                const float sum = total((c + i) * ROWS + r);
+                float *y = Y + (long long)(col + i) * ldy + row;
+                stream_store(y, sp_finish(beta == 0.f ? alpha * sum : beta * (*y) + alpha * sum, bias, 2, word));
+            }
+        }
+    };
+    if (ep.act == 2) {
+        const int share = CB * ROWS / (int)blockDim.x;
+        if (CB >= 4 && share >= 4) sampled(std::integral_constant<int, CB >= 4 ? 4 : 1>{});
+        else if (CB >= 2 && share >= 2) sampled(std::integral_constant<int, CB >= 2 ? 2 : 1>{});
+        else sampled(std::integral_constant<int, 1>{});
+        return;
+    }
     for (int e = threadIdx.x; e < CB * ROWS; e += blockDim.x) {
         const int c = e / ROWS, r = e - c * ROWS, row = row0 + r, col = col0 + c;
         if (row < first_row || row >= n_out || col >= batch) continue;
-        float sum = part[e];
-        for (int s = 1; s < slices; ++s) sum += part[s * CB * ROWS + e];
+        const float sum = total(e);
         float *y = Y + (long long)col * ldy + row;
         const float v = (beta == 0.f) ? alpha * sum : beta * (*y) + alpha * sum;
-        const unsigned word = ep.act == 2 ? sp_philox((unsigned)row, (unsigned)col >> 2, ep.seed_lo, ep.seed_hi).w[col & 3] : 0u;
-        stream_store(y, sp_finish(v, ep.bias ? ep.bias[row] : 0.f, ep.act, word));
+        stream_store(y, sp_finish(v, ep.bias ? ep.bias[row] : 0.f, ep.act));
     }
 }
 

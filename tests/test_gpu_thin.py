@@ -149,3 +149,49 @@ def test_values_above_2_gib():
         assert _lib.lib().cuvdia_last_kernel().decode().startswith("spmm_thin_kernel")
         ref, mag = _band_reference(A.vec.view(len(offsets), n), offsets, X, trans)
         assert torch.all((Y.double() - ref).abs() <= 1e-5 * mag)
+
+
+@pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch,trans,shape", [
+    (40, 41, 5, 1, 1, 1, "n", "<5, 1, 1>"),          # a block of the generator for one column, ...
+    (40, 41, 5, 1, 1, 7, "t", "<5, 2, 1>"),          # ... for one of two neighbours
+    (31, 33, 7, 3, 4, 6, "n", "<7, 2, 4>"),
+    (40, 41, 3, 1, 1, 6, "n", "<3, 2, 1>"),          # three waves: two columns of a row, the first or the third of a block
+    (200, 163, 9, 1, 1, 7, "n", "<9, 4, 1>"),        # eight waves: two of a lane's four
+    (231, 233, 9, 1, 1, 22, "t", "<9, 4, 1>"),       # four waves: a block whole; two columns at the end
+    (117, 117, 5, 3, 4, 27, "n", "<5, 8, 1>"),       # three at the end
+    (48, 48, 5, 1, 16, 4, "t", "<5, 4, 1>"),         # sixteen waves: one column
+])
+def test_sampled_exit_of_every_shape(oracle, px, py, fs, maps_in, maps_out, batch, trans, shape):
+    """The sample of an element is the one its row, column and seed name, however many columns a thread takes."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng = np.random.default_rng(px + batch)
+    h, w = px * py * maps_in, px * py * maps_out
+    A = _dia(oracle, rng, h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+    n_in, n_out = (h, w) if trans == "t" else (w, h)
+    B = np.asfortranarray(rng.uniform(-1, 1, (n_in, batch)).astype(np.float32))
+    dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
+    bias = rng.uniform(-1, 1, n_out).astype(np.float32)
+    u = oracle.sample_uniform(n_out, batch, 321)
+    dev, Bd = gu.make_dev_dia(A), D.to_device_colmajor(B)
+    L = _lib.lib()
+    _lib.check(L.cuvdia_set_path(_lib.PATH_THIN), "set_path")
+    try:
+        for beta, b in ((0.0, bias), (0.5, None)):
+            old = dst if beta else None
+            p = oracle.prod_bias_act(A, B, old, trans, 0.25, beta, b, True)
+            # a quarter (the sigmoid's steepest slope) of 1e-5 of the sum's terms, and the sigmoid's own rounding
+            tol = 0.25 * gu.REL_TOL * (oracle.prod_mag(A, B, old, trans, 0.25, beta) + 1.0) + 3e-7
+            out = torch.full((batch + 1, n_out + 3), -7.0, device="cuda:0")
+            view = out[:batch, :n_out]
+            view.copy_(D.to_device_colmajor(dst))
+            D.prod_bias_act(view, dev, Bd, trans, 0.25, beta, bias=None if b is None else torch.from_numpy(b).cuda(),
+                            act=_lib.ACT_SIGMOID_SAMPLE, seed=321)
+            assert L.cuvdia_last_kernel().decode() == "spmm_thin_kernel" + shape
+            decided = np.abs(p.astype(np.float64) - u) > tol
+            assert decided.mean() > 0.99
+            assert np.array_equal(D.to_host_colmajor(view)[decided], oracle.rnd_binarize(p, u)[decided])
+            assert torch.all(out[:, n_out:] == -7.0) and torch.all(out[batch] == -7.0)
+    finally:
+        L.cuvdia_set_path(_lib.PATH_AUTO)

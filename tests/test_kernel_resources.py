@@ -37,3 +37,10 @@ def test_rows_gradient_holds_its_registers():
     found = {n: m for n, m in _kernel_resources.kernels().items() if "dd2dia_rows_kernel" in n}
     assert len(found) >= 26
     assert {n: m[".vgpr_spill_count"] for n, m in found.items() if m[".vgpr_spill_count"] or m[".private_segment_fixed_size"]} == {}
+
+
+def test_rows_along_the_lanes_need_no_memory_of_their_own():
+    """The product's samples pick their word of a block of the generator from registers: no lane has an array in memory."""
+    found = {n: m for n, m in _kernel_resources.kernels().items() if "spmm_thin_kernel" in n}
+    assert len(found) == 13 * 6
+    assert [n for n, m in found.items() if m[".private_segment_fixed_size"]] == []
