@@ -1,4 +1,4 @@
-"""The automatic choice of the plane's walk on either side of its rule for well-filled tiles, its result and the tile-by-tile
+"""The automatic choice of the plane's walk on either side of its lines, its result and the tile-by-tile
 kernel's against 64 bits."""
 import pytest
 
@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch,trans,fused,taken", [
     (282, 282, 7, 2, 5, 128, "n", False, True),
-    (282, 282, 7, 2, 5, 128, "n", True, False),       # with a bias: 5 x 5 and 11 x 11 only
+    (282, 282, 7, 2, 5, 128, "n", True, False),       # with a bias and a sigmoid 7 x 7 have the lower line
     (282, 282, 7, 2, 5, 70, "n", False, False),       # most of the second column tile is empty
     (517, 517, 5, 3, 5, 64, "n", False, True),        # one column tile
     (300, 620, 11, 2, 1, 192, "t", True, True),

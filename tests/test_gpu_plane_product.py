@@ -217,3 +217,41 @@ def test_as_many_groups_as_a_table_has(oracle, plane, trans):
     for alpha, beta, old in ((1.0, 0.0, None), (0.75, -0.5, dst)):
         _, ran = gu.check_prod(oracle, A, B, old, trans, alpha, beta, _lib.PATH_PLANE, "51 groups")
         assert ran == _lib.PATH_PLANE
+
+
+@pytest.mark.parametrize("trans", ["n", "t"])
+@pytest.mark.parametrize("act", ["plain", "bias", "sigmoid", "sample"])
+@pytest.mark.parametrize("shape", [SHAPES[i] for i in (0, 1, 2, 3, 4, 5)], ids=lambda s: "x".join(map(str, s)))
+def test_padded_destination_that_is_read(oracle, plane, shape, act, trans):
+    """Old values and results go by 32-bit offsets from the destination's columns, apart by more than their length and on no 16-byte
+    boundary: what lies between and around them stays, and none of it is read."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng, A, B, dst = _case(oracle, 29 + sum(shape), *shape, trans)
+    n, batch = dst.shape
+    bias = rng.uniform(-1, 1, n).astype(np.float32) if act != "plain" else None
+    code = {"sigmoid": _lib.ACT_SIGMOID, "sample": _lib.ACT_SIGMOID_SAMPLE}.get(act, _lib.ACT_NONE)
+    dev = gu.make_dev_dia(A)
+    X = torch.full((batch + 1, B.shape[0] + 5), float("nan"), device="cuda:0")
+    X[:batch, 1:B.shape[0] + 1] = D.to_device_colmajor(B)
+    out = torch.full((batch + 2, n + 7), float("nan"), device="cuda:0")
+    view = out[1:batch + 1, 3:n + 3]
+    view.copy_(D.to_device_colmajor(dst))
+    D.prod_bias_act(view, dev, X[:batch, 1:B.shape[0] + 1], trans, 0.25, 0.5, bias=None if bias is None else torch.from_numpy(bias).cuda(),
+                    act=code, seed=11)
+    assert _ran()
+    got = D.to_host_colmajor(view)
+    mag = oracle.prod_mag(A, B, dst, trans, 0.25, 0.5) + (0 if bias is None else np.abs(bias)[:, None])
+    if code == _lib.ACT_NONE:
+        gu.assert_close_mag(got, oracle.prod(A, B, dst, trans, 0.25, 0.5) + (0 if bias is None else bias[:, None]), mag, "padded")
+    else:
+        p = oracle.prod_bias_act(A, B, dst, trans, 0.25, 0.5, bias, True)
+        tol = 0.25 * gu.REL_TOL * mag + 3e-7         # (the sigmoid's steepest slope, and its own rounding)
+        if act == "sample":
+            u = oracle.sample_uniform(n, batch, 11)
+            decided = np.abs(p.astype(np.float64) - u) > tol
+            assert decided.mean() > 0.99 and np.array_equal(got[decided], oracle.rnd_binarize(p, u)[decided])
+        else:
+            assert np.all(np.abs(got.astype(np.float64) - p) <= tol)
+    assert torch.isnan(out[0]).all() and torch.isnan(out[batch + 1]).all() and torch.isnan(out[1:-1, :3]).all() and torch.isnan(out[1:-1, n + 3:]).all()

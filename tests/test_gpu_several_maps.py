@@ -8,6 +8,8 @@ pytestmark = pytest.mark.gpu
 
 def _check(oracle, offsets, h, w, batch, trans, path, what):
     import _gpu_util as gu
+    from cuv_amd import _lib
+    kernel, ran_path = (b"spmm_walk_kernel", _lib.PATH_WALK) if path == _lib.PATH_WALK else (b"spmm_tiled_kernel", _lib.PATH_TILED)
     rng = np.random.default_rng(h + w + batch)
     A = oracle.Dia(h, w, np.asarray(offsets, np.int32), max(h, w), 1)
     A.vals[:] = np.nan                                   # padding must never be read
@@ -18,7 +20,7 @@ def _check(oracle, offsets, h, w, batch, trans, path, what):
     dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
     for alpha, beta, old in ((1.0, 0.0, None), (0.75, -0.5, dst)):
         _, ran = gu.check_prod(oracle, A, B, old, trans, alpha, beta, path, what)
-        assert ran == path or path != 3                  # (3: the walking kernel)
+        assert ran == ran_path and _lib.lib().cuvdia_last_kernel().startswith(kernel)
 
 
 @pytest.mark.parametrize("px,py,fs,maps_in,maps_out,batch", [
