@@ -5,9 +5,9 @@
 // A wave owns 256 rows of one chunk: a lane keeps 4 rows x LC diagonals of running sums and, per batch column, loads
 // its 4 values of A and of B (one 16-byte load each) and gets the LC - 1 values of B that follow its own from its
 // neighbours through a piece of LDS that belongs to the wave; the next CU columns (2, or 4 on launches of few waves) are in
-// flight meanwhile.  No barrier until the end, and 4-byte alignment is all the loads need -- the kernels that share staged operands between
-// waves take 16-byte pieces from 16-byte boundaries, and fall to single-element loads where a map's width, the leading
-// dimension or a pointer is no multiple of 4 -- and 64-bit addresses: no limit on the operands' sizes.  The waves of a
+// flight meanwhile.  No barrier until the end, and 4-byte alignment is all the loads need -- the kernels that share staged
+// operands between waves take 16-byte pieces from 16-byte boundaries, and fall to single-element loads where a map's width, the
+// leading dimension or a pointer is no multiple of 4 -- and 64-bit addresses: no limit on the operands' sizes.  The waves of a
 // workgroup take neighbouring chunks of the same rows (A's values come out of the L1) or, on launches of few tiles,
 // ranges of the batch, whose sums meet in LDS.
 //
@@ -282,21 +282,24 @@ bool dd2dia_rows_by_size(const DiaView &C, int batch, bool aligned, bool windowe
     // there, 0.85 - 1.1 above 8 columns of rows up to 4 wide and above 12 of 5 and 6 (5 x 5, 396 x 278, batch 15 11.5 and 13.5 us).
     // Pairs of chunks on up to 256 tiles: 1.1 - 1.5 up to batch 128 (rows 5 wide 0.96 - 1.05 above 96), 0.9 - 1 up to 256, 1.05 -
     // 1.25 where 16 ranges run, up to batch 2048, 0.79 - 0.95 above (8 x 8, 28 x 28, batch 4096 130 and 153 us), 0.9 - 0.96 for
-    // 3 columns, two steps of one wave; up to 1024 tiles 1.0 - 1.5 up to batch 48, of rows 5 and 6 wide up to 16 (5 x 5,
-    // 128 x 128, batch 64 6.8 and 8.2).
+    // 3 columns, two steps of one wave; up to 1024 tiles 1.0 - 1.5 up to batch 48, of bands of a few chunks up to 64 (mean
+    // 1.25; a band of 15 on 262 x 262, batch 64 16.4 -> 11.9), of rows 5 and 6 wide up to 16 (5 x 5, 128 x 128, batch 64 6.8 and
+    // 8.2).
     // 9 to 12 wide window rows in the plane's kernel: 1.1 - 1.6 up to batch 20, 0.6 - 0.85 above 32.
     // Of 1583 gradients that the lines without these distinctions had sent here 230 are left out, at 0.79 - 1.5 (mean 0.92); the
     // others are at a mean of 1.25, 1 % below 1.0, the least 0.94.
     const long long tiles = (long long)((C.h + DR_ROWS - 1) / DR_ROWS) * C.n_chunks_n;
     const int run = C.max_len_n;
     if (windowed) return C.walk_n.period % 64 != 0 && batch <= (C.walk_n.lck > CHUNK_MAX && C.walk_n.lck < 13 ? 20 : 8);
-    if (tiles > 1024 && run <= CHUNK_MAX && C.n_chunks_n > 1 && batch <= (run >= 7 || C.n_chunks_n > run ? 16 : run >= 5 ? 12 : 8)) return true;
+    const int short_batch = run >= 7 || C.n_chunks_n > run ? 16 : run >= 5 ? 12 : 8;
+    if (tiles > 1024 && run <= CHUNK_MAX && C.n_chunks_n > 1 && batch <= short_batch) return true;
     if (C.n_units < C.n_chunks_p && run <= CHUNK_MAX && run >= 5 && tiles <= 1024 && (batch != 3 || tiles > 256)) {
-        const int most = tiles <= 256 && C.n_chunks_n < 14 ? (run == 5 ? 96 : 128) : run >= 7 ? 48 : 16;
+        const int most = tiles <= 256 && C.n_chunks_n < 14 ? (run == 5 ? 96 : 128) : run < 7 ? 16 : C.n_chunks_n < run ? 64 : 48;
         if (batch <= most || (tiles <= 256 && batch > 256 && batch <= DR_WAVES_MOST * DR_BLOCK)) return true;
     }
     if (C.n_chunks_n >= 14) return batch <= 64;
-    const bool wide = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.pair_delta_max > PAIR_NARROW_DELTA && C.pair_delta_max <= PAIR_BAND_DELTA;
+    const bool wide = C.n_units < C.n_chunks_p && C.max_len_n <= CHUNK_MAX && C.pair_delta_max > PAIR_NARROW_DELTA &&
+                      C.pair_delta_max <= PAIR_BAND_DELTA;
     return wide && C.max_len_p >= 4 && batch <= 128;
 }
 

@@ -172,6 +172,7 @@ for M, yes, no in [
     (window(64, 64, 7, 1, 2), [64, 300], [65]),                                      # 14 chunks
     (window(120, 120, 7), [3, 48], [49, 300]),                                       # 399 tiles
     (window(128, 128, 5), [3, 16], [17, 300]),                                       # 320
+    (matrix(262 * 262, 262 * 262, list(range(-7, 8))), [64], [65, 300]),             # 538, two chunks
     (window(280, 280, 7), [16], [17]),                                               # 2149
     (window(356, 356, 5), [12], [13]),                                               # 2480
     (window(416, 217, 5, 1, 2), [16], [17]),                                         # ..., two maps
