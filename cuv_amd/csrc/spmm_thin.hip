@@ -249,6 +249,10 @@ hipError_t launch_lc(const ThinLaunch &L, int cb, int g, int waves)
     return cb == 1 ? launch_one<LC, 1, 4>(L, waves) : launch_one<LC, 2, 4>(L, waves);
 }
 
+// Few chunks per row block (launch_spmm_thin): 8 columns per lane only from so many workgroups of them on.
+bool thin_few_chunks(int nchunks, double chunks) { return chunks <= (nchunks < 16 ? 18 : 9); }
+constexpr int THIN_EIGHT_FROM = 4000;
+
 }  // namespace
 
 bool spmm_thin_ok(const DiaView &A, bool trans)
@@ -268,15 +272,26 @@ bool spmm_thin_by_size(const DiaView &A, bool trans, int batch)
     // percentile; median 1.37, 2.1 % below 0.97, most of them maps whose width is a multiple of 4); one step beyond these
     // lines a tenth of the products falls below 0.9.  On 2400 products of maps of any shape up to 640 wide, batch up to 640:
     // none and 1.5 % below 0.97, the least 0.90.
-    // Measured again on 3000 products and layers of the same maps, in turn with the lines below 14, 24 and 40 chunks at 90, 110
-    // and 120 tiles, above 40 at 190, and up to 35 columns decided by the tiles alone: 114 came here that had not, at 0.82 - 2.0
-    // times the rate (mean 1.22, 10 below 0.97).  (A second column tile that is nearly empty: 448 x 448, a band of 25, batch 67 59 ->
-    // 85 us.)
+    // Up to 35 columns of many tiles: measured on 2742 products and layers of maps up to 520 wide that meet fewer than 14 chunks.
+    // Rows 6 and 13 long are behind with 8 columns per lane (337 at a mean of 0.94, the least 0.65; 340 x 340, 6 x 6, 2 maps to 5,
+    // batch 25, transposed 184 us tile by tile, 217 here); from 7 on 33 - 35 columns with 8 per lane are a fifth group nearly empty
+    // (0.83 - 1.2).  Where a table holds twice the chunks that a row block meets -- one map to more, transposed -- the results are
+    // most of the traffic: of rows from 7 on and fewer than 1000 tiles 25 - 28 columns are ahead with an odd length (1.20; 0.88 at
+    // the least), not with 8 and 12 (0.71 - 1.3), and more are not (29 - 35: 1.02, a third below 0.97;
+    // 32 x 410, 8 x 8, 1 map to 8, batch 30, transposed 32 us tile by tile, 49 here).  The 1945 that come here are at 0.82 - 2.9
+    // (mean 1.32, 2 % below 0.97), the 797 left out at a mean of 1.00, half of them below 0.97.  (A second column tile that is
+    // nearly empty: 448 x 448, a band of 25, batch 67 59 and 85 us.)
     const double tiles = (n_out + 63) / 64 * (batch / 64.0);     // of the columns that exist
     const double chunks = (double)A.nnz / n_out / lc;            // per tile, those outside the operand left out
     const double there = batch / 64.0 / ((batch + 63) / 64);
     const double most = chunks < 6 ? 40 : chunks < 9.5 ? 56 : chunks < 14 ? 115 : chunks < 40 ? 130 : 250;
-    if (batch <= 35 && chunks >= 4 && tiles >= (chunks < 6 ? 1000 : 300)) return true;
+    if (batch <= 35 && chunks >= 4 && tiles >= (chunks < 6 ? 1000 : 300)) {
+        const int nchunks = trans ? A.n_chunks_t : A.n_chunks_n;
+        const long long groups = (n_out + 255) / 256 * (long long)((batch + 7) / 8);
+        const bool eight = !thin_few_chunks(nchunks, chunks) || groups >= THIN_EIGHT_FROM, wide = nchunks >= 1.9 * chunks;
+        const int most_columns = lc <= 5 ? 35 : !wide ? (eight ? 32 : 35) : tiles >= 1000 ? 32 : lc % 2 == 1 ? 28 : 24;
+        if (!(eight && (lc == 6 || lc == 13)) && batch <= most_columns) return true;
+    }
     return tiles < most || (chunks >= 14 && there <= (lc <= 5 ? 0.8 : 0.7));
 }
 
@@ -300,7 +315,7 @@ hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B,
     if (L.nchunks >= 16 && wgs(256, 2) <= 160) {
         g = 4;
         if (cb > 2) cb = 2;
-    } else if (cb == 8 && chunks <= (L.nchunks < 16 ? 18 : 9)) {
+    } else if (cb == 8 && thin_few_chunks(L.nchunks, chunks)) {
         // Few chunks per row block, however many the table has: 8 waves have nothing to share, and their sums' place in LDS
         // lets two workgroups into a CU.  Measured on 170 random products, up to 16 maps, batch 1 to 140, every shape: of those
         // that come here the choice below is at 1.00 - 2.4 times the rate of 8 columns by 4 or 8 waves (mean 1.35), within 1.2 of
@@ -308,7 +323,7 @@ hipError_t launch_spmm_thin(const DiaView &A, const float *vals, const float *B,
         // 0.99 is 144 x 144, 5 x 5, 2 maps to 1, batch 17: 8.4 -> 9.0 us).  448 x 448, 3 x 3, 1 map to 4, batch 23, transposed 94 -> 45 us; 388 x 388,
         // 7 x 7, batch 12, transposed 33 -> 17.  Tables of 16 chunks and more had 4 waves before: beyond 9 chunks a row block
         // 0.89 - 1.1.
-        if (wgs(256, 8) < 4000) cb = 4;
+        if (wgs(256, 8) < THIN_EIGHT_FROM) cb = 4;
         const long long n = wgs(256, cb);
         waves = n >= 16000 ? 1 : n >= 3000 || chunks <= 3 ? 2 : 4;
     } else if (cb == 8 && L.nchunks >= 16) {

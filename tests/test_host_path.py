@@ -187,6 +187,32 @@ for M, yes, no in [
 """)
 
 
+def test_the_products_of_few_columns_that_run_with_rows_along_the_lanes(tmp_path):
+    """Both sides of every limit of the choice on many tiles."""
+    _fake_hip.run(tmp_path, """
+def thin(M, trans, batch):
+    out, inner = (M.w, M.h) if trans == "t" else (M.h, M.w)
+    D.prod(tensor(batch, out, bytes_at=1 << 41), M, tensor(batch, inner, bytes_at=1 << 42), trans)
+    return L.cuvdia_last_kernel().startswith(b"spmm_thin_kernel")
+def window(px, py, fs, maps_in=1, maps_out=1):
+    return matrix(px * py * maps_in, px * py * maps_out, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+for M, trans, yes, no in [
+    (window(201, 260, 7), "n", [24, 32, 35], [36]),          # 4 columns per lane
+    (window(152, 152, 3, 4, 4), "n", [24, 35], [36]),        # 8
+    (window(332, 332, 7, 2, 2), "n", [24, 32], [33]),
+    (window(340, 340, 6, 2, 5), "t", [], [24, 25, 32]),      # 8, window rows of 6 and of 13 diagonals
+    (window(90, 90, 13, 1, 16), "t", [], [24, 32]),
+    (window(420, 420, 6), "n", [24, 35], [36]),              # 4
+    (window(32, 410, 8, 1, 8), "t", [24], [25, 30]),         # 15 chunks' rows, of which a row block meets 8
+    (window(164, 234, 8, 1, 8), "t", [24, 32], [33]),        # ..., on more than 1000 tiles
+    (window(57, 152, 7, 1, 8), "t", [28], [29]),
+    (window(96, 260, 5, 1, 8), "t", [24, 35], [36]),
+]:
+    for batch in yes + no:
+        assert thin(M, trans, batch) == (batch in yes), (M.h, M.w, M.num_dia, batch, L.cuvdia_last_kernel())
+""")
+
+
 def test_the_planned_walk_is_the_one_that_runs(tmp_path):
     """cuvdia_plan_walk_launch against the kernel and the grid of the product, over maps, windows and batches on both sides of
     its rules."""
