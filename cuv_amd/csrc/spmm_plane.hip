@@ -252,7 +252,8 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     const int my_row = 4 * (lane % 8), my_col = 16 * wave + lane / 8;
     // (what lies past the batch or before the rows of this walk is out of the resource's range)
     auto place = [&](int c, int r) { return c < cols && r >= skip ? (unsigned)c * ((unsigned)ldy * 4u) + 4u * r : OOB_OFFSET; };
-    const bool reads_old = beta != 0.f && !(EP && ep.act == 2);
+    const int sample_row = lane % 32, sample_col = 16 * wave + 8 * (lane / 32);   // sampled: a lane takes a row and 8 columns
+    const bool reads_old = beta != 0.f;
     f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     auto read_old = [&](int m) {
         const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
@@ -261,6 +262,15 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             if (skip == 0) {
                 old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
             } else {
+        // (sampled: all before the first store; one by one between the stores each waited for memory: 5 x 5, 272 x 63, 1 map to 8,
+        // batch 670, transposed 404 us like that, 276 now; 8 x 8, 364 x 364, batch 273 279 and 185; 9 x 9, 467 x 467, batch 860
+        // 1410 and 984; 11 x 11, 128 x 251, 1 to 8, batch 898 1955 and 1233)
+        if (EP && ep.act == 2) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                old[i / 4][i % 4] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(sample_col + i, sample_row), tile_at, 0));
+            return;
+        }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     old[k][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0));
@@ -277,8 +287,8 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (EP && ep.act == 2) {
-            // sampled: a lane takes a row and 8 columns, two blocks of the generator
-            const int r = lane % 32, c0 = 16 * wave + 8 * (lane / 32), row = row_first + m * period + r;
+            // sampled: two blocks of the generator
+            const int r = sample_row, c0 = sample_col, row = row_first + m * period + r;
             const float bias = ep.bias ? ep.bias[row] : 0.f;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -286,11 +296,9 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int c = c0 + 4 * h + i;
-                    const unsigned to = place(c, r);
                     const float t = alpha * out[c * OPITCH + r];
-                    const float was = beta == 0.f ? 0.f : __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, to, tile_at, 0));
-                    const float p = sp_finish(beta == 0.f ? t : beta * was + t, bias, 2, w.w[i]);
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(p), yrsrc, to, tile_at, 0);
+                    const float p = sp_finish(beta == 0.f ? t : beta * old[h][i] + t, bias, 2, w.w[i]);
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(p), yrsrc, place(c, r), tile_at, 0);
                 }
             }
             return;
