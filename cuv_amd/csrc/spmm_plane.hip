@@ -534,18 +534,24 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     // Taken by the steps, with the positions that only fill tiles up, over the work: up to these lines, for plain products,
     // with a bias and a sigmoid, and with a sample (on the vector unit, a few workgroups at a time).  Columns that only fill
     // tiles up are the tile-by-tile kernel's as well; where they are more than half of those that exist the kernel with rows
-    // along the lanes does without them, and is ahead on a single column tile.
-    // Fitted to 1841 random products and layers of 1 to 16 maps, 28 to 512 wide, batch 24 to 1024, all kernels timed on each.  Timed
-    // again against the kernel otherwise taken, on 1100 others: of 505 that come here the mean is 1.21, 1 % are below 0.93 (the
-    // least, 0.87, on 5 x 5 windows whose segments fill a round badly), 5 % below 0.99.  A sample is taken at every exit, and with
-    // one map there is an exit for every block: 9 x 9 1.0 - 1.1 up to 1.4, 0.77 - 1.1 (mean 0.96) from there to the line of several
-    // maps (396 x 396, batch 576 539 us here and 486).
-    static const struct { int k; double plain, fused, sample; } LINES[] = {
-        {5, 1.8, 1.85, 1.75}, {7, 2.4, 1.5, 1.45}, {8, 2.5, 2.2, 1.8}, {9, 2.2, 2.4, 1.7}, {11, 2.0, 1.8, 1.3}};
+    // along the lanes does without them, and is ahead on a single column tile (and, with a sample, up to 76 columns of 15 chunks
+    // and more: 0.72 - 0.95 of its rate, 310 x 310, 5 x 5, 3 maps to 4, batch 71 204 us here and 152).
+    // Fitted to random products and layers of 1 to 16 maps, 28 to 520 wide, batch 24 to 1024, all kernels timed on each; of 10700
+    // others within these lines the mean is 1.29 times the better other kernel's rate, 5 % are below 0.99, 3.6 % below 0.97 (2.0 %
+    // without samples added to old values, whose exit was slower then, and of up to 76 columns; the least, 0.63, on 5 x 5 windows
+    // of maps 32 wide).  A sample is taken at every exit, on the vector unit, and with one map there is
+    // an exit for every block: 9 x 9 1.05 on average from 1.4 to 1.5, 0.98 from there to 1.8; with several 1.19 and 1.17 around 1.7;
+    // 11 x 11 with several 1.22 from 1.4 to 1.5 and 1.18 to 1.6, with one 1.02 and 0.98.  7 x 7 with a sigmoid are at 1.1 - 1.6 up to
+    // 1.8, but their steps alone are looked at beyond 1.5.
+    static const struct { int k; double plain, fused, sample, sample_one; } LINES[] = {{5, 1.8, 1.85, 1.75, 1.75},
+                                                                                       {7, 2.4, 1.5, 1.55, 1.45},
+                                                                                       {8, 2.5, 2.2, 1.8, 1.8},
+                                                                                       {9, 2.2, 2.4, 1.7, 1.5},
+                                                                                       {11, 2.0, 1.8, 1.55, 1.3}};
     double line = 0;
     for (const auto &l : LINES)
-        if (l.k == wk.k) line = ep.act == 2 ? l.sample : fused ? l.fused : l.plain;
-    if (wk.k == 9 && ep.act == 2 && wk.ngroups == 1) line = 1.4;
+        if (l.k == wk.k) line = ep.act != 2 ? (fused ? l.fused : l.plain) : wk.ngroups > 1 ? l.sample : l.sample_one;
+    if (wk.k == 7 && fused && ep.act != 2 && over <= 1.4) line = 1.8;
     if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, wk.k >= 8 ? 1.65 : 1.45) : 0;
     bool ahead = over * L.tp * PLANE_ROWS / wk.period <= line;
     // (13 x 13: of what spmm_split.hip's rule leaves; with one column tile the values are most of the traffic, and the
@@ -553,6 +559,7 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     if (wk.k == 13) ahead = L.col_tiles >= 2 && over <= 1.65;
     if (!force && !ahead) return false;
     plane_cut(spans, walk_len, 1, L);
+    if (ep.act == 2 && batch <= 76 && L.col_tiles == 2 && (long long)spans.work * wk.k >= 15LL * walk_len) line = 0;
     return true;
 }
 

@@ -251,6 +251,29 @@ assert ran(509, 444, 1, 329, _lib.ACT_SIGMOID_SAMPLE)
 """)
 
 
+def test_layers_on_either_side_of_the_planes_lines(tmp_path):
+    """Samples of several maps, a sigmoid on tiles that the width fills badly, samples of a few columns more than a tile."""
+    _fake_hip.run(tmp_path, """
+def ran(px, py, fs, maps_in, maps_out, batch, trans, act):
+    h, w = px * py * maps_in, px * py * maps_out
+    A = matrix(h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+    out, inner = (w, h) if trans == "t" else (h, w)
+    D.prod_bias_act(tensor(batch, out, bytes_at=1 << 41), A, tensor(batch, inner, bytes_at=1 << 42), trans, act=act)
+    return L.cuvdia_last_kernel().decode().split("<")[0]
+for call, kernel in [
+    ((288, 318, 11, 4, 4, 154, "t", _lib.ACT_SIGMOID_SAMPLE), "spmm_plane_kernel"),
+    ((520, 520, 11, 1, 1, 537, "n", _lib.ACT_SIGMOID), "spmm_plane_kernel"),
+    ((171, 270, 7, 2, 5, 94, "t", _lib.ACT_SIGMOID), "spmm_plane_kernel"),
+    ((261, 261, 7, 4, 4, 128, "n", _lib.ACT_SIGMOID_SAMPLE), "spmm_plane_kernel"),
+    ((310, 310, 5, 3, 4, 71, "n", _lib.ACT_SIGMOID), "spmm_plane_kernel"),
+    ((310, 310, 5, 3, 4, 71, "n", _lib.ACT_SIGMOID_SAMPLE), "spmm_thin_kernel"),
+    ((310, 310, 5, 3, 4, 77, "n", _lib.ACT_SIGMOID_SAMPLE), "spmm_plane_kernel"),
+    ((160, 189, 7, 1, 16, 70, "t", _lib.ACT_SIGMOID_SAMPLE), "spmm_plane_kernel"),       # 7 chunks a tile
+]:
+    assert ran(*call) == kernel, (call, L.cuvdia_last_kernel())
+""")
+
+
 def test_an_empty_batch_is_launched_for_the_projection_alone(tmp_path):
     _fake_hip.run(tmp_path, """
 A = matrix(4096, 4096, [64 * dy + dx for dy in range(-2, 3) for dx in range(-2, 3)])
