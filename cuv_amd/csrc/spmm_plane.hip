@@ -73,7 +73,8 @@ struct PlaneShape {
     static constexpr int LDS_FLOATS = STAGE + std::max(STAGE, LAST_READ + 1);
     static constexpr int XIT = (XQ + PLANE_WAVES - 1) / PLANE_WAVES;    // load instructions per wave
     static constexpr int FIT = 160 * 1024 / ((4 * LDS_FLOATS + 4 * PLANE_TAB + 1279) / 1280 * 1280);
-    // Workgroups per CU, a wave per SIMD each: as many as fit in LDS and, with the registers that a wave needs, on a SIMD.
+    // Workgroups per CU, a wave per SIMD each: as many as fit in LDS and, with the registers that a wave needs, on a SIMD (fused
+    // 9 x 9 windows spill 4 there, and are faster all the same: `AHEAD`).
     static constexpr int per_cu(bool fused)
     {
         const int most = K <= 5 ? 4 : K <= 8 ? (fused ? 3 : 4) : 3;
@@ -133,7 +134,8 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     const float *const xbase = X + (long long)col0 * ldx;
     const sp_int4 xrsrc = raw_rsrc(xbase, (unsigned)(((long long)(cols - 1) * ldx + n_in) * 4));
     const sp_int4 arsrc = raw_rsrc(vals, a_bytes);
-    const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(Y + (long long)col0 * ldy, 0, (unsigned)(((long long)(cols - 1) * ldy + n_out) * 4), 0x00020000);
+    const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        Y + (long long)col0 * ldy, 0, (unsigned)(((long long)(cols - 1) * ldy + n_out) * 4), 0x00020000);
     const int amin = min(0, astep4 * (LC - 1));
     const unsigned lds0 = (unsigned)(unsigned long long)(__attribute__((address_space(3))) float *)&lds[0];
 
@@ -169,7 +171,9 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             // the block crosses an end of the operand: element by element, what does not exist is 0
             for (int i = wave; i < 4 * S::XQ; i += waves) {
                 const int p = 64 * i + lane, col = p / (4 * S::XQ), r = p - col * (4 * S::XQ), row = x0 + r;
-                lds_load_b32(xrsrc, base + 256u * i, r < 4 * nqx && (unsigned)row < (unsigned)n_in ? (unsigned)min(col, cols - 1) * ((unsigned)ldx * 4u) + 4u * row : OOB_OFFSET);
+                const bool there = r < 4 * nqx && (unsigned)row < (unsigned)n_in;
+                lds_load_b32(xrsrc, base + 256u * i,
+                             there ? (unsigned)min(col, cols - 1) * ((unsigned)ldx * 4u) + 4u * row : OOB_OFFSET);
             }
         }
         for (int s = wave; s < K; s += waves) {
@@ -185,8 +189,9 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             } else {
                 for (int it = 0; it < (LC * S::AROW + 63) / 64; ++it) {
                     const int p = 64 * it + lane, dx = p / S::AROW, r = p % S::AROW;
+                    const bool there = (unsigned)(x0 + r + dx) < (unsigned)n_in;
                     if (dx < LC)
-                        lds_load_b32(arsrc, to + 256u * it, (unsigned)(x0 + r + dx) < (unsigned)n_in ? (unsigned)(at + astep4 * dx + 4 * r) : OOB_OFFSET);
+                        lds_load_b32(arsrc, to + 256u * it, there ? (unsigned)(at + astep4 * dx + 4 * r) : OOB_OFFSET);
                 }
             }
         }
@@ -257,11 +262,6 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     f4 old[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     auto read_old = [&](int m) {
         const unsigned tile_at = (unsigned)(row_first + m * period) * 4u;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            if (skip == 0) {
-                old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
-            } else {
         // (sampled: all before the first store; one by one between the stores each waited for memory: 5 x 5, 272 x 63, 1 map to 8,
         // batch 670, transposed 404 us like that, 276 now; 8 x 8, 364 x 364, batch 273 279 and 185; 9 x 9, 467 x 467, batch 860
         // 1410 and 984; 11 x 11, 128 x 251, 1 to 8, batch 898 1955 and 1233)
@@ -271,6 +271,11 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                 old[i / 4][i % 4] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(sample_col + i, sample_row), tile_at, 0));
             return;
         }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            if (skip == 0) {
+                old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(yrsrc, place(my_col + 8 * k, my_row), tile_at, 0));
+            } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     old[k][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yrsrc, place(my_col + 8 * k, my_row + i), tile_at, 0));
@@ -506,7 +511,8 @@ void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
 bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpilogue &ep, bool force, PlaneLaunch &L)
 {
     const bool fused = ep.bias != nullptr || ep.act != 0;
-    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.ngroups * wk.k > PLANE_TAB || wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
+    if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.lck != wk.k || wk.ngroups * wk.k > PLANE_TAB) return false;
+    if (wk.period < PLANE_ROWS || (wk.k == 13 && fused)) return false;
     const PlaneSpans &spans = *wk.spans;
     if (spans.work == 0) return false;
     L.col_tiles = (batch + 63) / 64;
@@ -553,13 +559,13 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
         if (l.k == wk.k) line = ep.act != 2 ? (fused ? l.fused : l.plain) : wk.ngroups > 1 ? l.sample : l.sample_one;
     if (wk.k == 7 && fused && ep.act != 2 && over <= 1.4) line = 1.8;
     if (L.col_tiles * 64 > batch + batch / 2) line = L.col_tiles > 1 ? std::min(line, wk.k >= 8 ? 1.65 : 1.45) : 0;
+    if (ep.act == 2 && batch <= 76 && L.col_tiles == 2 && (long long)spans.work * wk.k >= 15LL * walk_len) line = 0;
     bool ahead = over * L.tp * PLANE_ROWS / wk.period <= line;
     // (13 x 13: of what spmm_split.hip's rule leaves; with one column tile the values are most of the traffic, and the
     // tile-by-tile kernel fetches them in pieces twice as long)
     if (wk.k == 13) ahead = L.col_tiles >= 2 && over <= 1.65;
     if (!force && !ahead) return false;
     plane_cut(spans, walk_len, 1, L);
-    if (ep.act == 2 && batch <= 76 && L.col_tiles == 2 && (long long)spans.work * wk.k >= 15LL * walk_len) line = 0;
     return true;
 }
 
