@@ -548,9 +548,10 @@ bool spmm_plane_plan(const WalkView &wk, long long n_out, int batch, const SpEpi
     // of maps 32 wide).  A sample is taken at every exit, on the vector unit, and with one map there is
     // an exit for every block: 9 x 9 1.05 on average from 1.4 to 1.5, 0.98 from there to 1.8; with several 1.19 and 1.17 around 1.7;
     // 11 x 11 with several 1.22 from 1.4 to 1.5 and 1.18 to 1.6, with one 1.02 and 0.98.  7 x 7 with a sigmoid are at 1.1 - 1.6 up to
-    // 1.8, but their steps alone are looked at beyond 1.5.
+    // 1.8, but their steps alone are looked at beyond 1.5; plain ones at 1.11 on average from 2.0 to 2.1, 1.06 to 2.2, 0.99 from
+    // there to 2.4, two fifths below 0.97 (56 x 152, batch 897 41 us here and 33).
     static const struct { int k; double plain, fused, sample, sample_one; } LINES[] = {{5, 1.8, 1.85, 1.75, 1.75},
-                                                                                       {7, 2.4, 1.5, 1.55, 1.45},
+                                                                                       {7, 2.2, 1.5, 1.55, 1.45},
                                                                                        {8, 2.5, 2.2, 1.8, 1.8},
                                                                                        {9, 2.2, 2.4, 1.7, 1.5},
                                                                                        {11, 2.0, 1.8, 1.55, 1.3}};

@@ -261,6 +261,9 @@ def ran(px, py, fs, maps_in, maps_out, batch, trans, act):
     D.prod_bias_act(tensor(batch, out, bytes_at=1 << 41), A, tensor(batch, inner, bytes_at=1 << 42), trans, act=act)
     return L.cuvdia_last_kernel().decode().split("<")[0]
 for call, kernel in [
+    ((150, 150, 7, 4, 6, 200, "n", _lib.ACT_NONE), "spmm_plane_kernel"),
+    ((56, 152, 7, 1, 1, 897, "n", _lib.ACT_NONE), "spmm_tiled_kernel"),                  # segments of few map rows
+    ((272, 60, 7, 1, 2, 569, "n", _lib.ACT_NONE), "spmm_tiled_kernel"),
     ((288, 318, 11, 4, 4, 154, "t", _lib.ACT_SIGMOID_SAMPLE), "spmm_plane_kernel"),
     ((520, 520, 11, 1, 1, 537, "n", _lib.ACT_SIGMOID), "spmm_plane_kernel"),
     ((171, 270, 7, 2, 5, 94, "t", _lib.ACT_SIGMOID), "spmm_plane_kernel"),
