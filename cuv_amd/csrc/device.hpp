@@ -156,6 +156,26 @@ __device__ __forceinline__ void lds_load_b32(sp_int4 rsrc, unsigned lds_byte_add
                  :: "s"(lds_byte_addr), "v"(voff), "s"(rsrc) : "memory");
 }
 
+// f(integral_constant<I>) ... f(integral_constant<N - 1>)
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// acc[r] += a(lane 16 n + LANE0 + r) * x[r]: the value broadcast inside each row of 16 lanes
+template <int LANE0>
+__device__ __forceinline__ void fma8_dpp(float (&acc)[8], float a, const float *x)
+{
+#define CUVDIA_FMA(r)                                                                                       \
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc[r]) : "v"(a), "v"(x[r]), "n"(LANE0 + r));
+    CUVDIA_FMA(0) CUVDIA_FMA(1) CUVDIA_FMA(2) CUVDIA_FMA(3) CUVDIA_FMA(4) CUVDIA_FMA(5) CUVDIA_FMA(6) CUVDIA_FMA(7)
+#undef CUVDIA_FMA
+}
+
 constexpr unsigned OOB_OFFSET = 0x80000000u;     // >= every resource size used here
 
 }  // namespace

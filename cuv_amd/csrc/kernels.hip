@@ -3128,23 +3128,24 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
         }
     }
     if (path == CUVDIA_PATH_WALK) return hipErrorNotSupported;
-    // One of another width, or with a larger window: the plane's walk on the matrix cores, 13 x 13 ones with split operands.
     if (path == CUVDIA_PATH_AUTO || path == CUVDIA_PATH_PLANE) {
+        // One of another width, or with a larger window: the plane's walk on the matrix cores, 13 x 13 ones with split operands.
         PlaneLaunch plane{}, other{};
         const bool force = path == CUVDIA_PATH_PLANE, walks = spmm_plane_plan(wk, n_out, batch, ep, force, plane);
         const bool split = spmm_split_plan(wk, n_out, batch, force, walks, other);
-        if (split || walks) {
+        if (force && !split && !walks) return hipErrorNotSupported;
+        // A smaller one: patch by patch, or with rows along the lanes.
+        const bool thin = !split && !walks && spmm_thin_by_size(A, trans, batch);
+        if (split || walks || spmm_patch_plan(wk, n_out, batch, thin)) {
             PlaneLaunch &P = split ? other : plane;
-            if (ran) *ran = CUVDIA_PATH_PLANE;
+            if (ran && (split || walks)) *ran = CUVDIA_PATH_PLANE;
             P.tab = wk.tab_dev; P.ngroups = wk.ngroups; P.period = wk.period; P.s0 = wk.s0; P.astep4 = wk.astep4; P.k = wk.k;
             P.vals = vals; P.B = B; P.ldb = ldb; P.dst = dst; P.ldd = ldd; P.n_out = n_out; P.n_in = n_in; P.batch = batch;
             P.alpha = alpha; P.beta = beta; P.a_bytes = (unsigned)((long long)A.nd * A.stride * 4); P.ep = ep; P.stream = stream;
-            return split ? spmm_split_launch(P) : spmm_plane_launch(P);
+            return split ? spmm_split_launch(P) : walks ? spmm_plane_launch(P) : spmm_patch_launch(P);
         }
-        if (path == CUVDIA_PATH_PLANE) return hipErrorNotSupported;
+        if (thin) return launch_spmm_thin(A, vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, stream);
     }
-    if (path == CUVDIA_PATH_AUTO && spmm_thin_by_size(A, trans, batch))
-        return launch_spmm_thin(A, vals, B, ldb, dst, ldd, batch, trans, alpha, beta, ep, stream);
     const SpLaunch L{trans ? A.chunks_t_dev : A.chunks_n_dev,
                      trans ? A.n_chunks_t : A.n_chunks_n,
                      vals, A.stride, trans ? 1 : 0, B, ldb, dst, ldd, n_out, n_in, batch, alpha, beta,

@@ -102,7 +102,8 @@ int spmm_walk_plan(int lck, int k, int s0, int period, long long n_out, long lon
 // values are broadcast across each 16-lane row by DPP.  Window tables on
 // products of many tiles go to the walking kernel, which stages a block of
 // dense rows once for all the window rows that read it, or to the plane's walk
-// on the matrix cores (below); products of few tiles and ragged batches to the
+// on the matrix cores (below), smaller ones of 3 x 3, 5 x 5 and 7 x 7 windows
+// patch by patch (below); products of few tiles and ragged batches to the
 // kernel with rows along the lanes.
 // path: CUVDIA_PATH_AUTO -- those choices are made by size; _TILED -- the
 // walking kernel by size, else tile by tile; _WALK, _PLANE -- that kernel or
@@ -153,6 +154,10 @@ void plane_cut(const PlaneSpans &spans, int walk_len, int every, PlaneLaunch &L)
 // walks: whether the former would be taken.
 bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force, bool walks, PlaneLaunch &L);
 hipError_t spmm_split_launch(const PlaneLaunch &L);
+// The same, tile by tile, a tile being a patch of the window's plane (spmm_patch.hip): windows of 3 x 3, 5 x 5 and 7 x 7 of one
+// group.  thin: whether the kernel with rows along the lanes would be taken.
+bool spmm_patch_plan(const WalkView &wk, long long n_out, int batch, bool thin);
+hipError_t spmm_patch_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.
 hipError_t launch_momentum(float *W, float *M, const float *dW, long long n, float lr, float mw, float l2,

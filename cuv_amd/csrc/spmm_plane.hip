@@ -82,25 +82,6 @@ struct PlaneShape {
     }
 };
 
-template <int I, int N, class F>
-__device__ __forceinline__ void plane_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        plane_for<I + 1, N>(f);
-    }
-}
-
-// acc[r] += a(lane 16 n + LANE0 + r) * x[r]: the value broadcast inside each row of 16 lanes
-template <int LANE0>
-__device__ __forceinline__ void plane_fma8(float (&acc)[8], float a, const float *x)
-{
-#define PLANE_FMA(r)                                                                                        \
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc[r]) : "v"(a), "v"(x[r]), "n"(LANE0 + r));
-    PLANE_FMA(0) PLANE_FMA(1) PLANE_FMA(2) PLANE_FMA(3) PLANE_FMA(4) PLANE_FMA(5) PLANE_FMA(6) PLANE_FMA(7)
-#undef PLANE_FMA
-}
-
 template <int LC, int K, bool EP>
 __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) void spmm_plane_kernel(
     const int *__restrict__ tab, int ngroups, int period, int s0, int astep4, int tp, int nseg, PlaneCuts cuts,
@@ -226,13 +207,13 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
         // tiles alive at this step: max(0, u - K + 1) .. min(u, tiles - 1)
         const int lo = max(0, u - K + 1), n = min(u, tiles - 1) - lo + 1, s_lo = lo % K;
         const unsigned ones = (1u << n) - 1u, alive = (ones << s_lo) | (ones >> (K - s_lo));
-        plane_for<0, S::NG>([&](auto g_) {
+        static_for<0, S::NG>([&](auto g_) {
             constexpr int g = decltype(g_)::value;
             if (!((alive >> (4 * g)) & 15u)) return;
-            plane_for<0, S::NQ>([&](auto q_) {
+            static_for<0, S::NQ>([&](auto q_) {
                 constexpr int q = decltype(q_)::value;
                 const float v = value(g, q);
-                plane_for<0, 16>([&](auto b_) {
+                static_for<0, 16>([&](auto b_) {
                     constexpr int b = decltype(b_)::value, r = b % 8, dx = 2 * q + b / 8;
                     if constexpr (dx < LC) acc[g][r] = __builtin_amdgcn_mfma_f32_4x4x1f32(v, x[r + dx], acc[g][r], 4, b, 0);
                 });
@@ -240,11 +221,11 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
         });
         if constexpr (S::TAIL) {
             if ((alive >> (4 * S::NG)) & 1u) {
-                plane_for<0, S::NQ>([&](auto q_) {
+                static_for<0, S::NQ>([&](auto q_) {
                     constexpr int q = decltype(q_)::value;
                     const float v = st[S::X_FLOATS + lane_t + 2 * q * S::AROW];
-                    plane_fma8<0>(tail, v, x + 2 * q);
-                    if constexpr (2 * q + 1 < LC) plane_fma8<8>(tail, v, x + 2 * q + 1);
+                    fma8_dpp<0>(tail, v, x + 2 * q);
+                    if constexpr (2 * q + 1 < LC) fma8_dpp<8>(tail, v, x + 2 * q + 1);
                 });
             }
         }
@@ -370,7 +351,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
     constexpr bool AHEAD = S::per_cu(EP) < 4 || (EP && K == 5);
     int slot = 0;                                    // u % K
     for (int u = 0; u < steps; ++u) {
-        plane_for<0, K>([&](auto s_) {
+        static_for<0, K>([&](auto s_) {
             constexpr int s = decltype(s_)::value;
             if (slot == s && u < tiles) {
 #pragma unroll
@@ -401,7 +382,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
             if (AHEAD && !old_read) read_old(done);
             const int leaving = slot + 1 == K ? 0 : slot + 1;
             float v[8];
-            plane_for<0, K>([&](auto s_) {
+            static_for<0, K>([&](auto s_) {
                 constexpr int s = decltype(s_)::value;
                 if (leaving == s) {
 #pragma unroll

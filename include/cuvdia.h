@@ -155,7 +155,7 @@ long long cuvdia_plan_window_launch(const int *offsets_host, int nd, int stride,
  * is not 0.  Returns 0: no window table; 1: a window table without a walking
  * kernel (its large products run on the matrix cores for square windows of 5,
  * 7, 8, 9, 11 or 13 rows, else tile by tile, with their row tiles numbered
- * period-major on launches of many rounds); 2: a window table with a walking kernel (centred 3x3, 5x5 or
+ * period-major on launches of many rounds, or as patches of the window's plane); 2: a window table with a walking kernel (centred 3x3, 5x5 or
  * 7x7 window, period a multiple of 64); negative: an error.  The answer is
  * about the TABLE only.  Whether a given product runs the walking kernel also
  * depends on its shape -- cuvdia_plan_walk_launch answers that.  No
@@ -320,8 +320,9 @@ int cuvdia_dd2dia_offsets_f32(float *C_vals_device, const int *offsets_host,
  * hipMalloc.  It has no counterpart in the reference.  Same arguments, same
  * argument rules, and the generic, tile-by-tile or rows-along-the-lanes kernels
  * chosen as there: bit-identical results wherever cuvdia_spmm_offsets_f32 does
- * not take one of its kernels for window tables (the walking one or the one on
- * the matrix cores, on large products; CUVDIA_PATH_TILED_NOWALK keeps it from
+ * not take one of its kernels for window tables (the walking one, the one on
+ * the matrix cores, the tile-by-tile one whose tiles are patches of the
+ * window's plane; CUVDIA_PATH_TILED_NOWALK keeps it from
  * doing so), within rounding of them where it does.  But the
  * device copy of the offset table and of the chunk table the kernels walk -- which a
  * descriptor keeps in memory it allocates -- lives in a static device array
