@@ -1896,8 +1896,9 @@ __device__ __forceinline__ void dd2dia_unit(
     // scalar offsets, and left alone the compiler derives them from a vector
     // copy of ldb and then has to loop over lanes to issue each load.
     unsigned lda4, ldb4;
-    asm("v_readfirstlane_b32 %0, %1" : "=s"(lda4) : "v"((unsigned)lda * 4u));
-    asm("v_readfirstlane_b32 %0, %1" : "=s"(ldb4) : "v"((unsigned)ldb * 4u));
+    // (the waits: the compiler knows of none that a register just written needs before it is read like this)
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(lda4) : "v"((unsigned)lda * 4u));
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(ldb4) : "v"((unsigned)ldb * 4u));
 
     float acc[NCH][4][LC];
 #pragma unroll
