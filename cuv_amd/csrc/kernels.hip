@@ -1742,7 +1742,6 @@ struct DdShape {
     static constexpr int NB = WIDE == DD_WIDE ? 3 : WIDE == DD_SHIFTED ? 1 : 2;   // 16-byte pieces a lane holds per column
     static constexpr int PITCH = 64 * NQ + (LONG ? 16 : 8);     // staged rows per column: 264, 272, 392 or 520
     static constexpr int WAVES = (NCH == 2 && WIDE != DD_SHIFTED) ? 8 : 4;
-    static constexpr int RED_PAD = LONG ? 4 : 8;              // a long chunk's sums then fit a third of a CU's LDS
     static constexpr int WAVE_FLOATS = 2 * DD_BG * PITCH + 4;   // two buffers + a slot idle lanes write to
     static constexpr int STAGE_FLOATS = WAVES * WAVE_FLOATS;
 };
@@ -1759,13 +1758,11 @@ struct DdStage {
     float a[NA][DD_BG][4];    // this lane's 4 rows of each column (a shifted pair: and the 4 rows delta above)
 };
 
-template <int LC, int NCH>
-constexpr int dd_red_floats() { return 4 * 4 * (NCH * LC * 64 + DdShape<NCH, LC>::RED_PAD); }
 template <int LC, int NCH, int WIDE = DD_NARROW>
 constexpr int dd_lds_floats()
 {
     // (a shifted pair adds its chunks' sums one chunk after the other, in the block of a single chunk)
-    constexpr int red = WIDE == DD_SHIFTED ? dd_red_floats<LC, 1>() : dd_red_floats<LC, NCH>();
+    constexpr int red = DdShape<NCH, LC, WIDE>::WAVES * (WIDE == DD_SHIFTED ? 1 : NCH) * LC * 64 * 4;
     return DdShape<NCH, LC, WIDE>::STAGE_FLOATS > red ? DdShape<NCH, LC, WIDE>::STAGE_FLOATS : red;
 }
 
@@ -1794,28 +1791,22 @@ __device__ __forceinline__ void dd2dia_unit(
     static_assert(!SHORT || TR + S::SPAN <= 256 || (S::LONG && TR + 16 <= 256), "a short tile's band is one piece per lane");
     constexpr int WIN = 4 + LC - 1;
     constexpr int WQ = (WIN + 3) / 4;
-    constexpr int RED_T = NRED * LC * 64 + S::RED_PAD;       // floats between the 4 rows a lane owns: keeps the
-                                                    // row-major read below free of bank conflicts
-    constexpr int RED_WAVE = 4 * RED_T;
-
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // each table entry in three (a long chunk: four) 16-byte scalar loads
-    typedef int int4v __attribute__((ext_vector_type(4)));
-    typedef const int4v __attribute__((address_space(4))) *sc_int4_ptr;
-    int s0[NCH], slots[NCH][S::SPAN];
+    typedef const int __attribute__((address_space(4))) *sc_int_ptr;         // (scalar loads)
+    // A wave's share of the output: positions wave, wave + WAVES, ... of the unit's NCH x LC (a shifted pair: of one chunk, then of
+    // the other), of which each lane combines and writes its own 4 rows.
+    constexpr int PASS = NRED * LC, SHARE = (PASS + WAVES - 1) / WAVES, PASSES = NCH / NRED;
+    int s0[NCH], slot[PASSES][SHARE];
 #pragma unroll
-    for (int n = 0; n < NCH; ++n) {
-        const sc_int4_ptr e = (sc_int4_ptr)(n == 0 ? ck1 : ck2);
-        const int4v e0 = e[0], e1 = e[1], e2 = e[2];
-        s0[n] = e0.x;
-        slots[n][0] = e0.z; slots[n][1] = e0.w; slots[n][2] = e1.x; slots[n][3] = e1.y;
-        slots[n][4] = e1.z; slots[n][5] = e1.w; slots[n][6] = e2.x; slots[n][7] = e2.y;
-        if constexpr (S::LONG) {
-            const int4v e3 = e[3];
-            slots[n][8] = e2.z; slots[n][9] = e2.w; slots[n][10] = e3.x; slots[n][11] = e3.y; slots[n][12] = e3.z;
+    for (int n = 0; n < NCH; ++n) s0[n] = ((sc_int_ptr)(n == 0 ? ck1 : ck2))[0];
+#pragma unroll
+    for (int n0 = 0; n0 < PASSES; ++n0)
+#pragma unroll
+        for (int i = 0; i < SHARE; ++i) {
+            const int nj = n0 * PASS + min(wave + WAVES * i, PASS - 1), n = NCH == 1 ? 0 : nj / LC;
+            slot[n0][i] = ((sc_int_ptr)(n == 0 ? ck1 : ck2))[2 + nj - n * LC];
         }
-    }
     const int delta = NCH == 2 ? s0[NCH - 1] - s0[0] : 0;      // rows between the two windows
     const int wdelta = SHIFTED ? 0 : delta;                     // .. inside the staged band
     const int need = TR + wdelta + S::SPAN;                     // staged rows that are ever read
@@ -1828,30 +1819,38 @@ __device__ __forceinline__ void dd2dia_unit(
     if (row0 - (SHIFTED ? delta : 0) >= h) return;
     const int myrow = row0 + 4 * lane;
 
-    // C values this lane will combine at the end: row row0 + 64*wave + lane of
-    // every diagonal of the unit (waves 0..3; a pair's waves 4..7 leave the
-    // output to them).  Byte offset of that slot, or the out-of-range marker
-    // where no matrix element sits.
-    auto c_offset = [&](int n, int j) -> unsigned {
-        const int sl = slots[n][j];
-        const int o = row0 + 64 * wave + lane - ((SHIFTED && n) ? delta : 0);
-        const int in = o + s0[n] + j;
-        const bool ok = (wave < 4) & (sl >= 0) & (o >= 0) & (o < h) & (in >= 0) & (in < w) & (64 * wave + lane < TR);
-        return ok ? ((unsigned)sl * (unsigned)stride + (unsigned)o) * 4u : OOB_OFFSET;
+    // Where a row of a quad has no matrix element there, it is worked element by element.
+    struct Quad { unsigned at, valid; };            // byte offset of the first row's slot; which of the 4 rows exist
+    auto out_quad = [&](int n0, int i) -> Quad {
+        const int nj = n0 * PASS + wave + WAVES * i, n = NCH == 1 ? 0 : nj / LC, j = nj - n * LC, sl = slot[n0][i];
+        const int o = myrow - ((SHIFTED && n) ? delta : 0), in = o + s0[0] + (n ? delta : 0) + j;
+        unsigned valid = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            valid |= ((o + t >= 0) & (o + t < h) & (in + t >= 0) & (in + t < w) & (4 * lane + t < TR)) ? 1u << t : 0u;
+        return Quad{((unsigned)sl * (unsigned)stride + (unsigned)o) * 4u, sl >= 0 ? valid : 0u};
     };
-    float cpre[NCH][LC];
+    typedef float f4q __attribute__((ext_vector_type(4)));
+    f4q cpre[PASSES][SHARE];
 #pragma unroll
-    for (int n = 0; n < NCH; ++n)
+    for (int n0 = 0; n0 < PASSES; ++n0)
 #pragma unroll
-        for (int j = 0; j < LC; ++j) cpre[n][j] = 0.f;
-    // beta == 0: C is not read; waves 4..7 of a pair write nothing and ask for nothing (a load costs the
-    // memory pipeline its slot even when every lane is out of range)
-    if ((beta != 0.f) & (wave < 4)) {
+        for (int i = 0; i < SHARE; ++i) cpre[n0][i] = f4q{0.f, 0.f, 0.f, 0.f};
+    // (beta == 0: C is not read)
+    if (beta != 0.f) {
         const __amdgpu_buffer_rsrc_t cr = make_rsrc(C, c_bytes);
 #pragma unroll
-        for (int n = 0; n < NCH; ++n)
+        for (int n0 = 0; n0 < PASSES; ++n0)
 #pragma unroll
-            for (int j = 0; j < LC; ++j) cpre[n][j] = buffer_load_f32(cr, c_offset(n, j));
+            for (int i = 0; i < SHARE; ++i) {
+                if (wave + WAVES * i >= PASS) continue;
+                const Quad q = out_quad(n0, i);
+                cpre[n0][i] = __builtin_bit_cast(f4q, __builtin_amdgcn_raw_buffer_load_b128(cr, q.valid == 15u ? q.at : OOB_OFFSET, 0, 0));
+                if (q.valid != 15u && q.valid != 0u) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) cpre[n0][i][t] = buffer_load_f32(cr, (q.valid >> t) & 1u ? q.at + 4u * t : OOB_OFFSET);
+                }
+            }
     }
 
     // The band of B travels as 16-byte pieces, a lane holding rows base + 4*lane
@@ -2060,59 +2059,46 @@ __device__ __forceinline__ void dd2dia_unit(
     }
     if (k < steps) step(k, 0, st0, st1);
 
-    // Combine the waves' partial sums.  8 waves: wave q + 4 hands its sums to
-    // wave q first (same lanes, same layout); then the four sums meet in wave
-    // order: total = ((p0 + p1) + p2) + p3 with p_q = s_q (+ s_{q+4}).
-    __syncthreads();
-    float *red = lds;                               // [wave][t][n][j][64 lanes], t blocks RED_T apart
-    if (WAVES == 8) {
-        if (wave >= 4) {
+    // Combine the waves' partial sums: every wave leaves its own in LDS, a lane's 4 rows side by side, and takes its share of the
+    // output (a shifted pair: one chunk after the other).  Summed in wave order: total = ((p0 + p1) + p2) + p3 with p_q = s_q, of
+    // 8 waves s_q + s_{q+4}.  (Before, four of 8 waves added the others' sums to theirs, 4 bytes at a time, and wrote the output:
+    // 5000 clocks of the 17500 of a one-round launch.  16384-unit layer, 7 x 7, batch 128 10.7 -> 9.5 us; 784 x 1568, 128
+    // diagonals, batch 96 9.0 -> 7.8; launches of many rounds 0 - 3 %.)
+    f4q *const red = reinterpret_cast<f4q *>(lds);           // [wave][position][64 lanes]
 #pragma unroll
-            for (int n = 0; n < NCH; ++n)
+    for (int n0 = 0; n0 < PASSES; ++n0) {
+        __syncthreads();                            // nobody uses the place any more
+#pragma unroll
+        for (int n = 0; n < NRED; ++n)
+#pragma unroll
+            for (int j = 0; j < LC; ++j)
+                red[(wave * PASS + n * LC + j) * 64 + lane] =
+                    f4q{acc[n0 + n][0][j], acc[n0 + n][1][j], acc[n0 + n][2][j], acc[n0 + n][3][j]};
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < SHARE; ++i) {
+            const int nj = wave + WAVES * i;
+            if (nj >= PASS) continue;
+            const Quad q = out_quad(n0, i);
+            f4q total;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                f4q v = red[(p * PASS + nj) * 64 + lane];
+                if constexpr (WAVES == 8) v += red[((p + 4) * PASS + nj) * 64 + lane];
+                total = p == 0 ? v : total + v;
+            }
+            f4q out;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) out[t] = (beta == 0.f) ? alpha * total[t] : beta * cpre[n0][i][t] + alpha * total[t];
+            float *const cd = reinterpret_cast<float *>(reinterpret_cast<char *>(C) + q.at);
+            if (q.valid == 15u) {
+                stream_store4(cd, out[0], out[1], out[2], out[3]);
+            } else {
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int j = 0; j < LC; ++j)
-                        red[(wave - 4) * RED_WAVE + t * RED_T + (n * LC + j) * 64 + lane] = acc[n][t][j];
-        }
-        __syncthreads();
-        if (wave >= 4) return;
-#pragma unroll
-        for (int n = 0; n < NCH; ++n)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int j = 0; j < LC; ++j)
-                    acc[n][t][j] += red[wave * RED_WAVE + t * RED_T + (n * LC + j) * 64 + lane];
-        // no barrier needed here: below, wave q overwrites only the block it has just read
-    }
-    // (a shifted pair: one chunk after the other through the block of a single chunk)
-#pragma unroll
-    for (int n0 = 0; n0 < NCH; n0 += NRED) {
-        if (n0 > 0) __syncthreads();                // the block is free again
-#pragma unroll
-        for (int n = 0; n < NRED; ++n)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int j = 0; j < LC; ++j)
-                    red[wave * RED_WAVE + t * RED_T + (n * LC + j) * 64 + lane] = acc[n0 + n][t][j];
-        __syncthreads();
-        const int r = 64 * wave + lane;             // row within the tile: lane r/4 owned it as its row r%4
-        const float *src = red + (r & 3) * RED_T + (r >> 2);
-#pragma unroll
-        for (int n = 0; n < NRED; ++n)
-#pragma unroll
-            for (int j = 0; j < LC; ++j) {
-                float total = src[(n * LC + j) * 64];
-#pragma unroll
-                for (int p = 1; p < 4; ++p) total += src[p * RED_WAVE + (n * LC + j) * 64];
-                const unsigned off = c_offset(n0 + n, j);
-                if (off != OOB_OFFSET) {
-                    float *cd = reinterpret_cast<float *>(reinterpret_cast<char *>(C) + off);
-                    stream_store(cd, (beta == 0.f) ? alpha * total : beta * cpre[n0 + n][j] + alpha * total);
-                }
+                    if ((q.valid >> t) & 1u) stream_store(cd + t, out[t]);
             }
+        }
     }
 }
 
