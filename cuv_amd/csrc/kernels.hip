@@ -1732,7 +1732,11 @@ constexpr int DD_BG = 4;           // batch columns per step
 //     one band of one piece (the tile is cut short, dd_short_rows), one window per column for both chunks, and two
 //     copies of A's rows.  Any distance that is a multiple of 4; 4 waves, three such workgroups to a CU.
 constexpr int DD_NARROW = 0, DD_WIDE = 1, DD_SHIFTED = 2;
-template <int NCH, int LC, int WIDE = DD_NARROW>
+// Waves of a workgroup: 4, of a launch of pairs that share A's rows 8, with its single units (which took 4: the 16384-unit layer at
+// batch 2048 99.3 us for 96.9).  12 would fit 7 diagonals with 8 registers spilled: 9.6 -> 11.5 us at batch 128, 99.9 at 2048.
+template <bool PAIRS, int WIDE>
+constexpr int dd_waves() { return !PAIRS || WIDE == DD_SHIFTED ? 4 : 8; }
+template <int NCH, int LC, int WIDE = DD_NARROW, int NW = (NCH == 2 && WIDE != DD_SHIFTED) ? 8 : 4>
 struct DdShape {
     static_assert(NCH == 1 || LC <= CHUNK_MAX, "pairs are made of short chunks");
     static_assert(NCH == 2 || WIDE == DD_NARROW, "only pairs come in forms");
@@ -1741,7 +1745,7 @@ struct DdShape {
     static constexpr int NQ = (NCH == 1 || WIDE == DD_SHIFTED) ? 4 : WIDE == DD_WIDE ? 8 : 6;   // 64-row blocks of the band
     static constexpr int NB = WIDE == DD_WIDE ? 3 : WIDE == DD_SHIFTED ? 1 : 2;   // 16-byte pieces a lane holds per column
     static constexpr int PITCH = 64 * NQ + (LONG ? 16 : 8);     // staged rows per column: 264, 272, 392 or 520
-    static constexpr int WAVES = (NCH == 2 && WIDE != DD_SHIFTED) ? 8 : 4;
+    static constexpr int WAVES = NW;
     static constexpr int WAVE_FLOATS = 2 * DD_BG * PITCH + 4;   // two buffers + a slot idle lanes write to
     static constexpr int STAGE_FLOATS = WAVES * WAVE_FLOATS;
 };
@@ -1758,12 +1762,12 @@ struct DdStage {
     float a[NA][DD_BG][4];    // this lane's 4 rows of each column (a shifted pair: and the 4 rows delta above)
 };
 
-template <int LC, int NCH, int WIDE = DD_NARROW>
+template <int LC, int NCH, int WIDE, int NW>
 constexpr int dd_lds_floats()
 {
     // (a shifted pair adds its chunks' sums one chunk after the other, in the block of a single chunk)
-    constexpr int red = DdShape<NCH, LC, WIDE>::WAVES * (WIDE == DD_SHIFTED ? 1 : NCH) * LC * 64 * 4;
-    return DdShape<NCH, LC, WIDE>::STAGE_FLOATS > red ? DdShape<NCH, LC, WIDE>::STAGE_FLOATS : red;
+    constexpr int red = NW * (WIDE == DD_SHIFTED ? 1 : NCH) * LC * 64 * 4;
+    return DdShape<NCH, LC, WIDE, NW>::STAGE_FLOATS > red ? DdShape<NCH, LC, WIDE, NW>::STAGE_FLOATS : red;
 }
 
 // Rows of a tile.  A launch of single chunks only (no pairs) cuts its tiles 8 (long chunks: 16) rows short of
@@ -1772,14 +1776,14 @@ constexpr int dd_lds_floats()
 template <int LC>
 constexpr int dd_short_rows() { return DD_ROWS - (LC > CHUNK_MAX ? 16 : 8); }
 
-template <int LC, int NCH, bool AVEC, int WIDE = DD_NARROW, bool SHORT = false>
+template <int LC, int NCH, bool AVEC, int WIDE, bool SHORT, int NW>
 __device__ __forceinline__ void dd2dia_unit(
     float *lds, int row0, const Chunk *ck1, const Chunk *ck2, float *__restrict__ C, int stride,
     const float *__restrict__ A, long long lda, const float *__restrict__ B, long long ldb,
     int h, int w, int batch, float alpha, float beta, unsigned a_bytes, unsigned b_bytes,
     unsigned c_bytes)
 {
-    typedef DdShape<NCH, LC, WIDE> S;
+    typedef DdShape<NCH, LC, WIDE, NW> S;
     constexpr bool SHIFTED = WIDE == DD_SHIFTED;
     static_assert(!SHORT || NCH == 1, "short tiles: launches of single chunks, and of shifted pairs (which say so)");
     static_assert(!SHIFTED || AVEC, "pairs are formed with 16-byte loads of A only");
@@ -2127,10 +2131,10 @@ struct DdBlock {
 };
 
 // PAIRS = false: every unit is a single chunk, 4 waves per workgroup.
-// PAIRS = true: 8 waves per workgroup; a workgroup whose unit is a single
-// chunk retires its upper four waves at once.
+// PAIRS = true: 8 waves per workgroup (a shifted pair 4), also of one whose unit is a single
+// chunk.
 template <int LC, bool AVEC, bool PAIRS, int WIDE = DD_NARROW>
-__global__ __launch_bounds__((PAIRS && WIDE != DD_SHIFTED) ? 512 : 256) void dd2dia_tiled_kernel(
+__global__ __launch_bounds__(64 * (dd_waves<PAIRS, WIDE>())) void dd2dia_tiled_kernel(
     const Chunk *__restrict__ chunks, const Unit *__restrict__ units, int nunits,
     float *__restrict__ C, int stride,
     const float *__restrict__ A, long long lda, const float *__restrict__ B, long long ldb,
@@ -2139,8 +2143,9 @@ __global__ __launch_bounds__((PAIRS && WIDE != DD_SHIFTED) ? 512 : 256) void dd2
 {
     constexpr int NCH_MAX = PAIRS ? 2 : 1;
     static_assert(PAIRS || WIDE == DD_NARROW, "only pairs come in forms");
-    constexpr int LDS_FLOATS = dd_lds_floats<LC, NCH_MAX, WIDE>() > dd_lds_floats<LC, 1>() ? dd_lds_floats<LC, NCH_MAX, WIDE>()
-                                                                                           : dd_lds_floats<LC, 1>();
+    constexpr int NW = dd_waves<PAIRS, WIDE>();
+    constexpr int LDS_PAIR = dd_lds_floats<LC, NCH_MAX, WIDE, NW>(), LDS_ONE = dd_lds_floats<LC, 1, DD_NARROW, NW>();
+    constexpr int LDS_FLOATS = LDS_PAIR > LDS_ONE ? LDS_PAIR : LDS_ONE;
     __shared__ __attribute__((aligned(16))) float lds[LDS_FLOATS];
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     // Tiles are numbered block by block: a block is DdBlock::rows(nunits) neighbouring row tiles x up to 16
@@ -2177,14 +2182,13 @@ __global__ __launch_bounds__((PAIRS && WIDE != DD_SHIFTED) ? 512 : 256) void dd2
     const int row0 = rowtile * TR;
     if constexpr (PAIRS) {
         if (c2 >= 0) {
-            dd2dia_unit<LC, 2, AVEC, WIDE>(lds, row0, chunks + c1, chunks + c2, C, stride, A, lda, B, ldb, h, w, batch,
+            dd2dia_unit<LC, 2, AVEC, WIDE, false, NW>(lds, row0, chunks + c1, chunks + c2, C, stride, A, lda, B, ldb, h, w, batch,
                                            alpha, beta, a_bytes, b_bytes, c_bytes);
             return;
         }
     }
-    if (PAIRS && threadIdx.x >= 256) return;
     if (row0 >= h) return;
-    dd2dia_unit<LC, 1, AVEC, DD_NARROW, !PAIRS || WIDE == DD_SHIFTED>(lds, row0, chunks + c1, chunks + c1, C, stride, A, lda, B, ldb, h, w, batch,
+    dd2dia_unit<LC, 1, AVEC, DD_NARROW, !PAIRS || WIDE == DD_SHIFTED, NW>(lds, row0, chunks + c1, chunks + c1, C, stride, A, lda, B, ldb, h, w, batch,
                              alpha, beta, a_bytes, b_bytes, c_bytes);
 }
 
@@ -3377,9 +3381,9 @@ hipError_t launch_dd2dia_tiled(const DiaView &C, float *vals, const float *A, lo
         if (shifted) {                                                                                   \
             launch_kernel((dd2dia_tiled_kernel<L, true, true, DD_SHIFTED>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
         } else if (wide) {                                                                               \
-            launch_kernel((dd2dia_tiled_kernel<L, true, true, DD_WIDE>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
+            launch_kernel((dd2dia_tiled_kernel<L, true, true, DD_WIDE>), grid, dim3(64 * dd_waves<true, DD_WIDE>()), 0, stream, CUVDIA_DD_ARGS);  \
         } else if (pairs) {                                                                              \
-            launch_kernel((dd2dia_tiled_kernel<L, true, true>), grid, dim3(512), 0, stream, CUVDIA_DD_ARGS);  \
+            launch_kernel((dd2dia_tiled_kernel<L, true, true>), grid, dim3(64 * dd_waves<true, DD_NARROW>()), 0, stream, CUVDIA_DD_ARGS);  \
         } else {                                                                                         \
             if (a_vec) launch_kernel((dd2dia_tiled_kernel<L, true, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);  \
             else launch_kernel((dd2dia_tiled_kernel<L, false, false>), grid, dim3(256), 0, stream, CUVDIA_DD_ARGS);       \
