@@ -11,14 +11,17 @@
 // every stage has some (4 maps of 256 x 256 to 4, batch 256: 4.0 ms).
 //
 // Per stage of 16 columns the loads of the next one are on their way to registers; the split, transposed, goes to LDS; a wave
-// works two patches of A.  No branch is taken in the products' loop: each taken branch cost about 30 clocks.
+// works two patches of A.  The products of a stage are one stretch of code without a branch, a patch's sums are added while the next
+// one's products are made.  (With a branch per patch of B to the fp32 way every sum was waited for, 4800 - 5100 clocks a stage.)
 //
-// Bound: the loads.  A stage's products take 4500 clocks of a CU, the split and its way to LDS 2300; with all CUs at work a stage
-// comes to 11000, for 80 KB in segments of 176 bytes (tiles 16 positions wide: 112 bytes, and half as long again).  Measured
-// against the kernel with a wave per window row: 4 channels of 256 x 256 maps, batch 256 981 -> 837 us (58 -> 68 TFLOP/s); 416 x 416,
-// batch 357 421 -> 322; 200 x 200, 2 maps to 2, batch 256 357 -> 228; 272 x 272 to 2, batch 388 413 -> 329.  (Parts cut off instead
-// of rounded: 825, 332, 228 and 331.)  Windows of 7 to 11 rows have fewer products for the same loads and fewer of them are
-// slots: 0.5 - 0.95 times the kernels that serve them.
+// Bound: the loads.  A stage's products take 3300 clocks of a wave that is first on its SIMD, 4500 of the other, the split and its way
+// to LDS 2500; with all CUs at work the loads have come 5000 after the products begin, 80 KB in segments of 176 bytes (tiles 16
+// positions wide: 112 bytes, and half as long again), a third of them from beyond the L2: 8400 a stage, 9300 before the branches went.
+// (The clock falls with every saving, 2.02 -> 1.92 GHz.)  Measured against the kernel with a wave per window row, in brackets with the
+// branches: 4 channels of 256 x 256 maps, batch 256 981 -> 815 us (838; 69 TFLOP/s); 416 x 416, batch 357 421 -> 314 (323); 200 x 200, 2
+// maps to 2, batch 256 357 -> 211 (228); 272 x 272 to 2, batch 388 413 -> 311 (329); 192 x 192 to 8, batch 160 266 (274).  (With the branches and
+// parts cut off instead of rounded: 825, 332, 228 and 331 on the first four.)  Windows of 7 to 11 rows have fewer products for the same
+// loads and fewer of them are slots: 0.5 - 0.95 times the kernels that serve them.
 //
 // Accumulation order: of every 16 columns the six products of all columns, smallest first, rounded as the matrix core does
 // (split.hpp); these sums in fp32, columns ascending.  Error against 64 bits (2-norm, relative; uniform operands in -1 .. 1) at
@@ -214,47 +217,73 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             for (int x = 0; x < S::BX; ++x) acc[i][y][x] = f4{0.f, 0.f, 0.f, 0.f};
 
     constexpr int TILES = (S::BY + 1) * S::BX;
-    request(std::integral_constant<int, 0>{}, std::integral_constant<int, S::LOADS>{}, 0);
-    for (int c = 0; c < batch; c += DS_COLS) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (the loads to LDS are not the compiler's)
-        barrier();                                   // nobody reads the last stage any more
-        place();
-        barrier();
-        const unsigned flag = flags[lane % DS_WAVES];
-        u4 af[2][3];
+    f4 sum[2][2];
+    auto add = [&](auto t_) __attribute__((always_inline)) {
+        constexpr int t = decltype(t_)::value, y = t / S::BX, x = t % S::BX;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            af[i][0] = *reinterpret_cast<const u4 *>(a13 + i * (DS_XT / 4) * S::PATCH);
-            af[i][1] = *reinterpret_cast<const u4 *>(a11 + i * (DS_XT / 4) * S::PATCH + S::PART);
-            af[i][2] = *reinterpret_cast<const u4 *>(a11 + i * (DS_XT / 4) * S::PATCH);
-        }
-        const bool exact = __any(flag);
-        u4 bf[2][2];
-        auto fetch = [&](auto t_) __attribute__((always_inline)) {
-            constexpr int t = decltype(t_)::value, at = (t / S::BX * S::NBX + t % S::BX) * S::PATCH;
-            if constexpr (t < TILES) {
-                bf[t % 2][0] = *reinterpret_cast<const u4 *>(b31 + at);
-                bf[t % 2][1] = *reinterpret_cast<const u4 *>(b21 + at);
+        for (int i = 0; i < 2; ++i)
+            if (y - i >= 0 && y - i < S::BY) {
+                acc[i][y - i][x] += sum[t % 2][i];
+                asm volatile("" : "+v"(acc[i][y - i][x]));       // (here, not where it is used next)
             }
-        };
-        fetch(std::integral_constant<int, 0>{});
-        // (the next stage's requests a few at a time, past the last one too: all at once they wait for each other)
-        ds_for<0, TILES>([&](auto t_) {
-            constexpr int t = decltype(t_)::value, y = t / S::BX, x = t % S::BX;
-            fetch(std::integral_constant<int, t + 1>{});
-            request(std::integral_constant<int, S::LOADS * t / TILES>{}, std::integral_constant<int, S::LOADS * (t + 1) / TILES>{}, c + DS_COLS);
-            f4 sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-            if (__builtin_expect(!exact, 1)) {
+    };
+    request(std::integral_constant<int, 0>{}, std::integral_constant<int, S::LOADS>{}, 0);
+    for (int c0 = 0; c0 < batch; c0 += 64 * DS_COLS) {
+        unsigned long long exact = 0;                // stages of these 64 that the split does not hold
+        const int c1 = min(c0 + 64 * DS_COLS, batch);
+        for (int c = c0; c < c1; c += DS_COLS) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (the loads to LDS are not the compiler's)
+            barrier();                                   // nobody reads the last stage any more
+            place();
+            barrier();
+            const unsigned flag = flags[lane % DS_WAVES];
+            u4 af[2][3], bf[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                af[i][0] = *reinterpret_cast<const u4 *>(a13 + i * (DS_XT / 4) * S::PATCH);
+                af[i][1] = *reinterpret_cast<const u4 *>(a11 + i * (DS_XT / 4) * S::PATCH + S::PART);
+                af[i][2] = *reinterpret_cast<const u4 *>(a11 + i * (DS_XT / 4) * S::PATCH);
+            }
+            auto fetch = [&](auto t_) __attribute__((always_inline)) {
+                constexpr int t = decltype(t_)::value, at = (t / S::BX * S::NBX + t % S::BX) * S::PATCH;
+                if constexpr (t < TILES) {
+                    bf[t % 2][0] = *reinterpret_cast<const u4 *>(b31 + at);
+                    bf[t % 2][1] = *reinterpret_cast<const u4 *>(b21 + at);
+                }
+            };
+            fetch(std::integral_constant<int, 0>{});
+            if (__builtin_expect(__any(flag), 0)) {
+                exact |= 1ull << ((c - c0) / DS_COLS);
+                request(std::integral_constant<int, 0>{}, std::integral_constant<int, S::LOADS>{}, c + DS_COLS);
+                continue;
+            }
+            // (the next stage's requests a few at a time, past the last one too, and by two thirds of the products: all at once they
+            // wait for each other, the last ones at the end are waited for)
+            ds_for<0, TILES>([&](auto t_) {
+                constexpr int t = decltype(t_)::value, y = t / S::BX;
+                constexpr int first = 3 * S::LOADS * t / (2 * TILES), last = 3 * S::LOADS * (t + 1) / (2 * TILES);
+                fetch(std::integral_constant<int, t + 1>{});
+                request(std::integral_constant<int, (first < S::LOADS ? first : S::LOADS)>{}, std::integral_constant<int, (last < S::LOADS ? last : S::LOADS)>{}, c + DS_COLS);
                 // the six products: a1 b3, a3 b1; a2 b2, a2 b1; a1 b2, a1 b1
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
-                        if (y - i >= 0 && y - i < S::BY) sum[i] = split_mfma(af[i][p], bf[t % 2][p > 0], sum[i]);
-            } else {
-                // An operand that the split does not hold exactly -- an infinity, a NaN, a number next to the smallest ones --:
-                // the stage in fp32, four columns at a time, from memory.
+                        if (y - i >= 0 && y - i < S::BY) sum[t % 2][i] = split_mfma(af[i][p], bf[t % 2][p > 0], p == 0 ? f4{0.f, 0.f, 0.f, 0.f} : sum[t % 2][i]);
+                if constexpr (t > 0) add(std::integral_constant<int, t - 1>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            add(std::integral_constant<int, TILES - 1>{});
+        }
+        // An operand that the split does not hold exactly -- an infinity, a NaN, a number next to the smallest ones --: its stage
+        // in fp32, four columns at a time, from memory.  (Behind the loop: a second way through it cost its registers' places.)
+        while (exact) {
+            const int c = c0 + DS_COLS * __builtin_ctzll(exact);
+            exact &= exact - 1;
+            ds_for<0, TILES>([&](auto t_) {
+                constexpr int t = decltype(t_)::value, y = t / S::BX, x = t % S::BX;
                 const int l = here(lane), row_a = i_tile + l % 16 / 4 * period + 4 * wave + l % 4, row_b = row_a + s_g + 4 * y * period + 4 * x;
+                sum[t % 2][0] = sum[t % 2][1] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma nounroll
                 for (int k = c; k < min(c + DS_COLS, batch); k += 4) {
                     const int col = k + l / 16;
@@ -262,17 +291,12 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
                         const float a_col = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ar, col < batch ? (unsigned)(row_a + 4 * i * period) * 4u + (unsigned)col * lda4 : OOB_OFFSET, 0, 0));
-                        sum[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_col, b_col, sum[i], 0, 0, 0);
+                        sum[t % 2][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_col, b_col, sum[t % 2][i], 0, 0, 0);
                     }
                 }
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                if (y - i >= 0 && y - i < S::BY) {
-                    acc[i][y - i][x] += sum[i];
-                    asm volatile("" : "+v"(acc[i][y - i][x]));       // (here, not where it is used next)
-                }
-        });
+                add(t_);
+            });
+        }
     }
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // (what was requested past the last stage)
