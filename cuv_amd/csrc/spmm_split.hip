@@ -15,9 +15,9 @@
 // registers, its work interleaved by hand (720 - 770 us on the first case below), the values and not the rows in two buffers (780).
 //
 // Bound: that chain, 7500 - 8500 clocks a step where the products take 1600 (rows of bfloat16 numbers) or 3200 of a SIMD's.
-// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256, binary rows 815 -> 692 us, uniform ones
-// 752 (six products of parts instead of three); 200 x 200, 2 maps to 4, batch 256 556 -> 415 and 450; 448 x 448, 2 maps to 3,
-// batch 64 560 -> 370 and 425.  (Parts cut off instead of rounded: 689, 407 and 367 with binary rows.)
+// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256, binary rows 815 -> 686 us, uniform ones
+// 752 (six products of parts instead of three); 200 x 200, 2 maps to 4, batch 256 556 -> 397 and 450; 448 x 448, 2 maps to 3,
+// batch 64 560 -> 365 and 425.  (Parts cut off instead of rounded: 689, 407 and 367 with binary rows.)
 // Windows of 11 rows use 47 % of a patch's products: level with the fp32 kernel.
 //
 // Accumulation order: of every 32 dense rows (16 of two map rows) the products of parts, smallest first, rounded as the matrix
@@ -537,26 +537,28 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
             u2 xq[3];
             PsPair ap, aq, xp;
             __builtin_amdgcn_sched_barrier(0);
-            auto product = [&](auto i_, auto pa_, auto pb_) __attribute__((always_inline)) {
+            auto product = [&](auto i_, auto pa_, auto pb_, auto first_) __attribute__((always_inline)) {
                 constexpr int r = decltype(i_)::value / 2 % 2, n = decltype(i_)::value % 2, pa = decltype(pa_)::value, pb = decltype(pb_)::value;
-                t[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(split_b8, af[pass][r][pa]), __builtin_bit_cast(split_b8, xf[n][r][pb]), t[n], 0, 0, 0);
+                t[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(split_b8, af[pass][r][pa]), __builtin_bit_cast(split_b8, xf[n][r][pb]), decltype(first_)::value ? f16{} : t[n], 0, 0, 0);
             };
-#pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-                for (int k = 0; k < 16; ++k) t[n][k] = 0.f;
-            // (dense rows of bfloat16 numbers, as a layer's binary units are, have no other parts to multiply)
+            // (dense rows of bfloat16 numbers, as a layer's binary units are, have no other parts to multiply; the first two products
+            // of the others are in either way, so that no zeros are written for them to add to)
+            constexpr std::integral_constant<int, 2> last_part{};
             if (x_more) {
                 constexpr int PA[3] = {0, 1, 0}, PB[3] = {2, 1, 1};
                 ps_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
                     constexpr int p = decltype(i_)::value / 4;
-                    product(i_, std::integral_constant<int, PA[p]>{}, std::integral_constant<int, PB[p]>{});
+                    product(i_, std::integral_constant<int, PA[p]>{}, std::integral_constant<int, PB[p]>{}, std::bool_constant<(decltype(i_)::value < 2)>{});
                     __builtin_amdgcn_sched_barrier(0);
                 });
+                ps_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::false_type{}); });
+            } else {
+                ps_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::true_type{}); });
             }
+            __builtin_amdgcn_sched_barrier(0);
             ps_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
                 constexpr int i = decltype(i_)::value;
-                product(i_, std::integral_constant<int, 2 - i / 4>{}, std::integral_constant<int, 0>{});
+                if constexpr (i >= 2) product(i_, std::integral_constant<int, 2 - i / 4>{}, std::integral_constant<int, 0>{}, std::false_type{});
                 // beside the products: in the first pass two pairs of the second pair's values per 3; a pair of the next dense rows per 3
                 if constexpr (pass == 0) {
                     constexpr int j = 2 * (i / 3), ar = j / 4, aj = j % 4;
