@@ -15,9 +15,9 @@
 // registers, its work interleaved by hand (720 - 770 us on the first case below), the values and not the rows in two buffers (780).
 //
 // Bound: that chain, 7500 - 8500 clocks a step where the products take 1600 (rows of bfloat16 numbers) or 3200 of a SIMD's.
-// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256, binary rows 815 -> 686 us, uniform ones
-// 752 (six products of parts instead of three); 200 x 200, 2 maps to 4, batch 256 556 -> 397 and 450; 448 x 448, 2 maps to 3,
-// batch 64 560 -> 365 and 425.  (Parts cut off instead of rounded: 689, 407 and 367 with binary rows.)
+// Measured against the kernels that served it: 4 channels of 256 x 256 maps, batch 256, binary rows 815 -> 667 us, uniform ones
+// 752 (six products of parts instead of three); 200 x 200, 2 maps to 4, batch 256 556 -> 385 and 450; 448 x 448, 2 maps to 3,
+// batch 64 560 -> 358 and 425.  (Parts cut off instead of rounded: 689, 407 and 367 with binary rows.)
 // Windows of 11 rows use 47 % of a patch's products: level with the fp32 kernel.
 //
 // Accumulation order: of every 32 dense rows (16 of two map rows) the products of parts, smallest first, rounded as the matrix
@@ -505,8 +505,8 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 values_at(std::integral_constant<int, 0>{}, r, u);
                 ps_for<0, 4>([&](auto j_) __attribute__((always_inline)) { values_of(j_, v[4 * r + decltype(j_)::value]); });
             });
-#pragma unroll
-            for (int s = 2; s >= 0; --s)
+            auto rows_of = [&](auto s_) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_)::value;
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -516,6 +516,12 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                         xf[n][r][s] = u4{q0[0], q0[1], q1[0], q1[1]};
                         __builtin_amdgcn_sched_barrier(0);       // (both quads by one instruction)
                     }
+            };
+            if (x_more) {                            // (read in any case: 686 us for 667 on the large layer's binary rows)
+                rows_of(std::integral_constant<int, 2>{});
+                rows_of(std::integral_constant<int, 1>{});
+            }
+            rows_of(std::integral_constant<int, 0>{});
             ps_for<0, 8>([&](auto j_) __attribute__((always_inline)) {
                 constexpr int j = decltype(j_)::value;
                 unsigned p0, p1, p2;
