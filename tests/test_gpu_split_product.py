@@ -44,6 +44,20 @@ def test_sizes(oracle, px, py, maps_in, maps_out, batch, binary, trans):
         assert _split_ran() and ran == _lib.PATH_PLANE
 
 
+@pytest.mark.parametrize("trans,maps_in,maps_out", [("n", 1, 1), ("t", 3, 2)])
+@pytest.mark.parametrize("every,columns", [(5, slice(0, 1)), (7, slice(40, 70)), (40, slice(3, 70, 16))])
+def test_bfloat16_rows_among_others(oracle, trans, maps_in, maps_out, every, columns):
+    """Second and third parts are read and multiplied only in steps where some dense row has them: some map rows of some columns
+    do, from step to step, from wave to wave, from map to map."""
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    rng, A, B, _ = _case(oracle, 36, 40, maps_in, maps_out, 70, trans, binary=True)
+    other = np.flatnonzero(np.arange(B.shape[0]) // 36 % every == 1)
+    B[other, columns] = rng.uniform(-1, 1, B[other, columns].shape).astype(np.float32)
+    gu.check_prod(oracle, A, B, None, trans, 1.0, 0.0, _lib.PATH_PLANE, "every %d" % every)
+    assert _split_ran()
+
+
 @pytest.mark.parametrize("where", ["rows", "values", "both"])
 def test_values_that_no_three_parts_hold(oracle, where):
     """Infinities and NaN reach the elements that have them in their sums and no others; small numbers keep all their bits."""
