@@ -178,5 +178,16 @@ __device__ __forceinline__ void fma8_dpp(float (&acc)[8], float a, const float *
 
 constexpr unsigned OOB_OFFSET = 0x80000000u;     // >= every resource size used here
 
+// Four floats as one 16-byte buffer store at a vector offset and a scalar one.  Such a store reads its registers up to two issue
+// slots late, and the compiler waits for that only where there is no scalar offset: the last lanes once stored the address that the
+// next instruction had written there.  The wait names the registers, so they are not written before it.
+template <int CPOL>
+__device__ __forceinline__ void buffer_store4(float __attribute__((ext_vector_type(4))) v, __amdgpu_buffer_rsrc_t rsrc, unsigned voff, unsigned soff)
+{
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rsrc, voff, soff, CPOL);
+    asm volatile("s_nop 1" :: "v"(v));
+}
+
 }  // namespace
 }  // namespace cuvdia

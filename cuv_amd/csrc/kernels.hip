@@ -1525,7 +1525,6 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
     constexpr int LPC = ROWS / 4, CPI = 64 / LPC, CPW = SP_COLS / WAVES, NST = CPW / CPI, OPITCH = ROWS + 4;
     static_assert(SP_COLS * OPITCH <= S::XFLOATS, "the transposition fits the dense rows' part of a buffer");
     typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-    typedef unsigned sp_u4 __attribute__((ext_vector_type(4)));
     // What a lane contributes to the addresses of a tile's final store, kept for the whole walk: where it writes
     // its sums in the transposition block and reads its 4 rows back (floats), and the byte offset of those rows in
     // the destination's column tile (the out-of-range marker for a column past the batch: the buffer store then
@@ -1613,7 +1612,7 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
             }
 #pragma unroll
             for (int q = 0; q < NST; ++q)       // non-temporal, like every result of the library
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(sp_u4, v[q]), yr, y_lane[q], tile_off, 2);
+                buffer_store4<2>(v[q], yr, y_lane[q], tile_off);
             __syncthreads();
         }
 #pragma unroll

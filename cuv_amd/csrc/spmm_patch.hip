@@ -34,7 +34,6 @@ namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef unsigned u4 __attribute__((ext_vector_type(4)));
 
 constexpr int PT_WAVES = 8, PT_THREADS = 64 * PT_WAVES, PT_COLS = 32;
 
@@ -331,7 +330,7 @@ __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled
             if (EP) s[j] = sp_finish(s[j], bias[j], ep.act);
         }
         constexpr int NT = 2;                        // streamed past the caches, as stream_store does (through them: 9.9 us for 9.1)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, s), ybuf, whole && column(k) ? place(k) : OOB_OFFSET, 4u * (unsigned)row0, NT);
+        buffer_store4<NT>(s, ybuf, whole && column(k) ? place(k) : OOB_OFFSET, 4u * (unsigned)row0);
         if (part) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -339,9 +338,6 @@ __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(e), ybuf, column(k) && element(j) ? place(k) + 4u * j : OOB_OFFSET, 4u * (unsigned)row0, NT);
             }
         }
-        // (16 bytes with a scalar offset leave their registers a clock late, and the compiler does not know: the last lanes stored the
-        // address that the next instruction wrote there)
-        asm volatile("s_nop 1" :: "v"(s));
     }
 }
 

@@ -46,7 +46,6 @@ namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef unsigned plane_u4 __attribute__((ext_vector_type(4)));
 
 // A workgroup's tile: 32 rows x 64 columns, 8 rows per wave.  Up to four workgroups share a CU, each with barriers of its
 // own: while one waits for its block the others multiply.
@@ -303,7 +302,7 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                 if (EP) s[i] = sp_finish(s[i], bias[i], ep.act);
             }
             if (skip == 0) {
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(plane_u4, s), yrsrc, place(my_col + 8 * k, my_row), tile_at, 0);
+                buffer_store4<0>(s, yrsrc, place(my_col + 8 * k, my_row), tile_at);
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)

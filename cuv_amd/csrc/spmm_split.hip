@@ -353,7 +353,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
         }
         if (skip == 0) {
 #pragma unroll
-            for (int it = 0; it < S::OIT; ++it) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, s[it]), yrsrc, at[it], first + it / PER_ROW * step, 0);
+            for (int it = 0; it < S::OIT; ++it) buffer_store4<0>(s[it], yrsrc, at[it], first + it / PER_ROW * step);
         } else {
 #pragma unroll
             for (int it = 0; it < S::OIT; ++it)

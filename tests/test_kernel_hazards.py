@@ -1,0 +1,103 @@
+"""Waits that the hardware needs and the compiler does not know of, in the sources and in the built library, without a GPU."""
+import glob
+import os
+import re
+import subprocess
+
+import pytest
+
+import _kernel_resources
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cuv_amd", "csrc")
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+WAIT = 2                                 # issue slots between the one instruction and the other
+
+
+def _sources():
+    for path in sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.hpp"))):
+        with open(path) as f:
+            yield os.path.basename(path), re.sub(r"//[^\n]*", "", f.read())
+
+
+def _arguments(text, at):
+    """The arguments of the call whose bracket opens at text[at]."""
+    depth, args, start = 0, [], at + 1
+    for i in range(at, len(text)):
+        if text[i] in "([{":
+            depth += 1
+        elif text[i] in ")]}":
+            depth -= 1
+        if depth == 1 and text[i] == "," or depth == 0:
+            args.append(text[start:i].strip())
+            start = i + 1
+        if depth == 0:
+            return args
+
+
+def test_wide_stores_with_a_scalar_offset_have_their_wait():
+    """A buffer store of more than 8 bytes with a scalar offset reads its registers late: only buffer_store4 makes one, with a wait."""
+    bare, waiting = [], 0
+    for name, text in _sources():
+        for m in re.finditer(r"raw_buffer_store_b(?:96|128)\(", text):
+            offset = _arguments(text, m.end() - 1)[3]
+            waits = re.match(r'[^;]*;\s*asm volatile\("s_nop 1" :: "v"\(v\)\);', text[m.end():]) is not None
+            waiting += waits
+            if offset != "0" and not waits:
+                bare.append((name, offset))
+    assert bare == [] and waiting == 1
+
+
+_VECTOR = re.compile(r"v\[(\d+):(\d+)\]$|v(\d+)$")
+
+
+def _registers(operand):
+    m = _VECTOR.match(operand.split()[0]) if operand else None
+    if m is None:
+        return set()
+    return set(range(int(m[1]), int(m[2]) + 1)) if m[1] else {int(m[3])}
+
+
+def _instructions(path):
+    """(operation, operands) of every kernel, in the order of their addresses."""
+    text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", path], capture_output=True, text=True, check=True).stdout
+    for line in text.splitlines():
+        if line.startswith("\t"):
+            operation, _, operands = line.partition("//")[0].strip().partition(" ")
+            if operation:
+                yield operation, [o.strip() for o in operands.split(",")]
+
+
+def _slots(operation, operands):
+    return int(operands[0]) + 1 if operation == "s_nop" else 1
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no disassembler")
+    at = tmp_path_factory.mktemp("code")
+    with open(_kernel_resources.LIBRARY, "rb") as f:
+        data = f.read()
+    found = []
+    for i, elf in enumerate(_kernel_resources._code_objects(data)):
+        path = at / ("%d.elf" % i)
+        path.write_bytes(elf)
+        found.append(list(_instructions(str(path))))
+    assert found
+    return found
+
+
+def test_no_register_of_a_wide_store_is_written_early(library):
+    stores = 0
+    for code in library:
+        for i, (operation, operands) in enumerate(code):
+            if re.match(r"buffer_store_dwordx[34]", operation) is None or not operands[3].startswith("s"):
+                continue
+            stores += 1
+            data, passed = _registers(operands[0]), 0
+            for after, written in code[i + 1:i + 1 + WAIT]:
+                if passed >= WAIT:
+                    break
+                assert not (after.startswith("v_") and _registers(written[0]) & data), (operation, operands, after, written)
+                passed += _slots(after, written)
+    assert stores > 0
