@@ -166,15 +166,29 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-// acc[r] += a(lane 16 n + LANE0 + r) * x[r]: the value broadcast inside each row of 16 lanes
-template <int LANE0>
+// acc[r] += a(lane 16 n + r) * x[r], r = 0..7: the values broadcast inside each row of 16 lanes; fma16_dpp after that
+// += a(lane 16 n + 8 + r) * x[1 + r].  A DPP operand must not have been written by a VALU instruction in the two preceding
+// issue slots, and the compiler does not look into a statement: hence the wait at its head.
+#define CUVDIA_FMA_DPP(r, x, lane) "v_fmac_f32_dpp %" #r ", %8, %" #x " row_newbcast:" #lane " row_mask:0xf bank_mask:0xf\n\t"
+#define CUVDIA_FMA8_DPP                                                                                     \
+    CUVDIA_FMA_DPP(0, 9, 0) CUVDIA_FMA_DPP(1, 10, 1) CUVDIA_FMA_DPP(2, 11, 2) CUVDIA_FMA_DPP(3, 12, 3)      \
+    CUVDIA_FMA_DPP(4, 13, 4) CUVDIA_FMA_DPP(5, 14, 5) CUVDIA_FMA_DPP(6, 15, 6) CUVDIA_FMA_DPP(7, 16, 7)
 __device__ __forceinline__ void fma8_dpp(float (&acc)[8], float a, const float *x)
 {
-#define CUVDIA_FMA(r)                                                                                       \
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc[r]) : "v"(a), "v"(x[r]), "n"(LANE0 + r));
-    CUVDIA_FMA(0) CUVDIA_FMA(1) CUVDIA_FMA(2) CUVDIA_FMA(3) CUVDIA_FMA(4) CUVDIA_FMA(5) CUVDIA_FMA(6) CUVDIA_FMA(7)
-#undef CUVDIA_FMA
+    asm("s_nop 1\n\t" CUVDIA_FMA8_DPP
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]), "+&v"(acc[6]), "+&v"(acc[7])
+        : "v"(a), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]));
 }
+__device__ __forceinline__ void fma16_dpp(float (&acc)[8], float a, const float *x)
+{
+    asm("s_nop 1\n\t" CUVDIA_FMA8_DPP
+        CUVDIA_FMA_DPP(0, 10, 8) CUVDIA_FMA_DPP(1, 11, 9) CUVDIA_FMA_DPP(2, 12, 10) CUVDIA_FMA_DPP(3, 13, 11)
+        CUVDIA_FMA_DPP(4, 14, 12) CUVDIA_FMA_DPP(5, 15, 13) CUVDIA_FMA_DPP(6, 16, 14) CUVDIA_FMA_DPP(7, 17, 15)
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5]), "+&v"(acc[6]), "+&v"(acc[7])
+        : "v"(a), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]));
+}
+#undef CUVDIA_FMA8_DPP
+#undef CUVDIA_FMA_DPP
 
 constexpr unsigned OOB_OFFSET = 0x80000000u;     // >= every resource size used here
 

@@ -5,7 +5,7 @@
 // 4 + K - 1 map rows around them and the K * K diagonals' values.  The kernel that takes 64 rows in a line (spmm_tiled_kernel in
 // kernels.hip, of which this is the form for such tables) stages 76 rows x 64 columns anew for every window row, 7 steps with a
 // barrier each where this one has 4, and 2.3 times the bytes.  A half of a wave owns a group of 8 positions, a lane a column:
-// its window is read by 16 bytes, the values are broadcast by DPP in every 16 lanes (fma8_dpp).
+// its window is read by 16 bytes, the values are broadcast by DPP in every 16 lanes (fma16_dpp).
 //
 // Bound: on one round of workgroups (the 16384-unit layer at batch 128: 512) everything happens at once on all CUs -- 1400
 // clocks until the first request, 4700 for the requests (a load that writes LDS costs 2.3 clocks per 128-byte line that it
@@ -278,8 +278,8 @@ __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled
                 float w[4 * S::XW];
 #pragma unroll
                 for (int i = 0; i < 4 * S::XW; ++i) w[i] = x[d % 2][i / 4][i % 4];
-                fma8_dpp<0>(acc, a[d % 2][q], w + 2 * q);
-                if constexpr (2 * q + 1 < LC) fma8_dpp<8>(acc, a[d % 2][q], w + 2 * q + 1);
+                if constexpr (2 * q + 1 < LC) fma16_dpp(acc, a[d % 2][q], w + 2 * q);
+                else fma8_dpp(acc, a[d % 2][q], w + 2 * q);
                 // between the first pair's products the requests, all of them before the first wait
                 constexpr int at = d * S::NQ + q, slots = 2 * S::NQ - 1, items = 3 * (S::PAIRS - 1);
                 if constexpr (at < slots)

@@ -223,8 +223,8 @@ __global__ __launch_bounds__(64 * PLANE_WAVES, (PlaneShape<LC, K>::per_cu(EP))) 
                 static_for<0, S::NQ>([&](auto q_) {
                     constexpr int q = decltype(q_)::value;
                     const float v = st[S::X_FLOATS + lane_t + 2 * q * S::AROW];
-                    fma8_dpp<0>(tail, v, x + 2 * q);
-                    if constexpr (2 * q + 1 < LC) fma8_dpp<8>(tail, v, x + 2 * q + 1);
+                    if constexpr (2 * q + 1 < LC) fma16_dpp(tail, v, x + 2 * q);
+                    else fma8_dpp(tail, v, x + 2 * q);
                 });
             }
         }

@@ -47,6 +47,22 @@ def test_wide_stores_with_a_scalar_offset_have_their_wait():
     assert bare == [] and waiting == 1
 
 
+def test_dpp_statements_begin_with_their_wait():
+    """An operand that DPP reads across lanes must not have been written in the two preceding issue slots: a statement that the
+    compiler cannot look into waits first."""
+    bare, waiting = [], 0
+    for name, text in _sources():
+        macros = {m for m, body in re.findall(r"#define (\w+)(?:\([^)]*\))?((?:[^\n]*\\\n)*[^\n]*)", text) if "dpp" in body.lower()}
+        for m in re.finditer(r"\basm(?: volatile)?\(", text):
+            code = _arguments(text, m.end() - 1)[0]
+            if "_dpp" in code or any(re.search(r"\b%s\b" % macro, code) for macro in macros):
+                if re.match(r'"s_nop 1\\n\\t"', code):
+                    waiting += 1
+                else:
+                    bare.append((name, code[:80]))
+    assert bare == [] and waiting > 0
+
+
 _VECTOR = re.compile(r"v\[(\d+):(\d+)\]$|v(\d+)$")
 
 
@@ -101,3 +117,20 @@ def test_no_register_of_a_wide_store_is_written_early(library):
                 assert not (after.startswith("v_") and _registers(written[0]) & data), (operation, operands, after, written)
                 passed += _slots(after, written)
     assert stores > 0
+
+
+def test_no_operand_of_dpp_is_written_late(library):
+    broadcasts = 0
+    for code in library:
+        for i, (operation, operands) in enumerate(code):
+            if not operation.endswith("_dpp"):
+                continue
+            broadcasts += 1
+            source, passed = _registers(operands[1]), 0
+            for before, written in reversed(code[max(0, i - WAIT):i]):
+                if passed >= WAIT:
+                    break
+                passed += _slots(before, written) if before == "s_nop" else 0
+                assert passed >= WAIT or not (before.startswith("v_") and _registers(written[0]) & source), (operation, operands, before, written)
+                passed += before != "s_nop"
+    assert broadcasts > 0
