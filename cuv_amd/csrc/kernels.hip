@@ -35,9 +35,10 @@
 #include "device.hpp"
 #include "kernels.hpp"
 
-// This file is compiled seven times (CUVDIA_PART = 1 .. 7, see the Makefile), each translation unit
+// This file is compiled ten times (CUVDIA_PART = 1 .. 10, see the Makefile), each translation unit
 // instantiating one share of the kernel templates, so that the shares compile in parallel: parts 1 - 3 hold
-// the tiled SpMM kernels by longest chunk (1 - 5, 6 - 9, 10 - 13), part 5 the walking SpMM kernels, part 6
+// the tiled SpMM kernels by longest chunk (1 - 5, 6 - 9, 10 - 13), parts 8 - 10 those of tables with shorter chunks as
+// well, which want other switches, part 5 the walking SpMM kernels, part 6
 // the window-table projection for window rows of at most 8 diagonals, part 7 the one for rows of 9 to 13, part 4
 // everything else.  Without the macro one unit holds everything.
 #ifndef CUVDIA_PART
@@ -2897,6 +2898,9 @@ hipError_t dd2dia_window_long_launch(const DwLaunch &L);      // (rows of 9 to 1
 hipError_t spmm_tiled_launch_1_5(const SpLaunch &L);
 hipError_t spmm_tiled_launch_6_9(const SpLaunch &L);
 hipError_t spmm_tiled_launch_10_13(const SpLaunch &L);
+hipError_t spmm_mixed_launch_2_5(const SpLaunch &L);
+hipError_t spmm_mixed_launch_6_9(const SpLaunch &L);
+hipError_t spmm_mixed_launch_10_13(const SpLaunch &L);
 
 // 8 rows per wave (8 waves per workgroup) keeps four waves on every SIMD
 // at the sizes this path is measured on.
@@ -2904,23 +2908,28 @@ hipError_t spmm_tiled_launch_10_13(const SpLaunch &L);
                          L.batch, L.alpha, L.beta, L.col_tiles, L.col_group, L.a_bytes, L.s_min, L.s_max, L.period_tiles, L.slot_step, L.ep
 #define CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, EP, MIXED)                                                                    \
     launch_kernel((spmm_tiled_kernel<K, 8, NTAB, EP, MIXED>), L.grid, dim3(512), 0, L.stream, CUVDIA_SPMM_ARGS)
-#define CUVDIA_SPMM_LAUNCH_TAB(K, NTAB)                                                                               \
+#define CUVDIA_SPMM_LAUNCH_TAB(K, NTAB, MIXED)                                                                        \
     do {                                                                                                              \
-        if (K > 1 && L.mixed) {                                                                                       \
-            if (fused) CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, true, (K > 1));                                                \
-            else CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, false, (K > 1));                                                     \
-        } else {                                                                                                      \
-            if (fused) CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, true, false);                                                  \
-            else CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, false, false);                                                       \
-        }                                                                                                             \
+        if (fused) CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, true, MIXED);                                                      \
+        else CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, false, MIXED);                                                           \
     } while (0)
-#define CUVDIA_SPMM_LAUNCH(K)                                                                                         \
+#define CUVDIA_SPMM_LAUNCH(K, MIXED)                                                                                  \
     case K:                                                                                                           \
-        note_kernel("spmm_tiled_kernel<%d, 8, %d, %s, %s>", K, L.nchunks <= 64 ? 1 : 4, fused ? "true" : "false",     \
-                    (K > 1 && L.mixed) ? "true" : "false");                                                           \
-        if (L.nchunks <= 64) CUVDIA_SPMM_LAUNCH_TAB(K, 1);                                                            \
-        else CUVDIA_SPMM_LAUNCH_TAB(K, 4);                                                                            \
+        note_kernel("spmm_tiled_kernel<%d, 8, %d, %s, " #MIXED ">", K, L.nchunks <= 64 ? 1 : 4, fused ? "true" : "false"); \
+        if (L.nchunks <= 64) CUVDIA_SPMM_LAUNCH_TAB(K, 1, MIXED);                                                     \
+        else CUVDIA_SPMM_LAUNCH_TAB(K, 4, MIXED);                                                                     \
         break;
+// A unit's launch: the kernels of these longest chunks
+#define CUVDIA_SPMM_UNIT(NAME, CASES)                                                                                 \
+    hipError_t NAME(const SpLaunch &L)                                                                                \
+    {                                                                                                                 \
+        const bool fused = L.ep.bias != nullptr || L.ep.act != 0;                                                     \
+        switch (L.lck) {                                                                                              \
+            CASES                                                                                                     \
+            default: return hipErrorInvalidValue;                                                                     \
+        }                                                                                                             \
+        return hipGetLastError();                                                                                     \
+    }
 #if CUVDIA_IN_PART(5)
 // rows per wave of the instantiation that serves a window of k rows of lck diagonals whose first shift is
 // s0 (0: none).  Instantiated: the centred 3x3, 5x5 and 7x7 windows.  (A 13x13 window needs 13 sets of running
@@ -3051,38 +3060,24 @@ hipError_t dd2dia_window_long_launch(const DwLaunch &L)
 }
 #endif
 #if CUVDIA_IN_PART(1)
-hipError_t spmm_tiled_launch_1_5(const SpLaunch &L)
-{
-    const bool fused = L.ep.bias != nullptr || L.ep.act != 0;
-    switch (L.lck) {
-        CUVDIA_SPMM_LAUNCH(1) CUVDIA_SPMM_LAUNCH(2) CUVDIA_SPMM_LAUNCH(3) CUVDIA_SPMM_LAUNCH(4) CUVDIA_SPMM_LAUNCH(5)
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_1_5, CUVDIA_SPMM_LAUNCH(1, false) CUVDIA_SPMM_LAUNCH(2, false) CUVDIA_SPMM_LAUNCH(3, false) CUVDIA_SPMM_LAUNCH(4, false) CUVDIA_SPMM_LAUNCH(5, false))
 #endif
 #if CUVDIA_IN_PART(2)
-hipError_t spmm_tiled_launch_6_9(const SpLaunch &L)
-{
-    const bool fused = L.ep.bias != nullptr || L.ep.act != 0;
-    switch (L.lck) {
-        CUVDIA_SPMM_LAUNCH(6) CUVDIA_SPMM_LAUNCH(7) CUVDIA_SPMM_LAUNCH(8) CUVDIA_SPMM_LAUNCH(9)
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_6_9, CUVDIA_SPMM_LAUNCH(6, false) CUVDIA_SPMM_LAUNCH(7, false) CUVDIA_SPMM_LAUNCH(8, false) CUVDIA_SPMM_LAUNCH(9, false))
 #endif
 #if CUVDIA_IN_PART(3)
-hipError_t spmm_tiled_launch_10_13(const SpLaunch &L)
-{
-    const bool fused = L.ep.bias != nullptr || L.ep.act != 0;
-    switch (L.lck) {
-        CUVDIA_SPMM_LAUNCH(10) CUVDIA_SPMM_LAUNCH(11) CUVDIA_SPMM_LAUNCH(12) CUVDIA_SPMM_LAUNCH(13)
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_10_13, CUVDIA_SPMM_LAUNCH(10, false) CUVDIA_SPMM_LAUNCH(11, false) CUVDIA_SPMM_LAUNCH(12, false) CUVDIA_SPMM_LAUNCH(13, false))
 #endif
+#if CUVDIA_IN_PART(8)
+CUVDIA_SPMM_UNIT(spmm_mixed_launch_2_5, CUVDIA_SPMM_LAUNCH(2, true) CUVDIA_SPMM_LAUNCH(3, true) CUVDIA_SPMM_LAUNCH(4, true) CUVDIA_SPMM_LAUNCH(5, true))
+#endif
+#if CUVDIA_IN_PART(9)
+CUVDIA_SPMM_UNIT(spmm_mixed_launch_6_9, CUVDIA_SPMM_LAUNCH(6, true) CUVDIA_SPMM_LAUNCH(7, true) CUVDIA_SPMM_LAUNCH(8, true) CUVDIA_SPMM_LAUNCH(9, true))
+#endif
+#if CUVDIA_IN_PART(10)
+CUVDIA_SPMM_UNIT(spmm_mixed_launch_10_13, CUVDIA_SPMM_LAUNCH(10, true) CUVDIA_SPMM_LAUNCH(11, true) CUVDIA_SPMM_LAUNCH(12, true) CUVDIA_SPMM_LAUNCH(13, true))
+#endif
+#undef CUVDIA_SPMM_UNIT
 #undef CUVDIA_SPMM_LAUNCH
 #undef CUVDIA_SPMM_LAUNCH_TAB
 #undef CUVDIA_SPMM_LAUNCH_ONE
@@ -3146,9 +3141,10 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
                      trans ? A.slot_step_t : A.slot_step_n, ep,
                      dim3((unsigned)(row_tiles * col_tiles)), stream, lck,
                      (trans ? A.min_len_t : A.min_len_n) != lck};
-    if (lck <= 5) return spmm_tiled_launch_1_5(L);
-    if (lck <= 9) return spmm_tiled_launch_6_9(L);
-    return spmm_tiled_launch_10_13(L);
+    const bool mixed = L.mixed && lck > 1;
+    if (lck <= 5) return mixed ? spmm_mixed_launch_2_5(L) : spmm_tiled_launch_1_5(L);
+    if (lck <= 9) return mixed ? spmm_mixed_launch_6_9(L) : spmm_tiled_launch_6_9(L);
+    return mixed ? spmm_mixed_launch_10_13(L) : spmm_tiled_launch_10_13(L);
 }
 
 hipError_t launch_dd2dia_generic(const DiaView &C, float *vals, const float *A, long long lda,

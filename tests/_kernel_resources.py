@@ -44,3 +44,25 @@ def kernels(library=LIBRARY):
     with open(library, "rb") as f:
         data = f.read()
     return {k[".name"]: k for elf in _code_objects(data) for note in _notes(elf) for k in note["amdhsa.kernels"]}
+
+
+def preloaded(library=LIBRARY):
+    """{mangled name: dwords of its arguments that come in registers}: bytes 58 and 59 of the descriptor `name`.kd, their low 7 bits"""
+    with open(library, "rb") as f:
+        data = f.read()
+    out = {}
+    for elf in _code_objects(data):
+        table, = struct.unpack_from("<Q", elf, 40)
+        size, count = struct.unpack_from("<HH", elf, 58)
+        sections = [struct.unpack_from("<IIQQQQIIQQ", elf, table + i * size) for i in range(count)]
+        for _, kind, _, _, offset, length, strings, _, _, entry in sections:
+            if kind != 11:                               # SHT_DYNSYM
+                continue
+            for at in range(offset, offset + length, entry):
+                name, _, _, section, value, _ = struct.unpack_from("<IBBHQQ", elf, at)
+                start = sections[strings][4] + name
+                symbol = elf[start:elf.index(b"\0", start)].decode()
+                if symbol.endswith(".kd"):
+                    _, _, _, address, place, _, _, _, _, _ = sections[section]
+                    out[symbol[:-3]] = struct.unpack_from("<H", elf, place + value - address + 58)[0] & 127
+    return out

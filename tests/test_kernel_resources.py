@@ -44,3 +44,14 @@ def test_rows_along_the_lanes_need_no_memory_of_their_own():
     found = {n: m for n, m in _kernel_resources.kernels().items() if "spmm_thin_kernel" in n}
     assert len(found) == 13 * 6
     assert [n for n, m in found.items() if m[".private_segment_fixed_size"]] == []
+
+
+def test_arguments_in_registers_only_where_they_are_ahead():
+    """The products tile by tile, as patches too, and the gradient chunk by chunk; not those that save scalar registers in vector ones
+    for it: the tables with shorter chunks as well, rows along the lanes."""
+    found = _kernel_resources.preloaded()
+    assert found.keys() == _kernel_resources.kernels().keys()
+    ahead = {n for n in found if ("spmm_tiled_kernel" in n and "ELb1EEEvPKNS_5Chunk" not in n) or "dd2dia_tiled_kernel" in n}
+    assert len(ahead) > 80 and [n for n in ahead if found[n] == 0] == []
+    apart = {n for n in found if n not in ahead and any(k in n for k in ("spmm_", "dd2dia_")) and "generic" not in n}
+    assert len(apart) > 200 and [n for n in apart if found[n] != 0] == []
