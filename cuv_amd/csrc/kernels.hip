@@ -3121,7 +3121,7 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
         if (force && !split && !walks) return hipErrorNotSupported;
         // A smaller one: patch by patch, or with rows along the lanes.
         const bool thin = !split && !walks && spmm_thin_by_size(A, trans, batch);
-        if (split || walks || spmm_patch_plan(wk, n_out, batch, thin)) {
+        if (split || walks || spmm_patch_plan(wk, n_out, n_in, batch, beta, ep, thin)) {
             PlaneLaunch &P = split ? other : plane;
             if (ran && (split || walks)) *ran = CUVDIA_PATH_PLANE;
             P.tab = wk.tab_dev; P.ngroups = wk.ngroups; P.period = wk.period; P.s0 = wk.s0; P.astep4 = wk.astep4; P.k = wk.k;

@@ -156,7 +156,7 @@ bool spmm_split_plan(const WalkView &wk, long long n_out, int batch, bool force,
 hipError_t spmm_split_launch(const PlaneLaunch &L);
 // The same, tile by tile, a tile being a patch of the window's plane (spmm_patch.hip): windows of 3 x 3, 5 x 5 and 7 x 7 of one
 // group.  thin: whether the kernel with rows along the lanes would be taken.
-bool spmm_patch_plan(const WalkView &wk, long long n_out, int batch, bool thin);
+bool spmm_patch_plan(const WalkView &wk, long long n_out, long long n_in, int batch, float beta, const SpEpilogue &ep, bool thin);
 hipError_t spmm_patch_launch(const PlaneLaunch &L);
 
 // m = mw*M[i] - lr*(dW[i] + l2*W[i]); W[i] += m; M[i] = m, i < n.

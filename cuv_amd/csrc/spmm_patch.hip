@@ -374,13 +374,21 @@ hipError_t spmm_patch_launch(const PlaneLaunch &L)
     }
 }
 
-// Measured on 1100 random products and layers of one map, 20 to 400 wide, batch 24 to 1024, against the kernels that would run.  In
-// place of the one that takes rows in a line: 3 x 3 and 5 x 5 at 1.24 times its rate on average, 5 of 230 below 0.97 (the least
-// 0.92); 7 x 7 at 1.11 where the launch is one round of two workgroups per CU or what fills up patches, map rows and columns does
-// not come to a tenth more than there (the least 0.84), 0.96 elsewhere.  In place of rows along the lanes, which have a column of
+// Measured on 16500 random products and layers of one map, 20 to 400 wide, batch 24 to 1024, against the kernels that would run.
+//
+// In place of the one that takes rows in a line, what counts is how many workgroups of either a CU gets one after the other, as a
+// round costs the same whether it is full: 7 x 7 1.10 of its rate where it is not more than there, 0.93 where it is (0.79 on 513 -
+// 768 patches, a third workgroup on a few CUs); with so few that every CU has one at most, or two, the other's are ahead on maps
+// from 72 wide whose ends its 16-byte pieces fit (one: 0.95; two: sampled ones 0.96, of a bias and widths that are no multiples of 4
+// 0.99, the others 1.01).  3 x 3 and 5 x 5, which fit a CU three and four times: 1.25 and 1.23; with more workgroups than there 1.05 - 1.2,
+// but 0.96 on a third, sampled ones on a second one too.  3 x 3 that only write a map whose rows are no multiples of 16 bytes leave half
+// lines to memory: 0.92 from a fourth workgroup on, unless the other has a quarter more of them, 1.02 - 1.16 on old values, which
+// bring the lines into the caches.  Of 7650 others 6100 come here, at 1.16 on average, 3.4 % below
+// 0.97 (the least 0.84); of those left out two thirds are below 0.97, 0.94 on average.
+// In place of rows along the lanes, which have a column of
 // their own for each: at 1.22 (1.05 - 1.57) on one column tile of 320 patches and more that the map's width fills; 0.7 - 1.1 on
 // fewer, 0.8 - 1.0 on a second column tile that is nearly empty.  The plane's walk is ahead where it runs (0.90).
-bool spmm_patch_plan(const WalkView &wk, long long n_out, int batch, bool thin)
+bool spmm_patch_plan(const WalkView &wk, long long n_out, long long n_in, int batch, float beta, const SpEpilogue &ep, bool thin)
 {
     if (wk.tab_dev == nullptr || wk.spans == nullptr || wk.spans->work == 0 || wk.ngroups != 1 || wk.lck != wk.k) return false;
     if (wk.k != 3 && wk.k != 5 && wk.k != 7) return false;
@@ -389,8 +397,18 @@ bool spmm_patch_plan(const WalkView &wk, long long n_out, int batch, bool thin)
     const long long tiles = tx * ((n_out / wk.period + S::PYG - 1) / S::PYG) * col_tiles;
     if (tiles > 0xffff) return false;                // (PtDiv)
     if (thin) return col_tiles == 1 && tiles >= 320 && 20 * wk.period >= 19 * S::WIDTH * tx;
-    const long long in_a_line = ((n_out + 63) / 64) * ((batch + 63) / 64);     // tiles of as many results there
-    return wk.k < 7 || tiles <= 512 || 10 * tiles <= 11 * in_a_line;
+    constexpr int CUS = 256;
+    const long long in_a_line = ((n_out + 63) / 64) * ((batch + 63) / 64);     // tiles there
+    const long long rounds = (tiles + CUS - 1) / CUS, rounds_there = (in_a_line + CUS - 1) / CUS;
+    const bool sampled = ep.act == 2, fused = ep.bias != nullptr || ep.act != 0, quads = wk.period % 4 == 0;
+    if (wk.k == 7) {
+        if (rounds > rounds_there) return false;
+        if (wk.period < 72 || n_in % 4 != 0 || rounds_there > 2) return true;
+        return rounds_there == 2 && !sampled && (quads || !fused);
+    }
+    if (rounds > rounds_there && (rounds == 3 || (rounds == 2 && sampled))) return false;
+    if (wk.k == 3 && rounds > 3 && !quads && !sampled) return beta == 0.f ? 5 * tiles <= 4 * in_a_line : rounds <= rounds_there;
+    return true;
 }
 
 }  // namespace cuvdia

@@ -29,3 +29,40 @@ for call, kernel in [
     assert ran(*call) == kernel, (call, ran(*call))
 assert ran(128, 128, 7, 128, path=_lib.PATH_TILED) == ran(128, 128, 7, 128, path=_lib.PATH_TILED_NOWALK) == "spmm_tiled_kernel<7, 8, 1, false, false>"
 """)
+
+
+def test_patches_only_where_they_are_ahead_of_rows_in_a_line(tmp_path):
+    """Rounds of 256 workgroups here and there, widths, ends and exits: a call on either side of every line of the rule."""
+    _fake_hip.run(tmp_path, """
+def patches(px, py, fs, batch, beta=0.0, act=None):
+    n = px * py
+    A = matrix(n, n, D.filter_factory_float(px, py, fs, 1, 1).offsets())
+    dst, X = tensor(batch, n, bytes_at=1 << 41), tensor(batch, n, bytes_at=1 << 42)
+    if act is None:
+        D.prod(dst, A, X, "n", "n", 1.0, beta)
+    else:
+        D.prod_bias_act(dst, A, X, "n", 1.0, beta, bias=tensor(n, bytes_at=1 << 43), act=act)
+    name = L.cuvdia_last_kernel().decode()
+    assert name.startswith("spmm_tiled_kernel<%d, " % fs)
+    return name in ("spmm_tiled_kernel<%d, %s>" % (fs, f) for f in ("true", "false"))
+SIGMOID, SAMPLE = _lib.ACT_SIGMOID, _lib.ACT_SIGMOID_SAMPLE
+for want, call in [
+    # 7 x 7: not more rounds than there
+    (False, (104, 104, 7, 156)),                 # 520 patches, 507 tiles
+    (False, (224, 146, 7, 61)),                  # 518 and 511
+    (True, (224, 144, 7, 64)),                   # 504 and 504
+    (True, (224, 147, 7, 64)),                   # 518 and 515
+    (False, (100, 154, 7, 64)),                  # 312 and 241
+    # one round, two rounds: the widest that are taken, ends of 16-byte pieces, exits
+    (True, (71, 72, 7, 64)), (False, (72, 72, 7, 64)), (True, (73, 73, 7, 64)),
+    (True, (128, 128, 7, 128)), (True, (128, 128, 7, 128, 0.0, SIGMOID)), (False, (128, 128, 7, 128, 0.0, SAMPLE)),
+    (False, (90, 90, 7, 170, 0.0, SIGMOID)), (True, (90, 90, 7, 170)),
+    (True, (91, 91, 7, 192, 0.0, SAMPLE)),
+    # 5 x 5: a third round that is not there in a line, a sample's second one
+    (False, (90, 90, 5, 256)), (True, (96, 96, 5, 256)), (True, (73, 73, 5, 192)), (False, (74, 86, 5, 128, 0.5, SAMPLE)), (True, (47, 64, 5, 942, 0.0, SIGMOID)),
+    # 3 x 3: map rows that are no multiples of 16 bytes, only written, from the fourth round on
+    (False, (127, 127, 3, 512)), (True, (124, 124, 3, 512)), (True, (127, 127, 3, 512, 0.5)), (True, (127, 127, 3, 512, 0.0, SAMPLE)),
+    (False, (186, 272, 3, 640, 0.5)), (True, (303, 303, 3, 80)), (False, (303, 303, 3, 160)), (True, (127, 127, 3, 128)),
+]:
+    assert patches(*call) == want, (call, L.cuvdia_last_kernel())
+""")
