@@ -7,8 +7,8 @@
 // others are sums of their own that nobody reads, so no value of theirs, infinite or not, reaches a slot.  Every number is split
 // into three bfloat16 ones where it is staged (split.hpp), six of their nine products are made: 16 columns of two pairs of parts
 // fill an instruction's 32, three instructions are 16 columns.  What the split does not hold exactly (an infinity, a NaN, a
-// number below 2^-110) is seen there, and the stage that has it is multiplied in fp32 from memory, 4.7 times as long where
-// every stage has some (4 maps of 256 x 256 to 4, batch 256: 4.0 ms).
+// number below 2^-110) is seen there, and the stage that has it is multiplied in fp32 from memory, behind the other stages of its 1024
+// columns: 4.0 ms where every stage has some, 0.99 where one of 16 has (4 maps of 256 x 256 to 4, batch 256; 0.82 without).
 //
 // Per stage of 16 columns the loads of the next one are on their way to registers; the split, transposed, goes to LDS; a wave
 // works two patches of A.  The products of a stage are one stretch of code without a branch, a patch's sums are added while the next
@@ -24,7 +24,8 @@
 // loads and fewer of them are slots: 0.5 - 0.95 times the kernels that serve them.
 //
 // Accumulation order: of every 16 columns the six products of all columns, smallest first, rounded as the matrix core does
-// (split.hpp); these sums in fp32, columns ascending.  Error against 64 bits (2-norm, relative; uniform operands in -1 .. 1) at
+// (split.hpp); these sums in fp32, within each 1024 columns those of the stages that the split holds, ascending, then the others',
+// each a chain of fp32 FMAs, ascending.  Error against 64 bits (2-norm, relative; uniform operands in -1 .. 1) at
 // batch 37, 128, 256 and 2048: 0.5, 0.7, 0.9 and 2.2e-7, where a chain of fp32 FMAs has 1.1, 2.0, 2.9 and 8.1e-7.  Sums of 1, 2,
 // 4, 8 and 16 products spread over 128 columns: 3.1, 4.1, 5.1, 5.9 and 6.6e-8, the chain 2.5, 3.1, 4.0, 5.4 and 7.4e-8: a sum of
 // few is rounded where the others' meet the first parts' products and again where the blocks of 16 columns meet.  (First parts'

@@ -78,6 +78,35 @@ def test_values_that_no_three_parts_hold(oracle):
     assert _split_ran()
 
 
+@pytest.mark.parametrize("columns", [(3,), (1023,), (1024,), (1045, 1056), (0, 500, 1023, 1024, 1059), (1008, 1039)])
+def test_such_values_in_batches_of_several_blocks(oracle, columns):
+    """Stages of 16 columns that the split does not hold are multiplied behind their block of 64: the first and the last of a block,
+    those of the second, of either operand, and the block that follows."""
+    import _gpu_util as gu
+    from cuv_amd import _lib
+    rng = np.random.default_rng(columns[0])
+    px, rows, batch = 32, 16, 1060
+    n = px * rows
+    C, valid = _dia(oracle, rng, n, n, _offsets(px, rows, 0, 1, 1))
+    A, B = _operands(rng, n, n, batch)
+    for i, c in enumerate(columns):
+        (A if i % 2 == 0 else B)[::7, c] = np.float32(1e-39)
+    gu.check_dd2dia(oracle, C, A, B, 1.0 / batch, 0.5, _lib.PATH_PLANE, "tiny numbers in columns %r" % (columns,))
+    assert _split_ran()
+    C.vals[valid] = 0.0
+    for i, c in enumerate(columns):
+        (B if i % 2 == 0 else A)[100 + 77 * i, c] = (np.inf, np.nan, -np.inf)[i % 3]
+    with np.errstate(invalid="ignore"):
+        ref = oracle.dd2dia(C, A, B, 1.0, 0.0)
+    got, ran = gu.gpu_dd2dia(C, A, B, path=_lib.PATH_PLANE)
+    assert _split_ran() and ran == _lib.PATH_PLANE
+    assert np.array_equal(np.isnan(got[valid]), np.isnan(ref[valid])) and np.array_equal(got[valid] == np.inf, ref[valid] == np.inf)
+    assert np.array_equal(got[valid] == -np.inf, ref[valid] == -np.inf)
+    fin = valid & np.isfinite(ref)
+    assert 0 < fin.sum() < valid.sum()
+    np.testing.assert_allclose(got[fin], ref[fin], rtol=0, atol=1e-5 * batch)          # 1e-5 of the terms' magnitudes, which are below 1
+
+
 @pytest.mark.parametrize("px,rows,batch,split", [(256, 256, 128, True), (256, 256, 127, False), (256, 264, 128, False)])
 def test_automatic_choice(oracle, px, rows, batch, split):
     import _gpu_util as gu
