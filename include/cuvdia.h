@@ -389,7 +389,9 @@ int cuvdia_last_path(void);
 
 /* Name of the kernel the most recent compute call on this thread launched
  * (the last one, where a call launches several), written as a profiler
- * prints it, e.g. "spmm_tiled_kernel<7, 8, 1, false>"; "" before any call.
+ * prints it, e.g. "spmm_tiled_kernel<7, 8, 1, false, false>", the tile-by-tile
+ * product of rows in a line, or "spmm_tiled_kernel<7, false>", the one whose
+ * tiles are patches: two arguments instead of five; "" before any call.
  * The string belongs to the library and is overwritten by the next call.
  * No counterpart in the reference. */
 const char *cuvdia_last_kernel(void);

@@ -66,3 +66,28 @@ for want, call in [
 ]:
     assert patches(*call) == want, (call, L.cuvdia_last_kernel())
 """)
+
+
+def test_which_of_the_two_tile_by_tile_kernels_runs(tmp_path):
+    """Both are called spmm_tiled_kernel: rows in a line have five template arguments, patches two.  The calls that other tests expect to
+    be served tile by tile."""
+    _fake_hip.run(tmp_path, """
+def ran(px, py, fs, maps_in, maps_out, batch, trans="n", path=_lib.PATH_AUTO):
+    h, w = px * py * maps_in, px * py * maps_out
+    A = matrix(h, w, D.filter_factory_float(px, py, fs, maps_in, maps_out).offsets())
+    out, inner = (w, h) if trans == "t" else (h, w)
+    L.cuvdia_set_path(path)
+    D.prod(tensor(batch, out, bytes_at=1 << 41), A, tensor(batch, inner, bytes_at=1 << 42), trans)
+    L.cuvdia_set_path(_lib.PATH_AUTO)
+    return L.cuvdia_last_kernel().decode()
+for call, kernel in [
+    ((40, 40, 7, 1, 1, 150), "spmm_tiled_kernel<7, false>"),
+    ((64, 64, 5, 3, 4, 128), "spmm_tiled_kernel<5, 8, 1, false, false>"),
+    ((64, 64, 13, 2, 2, 92), "spmm_tiled_kernel<13, 8, 1, false, false>"),
+    ((56, 152, 7, 1, 1, 897), "spmm_tiled_kernel<7, 8, 1, false, false>"),
+    ((272, 60, 7, 1, 2, 569), "spmm_tiled_kernel<7, 8, 1, false, false>"),
+    ((40, 40, 7, 1, 1, 150, "n", _lib.PATH_TILED), "spmm_tiled_kernel<7, 8, 1, false, false>"),
+    ((56, 152, 7, 1, 1, 897, "t", _lib.PATH_TILED_NOWALK), "spmm_tiled_kernel<7, 8, 1, false, false>"),
+]:
+    assert ran(*call) == kernel, (call, ran(*call))
+""")
