@@ -93,3 +93,88 @@ def test_non_finite_values(oracle, px, rows, rows_in, k, shift, batch):
         got, _ = gu.gpu_prod(A, B, None, trans)
         assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(got == np.inf, ref == np.inf)
         assert np.array_equal(got == -np.inf, ref == -np.inf)
+
+
+@pytest.mark.parametrize("px,rows,rows_in,k,shift,batch", CASES[:7])
+def test_operands_off_every_alignment(oracle, px, rows, rows_in, k, shift, batch):
+    """Bases of the values, the dense rows, the destination and the bias off 16 bytes by 1 to 3 floats, columns of odd pitch with NaN
+    between them, transposed and not, plain and with a sigmoid and a sample: each result, and nothing beside them."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng = np.random.default_rng(3 * px + batch)
+    n_in, n_out = px * rows_in, px * rows
+    u = oracle.sample_uniform(n_out, batch, 31)
+    for trans in "nt":
+        A = _layer(oracle, rng, px, rows, rows_in, k, shift, trans, trans == "t")
+        B = np.asfortranarray(rng.uniform(-1, 1, (n_in, batch)).astype(np.float32))
+        dst = np.asfortranarray(rng.uniform(-1, 1, (n_out, batch)).astype(np.float32))
+        bias = rng.uniform(-1, 1, n_out).astype(np.float32)
+        dev = gu.make_dev_dia(A)
+        vals = torch.full((dev.vec.numel() + 1,), float("nan"), device="cuda:0")
+        vals[1:] = dev.vec
+        dev.vec = vals[1:]
+        X = torch.full((batch, n_in + 5), float("nan"), device="cuda:0")
+        X[:, 3:3 + n_in] = D.to_device_colmajor(B)
+        X, bias_d = X[:, 3:3 + n_in], torch.cat([torch.zeros(2), torch.from_numpy(bias)]).cuda()[2:]
+        mag = oracle.prod_mag(A, B, dst, trans, 0.25, -0.5)
+        for act in (_lib.ACT_NONE, _lib.ACT_SIGMOID, _lib.ACT_SIGMOID_SAMPLE):
+            out = torch.full((batch, n_out + 7), -7.0, device="cuda:0")
+            view = out[:, 1:1 + n_out]
+            view.copy_(D.to_device_colmajor(dst))
+            if act == _lib.ACT_NONE:
+                D.prod(view, dev, X, trans, "n", 0.25, -0.5)
+            else:
+                D.prod_bias_act(view, dev, X, trans, 0.25, -0.5, bias=bias_d, act=act, seed=31)
+            ran = _lib.lib().cuvdia_last_kernel()
+            got = D.to_host_colmajor(view.contiguous()).astype(np.float64)
+            if act == _lib.ACT_NONE:
+                assert ran == b"spmm_tiled_kernel<%d, false>" % k
+                assert np.all(np.abs(got - oracle.prod(A, B, dst, trans, 0.25, -0.5)) <= gu.REL_TOL * mag)
+            else:
+                p = oracle.prod_bias_act(A, B, dst, trans, 0.25, -0.5, bias, True).astype(np.float64)
+                tol = 0.25 * gu.REL_TOL * (mag + 1.0) + 3e-7     # a quarter (the sigmoid's steepest slope) of the sum's, and its own rounding
+                assert ran == b"spmm_tiled_kernel<%d, true>" % k
+                if act == _lib.ACT_SIGMOID:
+                    assert np.all(np.abs(got - p) <= tol)
+                else:
+                    decided = np.abs(p - u) > tol
+                    assert decided.mean() > 0.99 and np.array_equal(got[decided], oracle.rnd_binarize(p.astype(np.float32), u)[decided])
+            assert torch.all(out[:, 0] == -7.0) and torch.all(out[:, 1 + n_out:] == -7.0)
+
+
+@pytest.mark.parametrize("px,rows,rows_in,k,shift,batch", [CASES[1], CASES[4]])
+def test_capture_and_replay(oracle, px, rows, rows_in, k, shift, batch):
+    """Added to old values, with a sample, transposed: a graph's replays against the eager calls, operands changed in between."""
+    import torch
+    import _gpu_util as gu
+    from cuv_amd import _lib, dia as D
+    rng = np.random.default_rng(px)
+    dev = gu.make_dev_dia(_layer(oracle, rng, px, rows, rows_in, k, shift, "t", False))
+    X, bias = torch.empty(batch, px * rows_in, device="cuda:0"), torch.randn(px * rows, device="cuda:0")
+    plain, layer = torch.empty(batch, px * rows, device="cuda:0"), torch.empty(batch, px * rows, device="cuda:0")
+
+    def calls():
+        D.prod(plain, dev, X, "t", "n", 0.5, 0.25, sync=False)
+        assert _lib.lib().cuvdia_last_kernel() == b"spmm_tiled_kernel<%d, false>" % k
+        D.prod_bias_act(layer, dev, X, "t", bias=bias, act=_lib.ACT_SIGMOID_SAMPLE, seed=5, sync=False)
+        assert _lib.lib().cuvdia_last_kernel() == b"spmm_tiled_kernel<%d, true>" % k
+
+    def refill(i):
+        X.copy_(torch.from_numpy(np.random.default_rng(i).uniform(-1, 1, tuple(X.shape)).astype(np.float32)))
+        plain.fill_(0.5 + i)
+        layer.fill_(-1.0)
+    refill(0)
+    calls()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls()
+    for i in range(1, 5):
+        refill(i)
+        calls()
+        eager = plain.clone(), layer.clone()
+        refill(i)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(plain, eager[0]) and torch.equal(layer, eager[1])
