@@ -56,15 +56,6 @@ struct DsTiles {
     int first_tile[DS_MAX_GROUPS + 1], first_block[DS_MAX_GROUPS];
 };
 
-template <int I, int N, class F>
-__device__ __forceinline__ void ds_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        ds_for<I + 1, N>(f);
-    }
-}
-
 template <int LC, int K>
 struct DsShape {
     static constexpr int BX = (LC + 3 + 3) / 4, BY = (K + 3 + 3) / 4;      // patches of B that a patch of A meets
@@ -149,7 +140,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
 
     f4 st[8];
     auto request = [&](auto first_, auto last_, int c) __attribute__((always_inline)) {
-        ds_for<decltype(first_)::value, decltype(last_)::value>([&](auto j_) {
+        static_for<decltype(first_)::value, decltype(last_)::value>([&](auto j_) {
             constexpr int j = decltype(j_)::value;
             if constexpr (j == 8) {
                 lds_load_b128(a_raw, raw_to, raw_row < h ? raw_off + (unsigned)c * lda4 : OOB_OFFSET, 0);
@@ -260,7 +251,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             }
             // (the next stage's requests a few at a time, past the last one too, and by two thirds of the products: all at once they
             // wait for each other, the last ones at the end are waited for)
-            ds_for<0, TILES>([&](auto t_) {
+            static_for<0, TILES>([&](auto t_) {
                 constexpr int t = decltype(t_)::value, y = t / S::BX;
                 constexpr int first = 3 * S::LOADS * t / (2 * TILES), last = 3 * S::LOADS * (t + 1) / (2 * TILES);
                 fetch(std::integral_constant<int, t + 1>{});
@@ -281,7 +272,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
         while (exact) {
             const int c = c0 + DS_COLS * __builtin_ctzll(exact);
             exact &= exact - 1;
-            ds_for<0, TILES>([&](auto t_) {
+            static_for<0, TILES>([&](auto t_) {
                 constexpr int t = decltype(t_)::value, y = t / S::BX, x = t % S::BX;
                 const int l = here(lane), row_a = i_tile + l % 16 / 4 * period + 4 * wave + l % 4, row_b = row_a + s_g + 4 * y * period + 4 * x;
                 sum[t % 2][0] = sum[t % 2][1] = f4{0.f, 0.f, 0.f, 0.f};
@@ -309,7 +300,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
     float *const there = out + (by * LC + bx) * S::PITCH + q4 * DS_XT + 4 * wave;
     constexpr int PLACES = DS_XT * DS_YT / 2 / 4, SLOTS = DS_THREADS / PLACES, ITS = (LC * K + SLOTS - 1) / SLOTS;
     const int place_y = thread % PLACES / (DS_XT / 4), place_x = 4 * (thread % (DS_XT / 4));
-    ds_for<0, 2>([&](auto half_) {
+    static_for<0, 2>([&](auto half_) {
         constexpr int half = decltype(half_)::value;
         const int to_row = i_tile + (4 * half + place_y) * period + place_x;
         const bool is_row = tx * DS_XT + place_x < period && to_row < h;
@@ -325,7 +316,7 @@ __global__ __launch_bounds__(DS_THREADS, 2) void dd2dia_split_kernel(
             if (beta != 0.f && whole) old[k] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(cr, to_off[k], 0, 0));
             if (is && !whole) over |= 1u << k;
         }
-        ds_for<0, S::BY * S::BX * 4>([&](auto e_) {
+        static_for<0, S::BY * S::BX * 4>([&](auto e_) {
             constexpr int e = decltype(e_)::value, y = e / (4 * S::BX), x = e / 4 % S::BX, i = e % 4;
             // (checked only where a patch of B reaches over the window's edge)
             const bool in_y = (4 * y >= 3 && 4 * y + 3 < K) || (unsigned)(4 * y + by) < (unsigned)K;

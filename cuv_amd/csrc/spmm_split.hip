@@ -79,15 +79,6 @@ struct PsShape {
     static_assert(2 * LDS <= 160 * 1024, "two workgroups per CU");
 };
 
-template <int I, int N, class F>
-__device__ __forceinline__ void ps_for(F &&f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        ps_for<I + 1, N>(f);
-    }
-}
-
 // lds_load_b128 for operands that are in scalar registers as it is
 __device__ __forceinline__ void ps_load(sp_int4 rsrc, unsigned to, unsigned voff, unsigned soff)
 {
@@ -276,7 +267,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
     // positions are written together.
     auto finish = [&](int y0, int leaving, int buf) __attribute__((always_inline)) {
         float *const out = reinterpret_cast<float *>(lds + buf * S::X_BYTES);
-        ps_for<0, NA>([&](auto a_) __attribute__((always_inline)) {
+        static_for<0, NA>([&](auto a_) __attribute__((always_inline)) {
             constexpr int a = decltype(a_)::value;
             if (leaving != a) return;
             asm volatile("" :: "n"(a));              // (four ways through, not one with an index)
@@ -370,7 +361,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
     Block cur = advance(), next = advance(), third = advance();
     __syncthreads();                                 // (the tables, the zeros)
     request(next);
-    ps_for<0, PIECES>([&](auto n_) __attribute__((always_inline)) { request_x(n_); });
+    static_for<0, PIECES>([&](auto n_) __attribute__((always_inline)) { request_x(n_); });
 
 
     // A block's flags: 1: not all of its dense rows are held exactly; 2: not all are bfloat16 numbers
@@ -427,7 +418,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
     auto exact = [&](auto p_) __attribute__((always_inline)) {
         constexpr int p = decltype(p_)::value;
         const int l = here(lane), sx = wave * PX;            // this lane's sums: positions sx .. sx + 3 of patch rows l / 32, + 2
-        ps_for<0, NT>([&](auto n_) __attribute__((always_inline)) {
+        static_for<0, NT>([&](auto n_) __attribute__((always_inline)) {
             constexpr int n = decltype(n_)::value;
             const unsigned col = (unsigned)min(32 * n + l % 32, cols - 1) * ldx4;
             auto piece = [&](int xr) __attribute__((always_inline)) {
@@ -500,10 +491,10 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
         // the first pair's values
         {
             unsigned low = 0;
-            ps_for<0, 2>([&](auto r_) __attribute__((always_inline)) {
+            static_for<0, 2>([&](auto r_) __attribute__((always_inline)) {
                 constexpr int r = decltype(r_)::value;
                 values_at(std::integral_constant<int, 0>{}, r, u);
-                ps_for<0, 4>([&](auto j_) __attribute__((always_inline)) { values_of(j_, v[4 * r + decltype(j_)::value]); });
+                static_for<0, 4>([&](auto j_) __attribute__((always_inline)) { values_of(j_, v[4 * r + decltype(j_)::value]); });
             });
             auto rows_of = [&](auto s_) __attribute__((always_inline)) {
                 constexpr int s = decltype(s_)::value;
@@ -522,7 +513,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 rows_of(std::integral_constant<int, 1>{});
             }
             rows_of(std::integral_constant<int, 0>{});
-            ps_for<0, 8>([&](auto j_) __attribute__((always_inline)) {
+            static_for<0, 8>([&](auto j_) __attribute__((always_inline)) {
                 constexpr int j = decltype(j_)::value;
                 unsigned p0, p1, p2;
                 split2(v[j][0], v[j][1], split_const, p0, p1, p2, low);
@@ -531,7 +522,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
             if (split_inexact<2>(low, [&](int i) __attribute__((always_inline)) { return af[0][i][2]; })) exact(std::integral_constant<int, 0>{});
         }
         request(third);
-        ps_for<0, 2>([&](auto pass_) __attribute__((always_inline)) {
+        static_for<0, 2>([&](auto pass_) __attribute__((always_inline)) {
             constexpr int pass = decltype(pass_)::value;
             unsigned low = 0;
             if constexpr (pass == 0) {
@@ -552,17 +543,17 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
             constexpr std::integral_constant<int, 2> last_part{};
             if (x_more) {
                 constexpr int PA[3] = {0, 1, 0}, PB[3] = {2, 1, 1};
-                ps_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
+                static_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
                     constexpr int p = decltype(i_)::value / 4;
                     product(i_, std::integral_constant<int, PA[p]>{}, std::integral_constant<int, PB[p]>{}, std::bool_constant<(decltype(i_)::value < 2)>{});
                     __builtin_amdgcn_sched_barrier(0);
                 });
-                ps_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::false_type{}); });
+                static_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::false_type{}); });
             } else {
-                ps_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::true_type{}); });
+                static_for<0, 2>([&](auto i_) __attribute__((always_inline)) { product(i_, last_part, std::integral_constant<int, 0>{}, std::true_type{}); });
             }
             __builtin_amdgcn_sched_barrier(0);
-            ps_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
+            static_for<0, 12>([&](auto i_) __attribute__((always_inline)) {
                 constexpr int i = decltype(i_)::value;
                 if constexpr (i >= 2) product(i_, std::integral_constant<int, 2 - i / 4>{}, std::integral_constant<int, 0>{}, std::false_type{});
                 // beside the products: in the first pass two pairs of the second pair's values per 3; a pair of the next dense rows per 3
@@ -610,7 +601,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
                 asm volatile("" : "+v"(xst[2]), "+v"(xst[3]));       // (come before the values are asked for)
                 request_values_of(next);
                 barrier();                           // (nobody reads the values any more)
-                ps_for<0, S::SLOTS>([&](auto i_) __attribute__((always_inline)) { request_values(i_); });
+                static_for<0, S::SLOTS>([&](auto i_) __attribute__((always_inline)) { request_values(i_); });
             }
         });
         raise(buf ^ 1, low_x, more_x);
