@@ -1694,8 +1694,9 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
 // length are computed and dropped).  A table with runs of more than 8 shifts
 // (window rows wider than 8) is walked in the products' chunks of up to 13
 // instead, every unit one such chunk: as many sums as a pair, one band, one
-// copy of A's rows.  A single chunk is worked by 4 waves, a pair by 8; wave
-// q walks the batch-column groups g = q, q + WAVES, ...
+// copy of A's rows.  A launch of single chunks, or of shifted pairs, has 4
+// waves per workgroup, one of pairs that share A's rows 8, its single chunks
+// too (dd_waves); wave q walks the batch-column groups g = q, q + WAVES, ...
 // (4 columns per group).  Per group and column the wave
 //   1. writes the column's rows [row0 + s0, row0 + s0 + 264 + delta) of B,
 //      fetched one step earlier as 16-byte pieces (a lane holds 4 consecutive
@@ -1712,8 +1713,8 @@ __global__ __launch_bounds__(512, (WalkShape<LCK, K, T, SH>::WAVES_PER_SIMD)) vo
 //   4. issues 4 x LC FMAs per chunk.  A pair needs A once and the two bands of
 //      B overlap, so it moves about 40 % fewer bytes per FMA than two singles.
 // At the end the waves' partial sums meet in LDS and are added in a fixed
-// order; the result is written with lanes along rows (the values of C that
-// beta scales were fetched at kernel start).
+// order; every wave writes a share of the diagonals, 4 rows per lane (the
+// values of C that beta scales were fetched at kernel start).
 
 constexpr int DD_ROWS = 256;
 constexpr int DD_BG = 4;           // batch columns per step
@@ -1722,7 +1723,7 @@ constexpr int DD_BG = 4;           // batch columns per step
 // SP_CHUNK_MAX shifts: a whole row of a wide 2-d window), never a pair.  It
 // keeps as many running sums as a pair but is worked by 4 waves: three such
 // workgroups share a CU (registers allow 3 waves per SIMD, and the block the
-// sums are added in is kept just under a third of the CU's LDS).
+// sums are added in, 52 KB, is just under a third of the CU's LDS).
 // WIDE says how a pair is served.  The two chunks of a pair start delta rows apart; for row i the first pairs it
 // with rows i + s0 + j of B, the second with rows i + s0 + delta + j.
 //   DD_NARROW, DD_WIDE -- both chunks work on the SAME rows of A: one copy of A's rows and one band of B that
