@@ -1763,11 +1763,15 @@ struct DdStage {
     float a[NA][DD_BG][4];    // this lane's 4 rows of each column (a shifted pair: and the 4 rows delta above)
 };
 
+// Chunks whose sums meet in LDS at a time: both of a pair, of a shifted one only if its three workgroups still fit a CU.  (One after
+// the other, one of four waves has 2 of 5 diagonals, the others 1, twice: 5 x 5, 32 x 32, 2 maps to 2, batch 96 8.5 us for 8.0.)
+template <int LC, int NCH, int WIDE>
+constexpr int dd_meet() { return WIDE == DD_SHIFTED && LC > 6 ? 1 : NCH; }
 template <int LC, int NCH, int WIDE, int NW>
 constexpr int dd_lds_floats()
 {
-    // (a shifted pair adds its chunks' sums one chunk after the other, in the block of a single chunk)
-    constexpr int red = NW * (WIDE == DD_SHIFTED ? 1 : NCH) * LC * 64 * 4;
+    constexpr int red = NW * dd_meet<LC, NCH, WIDE>() * LC * 64 * 4;
+    static_assert(WIDE != DD_SHIFTED || 4 * red <= 160 * 1024 / 3, "");
     return DdShape<NCH, LC, WIDE, NW>::STAGE_FLOATS > red ? DdShape<NCH, LC, WIDE, NW>::STAGE_FLOATS : red;
 }
 
@@ -1792,15 +1796,15 @@ __device__ __forceinline__ void dd2dia_unit(
     constexpr int PITCH = S::PITCH, WAVES = S::WAVES, NB = SHORT ? 1 : S::NB;
     constexpr int NA = SHIFTED ? 2 : 1;                      // copies of A's rows a lane holds per column
     constexpr int NWIN = SHIFTED ? 1 : NCH;                  // windows of B a lane reads per column
-    constexpr int NRED = SHIFTED ? 1 : NCH;                  // chunks whose sums meet in LDS at a time
+    constexpr int NRED = dd_meet<LC, NCH, WIDE>();
     static_assert(!SHORT || TR + S::SPAN <= 256 || (S::LONG && TR + 16 <= 256), "a short tile's band is one piece per lane");
     constexpr int WIN = 4 + LC - 1;
     constexpr int WQ = (WIN + 3) / 4;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     typedef const int __attribute__((address_space(4))) *sc_int_ptr;         // (scalar loads)
-    // A wave's share of the output: positions wave, wave + WAVES, ... of the unit's NCH x LC (a shifted pair: of one chunk, then of
-    // the other), of which each lane combines and writes its own 4 rows.
+    // A wave's share of the output: positions wave, wave + WAVES, ... of the unit's NCH x LC (a shifted pair of more than 6: of one
+    // chunk, then of the other), of which each lane combines and writes its own 4 rows.
     constexpr int PASS = NRED * LC, SHARE = (PASS + WAVES - 1) / WAVES, PASSES = NCH / NRED;
     int s0[NCH], slot[PASSES][SHARE];
 #pragma unroll
@@ -2069,7 +2073,7 @@ __device__ __forceinline__ void dd2dia_unit(
     if (k < steps) step(k, 0, st0, st1);
 
     // Combine the waves' partial sums: every wave leaves its own in LDS, a lane's 4 rows side by side, and takes its share of the
-    // output (a shifted pair: one chunk after the other).  Summed in wave order: total = ((p0 + p1) + p2) + p3 with p_q = s_q, of
+    // output (a shifted pair of more than 6: one chunk after the other).  Summed in wave order: total = ((p0 + p1) + p2) + p3 with p_q = s_q, of
     // 8 waves s_q + s_{q+4}.  (Before, four of 8 waves added the others' sums to theirs, 4 bytes at a time, and wrote the output:
     // 5000 clocks of the 17500 of a one-round launch.  16384-unit layer, 7 x 7, batch 128 10.7 -> 9.5 us; 784 x 1568, 128
     // diagonals, batch 96 9.0 -> 7.8; launches of many rounds 0 - 3 %.)
