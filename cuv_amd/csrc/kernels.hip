@@ -38,7 +38,7 @@
 // This file is compiled ten times (CUVDIA_PART = 1 .. 10, see the Makefile), each translation unit
 // instantiating one share of the kernel templates, so that the shares compile in parallel: parts 1 - 3 hold
 // the tiled SpMM kernels by longest chunk (1 - 5, 6 - 9, 10 - 13), parts 8 - 10 those of tables with shorter chunks as
-// well, which want other switches, part 5 the walking SpMM kernels, part 6
+// well or with more than 64, which want other switches, part 5 the walking SpMM kernels, part 6
 // the window-table projection for window rows of at most 8 diagonals, part 7 the one for rows of 9 to 13, part 4
 // everything else.  Without the macro one unit holds everything.
 #ifndef CUVDIA_PART
@@ -2907,9 +2907,9 @@ hipError_t dd2dia_window_long_launch(const DwLaunch &L);      // (rows of 9 to 1
 hipError_t spmm_tiled_launch_1_5(const SpLaunch &L);
 hipError_t spmm_tiled_launch_6_9(const SpLaunch &L);
 hipError_t spmm_tiled_launch_10_13(const SpLaunch &L);
-hipError_t spmm_mixed_launch_2_5(const SpLaunch &L);
-hipError_t spmm_mixed_launch_6_9(const SpLaunch &L);
-hipError_t spmm_mixed_launch_10_13(const SpLaunch &L);
+hipError_t spmm_other_launch_1_5(const SpLaunch &L);
+hipError_t spmm_other_launch_6_9(const SpLaunch &L);
+hipError_t spmm_other_launch_10_13(const SpLaunch &L);
 
 // 8 rows per wave (8 waves per workgroup) keeps four waves on every SIMD
 // at the sizes this path is measured on.
@@ -2922,11 +2922,32 @@ hipError_t spmm_mixed_launch_10_13(const SpLaunch &L);
         if (fused) CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, true, MIXED);                                                      \
         else CUVDIA_SPMM_LAUNCH_ONE(K, NTAB, false, MIXED);                                                           \
     } while (0)
-#define CUVDIA_SPMM_LAUNCH(K, MIXED)                                                                                  \
+#define CUVDIA_SPMM_NOTE(K, NTAB, MIXED)                                                                              \
+    note_kernel("spmm_tiled_kernel<%d, 8, %d, %s, " #MIXED ">", K, NTAB, fused ? "true" : "false")
+// A table of up to 64 chunks, all of one length
+#define CUVDIA_SPMM_LAUNCH(K)                                                                                         \
     case K:                                                                                                           \
-        note_kernel("spmm_tiled_kernel<%d, 8, %d, %s, " #MIXED ">", K, L.nchunks <= 64 ? 1 : 4, fused ? "true" : "false"); \
-        if (L.nchunks <= 64) CUVDIA_SPMM_LAUNCH_TAB(K, 1, MIXED);                                                     \
-        else CUVDIA_SPMM_LAUNCH_TAB(K, 4, MIXED);                                                                     \
+        CUVDIA_SPMM_NOTE(K, 1, false);                                                                                \
+        CUVDIA_SPMM_LAUNCH_TAB(K, 1, false);                                                                          \
+        break;
+// One of more chunks, or (from 2 diagonals on) of shorter ones as well
+#define CUVDIA_SPMM_LAUNCH_MANY(K)                                                                                    \
+    case K:                                                                                                           \
+        CUVDIA_SPMM_NOTE(K, 4, false);                                                                                \
+        CUVDIA_SPMM_LAUNCH_TAB(K, 4, false);                                                                          \
+        break;
+#define CUVDIA_SPMM_LAUNCH_OTHER(K)                                                                                   \
+    case K:                                                                                                           \
+        if (!L.mixed) {                                                                                               \
+            CUVDIA_SPMM_NOTE(K, 4, false);                                                                            \
+            CUVDIA_SPMM_LAUNCH_TAB(K, 4, false);                                                                      \
+        } else if (L.nchunks <= 64) {                                                                                 \
+            CUVDIA_SPMM_NOTE(K, 1, true);                                                                             \
+            CUVDIA_SPMM_LAUNCH_TAB(K, 1, true);                                                                       \
+        } else {                                                                                                      \
+            CUVDIA_SPMM_NOTE(K, 4, true);                                                                             \
+            CUVDIA_SPMM_LAUNCH_TAB(K, 4, true);                                                                       \
+        }                                                                                                             \
         break;
 // A unit's launch: the kernels of these longest chunks
 #define CUVDIA_SPMM_UNIT(NAME, CASES)                                                                                 \
@@ -3069,25 +3090,28 @@ hipError_t dd2dia_window_long_launch(const DwLaunch &L)
 }
 #endif
 #if CUVDIA_IN_PART(1)
-CUVDIA_SPMM_UNIT(spmm_tiled_launch_1_5, CUVDIA_SPMM_LAUNCH(1, false) CUVDIA_SPMM_LAUNCH(2, false) CUVDIA_SPMM_LAUNCH(3, false) CUVDIA_SPMM_LAUNCH(4, false) CUVDIA_SPMM_LAUNCH(5, false))
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_1_5, CUVDIA_SPMM_LAUNCH(1) CUVDIA_SPMM_LAUNCH(2) CUVDIA_SPMM_LAUNCH(3) CUVDIA_SPMM_LAUNCH(4) CUVDIA_SPMM_LAUNCH(5))
 #endif
 #if CUVDIA_IN_PART(2)
-CUVDIA_SPMM_UNIT(spmm_tiled_launch_6_9, CUVDIA_SPMM_LAUNCH(6, false) CUVDIA_SPMM_LAUNCH(7, false) CUVDIA_SPMM_LAUNCH(8, false) CUVDIA_SPMM_LAUNCH(9, false))
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_6_9, CUVDIA_SPMM_LAUNCH(6) CUVDIA_SPMM_LAUNCH(7) CUVDIA_SPMM_LAUNCH(8) CUVDIA_SPMM_LAUNCH(9))
 #endif
 #if CUVDIA_IN_PART(3)
-CUVDIA_SPMM_UNIT(spmm_tiled_launch_10_13, CUVDIA_SPMM_LAUNCH(10, false) CUVDIA_SPMM_LAUNCH(11, false) CUVDIA_SPMM_LAUNCH(12, false) CUVDIA_SPMM_LAUNCH(13, false))
+CUVDIA_SPMM_UNIT(spmm_tiled_launch_10_13, CUVDIA_SPMM_LAUNCH(10) CUVDIA_SPMM_LAUNCH(11) CUVDIA_SPMM_LAUNCH(12) CUVDIA_SPMM_LAUNCH(13))
 #endif
 #if CUVDIA_IN_PART(8)
-CUVDIA_SPMM_UNIT(spmm_mixed_launch_2_5, CUVDIA_SPMM_LAUNCH(2, true) CUVDIA_SPMM_LAUNCH(3, true) CUVDIA_SPMM_LAUNCH(4, true) CUVDIA_SPMM_LAUNCH(5, true))
+CUVDIA_SPMM_UNIT(spmm_other_launch_1_5, CUVDIA_SPMM_LAUNCH_MANY(1) CUVDIA_SPMM_LAUNCH_OTHER(2) CUVDIA_SPMM_LAUNCH_OTHER(3) CUVDIA_SPMM_LAUNCH_OTHER(4) CUVDIA_SPMM_LAUNCH_OTHER(5))
 #endif
 #if CUVDIA_IN_PART(9)
-CUVDIA_SPMM_UNIT(spmm_mixed_launch_6_9, CUVDIA_SPMM_LAUNCH(6, true) CUVDIA_SPMM_LAUNCH(7, true) CUVDIA_SPMM_LAUNCH(8, true) CUVDIA_SPMM_LAUNCH(9, true))
+CUVDIA_SPMM_UNIT(spmm_other_launch_6_9, CUVDIA_SPMM_LAUNCH_OTHER(6) CUVDIA_SPMM_LAUNCH_OTHER(7) CUVDIA_SPMM_LAUNCH_OTHER(8) CUVDIA_SPMM_LAUNCH_OTHER(9))
 #endif
 #if CUVDIA_IN_PART(10)
-CUVDIA_SPMM_UNIT(spmm_mixed_launch_10_13, CUVDIA_SPMM_LAUNCH(10, true) CUVDIA_SPMM_LAUNCH(11, true) CUVDIA_SPMM_LAUNCH(12, true) CUVDIA_SPMM_LAUNCH(13, true))
+CUVDIA_SPMM_UNIT(spmm_other_launch_10_13, CUVDIA_SPMM_LAUNCH_OTHER(10) CUVDIA_SPMM_LAUNCH_OTHER(11) CUVDIA_SPMM_LAUNCH_OTHER(12) CUVDIA_SPMM_LAUNCH_OTHER(13))
 #endif
 #undef CUVDIA_SPMM_UNIT
+#undef CUVDIA_SPMM_LAUNCH_OTHER
+#undef CUVDIA_SPMM_LAUNCH_MANY
 #undef CUVDIA_SPMM_LAUNCH
+#undef CUVDIA_SPMM_NOTE
 #undef CUVDIA_SPMM_LAUNCH_TAB
 #undef CUVDIA_SPMM_LAUNCH_ONE
 #undef CUVDIA_SPMM_ARGS
@@ -3150,10 +3174,10 @@ hipError_t launch_spmm_tiled(const DiaView &A, const float *vals, const float *B
                      trans ? A.slot_step_t : A.slot_step_n, ep,
                      dim3((unsigned)(row_tiles * col_tiles)), stream, lck,
                      (trans ? A.min_len_t : A.min_len_n) != lck};
-    const bool mixed = L.mixed && lck > 1;
-    if (lck <= 5) return mixed ? spmm_mixed_launch_2_5(L) : spmm_tiled_launch_1_5(L);
-    if (lck <= 9) return mixed ? spmm_mixed_launch_6_9(L) : spmm_tiled_launch_6_9(L);
-    return mixed ? spmm_mixed_launch_10_13(L) : spmm_tiled_launch_10_13(L);
+    const bool other = L.nchunks > 64 || (L.mixed && lck > 1);
+    if (lck <= 5) return other ? spmm_other_launch_1_5(L) : spmm_tiled_launch_1_5(L);
+    if (lck <= 9) return other ? spmm_other_launch_6_9(L) : spmm_tiled_launch_6_9(L);
+    return other ? spmm_other_launch_10_13(L) : spmm_tiled_launch_10_13(L);
 }
 
 hipError_t launch_dd2dia_generic(const DiaView &C, float *vals, const float *A, long long lda,

@@ -48,10 +48,10 @@ def test_rows_along_the_lanes_need_no_memory_of_their_own():
 
 def test_arguments_in_registers_only_where_they_are_ahead():
     """The products tile by tile, as patches too, and the gradient chunk by chunk; not those that save scalar registers in vector ones
-    for it: the tables with shorter chunks as well, rows along the lanes."""
+    for it: the tables with more than 64 chunks or with shorter ones as well, rows along the lanes."""
     found = _kernel_resources.preloaded()
     assert found.keys() == _kernel_resources.kernels().keys()
-    ahead = {n for n in found if ("spmm_tiled_kernel" in n and "ELb1EEEvPKNS_5Chunk" not in n) or "dd2dia_tiled_kernel" in n}
-    assert len(ahead) > 80 and [n for n in ahead if found[n] == 0] == []
+    ahead = {n for n in found if ("spmm_tiled_kernel" in n and "ELb1EEEvPKNS_5Chunk" not in n and "ELi8ELi4E" not in n) or "dd2dia_tiled_kernel" in n}
+    assert len(ahead) > 70 and [n for n in ahead if found[n] == 0] == []
     apart = {n for n in found if n not in ahead and any(k in n for k in ("spmm_", "dd2dia_")) and "generic" not in n}
     assert len(apart) > 200 and [n for n in apart if found[n] != 0] == []
