@@ -381,10 +381,10 @@ hipError_t spmm_patch_launch(const PlaneLaunch &L)
 // 768 patches, a third workgroup on a few CUs); with so few that every CU has one at most, or two, the other's are ahead on maps
 // from 72 wide whose ends its 16-byte pieces fit (one: 0.95; two: sampled ones 0.96, of a bias and widths that are no multiples of 4
 // 0.99, the others 1.01).  3 x 3 and 5 x 5, which fit a CU three and four times: 1.25 and 1.23; with more workgroups than there 1.05 - 1.2,
-// but 0.96 on a third, sampled ones on a second one too.  3 x 3 that only write a map whose rows are no multiples of 16 bytes leave half
-// lines to memory: 0.92 from a fourth workgroup on, unless the other has a quarter more of them, 1.02 - 1.16 on old values, which
-// bring the lines into the caches.  Of 7650 others 6100 come here, at 1.16 on average, 3.4 % below
-// 0.97 (the least 0.84); of those left out two thirds are below 0.97, 0.94 on average.
+// but on a third, sampled ones on a second one too, 0.92 on maps from 65 wide (1.04 on others, sampled 5 x 5 ones 0.99).  3 x 3 that only
+// write a map whose rows are no multiples of 16 bytes leave half lines to memory: 0.92 from a fourth workgroup on, unless the other
+// has a quarter more of them, 1.02 - 1.16 on old values, which bring the lines into the caches.  Of 7650 others 6100 come here, at
+// 1.16 on average, 3.4 % below 0.97 (the least 0.84); of those left out two thirds are below 0.97, 0.94 on average.
 // In place of rows along the lanes, which have a column of
 // their own for each: at 1.22 (1.05 - 1.57) on one column tile of 320 patches and more that the map's width fills; 0.7 - 1.1 on
 // fewer, 0.8 - 1.0 on a second column tile that is nearly empty.  The plane's walk is ahead where it runs (0.90).
@@ -406,7 +406,7 @@ bool spmm_patch_plan(const WalkView &wk, long long n_out, long long n_in, int ba
         if (wk.period < 72 || n_in % 4 != 0 || rounds_there > 2) return true;
         return rounds_there == 2 && !sampled && (quads || !fused);
     }
-    if (rounds > rounds_there && (rounds == 3 || (rounds == 2 && sampled))) return false;
+    if (rounds > rounds_there && (rounds == 3 || (rounds == 2 && sampled)) && (wk.period > 64 || (wk.k == 5 && sampled))) return false;
     if (wk.k == 3 && rounds > 3 && !quads && !sampled) return beta == 0.f ? 5 * tiles <= 4 * in_a_line : rounds <= rounds_there;
     return true;
 }

@@ -59,7 +59,7 @@ for want, call in [
     (False, (90, 90, 7, 170, 0.0, SIGMOID)), (True, (90, 90, 7, 170)),
     (True, (91, 91, 7, 192, 0.0, SAMPLE)),
     # 5 x 5: a third round that is not there in a line, a sample's second one
-    (False, (90, 90, 5, 256)), (True, (96, 96, 5, 256)), (True, (73, 73, 5, 192)), (False, (74, 86, 5, 128, 0.5, SAMPLE)), (True, (47, 64, 5, 942, 0.0, SIGMOID)),
+    (False, (90, 90, 5, 256)), (True, (62, 65, 5, 512)), (False, (48, 60, 5, 577, 0.0, SAMPLE)), (True, (40, 42, 3, 861)), (True, (96, 96, 5, 256)), (True, (73, 73, 5, 192)), (False, (74, 86, 5, 128, 0.5, SAMPLE)), (True, (47, 64, 5, 942, 0.0, SIGMOID)),
     # 3 x 3: map rows that are no multiples of 16 bytes, only written, from the fourth round on
     (False, (127, 127, 3, 512)), (True, (124, 124, 3, 512)), (True, (127, 127, 3, 512, 0.5)), (True, (127, 127, 3, 512, 0.0, SAMPLE)),
     (False, (186, 272, 3, 640, 0.5)), (True, (303, 303, 3, 80)), (False, (303, 303, 3, 160)), (True, (127, 127, 3, 128)),
