@@ -1854,11 +1854,10 @@ __device__ __forceinline__ void dd2dia_unit(
             for (int i = 0; i < SHARE; ++i) {
                 if (wave + WAVES * i >= PASS) continue;
                 const Quad q = out_quad(n0, i);
-                // (A quad of which a part exists is read whole as long as it lies in the buffer, and one way or the other by all lanes: rows
-                // read on top of the quads would wait for those to come, here, 0.4 - 1 us of a launch of few tiles.)
-                const bool some = q.valid != 0u, inside = q.at + 16u <= c_bytes;
-                if (!__any(some && !inside)) {
-                    cpre[n0][i] = __builtin_bit_cast(f4q, __builtin_amdgcn_raw_buffer_load_b128(cr, some ? q.at : OOB_OFFSET, 0, 0));
+                // (One way or the other for the whole wave: rows read on top of the quads would wait for those to come, here, 0.4 - 1 us
+                // of a launch of few tiles.)
+                if (!__any(q.valid != 15u && q.valid != 0u)) {
+                    cpre[n0][i] = __builtin_bit_cast(f4q, __builtin_amdgcn_raw_buffer_load_b128(cr, q.valid == 15u ? q.at : OOB_OFFSET, 0, 0));
                 } else {
 #pragma unroll
                     for (int t = 0; t < 4; ++t) cpre[n0][i][t] = buffer_load_f32(cr, (q.valid >> t) & 1u ? q.at + 4u * t : OOB_OFFSET);
