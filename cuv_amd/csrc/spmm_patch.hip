@@ -4,7 +4,8 @@
 // rows of K diagonals.  A workgroup owns 4 map rows x 32 positions x 32 batch columns and stages, once, all that they need: the
 // 4 + K - 1 map rows around them and the K * K diagonals' values.  The kernel that takes 64 rows in a line (spmm_tiled_kernel in
 // kernels.hip, of which this is the form for such tables) stages 76 rows x 64 columns anew for every window row, 7 steps with a
-// barrier each where this one has 4, and 2.3 times the bytes.  A half of a wave owns a group of 8 positions, a lane a column:
+// barrier each where this one has 4, and twice the bytes (2.7 times the dense rows, half the values); 1.76 times the accesses of
+// the L1 were counted.  A half of a wave owns a group of 8 positions, a lane a column:
 // its window is read by 16 bytes, the values are broadcast by DPP in every 16 lanes (fma16_dpp).
 //
 // Bound: on one round of workgroups (the 16384-unit layer at batch 128: 512) everything happens at once on all CUs -- 1400
@@ -17,9 +18,9 @@
 // them: a CU's two workgroups load and multiply in step); a map row's pieces of all columns dealt to the lanes (13.3: 600
 // instructions of addresses).
 //
-// Measured, us, operands that change from call to call (in a line -> this): 128 x 128, 7 x 7, batch 128 10.3 -> 9.1, added to half
-// of the old values, transposed 11.5 -> 10.1; 96 x 96, 5 x 5, batch 200 11.4 -> 6.9; 64 x 64, 5 x 5, batch 512 9.6 -> 6.8;
-// 128 x 128, 3 x 3, batch 128 6.9 -> 5.7.
+// Measured, us, 15 sets of operands in turn (in a line -> this): 128 x 128, 7 x 7, batch 128 10.4 -> 9.6, with a sigmoid 10.3 -> 9.9,
+// added to half of the old values, transposed 11.2 -> 10.7; 96 x 96, 5 x 5, batch 200 11.0 -> 6.6; 64 x 64, 5 x 5, batch 512 9.3 ->
+// 6.9; 128 x 128, 3 x 3, batch 128 6.4 -> 5.6; (rows along the lanes) 384 x 384, 7 x 7, batch 32 28.6 -> 22.2.
 //
 // Accumulation order per output element: window rows ascending, diagonals ascending, acc = fma(a, x, acc).
 #include <hip/hip_runtime.h>
