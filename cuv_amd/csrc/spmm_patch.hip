@@ -71,14 +71,6 @@ struct PtShape {
     static constexpr int PER_CU = 160 * 1024 / LDS < 4 ? 160 * 1024 / LDS : 4;
 };
 
-__device__ __forceinline__ void pt_load(sp_int4 rsrc, unsigned to, unsigned voff, unsigned soff)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(to), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-
 template <int K, bool EP>
 __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled_kernel(
     const float *__restrict__ X, unsigned ldx, int period, int tiles, unsigned group_tiles, unsigned group_magic,
@@ -179,14 +171,14 @@ __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled
         // a whole patch inside the operand: what the later window rows need is requested between the first ones' products
         const bool staged = inside && rows == PYG;
         auto request_x = [&](int r) __attribute__((always_inline)) {
-            if (x_lane) pt_load(xrsrc, x_to + 16u * (unsigned)(r * S::XROW), x_off, 4u * (unsigned)x0 + (unsigned)r * period4);
+            if (x_lane) lds_load_b128_scalar(xrsrc, x_to + 16u * (unsigned)(r * S::XROW), x_off, 4u * (unsigned)x0 + (unsigned)r * period4);
         };
         // values: diagonals 2 j, 2 j + 1 of window row d
         auto request_values = [&](int p) __attribute__((always_inline)) {
             if (wave >= S::loads(p)) return;
             const int d = 2 * p + wave / S::PER_ROW, j = wave % S::PER_ROW;
             if (vy < rows && vj < min(2, LC - 2 * j))
-                pt_load(arsrc, lds0 + 16u * (unsigned)(S::V0 + d * S::VROW + j * 4 * S::G), v_off + (unsigned)(2 * j * astep4), (unsigned)(starts[d] + 4 * row0 + amin));
+                lds_load_b128_scalar(arsrc, lds0 + 16u * (unsigned)(S::V0 + d * S::VROW + j * 4 * S::G), v_off + (unsigned)(2 * j * astep4), (unsigned)(starts[d] + 4 * row0 + amin));
         };
         f4 mend[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
         if (inside) {
@@ -201,7 +193,7 @@ __global__ __launch_bounds__(PT_THREADS, 2 * PtShape<K>::PER_CU) void spmm_tiled
 #pragma nounroll
             for (int r = 0; r < xrows; ++r) {
                 const int row = x0 + r * period + 4 * lq;
-                if (x_lane) pt_load(xrsrc, x_to + 16u * (unsigned)(r * S::XROW), row >= 0 && row + 4 <= n_in && xcol < cols ? (unsigned)xcol * ldx4 + 4u * (unsigned)row : OOB_OFFSET, 0u);
+                if (x_lane) lds_load_b128_scalar(xrsrc, x_to + 16u * (unsigned)(r * S::XROW), row >= 0 && row + 4 <= n_in && xcol < cols ? (unsigned)xcol * ldx4 + 4u * (unsigned)row : OOB_OFFSET, 0u);
             }
             // values: element by element, 0 where the dense row does not exist
             constexpr int E = 8 * S::G;

@@ -79,15 +79,6 @@ struct PsShape {
     static_assert(2 * LDS <= 160 * 1024, "two workgroups per CU");
 };
 
-// lds_load_b128 for operands that are in scalar registers as it is
-__device__ __forceinline__ void ps_load(sp_int4 rsrc, unsigned to, unsigned voff, unsigned soff)
-{
-    asm volatile("s_mov_b32 m0, %0\n\t"
-                 "s_nop 0\n\t"
-                 "buffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(to), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-
 // A pair of numbers on its way into three parts, a step at a time
 struct PsPair {
     float x0, x1;
@@ -222,7 +213,7 @@ __global__ __launch_bounds__(PS_THREADS, 2) void spmm_split_kernel(
             // (a slot whose output row is not of the segment, or that there is not: zeros)
             const bool have = 2 * i + 1 < K || slot_d == 0, alive = have && (unsigned)(values_top - 2 * i) < (unsigned)rows;
             const int at = __builtin_amdgcn_readlane(window_lane, i) + values_up;
-            ps_load(arsrc, have ? values_to + 2 * i * S::SLOTB : lds0 + S::NOWHERE, alive ? a_off : OOB_OFFSET, (unsigned)at);
+            lds_load_b128_scalar(arsrc, have ? values_to + 2 * i * S::SLOTB : lds0 + S::NOWHERE, alive ? a_off : OOB_OFFSET, (unsigned)at);
         }
     };
 

@@ -63,6 +63,23 @@ def test_dpp_statements_begin_with_their_wait():
     assert bare == [] and waiting > 0
 
 
+def test_loads_to_lds_have_their_wait():
+    """A load's scalar operands must not have been written by a vector instruction in the five preceding issue slots: a statement waits
+    for four behind its own write of M0."""
+    bare, waiting = [], 0
+    for name, text in _sources():
+        for m in re.finditer(r"\basm(?: volatile)?\(", text):
+            code = _arguments(text, m.end() - 1)[0]
+            for macro, body in re.findall(r"#define (\w+) (.*)", text):
+                code = re.sub(r"\b%s\b" % macro, lambda _: body, code)
+            if re.search(r"(buffer|global)_load", code):
+                if re.match(r's_mov_b32 m0, %0\\n\\ts_nop 3\\n\\t', code.replace('"', "")):
+                    waiting += 1
+                else:
+                    bare.append((name, code[:80]))
+    assert bare == [] and waiting > 0
+
+
 _VECTOR = re.compile(r"v\[(\d+):(\d+)\]$|v(\d+)$")
 
 
@@ -81,6 +98,16 @@ def _instructions(path):
             operation, _, operands = line.partition("//")[0].strip().partition(" ")
             if operation:
                 yield operation, [o.strip() for o in operands.split(",")]
+
+
+_SCALAR = re.compile(r"s\[(\d+):(\d+)\]$|s(\d+)$")
+
+
+def _scalars(operand):
+    m = _SCALAR.match(operand.split()[0]) if operand else None
+    if m is None:
+        return set()
+    return set(range(int(m[1]), int(m[2]) + 1)) if m[1] else {int(m[3])}
 
 
 def _slots(operation, operands):
@@ -134,3 +161,38 @@ def test_no_operand_of_dpp_is_written_late(library):
                 assert passed >= WAIT or not (before.startswith("v_") and _registers(written[0]) & source), (operation, operands, before, written)
                 passed += before != "s_nop"
     assert broadcasts > 0
+
+
+def test_no_operand_of_a_matrix_product_is_written_late(library):
+    """Two slots here as well, where a statement of assembly makes the operand."""
+    products = 0
+    for code in library:
+        for i, (operation, operands) in enumerate(code):
+            if not operation.startswith("v_mfma"):
+                continue
+            products += 1
+            source, passed = _registers(operands[1]) | _registers(operands[2]), 0
+            for before, written in reversed(code[max(0, i - WAIT):i]):
+                passed += _slots(before, written) if before == "s_nop" else 0
+                if passed >= WAIT:
+                    break
+                assert not (before.startswith("v_") and not before.startswith("v_mfma") and _registers(written[0]) & source), (operation, operands, before, written)
+                passed += before != "s_nop"
+    assert products > 0
+
+
+def test_no_scalar_operand_of_a_load_or_store_is_written_late(library):
+    accesses, need = 0, 5
+    for code in library:
+        for i, (operation, operands) in enumerate(code):
+            if re.match(r"(buffer|global)_(load|store|atomic)", operation) is None:
+                continue
+            source, passed = set().union(*(_scalars(o) for o in operands)), 0
+            accesses += bool(source)
+            for before, written in reversed(code[max(0, i - need):i]):
+                passed += _slots(before, written) if before == "s_nop" else 0
+                if passed >= need or not source:
+                    break
+                assert not (before.startswith("v_") and _scalars(written[0]) & source), (operation, operands, before, written)
+                passed += before != "s_nop"
+    assert accesses > 0
